@@ -133,28 +133,34 @@ static inline dim3 g16(int64_t len) { return dim3((unsigned)((len + 15) / 16)); 
 // ----------------------------------------------------------------------------------------
 // graph
 // ----------------------------------------------------------------------------------------
-__global__ void k_near_count(int64_t n, const int64_t *slice_ptr, const int32_t *cnt,
-                             const double *L, double lmax, int32_t *out)
+__global__ void k_near_count(int64_t n, pdx_rows rows, const int32_t *cnt, const uint32_t *bw,
+                             const double *L, const double4 *Xr, double lmax, int32_t *out)
 {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n) return;
-    const int64_t b0 = slice_ptr[p >> 6] + (p & 63);
+    const int64_t b0 = rows.row(p);
     int k = 0;
-    for (int t = 0; t < cnt[p]; t++) k += (L[b0 + 64 * (int64_t)t] <= lmax) ? 1 : 0;
+    const double4 Xi = Xr[p];
+    for (int t = 0; t < cnt[p]; t++) {
+        const int64_t b = rows.at(b0, t);
+        k += (pdx_ref_len(L, b, Xi, Xr[bw[b] & PDX_BW_NBR]) <= lmax) ? 1 : 0;
+    }
     out[p] = k;
 }
 
-__global__ void k_near_fill(int64_t n, const int64_t *slice_ptr, const int32_t *cnt,
-                            const uint32_t *bw, const double *L, double lmax,
+__global__ void k_near_fill(int64_t n, pdx_rows rows, const int32_t *cnt,
+                            const uint32_t *bw, const double *L, const double4 *Xr, double lmax,
                             const int64_t *near_ptr, int32_t *near)
 {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n) return;
-    const int64_t b0 = slice_ptr[p >> 6] + (p & 63);
+    const int64_t b0 = rows.row(p);
     int64_t o = near_ptr[p];
+    const double4 Xi = Xr[p];
     for (int t = 0; t < cnt[p]; t++) {
-        const int64_t b = b0 + 64 * (int64_t)t;
-        if (L[b] <= lmax) near[o++] = (int32_t)(bw[b] & PDX_BW_NBR);
+        const int64_t b = rows.at(b0, t);
+        const int32_t j = (int32_t)(bw[b] & PDX_BW_NBR);
+        if (pdx_ref_len(L, b, Xi, Xr[j]) <= lmax) near[o++] = j;
     }
 }
 
@@ -879,7 +885,7 @@ static pdx_status gnn_setup(pdx_ctx *c)
     const double lmax = G_NEAR_FRAC * c->P.delta;
     int32_t *dcnt = nullptr;
     PDX_TRY(pdx_alloc(c, &dcnt, n));
-    hipLaunchKernelGGL(k_near_count, g1(n), dim3(256), 0, c->stream, n, c->slice_ptr, c->cnt, c->L,
+    hipLaunchKernelGGL(k_near_count, g1(n), dim3(256), 0, c->stream, n, c->rows(), c->cnt, c->bw, c->L, c->Xr,
                        lmax, dcnt);
     PDX_HIP(c, hipGetLastError());
     std::vector<int32_t> nc(n), bc(n);
@@ -895,8 +901,8 @@ static pdx_status gnn_setup(pdx_ctx *c)
     PDX_TRY(pdx_alloc(c, &g->near_ptr, n + 1));
     PDX_TRY(pdx_alloc(c, &g->near, std::max<int64_t>(g->n_near, 1)));
     PDX_HIP(c, hipMemcpy(g->near_ptr, ptr.data(), sizeof(int64_t) * (n + 1), hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(k_near_fill, g1(n), dim3(256), 0, c->stream, n, c->slice_ptr, c->cnt, c->bw,
-                       c->L, lmax, g->near_ptr, g->near);
+    hipLaunchKernelGGL(k_near_fill, g1(n), dim3(256), 0, c->stream, n, c->rows(), c->cnt, c->bw,
+                       c->L, c->Xr, lmax, g->near_ptr, g->near);
     PDX_HIP(c, hipGetLastError());
     // input features from the reference positions
     std::vector<double> Xr(4 * n);

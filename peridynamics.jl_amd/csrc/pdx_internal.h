@@ -36,7 +36,38 @@
 #define PDX_F_BEXT 4        // b_ext is not all zero
 #define PDX_F_FORCE_ONLY 8  // calc_force_density! only: write b_int, damage, n_active
 #define PDX_F_SCALE_VOL 16  // force-only: write b_int * V (Newton-Krylov residual form)
+#define PDX_F_ORDER 64      // sums in the order of four lanes per point whatever the block size
 #define PDX_F_FP64 32       // FP64 kernels also in a mixed-precision context (Newton-Krylov)
+
+// Slots of the bonds.  A wave's 64 lanes serve a slice of 64 >> ls consecutive points, 1 << ls
+// lanes per point (ls = 0, 2, 3 or 4), and the slice's bonds come in row groups of 64 slots, one
+// slot per lane, so that a wave reads one contiguous run per group.  The bonds of a point are dealt
+// to its lanes in runs of 16: bond t goes to lane 4 ((t >> 4) mod m) + t mod 4 with m = lanes / 4,
+// group 4 ((t >> 4) / m) + (t >> 2) mod 4.  A lane's groups 4 g .. 4 g + 3 then hold bonds whose
+// numbers differ by 4 whatever the lanes per point, and a lane's bonds keep the row's order.
+// ls = 0 is one thread per point (SELL-64): bond t in group t.
+struct pdx_rows {
+    const int64_t *ptr;  // first slot of every slice
+    int ls;
+    __host__ __device__ __forceinline__ int64_t row(int64_t p) const
+    {
+        return ptr[p >> (6 - ls)] + ((p & ((64 >> ls) - 1)) << ls);
+    }
+    // slot of bond t of the point whose row() is b0
+    __host__ __device__ __forceinline__ int64_t at(int64_t b0, int t) const
+    {
+        if (ls == 0) return b0 + ((int64_t)t << 6);
+        const int k = t >> 4;
+        return b0 + ((int64_t)(((k >> (ls - 2)) << 2) + ((t >> 2) & 3)) << 6) + ((k & ((1 << (ls - 2)) - 1)) << 2) + (t & 3);
+    }
+    // row groups of a row of c bonds
+    __host__ __device__ __forceinline__ int groups(int c) const
+    {
+        if (ls == 0 || c == 0) return c;
+        const int k = (c - 1) >> 4, m = 1 << (ls - 2);
+        return ((k / m) << 2) + (k % m ? 4 : (((c - 1) >> 2) & 3) + 1);
+    }
+};
 
 struct pdx_crack {
     std::vector<int32_t> a, b;
@@ -63,8 +94,6 @@ struct pdx_gnn;  // learned preconditioner (pdx_gnn.hip)
 struct pdx_ctx {
     int device = 0;
     int precision = PDX_FP64;
-    // bonds per iteration of the BB thread (tuning knob PDX_BB_UNROLL = 2 | 4)
-    int bb_unroll = 0;  // bonds per lane and unrolled iteration of the BB step: 2, 4, 0 = default
     int64_t lds_limit = 160 * 1024;  // dynamic LDS bytes a workgroup may use
     int32_t lds_budget_env = 0;      // PDX_LDS_BUDGET (bytes), 0 = default
     hipStream_t stream = nullptr;
@@ -90,7 +119,7 @@ struct pdx_ctx {
     bool multi() const { return psets.size() > 1; }
     // EnergySurfaceCorrection (bond_system_corrections.jl:46-204): 0 none, 1 energy based
     int32_t corr = 0;
-    double *scf = nullptr;     // scfactor per bond slot (SELL-64, like L)
+    double *scf = nullptr;     // scfactor per bond slot (pdx_rows, like L)
     float *scf32 = nullptr;    // FP32 copy for the mixed step
     double *mfactor = nullptr; // 3 x n (internal order), mfactor[d * n + i]
     // export pipeline: two snapshot slots (device, pinned host) filled in turn; a snapshot
@@ -119,18 +148,30 @@ struct pdx_ctx {
     double *defgrad = nullptr, *cauchy = nullptr;  // 9n (CPD)
     int32_t *d_perm = nullptr, *d_iperm = nullptr;
     double *stage = nullptr;               // 9n staging for permuted transfers
-    // bonds in sliced ELL (SELL-64): bond t of point p at slice_ptr[p / 64] + 64 t + p % 64
-    int64_t *slice_ptr = nullptr;          // n_slices + 1
+    // bonds in sliced ELL (pdx_rows)
+    int64_t *slice_ptr = nullptr;          // n_slices() + 1
+    int ls = 0;                            // log2 of the lanes per point
+    int64_t n_slices() const { return (n + (64 >> ls) - 1) >> (6 - ls); }
+    pdx_rows rows() const { return {slice_ptr, ls}; }
     int32_t *cnt = nullptr;                // n: bonds of each point
     int64_t nb_alloc = 0;                  // entries including the padding of the slices
     uint32_t *bw = nullptr;                // bond words: neighbour | active | fail_permit
-    double *L = nullptr;                   // reference lengths (FP64 layout)
+    double *L = nullptr;                   // reference lengths, null with packed bonds (pdx_ref_len)
     float *Lf = nullptr;                   // reference lengths (mixed layout)
     // LDS-staged BB step: per block of PDX_BLOCK points, the sorted list of every point
     // its bonds reach (the halo); bonds then address the halo with 16-bit words
     // (bits 0-13 slot, bit 14 active, bit 15 fail_permit)
     bool lds_mode = false;
+    int cfg = -1;                          // points per block and lanes per point (choose_blocks)
+    int pb = PDX_BLOCK;                    // points per block of the LDS layout
     uint16_t *bw16 = nullptr;              // nb_alloc
+    // packed bonds (FP64 contexts, one parameter set, LDS layout): slot << pk_shift | length, the
+    // length as its bit pattern minus pk_base, all ones (pk_mask) = not active; they replace bw16
+    // and L (both null then)
+    unsigned long long *pk = nullptr;      // nb_alloc
+    int pk_shift = 0;
+    unsigned long long pk_mask = 0, pk_base = 0;
+    uint8_t *d_fp = nullptr;               // fail_permit of the points (internal order)
     int64_t *halo_ptr = nullptr;           // n_blocks + 1
     int32_t *halo = nullptr;               // halo entries (internal point indices)
     int32_t halo_max = 0;                  // largest halo of a block (LDS layout: every row's
@@ -240,6 +281,15 @@ __device__ __noinline__ double pdx_omega_other(int kid, double delta, double L)
 __device__ __forceinline__ double pdx_omega(int kid, double delta, double L, double rL)
 {
     return kid == PDX_KERNEL_LINEAR ? delta * rL : pdx_omega_other(kid, delta, L);
+}
+
+// Reference length of bond slot b between points at Xi, Xj: stored, or where the lengths are only
+// held in packed bonds (L null) formed again as the bond search formed it, bit for bit.
+__device__ __forceinline__ double pdx_ref_len(const double *L, int64_t b, const double4 &Xi, const double4 &Xj)
+{
+    if (L) return L[b];
+    const double p0 = Xi.x - Xj.x, p1 = Xi.y - Xj.y, p2 = Xi.z - Xj.z;
+    return sqrt((p0 * p0 + p1 * p1) + p2 * p2);
 }
 
 // finite-difference perturbation of J v (compute_perturbation, newton_krylov.jl:534-566):
@@ -402,7 +452,7 @@ struct pdx_step_args {
     int64_t step;
     int flags;
     double rho, dt, dth;
-    const int64_t *slice_ptr;
+    pdx_rows rows;
     const int32_t *cnt;
     uint32_t *bw;
     uint16_t *bw16;
@@ -427,6 +477,11 @@ struct pdx_step_args {
     const double *bcv;
     unsigned long long *flags_out;
     // material
+    unsigned long long *pk;  // packed bonds, or null
+    int pk_shift;
+    unsigned long long pk_mask, pk_base;
+    const uint8_t *fp;       // fail_permit of the points
+    double epsc_lo_min;      // the smallest epsc_lo of the parameter sets
     double bc, epsc, epsc_lo, epsc_hi, delta, G, K, lambda, mu, beta_zem, maxdmg, nu;
     int model;
     int kernel;  // influence function (PDX_KERNEL_*)

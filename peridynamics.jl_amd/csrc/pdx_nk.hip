@@ -217,27 +217,27 @@ __global__ void k_nk_update(int64_t n, const double *du, const uint8_t *cmask, d
 // Point-block Jacobi of the bond-based residual: J_ii = -V_i sum_j bc V_j
 // [ (1/L) n n^T + (eps/l) (I - n n^T) ] with n = dx/l (the derivative of r_i = b_i V_i with
 // respect to u_i).  Constrained dofs get identity rows/columns.  Stores the inverse.
-__global__ __launch_bounds__(256) void k_bb_block_jacobi(int64_t n, const int64_t *slice_ptr,
+__global__ __launch_bounds__(256) void k_bb_block_jacobi(int64_t n, pdx_rows rows,
                                                          const int32_t *cnt, const uint32_t *bw,
-                                                         const double *L, const double4 *rec,
+                                                         const double *L, const double4 *Xr, const double4 *rec,
                                                          double bc, const pdx_pset *ps,
                                                          const uint8_t *pid, const uint8_t *cmask,
                                                          double *dinv)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const int64_t b0 = slice_ptr[i >> 6] + (i & 63);
-    const double4 ri = rec[i];
+    const int64_t b0 = rows.row(i);
+    const double4 ri = rec[i], Xi = Xr[i];
     double D[6] = {0, 0, 0, 0, 0, 0};  // xx yx zx yy zy zz
     for (int t = 0; t < cnt[i]; t++) {
-        const int64_t b = b0 + (int64_t)t * 64;
+        const int64_t b = rows.at(b0, t);
         const uint32_t wd = bw[b];
         if (!(wd & PDX_BW_ACT)) continue;
         const double4 rj = rec[wd & PDX_BW_NBR];
         const double dx = rj.x - ri.x, dy = rj.y - ri.y, dz = rj.z - ri.z;
         const double l = sqrt((dx * dx + dy * dy) + dz * dz);
         const double nx = dx / l, ny = dy / l, nz = dz / l;
-        const double Lb = L[b];
+        const double Lb = pdx_ref_len(L, b, Xi, Xr[wd & PDX_BW_NBR]);
         const double eps = (l - Lb) / Lb;
         const double bcb = ps ? (ps[pid[i]].bc + ps[pid[wd & PDX_BW_NBR]].bc) / 2.0 : bc;
         const double a = bcb * rj.w / Lb, g = bcb * rj.w * eps / l;
@@ -647,9 +647,9 @@ __device__ __forceinline__ int nk_slot(int32_t *pj, int &ns, int64_t J, int *ove
 // Y[(i*TP + t)*nf + f][d] = sum over the bonds of i into slot t's aggregate of C_ij phi_j[f],
 // plus -sum_j C_ij phi_i[f] in slot 0 (the diagonal block J_ii).  C_ij is the bond's
 // stiffness dr_i/du_j = V_i bc V_j [(1/L) n n^T + (eps/l)(I - n n^T)].
-__global__ __launch_bounds__(256) void k_coarse_y(int64_t n, int agg, int nf, const int64_t *slice_ptr,
+__global__ __launch_bounds__(256) void k_coarse_y(int64_t n, int agg, int nf, pdx_rows rows,
                                                   const int32_t *cnt, const uint32_t *bw,
-                                                  const double *L, const double4 *rec, double bc,
+                                                  const double *L, const double4 *Xr, const double4 *rec, double bc,
                                                   const pdx_pset *ps, const uint8_t *pid,
                                                   const double *phi, int32_t *pJ, double *Y,
                                                   int *overflow)
@@ -657,8 +657,8 @@ __global__ __launch_bounds__(256) void k_coarse_y(int64_t n, int agg, int nf, co
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int64_t I = i / agg;
-    const int64_t b0 = slice_ptr[i >> 6] + (i & 63);
-    const double4 ri = rec[i];
+    const int64_t b0 = rows.row(i);
+    const double4 ri = rec[i], Xi = Xr[i];
     int32_t pj[NK_TP];
     for (int f0 = 0; f0 < nf; f0 += NK_FCH) {
         const int fn = min(NK_FCH, nf - f0);
@@ -682,7 +682,7 @@ __global__ __launch_bounds__(256) void k_coarse_y(int64_t n, int agg, int nf, co
                 for (int q = 0; q < NK_FCH; q++) S[d][q] = 0.0;
         };
         for (int t = 0; t < cnt[i]; t++) {
-            const int64_t b = b0 + (int64_t)t * 64;
+            const int64_t b = rows.at(b0, t);
             const uint32_t wd = bw[b];
             if (!(wd & PDX_BW_ACT)) continue;
             const int64_t j = wd & PDX_BW_NBR;
@@ -695,7 +695,7 @@ __global__ __launch_bounds__(256) void k_coarse_y(int64_t n, int agg, int nf, co
             const double dx = rj.x - ri.x, dy = rj.y - ri.y, dz = rj.z - ri.z;
             const double l = sqrt((dx * dx + dy * dy) + dz * dz);
             const double nv[3] = {dx / l, dy / l, dz / l};
-            const double Lb = L[b];
+            const double Lb = pdx_ref_len(L, b, Xi, Xr[j]);
             const double eps = (l - Lb) / Lb;
             const double bcb = ps ? (ps[pid[i]].bc + ps[pid[j]].bc) / 2.0 : bc;
             const double a = ri.w * bcb * rj.w / Lb, g = ri.w * bcb * rj.w * eps / l;
@@ -753,18 +753,18 @@ __global__ __launch_bounds__(256) void k_coarse_gather(int64_t n, int agg, int n
 
 // the number of aggregates (its own included) that the bonds of a point reach, maximised
 // over the points into *out
-__global__ void k_coarse_reach(int64_t n, int agg, const int64_t *slice_ptr, const int32_t *cnt,
+__global__ void k_coarse_reach(int64_t n, int agg, pdx_rows rows, const int32_t *cnt,
                                const uint32_t *bw, int *out)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int64_t I = i / agg;
-    const int64_t b0 = slice_ptr[i >> 6] + (i & 63);
+    const int64_t b0 = rows.row(i);
     int runs = 0;
     bool own = false;
     int64_t Jc = -1;
     for (int t = 0; t < cnt[i]; t++) {
-        const int64_t J = (int64_t)(bw[b0 + (int64_t)t * 64] & PDX_BW_NBR) / agg;
+        const int64_t J = (int64_t)(bw[rows.at(b0, t)] & PDX_BW_NBR) / agg;
         if (J != Jc) {
             runs++;
             own |= (J == I);
@@ -1026,7 +1026,7 @@ pdx_status pdx_nk_aggregates(pdx_ctx *c)
     if (!k->dflag) PDX_TRY(pdx_alloc(c, &k->dflag, 4));
     for (int64_t agg = pdx_nk_agg_size(n);; agg *= 2) {
         PDX_HIP(c, hipMemsetAsync(k->dflag, 0, sizeof(int), c->stream));
-        hipLaunchKernelGGL(k_coarse_reach, grid1(n), dim3(256), 0, c->stream, n, (int)agg, c->slice_ptr,
+        hipLaunchKernelGGL(k_coarse_reach, grid1(n), dim3(256), 0, c->stream, n, (int)agg, c->rows(),
                            c->cnt, c->bw, k->dflag);
         PDX_HIP(c, hipGetLastError());
         int reach = 0;
@@ -1089,8 +1089,8 @@ static pdx_status build_coarse(pdx_ctx *c, const float *learned_fields, int n_le
     hipLaunchKernelGGL(k_coarse_soa, grid1((n + 63) / 64 * 64), dim3(256), 0, s, n, nf, k->phi, k->phis);
     PDX_HIP(c, hipMemsetAsync(k->Ycs, 0, sizeof(double) * n * NK_TP * nf * 3, s));
     PDX_HIP(c, hipMemsetAsync(k->dflag, 0, sizeof(int) * 4, s));
-    hipLaunchKernelGGL(k_coarse_y, grid1(n), dim3(256), 0, s, n, k->agg, nf, c->slice_ptr, c->cnt, c->bw,
-                       c->L, c->rec[c->cur], c->P.bc, c->multi() ? c->d_psets : nullptr, c->d_pid,
+    hipLaunchKernelGGL(k_coarse_y, grid1(n), dim3(256), 0, s, n, k->agg, nf, c->rows(), c->cnt, c->bw,
+                       c->L, c->Xr, c->rec[c->cur], c->P.bc, c->multi() ? c->d_psets : nullptr, c->d_pid,
                        k->phi, k->pJ, k->Ycs, k->dflag);
     PDX_HIP(c, hipGetLastError());
     int ovf = 0;
@@ -1182,8 +1182,8 @@ pdx_status pdx_nk_coarse_add(pdx_ctx *c, const double *v, double *z, double alph
 static pdx_status build_jacobi(pdx_ctx *c)
 {
     if (c->kind != PDX_BB) return pdx_fail(c, PDX_ERR_UNSUPPORTED, "block Jacobi is built for BBMaterial");
-    hipLaunchKernelGGL(k_bb_block_jacobi, grid1(c->n), dim3(256), 0, c->stream, c->n, c->slice_ptr,
-                       c->cnt, c->bw, c->L, c->rec[c->cur], c->P.bc,
+    hipLaunchKernelGGL(k_bb_block_jacobi, grid1(c->n), dim3(256), 0, c->stream, c->n, c->rows(),
+                       c->cnt, c->bw, c->L, c->Xr, c->rec[c->cur], c->P.bc,
                        c->multi() ? c->d_psets : nullptr, c->d_pid, c->nk->cmask, c->nk->dinv);
     PDX_HIP(c, hipGetLastError());
     return PDX_OK;

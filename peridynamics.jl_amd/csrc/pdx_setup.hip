@@ -56,6 +56,8 @@ static void free_bonds(pdx_ctx *c)
     FREE(c->cnt);
     FREE(c->bw);
     FREE(c->bw16);
+    FREE(c->pk);
+    FREE(c->d_fp);
     FREE(c->halo_ptr);
     FREE(c->halo);
     c->lds_mode = false;
@@ -117,10 +119,6 @@ extern "C" pdx_status pdx_create(pdx_ctx **out, int32_t device, int32_t precisio
     pdx_ctx *c = new pdx_ctx();
     c->device = device;
     c->precision = precision;
-    if (const char *e = getenv("PDX_BB_UNROLL")) {
-        int v = atoi(e);
-        if (v == 2 || v == 4) c->bb_unroll = v;
-    }
     if (const char *e = getenv("PDX_LDS_BUDGET")) c->lds_budget_env = atoi(e);
     if (hipSetDevice(device) != hipSuccess || hipStreamCreate(&c->stream) != hipSuccess ||
         hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess) {
@@ -337,7 +335,7 @@ struct search_args {
     uint32_t filt_bits;       // bit 2k set: crack k filters its bonds
     const uint8_t *fp;        // fail_permit, internal order
     int32_t *counts;
-    const int64_t *slice_ptr;
+    pdx_rows rows;
     const int32_t *cnt;
     uint32_t *bw;
     double *L;
@@ -408,7 +406,7 @@ __global__ __launch_bounds__(PDX_BLOCK) void k_fill_bonds(search_args s)
     double4 xi = s.Xr[i];
     int cx = s.pcell[3 * i], cy = s.pcell[3 * i + 1], cz = s.pcell[3 * i + 2];
     uint32_t mi = s.cmask ? s.cmask[i] : 0;
-    const int64_t b0 = s.slice_ptr[i >> 6] + (i & 63);  // SELL-64: bond t at b0 + 64 t
+    const int64_t b0 = s.rows.row(i);
     const int want = s.cnt[i];                          // <= PDX_FILL_CAP, checked on the host
     int base = 0;
     for (int z = cz - 1; z <= cz + 1; z++) {
@@ -458,23 +456,29 @@ __global__ __launch_bounds__(PDX_BLOCK) void k_fill_bonds(search_args s)
         uint32_t h = s.cmask ? crack_hits(mi, s.cmask[j]) : 0u;
         const uint32_t fpb = (s.fp[i] & s.fp[j]) ? PDX_BW_FP : 0u;
         const uint32_t act = (h & ~s.filt_bits) ? 0u : PDX_BW_ACT;  // broken at t = 0 by a precrack
-        const int64_t b = b0 + (int64_t)rank * 64;
+        const int64_t b = s.rows.at(b0, rank);
         s.bw[b] = (uint32_t)j | act | fpb;
         s.L[b] = sqrt(d2);
     }
 }
 
-__global__ void k_init_point_state(int64_t n, const int64_t *slice_ptr, const int32_t *cnt,
+__global__ void k_init_point_state(int64_t n, pdx_rows rows, const int32_t *cnt,
                                    const uint32_t *bw, int32_t *nact, double *damage)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const int64_t b0 = slice_ptr[i >> 6] + (i & 63);
+    const int64_t b0 = rows.row(i);
     int na = 0;
-    for (int t = 0; t < cnt[i]; t++) na += (bw[b0 + (int64_t)t * 64] & PDX_BW_ACT) ? 1 : 0;
+    for (int t = 0; t < cnt[i]; t++) na += (bw[rows.at(b0, t)] & PDX_BW_ACT) ? 1 : 0;
     nact[i] = na;
     // calc_damage!: 1 - n_active / n_neighbors (NaN for a point without bonds)
     damage[i] = 1.0 - (double)na / (double)cnt[i];
+}
+
+__global__ void k_fill_value(int64_t n, double v, double *out)
+{
+    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < n) out[k] = v;
 }
 
 __global__ void k_L_to_float(int64_t nb, const double *L, float *Lf)
@@ -541,6 +545,82 @@ pdx_status pdx_download_vec(pdx_ctx *c, const double *dev, double *host, int com
 }
 
 // ----------------------------------------------------------------------------------------
+// packed bonds
+// ----------------------------------------------------------------------------------------
+// bit patterns of the shortest and the longest bond (positive doubles order as their bits do):
+// range[0] starts at ~0, range[1] at 0
+__global__ __launch_bounds__(256) void k_len_range(int64_t n, pdx_rows rows, const int32_t *cnt,
+                                                   const double *L, unsigned long long *range)
+{
+    unsigned long long lo = ~0ULL, hi = 0ULL;
+    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p < n) {
+        const int64_t b0 = rows.row(p);
+        for (int t = 0; t < cnt[p]; t++) {
+            const unsigned long long v = (unsigned long long)__double_as_longlong(L[rows.at(b0, t)]);
+            lo = v < lo ? v : lo;
+            hi = v > hi ? v : hi;
+        }
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        const unsigned long long a = __shfl_xor(lo, o), b = __shfl_xor(hi, o);
+        lo = a < lo ? a : lo;
+        hi = b > hi ? b : hi;
+    }
+    if ((threadIdx.x & 63) == 0) {
+        atomicMin(&range[0], lo);
+        atomicMax(&range[1], hi);
+    }
+}
+
+// in place: the packed word of a slot takes its length's 8 bytes
+__global__ void k_pack_bonds(int64_t nb, const uint16_t *w16, double *L, int shift, unsigned long long mask,
+                             unsigned long long base)
+{
+    const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (b >= nb) return;
+    const uint32_t w = w16[b];
+    const unsigned long long v = (unsigned long long)__double_as_longlong(L[b]) - base;
+    L[b] = __longlong_as_double(
+        (long long)((unsigned long long)(w & PDX_W16_SLOT) << shift | ((w & PDX_W16_ACT) ? v : mask)));
+}
+
+// One 64-bit word per bond in place of the 16-bit word and the FP64 length (FP64 contexts with
+// one parameter set): taken when the table slots and the span of the length patterns share 64
+// bits, which the usual horizons do (3.015 spacings: 11 bits of slot, lengths within a factor of
+// 4).  The words carry the bond state and take the place of the lengths in memory (12 bytes per
+// slot with the 32-bit word, 14 unpacked); the passes that are not per step form a length again
+// from the reference positions (pdx_ref_len).
+static pdx_status pack_bonds(pdx_ctx *c)
+{
+    if (c->precision != PDX_FP64 || c->multi() || c->nb <= 0) return PDX_OK;
+    unsigned long long *range = c->d_flags + 4, h[2] = {~0ULL, 0ULL};
+    PDX_HIP(c, hipMemcpyAsync(range, h, sizeof h, hipMemcpyHostToDevice, c->stream));
+    hipLaunchKernelGGL(k_len_range, dim3((unsigned)((c->n + 255) / 256)), dim3(256), 0, c->stream, c->n,
+                       c->rows(), c->cnt, c->L, range);
+    PDX_HIP(c, hipGetLastError());
+    PDX_HIP(c, hipMemcpyAsync(h, range, sizeof h, hipMemcpyDeviceToHost, c->stream));
+    PDX_HIP(c, hipStreamSynchronize(c->stream));
+    int sb = 1;
+    while ((1 << sb) < c->halo_max) sb++;
+    const int shift = 64 - sb;
+    const unsigned long long mask = (1ULL << shift) - 1;
+    if (h[1] - h[0] >= mask) return PDX_OK;
+    c->pk_shift = shift;
+    c->pk_mask = mask;
+    c->pk_base = h[0];
+    hipLaunchKernelGGL(k_pack_bonds, dim3((unsigned)((c->nb_alloc + 255) / 256)), dim3(256), 0, c->stream,
+                       c->nb_alloc, c->bw16, c->L, shift, mask, h[0]);
+    PDX_HIP(c, hipGetLastError());
+    PDX_HIP(c, hipStreamSynchronize(c->stream));
+    c->pk = reinterpret_cast<unsigned long long *>(c->L);
+    c->L = nullptr;
+    FREE(c->bw16);
+    c->dev_bytes -= (int64_t)sizeof(uint16_t) * c->nb_alloc;
+    return PDX_OK;
+}
+
+// ----------------------------------------------------------------------------------------
 // LDS halos of the BB step.  For every block of PDX_BLOCK consecutive (Morton) points the
 // sorted, de-duplicated list of the points its bonds reach; every bond is rewritten as a
 // 16-bit slot into its block's list.  Built on the host, in parallel over blocks, once.
@@ -550,8 +630,9 @@ static pdx_status build_halos(pdx_ctx *c, bool *ok)
 {
     *ok = false;
     const int64_t n = c->n, nba = c->nb_alloc;
-    const int64_t n_slices = (n + 63) / 64;
-    const int64_t nblk = (n + PDX_BLOCK - 1) / PDX_BLOCK;
+    const int64_t n_slices = c->n_slices();
+    const int64_t PB = c->pb;
+    const int64_t nblk = (n + PB - 1) / PB;
     hipDeviceProp_t prop;
     PDX_HIP(c, hipGetDeviceProperties(&prop, c->device));
     const int64_t lds_limit = std::min<int64_t>((int64_t)prop.sharedMemPerBlock, 160 * 1024);
@@ -565,19 +646,21 @@ static pdx_status build_halos(pdx_ctx *c, bool *ok)
     std::vector<uint32_t> w(nba);
     PDX_HIP(c, hipMemcpy(sp.data(), c->slice_ptr, sizeof(int64_t) * (n_slices + 1), hipMemcpyDeviceToHost));
     PDX_HIP(c, hipMemcpy(cn.data(), c->cnt, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
+    const pdx_rows hr{sp.data(), c->ls};
     PDX_HIP(c, hipMemcpy(w.data(), c->bw, sizeof(uint32_t) * nba, hipMemcpyDeviceToHost));
     std::vector<std::vector<int32_t>> tab(nblk);
     std::vector<uint16_t> w16(nba, 0);
+    std::vector<uint8_t> used(nba, 0);
     std::vector<int> too_big(nblk, 0), unsorted(nblk, 0);
     unsigned nth = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
     auto work = [&](int64_t k0, int64_t k1) {
         std::vector<int32_t> tmp;
         for (int64_t k = k0; k < k1; k++) {
             tmp.clear();
-            const int64_t pe = std::min(n, (k + 1) * PDX_BLOCK);
-            for (int64_t p = k * PDX_BLOCK; p < pe; p++) {
-                const int64_t b0 = sp[p >> 6] + (p & 63);
-                for (int t = 0; t < cn[p]; t++) tmp.push_back((int32_t)(w[b0 + 64 * (int64_t)t] & PDX_BW_NBR));
+            const int64_t pe = std::min(n, (k + 1) * PB);
+            for (int64_t p = k * PB; p < pe; p++) {
+                const int64_t b0 = hr.row(p);
+                for (int t = 0; t < cn[p]; t++) tmp.push_back((int32_t)(w[hr.at(b0, t)] & PDX_BW_NBR));
             }
             std::sort(tmp.begin(), tmp.end());
             tmp.erase(std::unique(tmp.begin(), tmp.end()), tmp.end());
@@ -585,18 +668,24 @@ static pdx_status build_halos(pdx_ctx *c, bool *ok)
                 too_big[k] = 1;
                 continue;
             }
-            for (int64_t p = k * PDX_BLOCK; p < pe; p++) {
-                const int64_t b0 = sp[p >> 6] + (p & 63);
+            for (int64_t p = k * PB; p < pe; p++) {
+                const int64_t b0 = hr.row(p);
                 int64_t prev = -1;
                 for (int t = 0; t < cn[p]; t++) {
-                    const int64_t b = b0 + 64 * (int64_t)t;
+                    const int64_t b = hr.at(b0, t);
                     const int32_t j = (int32_t)(w[b] & PDX_BW_NBR);
                     const uint32_t slot = (uint32_t)(std::lower_bound(tmp.begin(), tmp.end(), j) - tmp.begin());
                     if ((int64_t)slot <= prev) unsorted[k] = 1;
                     prev = slot;
+                    used[b] = 1;
                     w16[b] = (uint16_t)(slot | ((w[b] & PDX_BW_ACT) ? PDX_W16_ACT | PDX_W16_RACT : 0u) |
                                         ((w[b] & PDX_BW_FP) ? PDX_W16_FP : 0u));
                 }
+                // the slots past the row's end repeat its last neighbour, inactive
+                const int64_t ng = (sp[(p >> (6 - c->ls)) + 1] - sp[p >> (6 - c->ls)]) >> 6;
+                for (int64_t g = 0; g < ng; g++)
+                    for (int l = 0; l < (1 << c->ls); l++)
+                        if (!used[b0 + 64 * g + l]) w16[b0 + 64 * g + l] = (uint16_t)(prev < 0 ? 0 : prev);
             }
             tab[k] = tmp;
         }
@@ -630,6 +719,74 @@ static pdx_status build_halos(pdx_ctx *c, bool *ok)
     c->halo_total = hp[nblk];
     c->lds_mode = true;
     *ok = true;
+    return pack_bonds(c);
+}
+
+// Points per block and lanes per point of the LDS-staged kernels (pdx_step.hip, with_cfg): 256 x 4,
+// 128 x 4, 64 x 8 or 32 x 16.  A small body needs many small blocks (a 6400-point one is 25 blocks of
+// 256 points on 256 CUs) and many lanes per point (its step is one chain of load latencies per
+// lane); a large one wants the larger blocks' smaller neighbour tables per point.  Measured, us
+// per step, blocks of 256 / 128 / 64 / 32 points (3.015 spacings):
+//   BB FP64   6 k 14.3 /  9.8 /  7.1 /  6.4    14 k 16.7 / 11.8 /  8.7 /  8.8
+//            25 k 17.2 / 12.4 / 12.5 / 13.4   100 k 31.5 / 30.6 / 30.5 / 35.0
+//             2 M  560 /  515 /  598 /  729
+//   CPD FP64  6 k 44.8 / 30.9 / 24.1 / 21.7    14 k 52.9 / 36.5 / 28.8 / 32.0
+//            25 k 55.4 / 37.8 / 46.5 / 53.5    54 k 63.6 / 65.4 / 84.8 / 91.4
+// so the blocks are the largest that still give 160 of them.  The correspondence kernels go up to
+// 256 points (one block of 1024 threads per CU by their registers; 128 points: 2658 against 2034
+// at 2 M), as do the mixed steps of bodies beyond a million points (334 against 356 at 2 M); the
+// others stop at 128, whose blocks share a CU three at a time.  Horizons beyond about 4 spacings stop
+// at 64 points, whose neighbour tables still fit a block's share of the LDS (5.015 spacings, 121 k
+// points, BB: 216 / 169 / 157 / 159; OSB at 400 k: 1042 / 1074 / 897 / 942).
+static void choose_blocks(pdx_ctx *c, bool lds)
+{
+    if (!lds) {
+        c->cfg = -1;
+        c->ls = 0;
+        c->pb = PDX_BLOCK;
+        return;
+    }
+    static const int pbs[4] = {256, 128, 64, 32}, lss[4] = {2, 2, 3, 4};
+    int first = 1;
+    if (c->kind == PDX_CPD || (c->precision == PDX_MIXED && c->n > 1000000)) first = 0;
+    else if (c->nb > 180 * c->n) first = 2;
+    int k = first;
+    while (k < 3 && c->n < (int64_t)160 * pbs[k]) k++;
+    c->cfg = k;
+    c->pb = pbs[k];
+    c->ls = lss[k];
+}
+
+// the rows of the chosen layout: slice pointers, bond words and lengths
+static pdx_status fill_rows(pdx_ctx *c, search_args &s, const std::vector<int32_t> &counts)
+{
+    if (c->bw) c->dev_bytes -= (int64_t)(sizeof(uint32_t) + sizeof(double)) * c->nb_alloc;
+    FREE(c->slice_ptr);
+    FREE(c->bw);
+    FREE(c->L);
+    const int64_t n = c->n, n_slices = c->n_slices(), P = 64 >> c->ls;
+    std::vector<int64_t> slice_ptr(n_slices + 1, 0);
+    for (int64_t sl = 0; sl < n_slices; sl++) {
+        int32_t w = 0;
+        for (int64_t m = P * sl; m < std::min(n, P * sl + P); m++) w = std::max(w, counts[m]);
+        slice_ptr[sl + 1] = slice_ptr[sl] + 64 * (int64_t)c->rows().groups(w);
+    }
+    const int64_t nba = c->nb_alloc = slice_ptr[n_slices];
+    if (nba >= ((int64_t)1 << 40)) return pdx_fail(c, PDX_ERR_UNSUPPORTED, "too many bonds");
+    PDX_TRY(pdx_alloc(c, &c->slice_ptr, n_slices + 1));
+    PDX_TRY(pdx_alloc(c, &c->bw, nba));
+    PDX_TRY(pdx_alloc(c, &c->L, nba));
+    PDX_HIP(c, hipMemcpy(c->slice_ptr, slice_ptr.data(), sizeof(int64_t) * (n_slices + 1), hipMemcpyHostToDevice));
+    // padding slots: bond word 0, length 1
+    PDX_HIP(c, hipMemsetAsync(c->bw, 0, sizeof(uint32_t) * nba, c->stream));
+    hipLaunchKernelGGL(k_fill_value, dim3((unsigned)((nba + 255) / 256)), dim3(256), 0, c->stream, nba, 1.0, c->L);
+    s.rows = c->rows();
+    s.cnt = c->cnt;
+    s.bw = c->bw;
+    s.L = c->L;
+    hipLaunchKernelGGL(k_fill_bonds, dim3((unsigned)pdx_wave_grid(n)), dim3(PDX_BLOCK), 0, c->stream, s);
+    PDX_HIP(c, hipGetLastError());
+    PDX_HIP(c, hipStreamSynchronize(c->stream));
     return PDX_OK;
 }
 
@@ -725,14 +882,12 @@ extern "C" pdx_status pdx_build_bonds(pdx_ctx *c, int64_t *n_bonds_out)
     int32_t *d_pcell = nullptr, *d_cell_pts = nullptr, *d_counts = nullptr;
     int64_t *d_cell_start = nullptr;
     uint16_t *d_cmask = nullptr;
-    uint8_t *d_fp = nullptr;
     auto cleanup = [&]() {
         FREE(d_pcell);
         FREE(d_cell_pts);
         FREE(d_counts);
         FREE(d_cell_start);
         FREE(d_cmask);
-        FREE(d_fp);
     };
 #define TRY_C(expr)                                                                         \
     do {                                                                                    \
@@ -754,7 +909,7 @@ extern "C" pdx_status pdx_build_bonds(pdx_ctx *c, int64_t *n_bonds_out)
     HIP_C(hipMalloc((void **)&d_cell_pts, sizeof(int32_t) * n));
     HIP_C(hipMalloc((void **)&d_counts, sizeof(int32_t) * n));
     HIP_C(hipMalloc((void **)&d_cell_start, sizeof(int64_t) * (ncell + 1)));
-    HIP_C(hipMalloc((void **)&d_fp, n));
+    TRY_C(pdx_alloc(c, &c->d_fp, n));
     if (!cmask.empty()) HIP_C(hipMalloc((void **)&d_cmask, sizeof(uint16_t) * n));
     HIP_C(hipMemcpy(c->Xr, Xm.data(), sizeof(double4) * n, hipMemcpyHostToDevice));
     HIP_C(hipMemcpy(c->rec[0], Xm.data(), sizeof(double4) * n, hipMemcpyHostToDevice));
@@ -765,7 +920,7 @@ extern "C" pdx_status pdx_build_bonds(pdx_ctx *c, int64_t *n_bonds_out)
     HIP_C(hipMemcpy(d_cell_pts, cell_pts.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice));
     HIP_C(hipMemcpy(d_cell_start, cell_start.data(), sizeof(int64_t) * (ncell + 1),
                     hipMemcpyHostToDevice));
-    HIP_C(hipMemcpy(d_fp, fpm.data(), n, hipMemcpyHostToDevice));
+    HIP_C(hipMemcpy(c->d_fp, fpm.data(), n, hipMemcpyHostToDevice));
     if (d_cmask)
         HIP_C(hipMemcpy(d_cmask, cmask.data(), sizeof(uint16_t) * n, hipMemcpyHostToDevice));
     HIP_C(hipMemset(c->d_flags, 0, 8 * sizeof(unsigned long long)));
@@ -785,11 +940,10 @@ extern "C" pdx_status pdx_build_bonds(pdx_ctx *c, int64_t *n_bonds_out)
     s.perm = c->d_perm;
     s.cmask = d_cmask;
     s.filt_bits = filt_bits;
-    s.fp = d_fp;
+    s.fp = c->d_fp;
     s.counts = d_counts;
     s.flags = c->d_flags;
-    int64_t grid = pdx_wave_grid(n);
-    hipLaunchKernelGGL(k_count_bonds, dim3(grid), dim3(PDX_BLOCK), 0, c->stream, s);
+    hipLaunchKernelGGL(k_count_bonds, dim3((unsigned)pdx_wave_grid(n)), dim3(PDX_BLOCK), 0, c->stream, s);
     HIP_C(hipGetLastError());
     std::vector<int32_t> counts(n);
     HIP_C(hipMemcpyAsync(counts.data(), d_counts, sizeof(int32_t) * n, hipMemcpyDeviceToHost,
@@ -803,50 +957,32 @@ extern "C" pdx_status pdx_build_bonds(pdx_ctx *c, int64_t *n_bonds_out)
                         "point duplicate found! Point #%llu has a duplicate #%llu which will lead to NaNs",
                         hflags[2] + 1, hflags[3] + 1);
     }
-    // SELL-64 slices: slice s holds points 64 s .. 64 s + 63, as wide as its widest row
-    const int64_t n_slices = (n + 63) / 64;
-    std::vector<int64_t> slice_ptr(n_slices + 1, 0);
     int32_t maxc = 0;
-    int64_t nb_real = 0;
-    for (int64_t sl = 0; sl < n_slices; sl++) {
-        int32_t w = 0;
-        for (int64_t m = 64 * sl; m < std::min(n, 64 * sl + 64); m++) {
-            w = std::max(w, counts[m]);
-            nb_real += counts[m];
-        }
-        maxc = std::max(maxc, w);
-        slice_ptr[sl + 1] = slice_ptr[sl] + 64 * (int64_t)w;
+    int64_t nb = 0;
+    for (int64_t m = 0; m < n; m++) {
+        maxc = std::max(maxc, counts[m]);
+        nb += counts[m];
     }
     if (maxc > PDX_FILL_CAP) {
         cleanup();
         return pdx_fail(c, PDX_ERR_UNSUPPORTED, "a point has %d bonds (> %d)", maxc, PDX_FILL_CAP);
     }
-    const int64_t nb = nb_real;
-    const int64_t nb_alloc = slice_ptr[n_slices];
-    if (nb_alloc >= ((int64_t)1 << 40)) {
-        cleanup();
-        return pdx_fail(c, PDX_ERR_UNSUPPORTED, "too many bonds");
-    }
     c->nb = nb;
-    c->nb_alloc = nb_alloc;
-    TRY_C(pdx_alloc(c, &c->slice_ptr, n_slices + 1));
+    choose_blocks(c, !getenv("PDX_NO_LDS"));
     TRY_C(pdx_alloc(c, &c->cnt, n));
-    TRY_C(pdx_alloc(c, &c->bw, nb_alloc));
-    TRY_C(pdx_alloc(c, &c->L, nb_alloc));
-    HIP_C(hipMemcpy(c->slice_ptr, slice_ptr.data(), sizeof(int64_t) * (n_slices + 1),
-                    hipMemcpyHostToDevice));
     HIP_C(hipMemcpy(c->cnt, counts.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice));
-    // padding entries of a slice stay zero (never read: t < cnt)
-    HIP_C(hipMemsetAsync(c->bw, 0, sizeof(uint32_t) * nb_alloc, c->stream));
-    HIP_C(hipMemsetAsync(c->L, 0, sizeof(double) * nb_alloc, c->stream));
-    s.slice_ptr = c->slice_ptr;
-    s.cnt = c->cnt;
-    s.bw = c->bw;
-    s.L = c->L;
-    hipLaunchKernelGGL(k_fill_bonds, dim3(grid), dim3(PDX_BLOCK), 0, c->stream, s);
-    HIP_C(hipGetLastError());
+    TRY_C(fill_rows(c, s, counts));
+    // the LDS-staged layout; tables it cannot address go to the global-gather layout
+    if (c->ls > 0) {
+        bool ok = false;
+        TRY_C(build_halos(c, &ok));
+        if (!ok) {
+            choose_blocks(c, false);
+            TRY_C(fill_rows(c, s, counts));
+        }
+    }
     hipLaunchKernelGGL(k_init_point_state, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
-                       c->stream, n, c->slice_ptr, c->cnt, c->bw, c->nact, c->damage);
+                       c->stream, n, c->rows(), c->cnt, c->bw, c->nact, c->damage);
     HIP_C(hipGetLastError());
     // zero dynamic state
     for (double *p : {c->u, c->vh, c->v, c->a, c->bint, c->bext})
@@ -873,12 +1009,6 @@ extern "C" pdx_status pdx_build_bonds(pdx_ctx *c, int64_t *n_bonds_out)
         HIP_C(hipStreamSynchronize(c->stream));
     }
     cleanup();
-    // LDS-staged layouts: BB (x|V per neighbour-table entry), OSB (x|V and c1, c2), CPD
-    // (tables staged in tiles)
-    if (!getenv("PDX_NO_LDS")) {
-        bool ok = false;
-        PDX_TRY(build_halos(c, &ok));
-    }
     // FP32 lengths for the global-gather mixed BB step (the LDS-staged steps take L = |D|)
     if (c->precision == PDX_MIXED && !c->lds_mode) {
         const int64_t nba = c->nb_alloc;
@@ -908,22 +1038,23 @@ extern "C" pdx_status pdx_build_bonds(pdx_ctx *c, int64_t *n_bonds_out)
 pdx_status pdx_caller_bond_slots(pdx_ctx *c, std::vector<int64_t> &slots)
 {
     const int64_t n = c->n, nba = c->nb_alloc;
-    const int64_t n_slices = (n + 63) / 64;
+    const int64_t n_slices = c->n_slices();
     std::vector<int64_t> sp(n_slices + 1);
     std::vector<int32_t> cn(n);
     std::vector<uint32_t> w(nba);
     PDX_HIP(c, hipStreamSynchronize(c->stream));
     PDX_HIP(c, hipMemcpy(sp.data(), c->slice_ptr, sizeof(int64_t) * (n_slices + 1), hipMemcpyDeviceToHost));
     PDX_HIP(c, hipMemcpy(cn.data(), c->cnt, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
+    const pdx_rows hr{sp.data(), c->ls};
     PDX_HIP(c, hipMemcpy(w.data(), c->bw, sizeof(uint32_t) * nba, hipMemcpyDeviceToHost));
     slots.clear();
     std::vector<std::pair<int32_t, int64_t>> row;
     for (int64_t i = 0; i < n; i++) {
         const int64_t m = c->iperm[i];
-        const int64_t b0 = sp[m >> 6] + (m & 63);
+        const int64_t b0 = hr.row(m);
         row.clear();
         for (int t = 0; t < cn[m]; t++) {
-            const int64_t b = b0 + (int64_t)t * 64;
+            const int64_t b = hr.at(b0, t);
             row.push_back({c->perm[w[b] & PDX_BW_NBR], b});
         }
         std::sort(row.begin(), row.end());
@@ -938,18 +1069,24 @@ extern "C" pdx_status pdx_get_bonds(pdx_ctx *c, int64_t *row_ptr, int32_t *nbr, 
     if (!c) return PDX_ERR_ARG;
     if (!c->bonds_built) return pdx_fail(c, PDX_ERR_STATE, "pdx_build_bonds first");
     const int64_t n = c->n, nba = c->nb_alloc;
-    const int64_t n_slices = (n + 63) / 64;
+    const int64_t n_slices = c->n_slices();
     std::vector<int64_t> sp(n_slices + 1);
     std::vector<int32_t> cn(n);
     std::vector<uint32_t> w(nba);
-    std::vector<double> L_dev(L ? nba : 0);
+    std::vector<double> L_dev(L && c->L ? nba : 0);
     PDX_HIP(c, hipStreamSynchronize(c->stream));
     PDX_HIP(c, hipMemcpy(sp.data(), c->slice_ptr, sizeof(int64_t) * (n_slices + 1),
                          hipMemcpyDeviceToHost));
     PDX_HIP(c, hipMemcpy(cn.data(), c->cnt, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
+    const pdx_rows hr{sp.data(), c->ls};
     PDX_HIP(c, hipMemcpy(w.data(), c->bw, sizeof(uint32_t) * nba, hipMemcpyDeviceToHost));
-    if (L) PDX_HIP(c, hipMemcpy(L_dev.data(), c->L, sizeof(double) * nba, hipMemcpyDeviceToHost));
-    if (c->lds_mode) {
+    if (L && c->L) PDX_HIP(c, hipMemcpy(L_dev.data(), c->L, sizeof(double) * nba, hipMemcpyDeviceToHost));
+    if (c->pk) {  // the packed words keep the bond state
+        std::vector<unsigned long long> pk(nba);
+        PDX_HIP(c, hipMemcpy(pk.data(), c->pk, sizeof(unsigned long long) * nba, hipMemcpyDeviceToHost));
+        for (int64_t b = 0; b < nba; b++)
+            w[b] = (w[b] & ~PDX_BW_ACT) | ((pk[b] & c->pk_mask) != c->pk_mask ? PDX_BW_ACT : 0u);
+    } else if (c->lds_mode) {
         // the LDS-staged step keeps the bond state in the 16-bit words
         std::vector<uint16_t> w16(nba);
         PDX_HIP(c, hipMemcpy(w16.data(), c->bw16, sizeof(uint16_t) * nba, hipMemcpyDeviceToHost));
@@ -973,16 +1110,24 @@ extern "C" pdx_status pdx_get_bonds(pdx_ctx *c, int64_t *row_ptr, int32_t *nbr, 
         int64_t m = c->iperm[i];
         int64_t o = out_rp[i];
         row.clear();
-        const int64_t b0 = sp[m >> 6] + (m & 63);
+        const int64_t b0 = hr.row(m);
         for (int t = 0; t < cn[m]; t++) {
-            const int64_t b = b0 + (int64_t)t * 64;
+            const int64_t b = hr.at(b0, t);
             row.push_back({c->perm[w[b] & PDX_BW_NBR], b});
         }
         std::sort(row.begin(), row.end());
         for (auto &e : row) {
             const int64_t b = e.second;
             if (nbr) nbr[o] = e.first;
-            if (L) L[o] = L_dev[b];
+            if (L) {
+                if (c->L) {
+                    L[o] = L_dev[b];
+                } else {  // as the search formed it
+                    const double *xi = &c->X[3 * i], *xj = &c->X[3 * (int64_t)e.first];
+                    const double p0 = xi[0] - xj[0], p1 = xi[1] - xj[1], p2 = xi[2] - xj[2];
+                    L[o] = std::sqrt((p0 * p0 + p1 * p1) + p2 * p2);
+                }
+            }
             if (fp) fp[o] = (w[b] & PDX_BW_FP) ? 1 : 0;
             if (active) active[o] = ((w[b] & PDX_BW_ACT) && !killed[m]) ? 1 : 0;
             o++;
@@ -1115,7 +1260,7 @@ extern "C" pdx_status pdx_set_field(pdx_ctx *c, int32_t field, const double *hos
 // LDS and summed in that order by one lane, so that the value equals the reference's bit
 // for bit.
 // ----------------------------------------------------------------------------------------
-__global__ __launch_bounds__(PDX_BLOCK) void k_timestep(int64_t n, const int64_t *slice_ptr,
+__global__ __launch_bounds__(PDX_BLOCK) void k_timestep(int64_t n, pdx_rows rows,
                                                          const int32_t *cnts,
                                                          const uint32_t *bw, const double *L,
                                                          const double4 *Xr, const int32_t *perm,
@@ -1128,25 +1273,27 @@ __global__ __launch_bounds__(PDX_BLOCK) void k_timestep(int64_t n, const int64_t
     const int64_t i = pdx_wave_point();
     if (i >= n) return;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int64_t b0 = slice_ptr[i >> 6] + (i & 63);
+    const int64_t b0 = rows.row(i);
     const int cnt = cnts[i];  // <= PDX_FILL_CAP (checked when built)
+    const double4 Xi = Xr[i];
     if (psets) {  // the point's own parameter set (get_params(chunk, point_id))
         bc = psets[pid[i]].bc;
         rho = psets[pid[i]].rho;
     }
     for (int k = lane; k < cnt; k += 64) {
-        const uint32_t j = bw[b0 + (int64_t)k * 64] & PDX_BW_NBR;
+        const uint32_t j = bw[rows.at(b0, k)] & PDX_BW_NBR;
         key[w][k] = perm[j];
     }
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     __builtin_amdgcn_wave_barrier();
     for (int k = lane; k < cnt; k += 64) {
-        const int64_t b = b0 + (int64_t)k * 64;
+        const int64_t b = rows.at(b0, k);
         const uint32_t j = bw[b] & PDX_BW_NBR;
         const int32_t kk = key[w][k];
         int rank = 0;
         for (int m = 0; m < cnt; m++) rank += (key[w][m] < kk) ? 1 : 0;
-        term[w][rank] = Xr[j].w * bc / L[b];
+        const double4 Xj = Xr[j];
+        term[w][rank] = Xj.w * bc / pdx_ref_len(L, b, Xi, Xj);
     }
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -1166,7 +1313,7 @@ extern "C" pdx_status pdx_stable_timestep(pdx_ctx *c, double safety, double *dt_
     PDX_HIP(c, hipSetDevice(c->device));
     double *tmp = c->stage;
     hipLaunchKernelGGL(k_timestep, dim3((unsigned)pdx_wave_grid(c->n)), dim3(PDX_BLOCK), 0,
-                       c->stream, c->n, c->slice_ptr, c->cnt, c->bw, c->L, c->Xr, c->d_perm, c->P.bc,
+                       c->stream, c->n, c->rows(), c->cnt, c->bw, c->L, c->Xr, c->d_perm, c->P.bc,
                        c->P.rho, c->multi() ? c->d_psets : nullptr, c->multi() ? c->d_pid : nullptr, tmp);
     PDX_HIP(c, hipGetLastError());
     std::vector<double> dt(c->n);

@@ -1,11 +1,10 @@
 // Force density and the fused Velocity Verlet step: BB, OSB and CPD.
 //
-// Bond storage is sliced ELL with slices of 64 Morton-consecutive points (SELL-64): bond t
-// of point p sits at slice_ptr[p / 64] + 64 t + p % 64, so bond t of the 64 points of a
-// slice is one contiguous 64-entry row.  One thread owns one point: it walks its bonds
-// with fully coalesced loads of the bond words and lengths, gathers the neighbours'
-// records (Morton order keeps them in the L1/L2 of the CU), and accumulates its own
-// force density in registers -- no atomics and no cross-lane reductions.
+// The production kernels (LDS-staged) give a block of 32 to 256 Morton-consecutive points 4 to 16
+// lanes per point; its bonds come in row groups of 64 slots (pdx_rows), one contiguous run per
+// wave and load, and its neighbours' records are staged in LDS once per launch.  Bodies whose
+// neighbour tables 13-bit slots cannot address run the global-gather kernels: one thread per
+// point (CPD: four lanes) over SELL-64 rows, neighbours through the caches.
 //
 // The scatter of the reference's OSB and CPD force densities (b_int[j] -= ...,
 // ordinary_state_based.jl:145-146, correspondence.jl:248-249) is rewritten as a gather: a
@@ -30,7 +29,7 @@
 
 #include "pdx_internal.h"
 
-#define PDX_LDS_LANES 4  // lanes per point in the LDS-staged BB kernels
+#define PDX_LDS_LANES 4  // lanes per point of the global-gather CPD kernels
 
 // thread index of the calling point; blocks are remapped so that each XCD gets a
 // contiguous range of points (see pdx_xcd_block)
@@ -39,7 +38,6 @@ __device__ __forceinline__ int64_t pdx_thread_point()
     return pdx_xcd_block() * PDX_BLOCK + threadIdx.x;
 }
 
-// first bond entry of point p in the SELL-64 arrays; bond t is at + 64 t
 // Neighbour-table entries a block stages in LDS: all of them up to a budget that leaves
 // room for two 1024-thread blocks per CU; a block whose table is longer reads the entries
 // past the budget from global memory (through the caches).  ENTRY = LDS bytes per entry.
@@ -47,63 +45,6 @@ __host__ __device__ __forceinline__ int pdx_lds_entries(int halo_max, int budget
 {
     const int cap = budget / entry;
     return halo_max < cap ? (halo_max > 0 ? halo_max : 1) : cap;
-}
-
-__device__ __forceinline__ int64_t pdx_bond0(const int64_t *slice_ptr, int64_t p)
-{
-    return slice_ptr[p >> 6] + (p & 63);
-}
-
-// Bond words and lengths of G bonds of a lane's row: t, t + S, ..., t + (G - 1) S.  Bonds
-// past the row's end read its last bond (bond 0 of an empty row), an in-range address whose
-// value the caller never uses, so the loads need no branch and can be issued a whole group
-// ahead of their use.
-template <int G, int S>
-__device__ __forceinline__ void pdx_load_group(const uint16_t *wbase, const double *Lbase, int t, int c,
-                                               uint32_t (&w)[G], double (&L)[G])
-{
-    const int last = c > 0 ? c - 1 : 0;
-#pragma unroll
-    for (int u = 0; u < G; u++) {
-        const int tt = t + u * S < c ? t + u * S : last;
-        w[u] = wbase[(int64_t)tt * 64];
-        L[u] = Lbase[(int64_t)tt * 64];
-    }
-}
-
-// The bonds of a lane's row whose neighbour slots lie below the staged tile's end T1, in row
-// order from bond t, as groups of G: the words and lengths of the next group are loaded
-// before the current group is evaluated, so their latency hides behind G bond evaluations.
-// Returns the first bond not evaluated (past the tile, or c).  BOND(wd, L, t) evaluates one.
-template <int G, int S, class BOND>
-__device__ __forceinline__ int pdx_walk_tile(const uint16_t *wbase, const double *Lbase, int t, int c,
-                                             int T1, BOND &&bond)
-{
-    if (t >= c) return t;
-    uint32_t gw[G];
-    double gL[G];
-    pdx_load_group<G, S>(wbase, Lbase, t, c, gw, gL);
-    while (true) {
-        uint32_t nw[G];
-        double nL[G];
-        pdx_load_group<G, S>(wbase, Lbase, t + G * S, c, nw, nL);
-        // the leading bonds of the group inside the row and the tile (slots increase along
-        // the row, so every bond after the first one past T1 is past it too)
-        int kk = 0;
-#pragma unroll
-        for (int u = 0; u < G; u++)
-            if (kk == u && t + u * S < c && (int)(gw[u] & PDX_W16_SLOT) < T1) kk = u + 1;
-#pragma unroll
-        for (int u = 0; u < G; u++)
-            if (u < kk) bond(gw[u], gL[u], t + u * S);
-        t += kk * S;
-        if (kk < G) return t;
-#pragma unroll
-        for (int u = 0; u < G; u++) {
-            gw[u] = nw[u];
-            gL[u] = nL[u];
-        }
-    }
 }
 
 // ----------------------------------------------------------------------------------------
@@ -286,7 +227,7 @@ __global__ __launch_bounds__(PDX_BLOCK) void k_bb_step(pdx_step_args A)
     const int64_t p = pdx_thread_point();
     if (p >= A.n) return;
     const int c = A.cnt[p];
-    const int64_t b0 = pdx_bond0(A.slice_ptr, p);
+    const int64_t b0 = A.rows.row(p);
     uint32_t *const wbase = A.bw + b0;
     const double4 ri = A.rec_in[p];
     double4 Xi = make_double4(0, 0, 0, 0);
@@ -373,263 +314,376 @@ __global__ __launch_bounds__(PDX_BLOCK) void k_bb_step(pdx_step_args A)
     point_tail(A, p, ri, b, T, A.rho);
 }
 
-// ----------------------------------------------------------------------------------------
-// BB, LDS-staged (the production kernel).  A workgroup owns PDX_BLOCK consecutive Morton
-// points.  It first copies the records of its halo (every point its bonds reach, ~2000
-// for a 3.015-spacing horizon) from global memory into LDS with one coalesced pass, then
-// each thread walks its point's bonds: 16-bit bond words (slot into the halo, active,
-// fail_permit) and reference lengths stream from HBM, neighbour records come from LDS.
-// Arithmetic as k_bb_step (FP64); MIXED takes the stretch from the FP64 difference
-// d2 - L^2 (fused, one rounding) and does the rest in FP32 with FP64 sums.
-// ----------------------------------------------------------------------------------------
-__device__ __forceinline__ bool bond_fail16(uint16_t *wp, uint32_t wd, double e, double Lb, double eps,
-                                            double epsc, double epsc_lo, double epsc_hi)
-{
-    bool act = (wd & PDX_W16_ACT) != 0;
-    if (act && (wd & PDX_W16_FP) && eps >= epsc_lo) {
-        const bool brk = (eps > epsc_hi) ? true : ((e / Lb) > epsc);
-        if (brk) {
-            act = false;
-            *wp = (uint16_t)(wd & ~PDX_W16_ACT);
-        }
-    }
-    return act;
-}
-
-// One bond of the FP64 BB step (bond_based.jl:125-161): failure against the point's eps_c,
-// then the force term (w bc) eps V_j dx / l accumulated into b; bcb = the bond's bc,
-// sc = its surface-correction factor (1 without).
-// (rL = pdx_rcp1(Lb), passed in where one bond is evaluated at two states)
-__device__ __forceinline__ void bb_bond64_r(double4 ri, double4 rj, uint16_t *wp, uint32_t wd, double Lb,
-                                            double rL, double sc, double bcb, double epsc, double epsc_lo,
-                                            double epsc_hi, double &bx, double &by, double &bz, int &na)
-{
-    const double dx = rj.x - ri.x, dy = rj.y - ri.y, dz = rj.z - ri.z;
-    const double d2 = (dx * dx + dy * dy) + dz * dz;
-    double rl;
-    const double l = pdx_sqrt_rsq(d2, rl);
-    const double e = l - Lb;
-    const double eps = e * rL;
-    const bool act = bond_fail16(wp, wd, e, Lb, eps, epsc, epsc_lo, epsc_hi);
-    const double wbc = act ? sc * bcb : 0.0;  // (w * bc), w = active * sc
-    const double s = ((wbc * eps) * rj.w) * rl;
-    bx = __builtin_fma(s, dx, bx);
-    by = __builtin_fma(s, dy, by);
-    bz = __builtin_fma(s, dz, bz);
-    na += act ? 1 : 0;
-}
-
-__device__ __forceinline__ void bb_bond64(double4 ri, double4 rj, uint16_t *wp, uint32_t wd, double Lb,
-                                          double sc, double bcb, double epsc, double epsc_lo,
-                                          double epsc_hi, double &bx, double &by, double &bz, int &na)
-{
-    bb_bond64_r(ri, rj, wp, wd, Lb, pdx_rcp1(Lb), sc, bcb, epsc, epsc_lo, epsc_hi, bx, by, bz, na);
-}
-
-// The same bond with one parameter set, whose neighbour record carries V_j bc in its fourth
-// word (the neighbour-table staging forms it once per entry): one multiply fewer per bond.
-__device__ __forceinline__ void bb_bond64_vbc(double4 ri, double4 rj, uint16_t *wp, uint32_t wd, double Lb,
-                                              double rL, double sc, double epsc, double epsc_lo,
-                                              double epsc_hi, double &bx, double &by, double &bz, int &na)
-{
-    const double dx = rj.x - ri.x, dy = rj.y - ri.y, dz = rj.z - ri.z;
-    const double d2 = (dx * dx + dy * dy) + dz * dz;
-    double rl;
-    const double l = pdx_sqrt_rsq(d2, rl);
-    const double e = l - Lb;
-    const double eps = e * rL;
-    const bool act = bond_fail16(wp, wd, e, Lb, eps, epsc, epsc_lo, epsc_hi);
-    const double s = ((act ? sc * eps : 0.0) * rj.w) * rl;  // w eps (V_j bc) / l, w = active * sc
-    bx = __builtin_fma(s, dx, bx);
-    by = __builtin_fma(s, dy, by);
-    bz = __builtin_fma(s, dz, bz);
-    na += act ? 1 : 0;
-}
-
-// a neighbour record (x, V) with V_j bc in the fourth word, for bb_bond64_vbc
+// a neighbour record (x, V) with V_j bc in the fourth word
 __device__ __forceinline__ double4 pdx_rec_vbc(double4 r, double bc) { return make_double4(r.x, r.y, r.z, r.w * bc); }
 
+// ----------------------------------------------------------------------------------------
+// The bonds of the LDS-staged kernels.  A wave of 64 lanes serves 64 / S points, S adjacent
+// lanes per point, and walks its slice's row groups (pdx_rows) from the first to the last: every
+// load of the walk is one contiguous run of 64 slots at a wave-uniform address, the loop count is
+// wave-uniform, and lanes whose row is shorter evaluate padding slots (inactive, the row's last
+// neighbour), which add zero.
+//
+// Measured, FP64 steps at 2 M points (3.015 spacings), us: per-lane loops over rows interleaved by
+// 64 points, 256 x 4 blocks BB 642, OSB 1295; the same loops over row groups BB 578; this walk
+// with words and lengths apart BB 578 (128 x 4 blocks; 626 with 256 x 4), OSB 1133; with packed
+// bonds BB 515, OSB 1010 (a slot costs 8 bytes instead of 10, 232 M of them: 4.3 TB/s of the
+// 5.0 TB/s that a device copy reaches).  The look-ahead is worth 5 to 10 % (BB 100 k points 33.0
+// without, 30.6 with), and two bonds per step of the walk 5 % over one (BB 1 M 266 against 261 at
+// 76 against 54 VGPRs); forcing 64 VGPRs spills and triples the time.
+//
+// Two forms of a bond's data.  PK = false: a 16-bit word (slot in the block's neighbour table and
+// state bits) and the FP64 length.  PK = true (one parameter set, FP64 contexts): one 64-bit
+// word, the slot in the upper bits and below it the length as the distance of its bit pattern
+// from that of the body's shortest bond; all ones there mark a bond that is not active.
+// ----------------------------------------------------------------------------------------
+template <bool PK>
+struct bond_data {
+    uint32_t w;
+    double L;
+};
+template <>
+struct bond_data<true> {
+    unsigned long long w;
+};
+
+__device__ __forceinline__ int bond_slot(const pdx_step_args &, const bond_data<false> &b)
+{
+    return (int)(b.w & PDX_W16_SLOT);
+}
+__device__ __forceinline__ int bond_slot(const pdx_step_args &A, const bond_data<true> &b)
+{
+    return (int)(b.w >> A.pk_shift);
+}
+__device__ __forceinline__ bool bond_act(const pdx_step_args &, const bond_data<false> &b)
+{
+    return (b.w & PDX_W16_ACT) != 0;
+}
+__device__ __forceinline__ bool bond_act(const pdx_step_args &A, const bond_data<true> &b)
+{
+    return (b.w & A.pk_mask) != A.pk_mask;
+}
+__device__ __forceinline__ double bond_len(const pdx_step_args &, const bond_data<false> &b) { return b.L; }
+__device__ __forceinline__ double bond_len(const pdx_step_args &A, const bond_data<true> &b)
+{
+    return __longlong_as_double((long long)((b.w & A.pk_mask) + A.pk_base));
+}
+
+template <int S>
+__host__ __device__ constexpr int pdx_log2() { return S == 4 ? 2 : S == 8 ? 3 : 4; }
+
+// The calling lane's bonds: the slice's first slot and the number of bonds to walk, both uniform
+// over the wave.  With more than four lanes per point PDX_F_ORDER makes each group of four lanes walk
+// the whole row, so that the four sums of a point are those of four lanes per point, bit for bit
+// (the lanes 4 .. S - 1 repeat the work of lanes 0 .. 3 and pdx_fold drops their sums).
+template <int S, bool PK>
+struct pdx_lane {
+    int64_t b0;
+    int ng, lane;
+    bool order;
+    // slot of the lane's i-th bond (past the end: its last one)
+    __device__ __forceinline__ int64_t at(int i) const
+    {
+        i = i < ng ? i : ng - 1;
+        if (S > 4 && order) {
+            constexpr int M = S / 4;
+            const int k = i >> 2;
+            return b0 + (int64_t)(4 * (k / M) + (i & 3)) * 64 + 4 * (k % M) + lane;
+        }
+        return b0 + (int64_t)i * 64 + lane;
+    }
+    __device__ __forceinline__ bond_data<PK> load(const pdx_step_args &A, int i) const
+    {
+        const int64_t o = at(i);
+        bond_data<PK> b;
+        if constexpr (PK) {
+            b.w = A.pk[o];
+        } else {
+            b.w = A.bw16[o];
+            b.L = A.L[o];
+        }
+        return b;
+    }
+    // marks the lane's i-th bond as broken
+    __device__ __forceinline__ void kill(const pdx_step_args &A, int i, const bond_data<PK> &b) const
+    {
+        if constexpr (PK) A.pk[at(i)] = b.w | A.pk_mask;
+        else A.bw16[at(i)] = (uint16_t)(b.w & ~PDX_W16_ACT);
+    }
+};
+
+// p0 = the block's first point; waves past the last point have no bonds
+template <int S, bool PK>
+__device__ __forceinline__ pdx_lane<S, PK> pdx_lane_of(const pdx_step_args &A, int64_t p0)
+{
+    constexpr int LS = pdx_log2<S>();
+    const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    pdx_lane<S, PK> R;
+    R.lane = threadIdx.x & 63;
+    R.ng = 0;
+    R.b0 = 0;
+    R.order = S > 4 && (A.flags & PDX_F_ORDER) != 0;
+    if (p0 + wv * (64 / S) < A.n) {
+        const int64_t *const q = A.rows.ptr + (p0 >> (6 - LS)) + wv;
+        R.b0 = q[0];
+        R.ng = (int)((q[1] - R.b0) >> 6);
+        if (R.order) {
+            R.ng = (S / 4) * (R.ng & ~3) + (R.ng & 3);  // a last incomplete group of four is lane 0's
+            R.lane &= ~(S - 1) | 3;
+        }
+    }
+    return R;
+}
+
+// sum over a point's lanes, in every one of them
+template <int S, bool PK, class T>
+__device__ __forceinline__ void pdx_fold(const pdx_lane<S, PK> &R, T &x)
+{
+    if (S > 4 && R.order && (threadIdx.x & (S - 1)) >= 4) x = 0;
+#pragma unroll
+    for (int o = 1; o < S; o <<= 1) x += __shfl_xor(x, o);
+}
+
+// Walks the lane's bonds U at a time, the next U loaded before the current ones are evaluated.
+// GROUP(b, i): bonds i .. i + U - 1 (those past R.ng repeat the last one and must not count).
+template <int U, int S, bool PK, class GROUP>
+__device__ __forceinline__ void pdx_walk(const pdx_step_args &A, const pdx_lane<S, PK> &R, GROUP &&group)
+{
+    if (R.ng == 0) return;
+    bond_data<PK> c[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) c[u] = R.load(A, u);
+    for (int i = 0; i < R.ng; i += U) {
+        bond_data<PK> nx[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) nx[u] = R.load(A, i + U + u);
+        group(c, i);
+#pragma unroll
+        for (int u = 0; u < U; u++) c[u] = nx[u];
+    }
+}
+
+// l - L and 1/(l L) of an OSB bond with l = sqrt(d2): l is correctly rounded (one Goldschmidt step and
+// two residual corrections from the hardware's 1/sqrt estimate), the reciprocal is within about
+// two ulp.  The estimate is taken of d2 L^2, so that no reciprocal of L is formed.
+__device__ __forceinline__ double pdx_elong(double d2, double L, double &rlL)
+{
+    const double r = __builtin_amdgcn_rsq((L * L) * d2);
+    const double Lr = L * r;
+    double h = 0.5 * Lr;
+    double g = d2 * Lr;
+    const double e = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, e, g);
+    h = __builtin_fma(h, e, h);
+    rlL = __builtin_fma(r, e, r);
+    double d = __builtin_fma(-g, g, d2);
+    g = __builtin_fma(d, h, g);
+    d = __builtin_fma(-g, g, d2);
+    return __builtin_fma(d, h, g) - L;
+}
+
+// A bond that reaches the failure window [epsc_lo, inf): does it break (calc_failure!,
+// bond_based.jl:125-144)?  The stretch is the correctly rounded quotient, and both ends must
+// permit failure.
+template <bool PK>
+__device__ __forceinline__ bool bond_breaks(const pdx_step_args &A, const int32_t *hidx, const bond_data<PK> &b,
+                                            double el, double L, double epsc)
+{
+    bool permit;
+    if constexpr (PK) permit = A.fp[hidx[bond_slot(A, b)]] != 0;
+    else permit = (b.w & PDX_W16_FP) != 0;
+    return permit && (el / L) > epsc;
+}
+
+// The lane's bonds whose neighbours lie in the staged tile of the block's table (entries below
+// T1), from row group i: rows and tables are sorted by neighbour, so each lane meets the tiles in
+// order.  Returns the first group not evaluated.  BOND(b, i) evaluates one; two are in flight.
+template <int G, int S, bool PK, class BOND>
+__device__ __forceinline__ int pdx_walk_tile(const pdx_step_args &A, const pdx_lane<S, PK> &R, int i, int T1, BOND &&bond)
+{
+    if (i >= R.ng) return i;
+    bond_data<PK> c[G];
+#pragma unroll
+    for (int u = 0; u < G; u++) c[u] = R.load(A, i + u);
+    while (true) {
+        bond_data<PK> nx[G];
+#pragma unroll
+        for (int u = 0; u < G; u++) nx[u] = R.load(A, i + G + u);
+        // slots increase along the row: every bond after the first one past T1 is past it too
+        int kk = 0;
+#pragma unroll
+        for (int u = 0; u < G; u++)
+            if (kk == u && i + u < R.ng && bond_slot(A, c[u]) < T1) kk = u + 1;
+#pragma unroll
+        for (int u = 0; u < G; u++)
+            if (u < kk) bond(c[u], i + u);
+        i += kk;
+        if (kk < G) return i;
+#pragma unroll
+        for (int u = 0; u < G; u++) c[u] = nx[u];
+    }
+}
+
+// ----------------------------------------------------------------------------------------
+// BB: calc_failure! (bond_based.jl:125-144), calc_damage! (bond_system.jl:338-343),
+// force_density_point! (bond_based.jl:146-161) and the fused tail.  A workgroup owns PB
+// consecutive Morton points.  It first copies the records of its neighbour table (every point
+// its bonds reach) from global memory into LDS with one coalesced pass, then walks the bonds:
+// their data stream from HBM, the neighbour records come from LDS.
+//
 // F = feature mask.  PDX_FEAT_MULTI: several parameter sets (force_density_point! with a
 // ParameterHandler, bond_based.jl:163-180): eps_c of the row's point, (bc_i + bc_j) / 2 per
-// bond, rho_i.  PDX_FEAT_SC: EnergySurfaceCorrection, w = bond_active * scfactor[bond]
-// (bond_based.jl:156, bond_system_corrections.jl:71-74).  PDX_FEAT_CAP: the table may be
-// longer than the LDS budget; it is staged in tiles of HL entries.  Rows and table are both
-// sorted by neighbour, so each lane meets the tiles in order: it walks its bonds while their
-// slots lie in the staged tile and resumes there after the next tile is staged.
-template <int U, int S, int F>
-__global__ __launch_bounds__(PDX_BLOCK * S) void k_bb_lds(pdx_step_args A)
+// bond, rho_i; the table holds V_j / 2 and V_j bc_j / 2.  Otherwise its fourth word is V_j bc.
+// PDX_FEAT_SC: EnergySurfaceCorrection, w = bond_active * scfactor[bond] (bond_based.jl:156,
+// bond_system_corrections.jl:71-74).  PDX_FEAT_CAP: the table may be longer than the LDS budget;
+// it is staged in tiles of HL entries.
+// ----------------------------------------------------------------------------------------
+
+// the accumulated force density of one point and its active bonds
+struct bb_sum {
+    double x = 0.0, y = 0.0, z = 0.0;
+    int na = 0;
+};
+
+// U bonds of the lane: all stretches first, then the rare failure branch once for the group, then
+// the sums; a bond that is not active takes part with weight 0 (a NaN position still shows).
+template <int U, int F, int S, bool PK>
+__device__ __forceinline__ void bb_group(const pdx_step_args &A, const pdx_lane<S, PK> &R, const int32_t *hidx,
+                                         const double4 *hrec, const double *hb, int T0, double4 ri, double bci,
+                                         double thr, double epsc, const bond_data<PK> (&b)[U], int i, bb_sum &f)
+{
+    double dx[U], dy[U], dz[U], el[U], rr[U], vb[U], sc[U];
+    bool act[U], any = false;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const int slot = bond_slot(A, b[u]) - T0;
+        const double4 rj = hrec[slot];
+        dx[u] = rj.x - ri.x;
+        dy[u] = rj.y - ri.y;
+        dz[u] = rj.z - ri.z;
+        vb[u] = (F & PDX_FEAT_MULTI) ? __builtin_fma(bci, rj.w, hb[slot]) : rj.w;
+        sc[u] = (F & PDX_FEAT_SC) ? A.scf[R.at(i + u)] : 1.0;
+        const double L = bond_len(A, b[u]);
+        el[u] = pdx_sqrt_rsq((dx[u] * dx[u] + dy[u] * dy[u]) + dz[u] * dz[u], rr[u]) - L;
+        act[u] = (U == 1 || i + u < R.ng) && bond_act(A, b[u]);
+        any |= act[u] && el[u] >= thr * L;
+    }
+    if (any) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const double L = bond_len(A, b[u]);
+            if (act[u] && el[u] >= thr * L && bond_breaks<PK>(A, hidx, b[u], el[u], L, epsc)) {
+                act[u] = false;
+                R.kill(A, i + u, b[u]);
+            }
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const double eps = el[u] * pdx_rcp1(bond_len(A, b[u]));
+        const double s = ((act[u] ? ((F & PDX_FEAT_SC) ? sc[u] * eps : eps) : 0.0) * vb[u]) * rr[u];
+        f.x = __builtin_fma(s, dx[u], f.x);
+        f.y = __builtin_fma(s, dy[u], f.y);
+        f.z = __builtin_fma(s, dz[u], f.z);
+        f.na += act[u] ? 1 : 0;
+    }
+}
+
+// lower end of a point's failure window on e / L (its stretch may exceed eps_c from there on);
+// infinite where the point does not permit failure
+template <bool PK>
+__device__ __forceinline__ double fail_window(const pdx_step_args &A, int64_t p, double epsc_lo)
+{
+    return PK && !A.fp[p] ? INFINITY : epsc_lo;
+}
+
+template <int U, int S, int F, int PB, bool PK>
+__global__ __launch_bounds__(PB * S) void k_bb_lds(pdx_step_args A)
 {
     constexpr bool MULTI = (F & PDX_FEAT_MULTI) != 0;
-    constexpr bool SC = (F & PDX_FEAT_SC) != 0;
     constexpr bool CAP = (F & PDX_FEAT_CAP) != 0;
     extern __shared__ double4 hrec[];
     const int64_t k = pdx_xcd_block();
-    const int64_t p0 = k * PDX_BLOCK;
+    const int64_t p0 = k * PB;
     if (p0 >= A.n) return;  // whole workgroup
     const int64_t h0 = A.halo_ptr[k];
     const int H = (int)(A.halo_ptr[k + 1] - h0);
-    const int HL = CAP ? pdx_lds_entries(A.halo_max, A.lds_budget, 32 + (MULTI ? 1 : 0)) : A.halo_max;
+    const int HL = CAP ? pdx_lds_entries(A.halo_max, A.lds_budget, 32 + (MULTI ? 8 : 0)) : A.halo_max;
     const int32_t *const hidx = A.halo + h0;
-    uint8_t *const hpid = reinterpret_cast<uint8_t *>(hrec + HL);
-    // S adjacent lanes share a point; lane s takes its bonds s, s + S, s + 2S, ...
+    double *const hb = reinterpret_cast<double *>(hrec + HL);
+    auto stage = [&](int T0, int T1) {
+        for (int h = T0 + (int)threadIdx.x; h < T1; h += PB * S) {
+            const int32_t j = hidx[h];
+            const double4 r = A.rec_in[j];
+            if (MULTI) {
+                hrec[h - T0] = make_double4(r.x, r.y, r.z, 0.5 * r.w);
+                hb[h - T0] = 0.5 * (r.w * A.psets[A.pid[j]].bc);
+            } else {
+                hrec[h - T0] = pdx_rec_vbc(r, A.bc);
+            }
+        }
+    };
     const int sub = threadIdx.x % S;
     const int64_t p = p0 + threadIdx.x / S;
-    double bx = 0.0, by = 0.0, bz = 0.0;
-    int na = 0;
-    int c = 0;
-    double4 ri = make_double4(0.0, 0.0, 0.0, 0.0);
-    double rho = A.rho;
+    const int64_t q = p < A.n ? p : A.n - 1;  // lanes past the last point walk its slice's padding
+    const pdx_lane<S, PK> R = pdx_lane_of<S, PK>(A, p0);
+    const double4 ri = A.rec_in[q];
+    double bc = A.bc, epsc = A.epsc, epsc_lo = A.epsc_lo, rho = A.rho;
+    if (MULTI) {
+        const pdx_pset Pi = A.psets[A.pid[q]];
+        bc = Pi.bc;
+        epsc = Pi.epsc;
+        epsc_lo = Pi.epsc_lo;
+        rho = Pi.rho;
+    }
+    const double thr = fail_window<PK>(A, q, epsc_lo);
+    bb_sum f;
     if constexpr (!CAP) {
-        // the whole table fits: stage it once
-        for (int h = threadIdx.x; h < H; h += PDX_BLOCK * S) {
-            const int32_t j = hidx[h];
-            hrec[h] = MULTI ? A.rec_in[j] : pdx_rec_vbc(A.rec_in[j], A.bc);
-            if (MULTI) hpid[h] = A.pid[j];
-        }
+        stage(0, H);
         __syncthreads();
-        if (p >= A.n) return;  // all S lanes of the point together
-        c = A.cnt[p];
-        const int64_t b0 = pdx_bond0(A.slice_ptr, p);
-        uint16_t *const wbase = A.bw16 + b0;
-        const double *const Lbase = A.L + b0;
-        ri = A.rec_in[p];
-        double bc = A.bc, epsc = A.epsc, epsc_lo = A.epsc_lo, epsc_hi = A.epsc_hi;
-        if (MULTI) {
-            const pdx_pset Pi = A.psets[A.pid[p]];
-            bc = Pi.bc;
-            epsc = Pi.epsc;
-            epsc_lo = Pi.epsc_lo;
-            epsc_hi = Pi.epsc_hi;
-            rho = Pi.rho;
-        }
-        for (int t = sub; t < c; t += U * S) {
-            uint32_t wd[U];
-            double Ld[U], Sd[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                wd[u] = 0;
-                Ld[u] = 1.0;
-                Sd[u] = 1.0;
-                if (t + u * S < c) {
-                    const int64_t o = (int64_t)(t + u * S) * 64;
-                    wd[u] = wbase[o];
-                    Ld[u] = Lbase[o];
-                    if (SC) Sd[u] = A.scf[b0 + o];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                if (t + u * S >= c) continue;
-                const int slot = (int)(wd[u] & PDX_W16_SLOT);
-                if (MULTI)
-                    bb_bond64(ri, hrec[slot], wbase + (int64_t)(t + u * S) * 64, wd[u], Ld[u], Sd[u],
-                              (bc + A.psets[hpid[slot]].bc) / 2.0, epsc, epsc_lo, epsc_hi, bx, by, bz, na);
-                else
-                    bb_bond64_vbc(ri, hrec[slot], wbase + (int64_t)(t + u * S) * 64, wd[u], Ld[u],
-                                  pdx_rcp1(Ld[u]), Sd[u], epsc, epsc_lo, epsc_hi, bx, by, bz, na);
-            }
-        }
+        pdx_walk<U>(A, R, [&](const bond_data<PK> (&b)[U], int i) {
+            bb_group<U, F>(A, R, hidx, hrec, hb, 0, ri, bc, thr, epsc, b, i, f);
+        });
     } else {
-        // tiles of HL entries; all threads of the block take part in the staging barriers
-        const bool valid = p < A.n;
-        c = valid ? A.cnt[p] : 0;
-        const int64_t b0 = valid ? pdx_bond0(A.slice_ptr, p) : 0;
-        uint16_t *const wbase = A.bw16 + b0;
-        const double *const Lbase = A.L + b0;
-        if (valid) ri = A.rec_in[p];
-        double bc = A.bc, epsc = A.epsc, epsc_lo = A.epsc_lo, epsc_hi = A.epsc_hi;
-        if (MULTI && valid) {
-            const pdx_pset Pi = A.psets[A.pid[p]];
-            bc = Pi.bc;
-            epsc = Pi.epsc;
-            epsc_lo = Pi.epsc_lo;
-            epsc_hi = Pi.epsc_hi;
-            rho = Pi.rho;
-        }
-        int t = sub;
+        int i = 0;
         for (int T0 = 0; T0 < H; T0 += HL) {
             const int T1 = H < T0 + HL ? H : T0 + HL;
             if (T0 > 0) __syncthreads();  // the previous tile is consumed
-            for (int h = T0 + (int)threadIdx.x; h < T1; h += PDX_BLOCK * S) {
-                const int32_t j = hidx[h];
-                hrec[h - T0] = MULTI ? A.rec_in[j] : pdx_rec_vbc(A.rec_in[j], A.bc);
-                if (MULTI) hpid[h - T0] = A.pid[j];
-            }
+            stage(T0, T1);
             __syncthreads();
-            for (; t < c; t += U * S) {
-                uint32_t wd[U];
-                double Ld[U], Sd[U];
-#pragma unroll
-                for (int u = 0; u < U; u++) {
-                    wd[u] = 0;
-                    Ld[u] = 1.0;
-                    Sd[u] = 1.0;
-                    if (t + u * S < c) {
-                        const int64_t o = (int64_t)(t + u * S) * 64;
-                        wd[u] = wbase[o];
-                        Ld[u] = Lbase[o];
-                        if (SC) Sd[u] = A.scf[b0 + o];
-                    }
-                }
-                // the leading bonds of the group whose neighbours lie in the staged tile
-                int kk = 0;
-#pragma unroll
-                for (int u = 0; u < U; u++)
-                    if (kk == u && t + u * S < c && (int)(wd[u] & PDX_W16_SLOT) < T1) kk = u + 1;
-#pragma unroll
-                for (int u = 0; u < U; u++) {
-                    if (u >= kk) continue;
-                    const int ls = (int)(wd[u] & PDX_W16_SLOT) - T0;
-                    if (MULTI)
-                        bb_bond64(ri, hrec[ls], wbase + (int64_t)(t + u * S) * 64, wd[u], Ld[u], Sd[u],
-                                  (bc + A.psets[hpid[ls]].bc) / 2.0, epsc, epsc_lo, epsc_hi, bx, by, bz, na);
-                    else
-                        bb_bond64_vbc(ri, hrec[ls], wbase + (int64_t)(t + u * S) * 64, wd[u], Ld[u],
-                                      pdx_rcp1(Ld[u]), Sd[u], epsc, epsc_lo, epsc_hi, bx, by, bz, na);
-                }
-                if (kk < U) {
-                    t += kk * S;  // resume at the first bond past the tile (or the row's end)
-                    break;
-                }
-            }
-        }
-#pragma unroll
-        for (int o = 1; o < S; o <<= 1) {
-            bx += __shfl_xor(bx, o);
-            by += __shfl_xor(by, o);
-            bz += __shfl_xor(bz, o);
-            na += __shfl_xor(na, o);
-        }
-        if (!valid) return;
-    }
-    if constexpr (!CAP) {
-#pragma unroll
-        for (int o = 1; o < S; o <<= 1) {
-            bx += __shfl_xor(bx, o);
-            by += __shfl_xor(by, o);
-            bz += __shfl_xor(bz, o);
-            na += __shfl_xor(na, o);
+            i = pdx_walk_tile<2>(A, R, i, T1, [&](const bond_data<PK> &b, int ib) {
+                const bond_data<PK> one[1] = {b};
+                bb_group<1, F>(A, R, hidx, hrec, hb, T0, ri, bc, thr, epsc, one, ib, f);
+            });
         }
     }
+    pdx_fold(R, f.x);
+    pdx_fold(R, f.y);
+    pdx_fold(R, f.z);
+    pdx_fold(R, f.na);
+    if (p >= A.n) return;
+    const int c = A.cnt[p];
+    if (c == 0) f.x = f.y = f.z = 0.0;  // a point without bonds walked another row's padding
     if (sub == 0 && (A.flags & (PDX_F_STORE | PDX_F_FORCE_ONLY))) {
-        A.nact_out[p] = na;
-        A.dmg_out[p] = 1.0 - (double)na / (double)c;
+        A.nact_out[p] = f.na;
+        A.dmg_out[p] = 1.0 - (double)f.na / (double)c;
     }
-    static_assert(S == 4, "the tail takes four lanes per point");
-    const double b[3] = {bx, by, bz};
+    if (sub >= 4) return;  // the tail takes four lanes per point
+    const double b[3] = {f.x, f.y, f.z};
     point_tail4(A, p, ri, b, sub, rho);
 }
 
 // ----------------------------------------------------------------------------------------
 // J v of the bond-based material by central differences (jacobian_vector_product!,
 // newton_krylov.jl:504-532) in one kernel: the block stages its neighbour table at the
-// positions X + (u + e v), walks its bonds, stages the table again at X + (u - e v) and
-// walks them again, and combines the two force densities (times the volume) into
-// (F+ - F-) / (2 e); constrained rows take v.  The positions are formed as the reference
-// forms them (u +- e v, then X + u, two roundings each), the bond arithmetic is that of
-// k_bb_lds, so the result equals the two force evaluations of the step kernel bit for bit.
-// Bonds that break at the + state stay broken at the - state, as in two successive
-// calc_force_density! calls; n_active and damage keep the - state's values.
+// positions X + (u + e v) and X + (u - e v), evaluates every bond at both states, and combines
+// the two force densities (times the volume) into (F+ - F-) / (2 e); constrained rows take v.
+// The positions are formed as the reference forms them (u +- e v, then X + u, two roundings
+// each), the bond arithmetic and its order are those of k_bb_lds, so the result equals the two
+// force evaluations of the step kernel bit for bit.  Bonds that break at the + state are broken
+// at the - state, as in two successive calc_force_density! calls; n_active and damage keep the
+// - state's values.  ONE = true stages both tables at once (twice the LDS) and reads every bond
+// once; ONE = false stages the two states one after the other.
 // ----------------------------------------------------------------------------------------
 __device__ __forceinline__ double4 jv_position(const double4 X, const double *u, const double *v,
                                                int64_t j, double e)
@@ -640,15 +694,15 @@ __device__ __forceinline__ double4 jv_position(const double4 X, const double *u,
     return make_double4(X.x + u0, X.y + u1, X.z + u2, X.w);
 }
 
-template <int U, int S>
-__global__ __launch_bounds__(PDX_BLOCK * S) void k_bb_jv(pdx_step_args A, const double *u, const double *v,
-                                                          const double *un2, const double *parts, int np,
-                                                          double sc, const uint8_t *cmask, double *jv)
+template <int S, int PB, bool PK, bool ONE>
+__global__ __launch_bounds__(PB * S) void k_bb_jv(pdx_step_args A, const double *u, const double *v,
+                                                  const double *un2, const double *parts, int np,
+                                                  double sc, const uint8_t *cmask, double *jv)
 {
-    extern __shared__ double4 hrec[];
-    __shared__ double shs[PDX_BLOCK * S / 64];
+    extern __shared__ double4 hrec[];  // ONE: [0, H) + positions, [H, 2H) - positions
+    __shared__ double shs[PB * S / 64];
     const int64_t k = pdx_xcd_block();
-    const int64_t p0 = k * PDX_BLOCK;
+    const int64_t p0 = k * PB;
     if (p0 >= A.n) return;  // whole workgroup
     const double vn2 = pdx_block_sum_parts(parts, np, shs);
     const int64_t h0 = A.halo_ptr[k];
@@ -656,214 +710,163 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_bb_jv(pdx_step_args A, const 
     const int32_t *const hidx = A.halo + h0;
     const int sub = threadIdx.x % S;
     const int64_t p = p0 + threadIdx.x / S;
-    const bool valid = p < A.n;
+    const int64_t q = p < A.n ? p : A.n - 1;
     const double e = pdx_nk_perturbation_v(*un2, vn2, sc);
-    const int c = valid ? A.cnt[p] : 0;
-    const int64_t b0 = valid ? pdx_bond0(A.slice_ptr, p) : 0;
-    uint16_t *const wbase = A.bw16 + b0;
-    const double *const Lbase = A.L + b0;
-    // lane d < 3 keeps component d of F+ (the first pass); after the second, of F-
-    double fpd = 0.0, fmd = 0.0;
-    bool bad = false;
-    int na = 0;
-#pragma unroll 1
-    for (int pass = 0; pass < 2; pass++) {
-        const double es = pass == 0 ? e : -e;
-        if (pass == 1) __syncthreads();  // the + table is consumed
-        for (int h = threadIdx.x; h < H; h += PDX_BLOCK * S) {
+    const pdx_lane<S, PK> R = pdx_lane_of<S, PK>(A, p0);
+    const double4 Xi = A.Xr[q];
+    const double thr = fail_window<PK>(A, q, A.epsc_lo);
+    bb_sum fp, fm;
+    if constexpr (ONE) {
+        for (int h = threadIdx.x; h < H; h += PB * S) {
             const int32_t j = hidx[h];
-            hrec[h] = pdx_rec_vbc(jv_position(A.Xr[j], u, v, j, es), A.bc);
+            const double4 X = A.Xr[j];
+            hrec[h] = pdx_rec_vbc(jv_position(X, u, v, j, e), A.bc);
+            hrec[H + h] = pdx_rec_vbc(jv_position(X, u, v, j, -e), A.bc);
         }
         __syncthreads();
-        if (!valid) continue;  // all S lanes of the point together
-        const double4 ri = jv_position(A.Xr[p], u, v, p, es);
-        double bx = 0.0, by = 0.0, bz = 0.0;
-        int nap = 0;
-        for (int t = sub; t < c; t += U * S) {
-            uint32_t wd[U];
-            double Ld[U];
+        const double4 rp = jv_position(Xi, u, v, q, e), rm = jv_position(Xi, u, v, q, -e);
+        pdx_walk<2>(A, R, [&](const bond_data<PK> (&b)[2], int i) {
 #pragma unroll
-            for (int q = 0; q < U; q++) {
-                wd[q] = 0;
-                Ld[q] = 1.0;
-                if (t + q * S < c) {
-                    const int64_t o = (int64_t)(t + q * S) * 64;
-                    wd[q] = wbase[o];
-                    Ld[q] = Lbase[o];
-                }
+            for (int w = 0; w < 2; w++) {
+                if (i + w >= R.ng) continue;  // uniform
+                bond_data<PK> one[1] = {b[w]};
+                const int before = fp.na;
+                bb_group<1, 0>(A, R, hidx, hrec, nullptr, 0, rp, 0.0, thr, A.epsc, one, i + w, fp);
+                const bool gone = fp.na == before;
+                if constexpr (PK) one[0].w = gone ? (one[0].w | A.pk_mask) : one[0].w;
+                else one[0].w = gone ? (one[0].w & ~(uint32_t)PDX_W16_ACT) : one[0].w;
+                bb_group<1, 0>(A, R, hidx, hrec + H, nullptr, 0, rm, 0.0, thr, A.epsc, one, i + w, fm);
             }
-#pragma unroll
-            for (int q = 0; q < U; q++) {
-                if (t + q * S >= c) continue;
-                const int slot = (int)(wd[q] & PDX_W16_SLOT);
-                bb_bond64_vbc(ri, hrec[slot], wbase + (int64_t)(t + q * S) * 64, wd[q], Ld[q],
-                              pdx_rcp1(Ld[q]), 1.0, A.epsc, A.epsc_lo, A.epsc_hi, bx, by, bz, nap);
+        });
+    } else {
+#pragma unroll 1
+        for (int pass = 0; pass < 2; pass++) {
+            const double es = pass == 0 ? e : -e;
+            if (pass == 1) __syncthreads();  // the + table is consumed
+            for (int h = threadIdx.x; h < H; h += PB * S) {
+                const int32_t j = hidx[h];
+                hrec[h] = pdx_rec_vbc(jv_position(A.Xr[j], u, v, j, es), A.bc);
             }
+            __syncthreads();
+            const double4 ri = jv_position(Xi, u, v, q, es);
+            bb_sum f;
+            pdx_walk<2>(A, R, [&](const bond_data<PK> (&b)[2], int i) {
+                bb_group<2, 0>(A, R, hidx, hrec, nullptr, 0, ri, 0.0, thr, A.epsc, b, i, f);
+            });
+            if (pass == 0) fp = f;
+            else fm = f;
         }
-#pragma unroll
-        for (int o = 1; o < S; o <<= 1) {
-            bx += __shfl_xor(bx, o);
-            by += __shfl_xor(by, o);
-            bz += __shfl_xor(bz, o);
-            nap += __shfl_xor(nap, o);
-        }
-        bad = bad || isnan(bx) || isnan(by) || isnan(bz);
-        const double fd = sub == 0 ? bx : (sub == 1 ? by : bz);
-        if (pass == 0) fpd = fd;
-        else fmd = fd;
-        na = nap;
     }
-    if (!valid) return;
+    pdx_fold(R, fp.x);
+    pdx_fold(R, fp.y);
+    pdx_fold(R, fp.z);
+    pdx_fold(R, fm.x);
+    pdx_fold(R, fm.y);
+    pdx_fold(R, fm.z);
+    pdx_fold(R, fm.na);
+    if (p >= A.n) return;
+    const int c = A.cnt[p];
+    if (c == 0) fp = fm = bb_sum();
     if (sub == 0) {
-        A.nact_out[p] = na;
-        A.dmg_out[p] = 1.0 - (double)na / (double)c;
-        if (bad) atomicMin(A.flags_out, (unsigned long long)A.step);
+        A.nact_out[p] = fm.na;
+        A.dmg_out[p] = 1.0 - (double)fm.na / (double)c;
+        if (isnan(fp.x) || isnan(fp.y) || isnan(fp.z) || isnan(fm.x) || isnan(fm.y) || isnan(fm.z))
+            atomicMin(A.flags_out, (unsigned long long)A.step);
     }
     if (sub < 3) {
         const int64_t kk = 3 * p + sub;
-        const double w = A.Xr[p].w;
-        jv[kk] = cmask[kk] ? v[kk] : (fpd * w - fmd * w) / (2.0 * e);
-    }
-}
-
-// The same J v with both tables staged at once (twice the LDS of k_bb_jv, one block per CU
-// for a typical table): each bond's word and length are read once and the bond is
-// evaluated at both states.  A bond that breaks at the + state is evaluated broken at the
-// - state, as above.
-template <int U, int S>
-__global__ __launch_bounds__(PDX_BLOCK * S) void k_bb_jv1(pdx_step_args A, const double *u, const double *v,
-                                                           const double *un2, const double *parts, int np,
-                                                           double sc, const uint8_t *cmask, double *jv)
-{
-    extern __shared__ double4 hrec[];  // [0, H): + positions, [H, 2H): - positions
-    __shared__ double shs[PDX_BLOCK * S / 64];
-    const int64_t k = pdx_xcd_block();
-    const int64_t p0 = k * PDX_BLOCK;
-    if (p0 >= A.n) return;  // whole workgroup
-    const double vn2 = pdx_block_sum_parts(parts, np, shs);
-    const int64_t h0 = A.halo_ptr[k];
-    const int H = (int)(A.halo_ptr[k + 1] - h0);
-    const int32_t *const hidx = A.halo + h0;
-    const int sub = threadIdx.x % S;
-    const int64_t p = p0 + threadIdx.x / S;
-    const bool valid = p < A.n;  // the same for the S lanes of a point
-    const double e = pdx_nk_perturbation_v(*un2, vn2, sc);
-    for (int h = threadIdx.x; h < H; h += PDX_BLOCK * S) {
-        const int32_t j = hidx[h];
-        const double4 X = A.Xr[j];
-        hrec[h] = pdx_rec_vbc(jv_position(X, u, v, j, e), A.bc);
-        hrec[H + h] = pdx_rec_vbc(jv_position(X, u, v, j, -e), A.bc);
-    }
-    __syncthreads();
-    if (valid) {
-        const int c = A.cnt[p];
-        const int64_t b0 = pdx_bond0(A.slice_ptr, p);
-        uint16_t *const wbase = A.bw16 + b0;
-        const double *const Lbase = A.L + b0;
-        const double4 Xi = A.Xr[p];
-        const double4 rp = jv_position(Xi, u, v, p, e), rm = jv_position(Xi, u, v, p, -e);
-        double px = 0.0, py = 0.0, pz = 0.0, mx = 0.0, my = 0.0, mz = 0.0;
-        int nap = 0, nam = 0;
-        for (int t = sub; t < c; t += U * S) {
-            uint32_t wd[U];
-            double Ld[U];
-#pragma unroll
-            for (int q = 0; q < U; q++) {
-                wd[q] = 0;
-                Ld[q] = 1.0;
-                if (t + q * S < c) {
-                    const int64_t o = (int64_t)(t + q * S) * 64;
-                    wd[q] = wbase[o];
-                    Ld[q] = Lbase[o];
-                }
-            }
-#pragma unroll
-            for (int q = 0; q < U; q++) {
-                if (t + q * S >= c) continue;
-                const int slot = (int)(wd[q] & PDX_W16_SLOT);
-                uint16_t *const wp = wbase + (int64_t)(t + q * S) * 64;
-                const int before = nap;
-                const double rL = pdx_rcp1(Ld[q]);
-                bb_bond64_vbc(rp, hrec[slot], wp, wd[q], Ld[q], rL, 1.0, A.epsc, A.epsc_lo, A.epsc_hi,
-                              px, py, pz, nap);
-                const uint32_t wm = nap != before ? wd[q] : (wd[q] & ~(uint32_t)PDX_W16_ACT);
-                bb_bond64_vbc(rm, hrec[H + slot], wp, wm, Ld[q], rL, 1.0, A.epsc, A.epsc_lo, A.epsc_hi,
-                              mx, my, mz, nam);
-            }
-        }
-#pragma unroll
-        for (int o = 1; o < S; o <<= 1) {
-            px += __shfl_xor(px, o);
-            py += __shfl_xor(py, o);
-            pz += __shfl_xor(pz, o);
-            mx += __shfl_xor(mx, o);
-            my += __shfl_xor(my, o);
-            mz += __shfl_xor(mz, o);
-            nam += __shfl_xor(nam, o);
-        }
-        if (sub == 0) {
-            A.nact_out[p] = nam;
-            A.dmg_out[p] = 1.0 - (double)nam / (double)c;
-            if (isnan(px) || isnan(py) || isnan(pz) || isnan(mx) || isnan(my) || isnan(mz))
-                atomicMin(A.flags_out, (unsigned long long)A.step);
-        }
-        if (sub < 3) {
-            const int64_t kk = 3 * p + sub;
-            const double a = sub == 0 ? px : (sub == 1 ? py : pz);
-            const double b = sub == 0 ? mx : (sub == 1 ? my : mz);
-            jv[kk] = cmask[kk] ? v[kk] : (a * Xi.w - b * Xi.w) / (2.0 * e);
-        }
+        const double a = sub == 0 ? fp.x : (sub == 1 ? fp.y : fp.z);
+        const double b = sub == 0 ? fm.x : (sub == 1 ? fm.y : fm.z);
+        jv[kk] = cmask[kk] ? v[kk] : (a * Xi.w - b * Xi.w) / (2.0 * e);
     }
 }
 
 // ----------------------------------------------------------------------------------------
 // Mixed-precision BB step on the LDS-staged layout.  The stretch is formed without
 // cancellation from the reference bond vector D = X_j - X_i and the displacement difference
-// U = u_j - u_i (u = x - X of the positions the step receives):  l^2 - L^2 = 2 D.U + U.U,  eps = (l^2 - L^2) / (L (l + L)),  L = |D|,
-// l = |D + U|.  Both are staged per block in FP32 relative to the block's first point
-// (subtracted in FP64 first), so their rounding is relative to the block's extent, not to
-// the absolute coordinates, and a rigid motion of the body costs no precision.  Every
-// bond operation is FP32; the per-point sums are FP64 (each FP32 term is added with FP64
-// rounding, the effect of a compensated FP32 sum).  Per bond only the 16-bit bond word is
-// read: L comes from D.  The Velocity Verlet tail stays FP64.
+// U = u_j - u_i (u = x - X of the positions the step receives):  l^2 - L^2 = 2 D.U + U.U,
+// eps = (l^2 - L^2) / (L (l + L)),  L = |D|, l = |D + U|.  Both are staged per block in FP32
+// relative to a point of the block's run of 256 (subtracted in FP64 first), so their rounding is
+// relative to the run's extent, not to the absolute coordinates, and a rigid motion of the body
+// costs no precision.  Every bond operation is FP32; a lane's four bonds of a row-group quadruple
+// are summed in FP32 and then once into the FP64 sums (pdx_rows deals the bonds to the lanes so
+// that these four are the same bonds with 4, 8 or 16 lanes per point, so the FP32 results do not
+// depend on the block size).  Per bond only the 16-bit
+// bond word is read: L comes from D.  The Velocity Verlet tail stays FP64.
 // ----------------------------------------------------------------------------------------
-template <int U, int S, int F>
-__global__ __launch_bounds__(PDX_BLOCK * S) void k_bb_lds_mx(pdx_step_args A)
+
+// the lane's bond words, four row groups at a time, the next four in flight
+template <int S, class GROUP>
+__device__ __forceinline__ void pdx_walk4_mx(const pdx_step_args &A, const pdx_lane<S, false> &R, GROUP &&group)
+{
+    if (R.ng == 0) return;
+    uint32_t c[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) c[u] = A.bw16[R.at(u)];
+    for (int i = 0; i < R.ng; i += 4) {
+        uint32_t nx[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) nx[u] = A.bw16[R.at(i + 4 + u)];
+        group(c, i);
+#pragma unroll
+        for (int u = 0; u < 4; u++) c[u] = nx[u];
+    }
+}
+
+__device__ __forceinline__ void mx_stage_xu(const pdx_step_args &A, int64_t j, double4 O,
+                                            double uo0, double uo1, double uo2, float4 &a, float4 &b)
+{
+    const double4 X = A.Xr[j], x = A.rec_in[j];
+    a = make_float4((float)(X.x - O.x), (float)(X.y - O.y), (float)(X.z - O.z), (float)X.w);
+    b = make_float4((float)((x.x - X.x) - uo0), (float)((x.y - X.y) - uo1), (float)((x.z - X.z) - uo2), 0.f);
+}
+
+// FP32 stretches within 1e-4 of eps_c are decided on the FP64 stretch, so that a bond breaks in
+// the step in which the FP64 step would break it (the FP32 stretch is good to ~1e-6 relative)
+__device__ __forceinline__ bool mx_breaks(const pdx_step_args &A, const int32_t *hidx, uint32_t w, int64_t slot,
+                                          double4 ri, float eps, float win_hi, double epsc)
+{
+    if (eps > win_hi) return true;
+    const double L = A.L[slot];
+    const double4 xj = A.rec_in[hidx[w & PDX_W16_SLOT]];
+    const double dx = xj.x - ri.x, dy = xj.y - ri.y, dz = xj.z - ri.z;
+    double rl;
+    const double l = pdx_sqrt_rsq((dx * dx + dy * dy) + dz * dz, rl);
+    return ((l - L) / L) > epsc;
+}
+
+template <int S, int F, int PB>
+__global__ __launch_bounds__(PB * S) void k_bb_lds_mx(pdx_step_args A)
 {
     constexpr bool MULTI = (F & PDX_FEAT_MULTI) != 0;
     constexpr bool SC = (F & PDX_FEAT_SC) != 0;
     constexpr bool CAP = (F & PDX_FEAT_CAP) != 0;
     extern __shared__ float4 hmx[];  // [2 H]: (X - O, V), (u - u_O, 0)
     const int64_t k = pdx_xcd_block();
-    const int64_t p0 = k * PDX_BLOCK;
+    const int64_t p0 = k * PB;
     if (p0 >= A.n) return;  // whole workgroup
     const int64_t h0 = A.halo_ptr[k];
     const int H = (int)(A.halo_ptr[k + 1] - h0);
     // displacements are taken as x - X of the positions the step receives, so that the
     // perturbed positions of the Newton-Krylov products work like the Verlet state
-    const double4 O = A.Xr[p0], xo = A.rec_in[p0];
+    const int64_t po = p0 & ~(int64_t)(PDX_BLOCK - 1);
+    const double4 O = A.Xr[po], xo = A.rec_in[po];
     const double uo0 = xo.x - O.x, uo1 = xo.y - O.y, uo2 = xo.z - O.z;
     const int HL = CAP ? pdx_lds_entries(A.halo_max, A.lds_budget, 32 + (MULTI ? 1 : 0)) : A.halo_max;
     const int Hs = H < HL ? H : HL;
     const int32_t *const hidx = A.halo + h0;
     uint8_t *const hpid = reinterpret_cast<uint8_t *>(hmx + 2 * HL);
-    for (int h = threadIdx.x; h < Hs; h += PDX_BLOCK * S) {
+    for (int h = threadIdx.x; h < Hs; h += PB * S) {
         const int64_t j = hidx[h];
         if (MULTI) hpid[h] = A.pid[j];
-        const double4 X = A.Xr[j], x = A.rec_in[j];
-        hmx[2 * h] = make_float4((float)(X.x - O.x), (float)(X.y - O.y), (float)(X.z - O.z), (float)X.w);
-        hmx[2 * h + 1] = make_float4((float)((x.x - X.x) - uo0), (float)((x.y - X.y) - uo1),
-                                     (float)((x.z - X.z) - uo2), 0.f);
+        mx_stage_xu(A, j, O, uo0, uo1, uo2, hmx[2 * h], hmx[2 * h + 1]);
     }
-    __syncthreads();
     const int sub = threadIdx.x % S;
     const int64_t p = p0 + threadIdx.x / S;
-    if (p >= A.n) return;  // all S lanes of the point together
-    const int c = A.cnt[p];
-    const int64_t b0 = pdx_bond0(A.slice_ptr, p);
-    uint16_t *const wbase = A.bw16 + b0;
-    const double4 ri = A.rec_in[p];
-    const double4 Xi = A.Xr[p];
+    const int64_t q = p < A.n ? p : A.n - 1;
+    const pdx_lane<S, false> R = pdx_lane_of<S, false>(A, p0);
+    const double4 ri = A.rec_in[q];
+    const double4 Xi = A.Xr[q];
     const float xi = (float)(Xi.x - O.x), yi = (float)(Xi.y - O.y), zi = (float)(Xi.z - O.z);
     const float ui = (float)((ri.x - Xi.x) - uo0), vi = (float)((ri.y - Xi.y) - uo1),
                 wi = (float)((ri.z - Xi.z) - uo2);
@@ -872,29 +875,21 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_bb_lds_mx(pdx_step_args A)
     float bcf = (float)A.bc, epscf = (float)A.epsc;
     double rho = A.rho, epsc = A.epsc;
     if (MULTI) {
-        const pdx_pset Pi = A.psets[A.pid[p]];
+        const pdx_pset Pi = A.psets[A.pid[q]];
         bcf = (float)Pi.bc;
         epscf = (float)Pi.epsc;
         epsc = Pi.epsc;
         rho = Pi.rho;
     }
-    // FP32 stretches within 1e-4 of eps_c are decided on the FP64 stretch, so that a bond
-    // breaks in the step in which the FP64 step would break it (the FP32 stretch is good to
-    // ~1e-6 relative)
     const float win_lo = epscf * 0.9999f, win_hi = epscf * 1.0001f;
-    for (int t = sub; t < c; t += U * S) {
-        uint32_t wd[U];
-        float sc[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            wd[u] = (t + u * S < c) ? wbase[(int64_t)(t + u * S) * 64] : 0u;
-            sc[u] = (SC && t + u * S < c) ? A.scf32[b0 + (int64_t)(t + u * S) * 64] : 1.f;
-        }
+    __syncthreads();
+    pdx_walk4_mx(A, R, [&](const uint32_t (&wd)[4], int i) {
         // the group's bond forces are summed in FP32 (fused), then once into the FP64 sums
         float gx = 0.f, gy = 0.f, gz = 0.f;
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            if (t + u * S >= c) continue;
+        for (int u = 0; u < 4; u++) {
+            if (i + u >= R.ng) continue;  // uniform
+            const int64_t o = R.at(i + u);
             const int slot = (int)(wd[u] & PDX_W16_SLOT);
             float4 a, b;
             int32_t jg = 0;
@@ -903,10 +898,7 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_bb_lds_mx(pdx_step_args A)
                 b = hmx[2 * slot + 1];
             } else {  // past the staged entries: the same values from global memory
                 jg = hidx[slot];
-                const double4 X = A.Xr[jg], x = A.rec_in[jg];
-                a = make_float4((float)(X.x - O.x), (float)(X.y - O.y), (float)(X.z - O.z), (float)X.w);
-                b = make_float4((float)((x.x - X.x) - uo0), (float)((x.y - X.y) - uo1),
-                                (float)((x.z - X.z) - uo2), 0.f);
+                mx_stage_xu(A, jg, O, uo0, uo1, uo2, a, b);
             }
             const float Dx = a.x - xi, Dy = a.y - yi, Dz = a.z - zi;
             const float Ux = b.x - ui, Uy = b.y - vi, Uz = b.z - wi;
@@ -918,23 +910,12 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_bb_lds_mx(pdx_step_args A)
             const float l = __builtin_amdgcn_sqrtf(L2 + num);
             const float eps = num * __builtin_amdgcn_rcpf(Lb * (l + Lb));
             bool act = (wd[u] & PDX_W16_ACT) != 0;
-            if (act && (wd[u] & PDX_W16_FP) && eps > win_lo) {
-                bool brk = eps > win_hi;
-                if (!brk) {
-                    const double Lb = A.L[b0 + (int64_t)(t + u * S) * 64];
-                    const double4 xj = A.rec_in[hidx[slot]];
-                    const double dx = xj.x - ri.x, dy = xj.y - ri.y, dz = xj.z - ri.z;
-                    double rl;
-                    const double l64 = pdx_sqrt_rsq((dx * dx + dy * dy) + dz * dz, rl);
-                    brk = ((l64 - Lb) / Lb) > epsc;
-                }
-                if (brk) {
-                    act = false;
-                    wbase[(int64_t)(t + u * S) * 64] = (uint16_t)(wd[u] & ~PDX_W16_ACT);
-                }
+            if (act && (wd[u] & PDX_W16_FP) && eps > win_lo && mx_breaks(A, hidx, wd[u], o, ri, eps, win_hi, epsc)) {
+                act = false;
+                A.bw16[o] = (uint16_t)(wd[u] & ~PDX_W16_ACT);
             }
             const float bcb = MULTI ? (bcf + (float)A.psets[(!CAP || slot < HL) ? hpid[slot] : A.pid[jg]].bc) * 0.5f : bcf;
-            const float sf = act ? (((SC ? sc[u] * bcb : bcb) * eps) * a.w) * __builtin_amdgcn_rcpf(l) : 0.f;
+            const float sf = act ? (((SC ? A.scf32[o] * bcb : bcb) * eps) * a.w) * __builtin_amdgcn_rcpf(l) : 0.f;
             gx = __builtin_fmaf(sf, Dx + Ux, gx);
             gy = __builtin_fmaf(sf, Dy + Uy, gy);
             gz = __builtin_fmaf(sf, Dz + Uz, gz);
@@ -943,19 +924,19 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_bb_lds_mx(pdx_step_args A)
         bx += (double)gx;
         by += (double)gy;
         bz += (double)gz;
-    }
-#pragma unroll
-    for (int o = 1; o < S; o <<= 1) {
-        bx += __shfl_xor(bx, o);
-        by += __shfl_xor(by, o);
-        bz += __shfl_xor(bz, o);
-        na += __shfl_xor(na, o);
-    }
+    });
+    pdx_fold(R, bx);
+    pdx_fold(R, by);
+    pdx_fold(R, bz);
+    pdx_fold(R, na);
+    if (p >= A.n) return;
+    const int c = A.cnt[p];
+    if (c == 0) bx = by = bz = 0.0;
     if (sub == 0 && (A.flags & (PDX_F_STORE | PDX_F_FORCE_ONLY))) {
         A.nact_out[p] = na;
         A.dmg_out[p] = 1.0 - (double)na / (double)c;
     }
-    static_assert(S == 4, "the tail takes four lanes per point");
+    if (sub >= 4) return;  // the tail takes four lanes per point
     const double bb[3] = {bx, by, bz};
     point_tail4(A, p, ri, bb, sub, rho);
 }
@@ -971,46 +952,32 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_bb_lds_mx(pdx_step_args A)
 // carries no force sums.  Failure: FP32 stretches within 1e-4 of eps_c are decided on the
 // FP64 stretch.
 // ----------------------------------------------------------------------------------------
-__device__ __forceinline__ void mx_stage_xu(const pdx_step_args &A, int64_t j, double4 O,
-                                            double uo0, double uo1, double uo2, float4 &a, float4 &b)
-{
-    const double4 X = A.Xr[j], x = A.rec_in[j];
-    a = make_float4((float)(X.x - O.x), (float)(X.y - O.y), (float)(X.z - O.z), (float)X.w);
-    b = make_float4((float)((x.x - X.x) - uo0), (float)((x.y - X.y) - uo1), (float)((x.z - X.z) - uo2), 0.f);
-}
-
-template <int U, int S, int F>
-__global__ __launch_bounds__(PDX_BLOCK * S) void k_osb_lds1_mx(pdx_step_args A)
+template <int S, int F, int PB>
+__global__ __launch_bounds__(PB * S) void k_osb_lds1_mx(pdx_step_args A)
 {
     static_assert((F & PDX_FEAT_MULTI) == 0, "mixed OSB takes one parameter set");
     constexpr bool SC = (F & PDX_FEAT_SC) != 0;
     constexpr bool CAP = (F & PDX_FEAT_CAP) != 0;
     extern __shared__ float4 hmx[];
     const int64_t k = pdx_xcd_block();
-    const int64_t p0 = k * PDX_BLOCK;
+    const int64_t p0 = k * PB;
     if (p0 >= A.n) return;  // whole workgroup
     const int64_t h0 = A.halo_ptr[k];
     const int H = (int)(A.halo_ptr[k + 1] - h0);
-    const double4 O = A.Xr[p0], xo = A.rec_in[p0];
+    const int64_t po = p0 & ~(int64_t)(PDX_BLOCK - 1);
+    const double4 O = A.Xr[po], xo = A.rec_in[po];
     const double uo0 = xo.x - O.x, uo1 = xo.y - O.y, uo2 = xo.z - O.z;
     const int HL = CAP ? pdx_lds_entries(A.halo_max, A.lds_budget, 32) : A.halo_max;
     const int Hs = H < HL ? H : HL;
     const int32_t *const hidx = A.halo + h0;
-    for (int h = threadIdx.x; h < Hs; h += PDX_BLOCK * S) {
-        float4 a, b;
-        mx_stage_xu(A, hidx[h], O, uo0, uo1, uo2, a, b);
-        hmx[2 * h] = a;
-        hmx[2 * h + 1] = b;
-    }
-    __syncthreads();
+    for (int h = threadIdx.x; h < Hs; h += PB * S)
+        mx_stage_xu(A, hidx[h], O, uo0, uo1, uo2, hmx[2 * h], hmx[2 * h + 1]);
     const int sub = threadIdx.x % S;
     const int64_t p = p0 + threadIdx.x / S;
-    if (p >= A.n) return;  // all S lanes of the point together
-    const int c = A.cnt[p];
-    const int64_t b0 = pdx_bond0(A.slice_ptr, p);
-    uint16_t *const wbase = A.bw16 + b0;
-    const double4 ri = A.rec_in[p];
-    const double4 Xi = A.Xr[p];
+    const int64_t q = p < A.n ? p : A.n - 1;
+    const pdx_lane<S, false> R = pdx_lane_of<S, false>(A, p0);
+    const double4 ri = A.rec_in[q];
+    const double4 Xi = A.Xr[q];
     const float xi = (float)(Xi.x - O.x), yi = (float)(Xi.y - O.y), zi = (float)(Xi.z - O.z);
     const float ui = (float)((ri.x - Xi.x) - uo0), vi = (float)((ri.y - Xi.y) - uo1),
                 wi = (float)((ri.z - Xi.z) - uo2);
@@ -1019,19 +986,14 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_osb_lds1_mx(pdx_step_args A)
     const double epsc = A.epsc;
     const float epscf = (float)epsc, deltaf = (float)A.delta;
     const float win_lo = epscf * 0.9999f, win_hi = epscf * 1.0001f;
-    for (int t = sub; t < c; t += U * S) {
-        uint32_t wd[U];
-        float sc[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            wd[u] = (t + u * S < c) ? wbase[(int64_t)(t + u * S) * 64] : 0u;
-            sc[u] = (SC && t + u * S < c) ? A.scf32[b0 + (int64_t)(t + u * S) * 64] : 1.f;
-        }
+    __syncthreads();
+    pdx_walk4_mx(A, R, [&](const uint32_t (&wd)[4], int i) {
         // the group's sums in FP32 (fused), then once into the FP64 sums
         float gv = 0.f, gs = 0.f;
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            if (t + u * S >= c) continue;
+        for (int u = 0; u < 4; u++) {
+            if (i + u >= R.ng) continue;  // uniform
+            const int64_t o = R.at(i + u);
             const int slot = (int)(wd[u] & PDX_W16_SLOT);
             float4 a, b;
             if (!CAP || slot < HL) {
@@ -1052,24 +1014,13 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_osb_lds1_mx(pdx_step_args A)
             const float e = num * __builtin_amdgcn_rcpf(l + Lb);
             const float eps = e * rL;
             bool act = (wd[u] & PDX_W16_ACT) != 0;
-            if (act && (wd[u] & PDX_W16_FP) && eps > win_lo) {
-                bool brk = eps > win_hi;
-                if (!brk) {
-                    const double L64 = A.L[b0 + (int64_t)(t + u * S) * 64];
-                    const double4 xj = A.rec_in[hidx[slot]];
-                    const double dx = xj.x - ri.x, dy = xj.y - ri.y, dz = xj.z - ri.z;
-                    double rl;
-                    const double l64 = pdx_sqrt_rsq((dx * dx + dy * dy) + dz * dz, rl);
-                    brk = ((l64 - L64) / L64) > epsc;
-                }
-                if (brk) {
-                    act = false;
-                    wbase[(int64_t)(t + u * S) * 64] = (uint16_t)(wd[u] & ~PDX_W16_ACT);
-                }
+            if (act && (wd[u] & PDX_W16_FP) && eps > win_lo && mx_breaks(A, hidx, wd[u], o, ri, eps, win_hi, epsc)) {
+                act = false;
+                A.bw16[o] = (uint16_t)(wd[u] & ~PDX_W16_ACT);
             }
             if (act) {
                 float w = deltaf * rL;  // linear_kernel(delta, L)
-                if (SC) w *= sc[u];
+                if (SC) w *= A.scf32[o];
                 const float wVL = (w * a.w) * Lb;
                 gv = __builtin_fmaf(wVL, Lb, gv);
                 gs = __builtin_fmaf(wVL, e, gs);
@@ -1078,14 +1029,11 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_osb_lds1_mx(pdx_step_args A)
         }
         wvol += (double)gv;
         Ssum += (double)gs;
-    }
-#pragma unroll
-    for (int o = 1; o < S; o <<= 1) {
-        wvol += __shfl_xor(wvol, o);
-        Ssum += __shfl_xor(Ssum, o);
-        na += __shfl_xor(na, o);
-    }
-    if (sub != 0) return;
+    });
+    pdx_fold(R, wvol);
+    pdx_fold(R, Ssum);
+    pdx_fold(R, na);
+    if (p >= A.n || sub != 0) return;
     double c1 = 0.0, c2 = 0.0;
     if (wvol != 0.0) {
         const double dil = (3.0 / wvol) * Ssum;
@@ -1095,30 +1043,31 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_osb_lds1_mx(pdx_step_args A)
     reinterpret_cast<double2 *>(A.pstate)[p] = make_double2(c1, c2);
     if (A.flags & (PDX_F_STORE | PDX_F_FORCE_ONLY)) {
         A.nact_out[p] = na;
-        A.dmg_out[p] = 1.0 - (double)na / (double)c;
+        A.dmg_out[p] = 1.0 - (double)na / (double)A.cnt[p];
     }
 }
 
-template <int U, int S, int F>
-__global__ __launch_bounds__(PDX_BLOCK * S) void k_osb_lds2_mx(pdx_step_args A)
+template <int S, int F, int PB>
+__global__ __launch_bounds__(PB * S) void k_osb_lds2_mx(pdx_step_args A)
 {
     static_assert((F & PDX_FEAT_MULTI) == 0, "mixed OSB takes one parameter set");
     constexpr bool SC = (F & PDX_FEAT_SC) != 0;
     constexpr bool CAP = (F & PDX_FEAT_CAP) != 0;
     extern __shared__ float4 hmx[];
     const int64_t k = pdx_xcd_block();
-    const int64_t p0 = k * PDX_BLOCK;
+    const int64_t p0 = k * PB;
     if (p0 >= A.n) return;  // whole workgroup
     const int64_t h0 = A.halo_ptr[k];
     const int H = (int)(A.halo_ptr[k + 1] - h0);
-    const double4 O = A.Xr[p0], xo = A.rec_in[p0];
+    const int64_t po = p0 & ~(int64_t)(PDX_BLOCK - 1);
+    const double4 O = A.Xr[po], xo = A.rec_in[po];
     const double uo0 = xo.x - O.x, uo1 = xo.y - O.y, uo2 = xo.z - O.z;
     const int HL = CAP ? pdx_lds_entries(A.halo_max, A.lds_budget, 36) : A.halo_max;
     const int Hs = H < HL ? H : HL;
     const int32_t *const hidx = A.halo + h0;
     const double2 *const cst = reinterpret_cast<const double2 *>(A.pstate);
     float *const hc2 = reinterpret_cast<float *>(hmx + 2 * HL);
-    for (int h = threadIdx.x; h < Hs; h += PDX_BLOCK * S) {
+    for (int h = threadIdx.x; h < Hs; h += PB * S) {
         const int64_t j = hidx[h];
         float4 a, b;
         mx_stage_xu(A, j, O, uo0, uo1, uo2, a, b);
@@ -1129,35 +1078,26 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_osb_lds2_mx(pdx_step_args A)
         hmx[2 * h + 1] = b;
         hc2[h] = (float)(cj.y * Vj);
     }
-    __syncthreads();
     const int sub = threadIdx.x % S;
     const int64_t p = p0 + threadIdx.x / S;
-    if (p >= A.n) return;  // all S lanes of the point together
-    const int c = A.cnt[p];
-    const int64_t b0 = pdx_bond0(A.slice_ptr, p);
-    const uint16_t *const wbase = A.bw16 + b0;
-    const double4 ri = A.rec_in[p];
-    const double4 Xi = A.Xr[p];
+    const int64_t q = p < A.n ? p : A.n - 1;
+    const pdx_lane<S, false> R = pdx_lane_of<S, false>(A, p0);
+    const double4 ri = A.rec_in[q];
+    const double4 Xi = A.Xr[q];
     const float xi = (float)(Xi.x - O.x), yi = (float)(Xi.y - O.y), zi = (float)(Xi.z - O.z);
     const float ui = (float)((ri.x - Xi.x) - uo0), vi = (float)((ri.y - Xi.y) - uo1),
                 wi = (float)((ri.z - Xi.z) - uo2);
     double bx = 0.0, by = 0.0, bz = 0.0;
-    const double2 ci = cst[p];
+    const double2 ci = cst[q];
     const float c1i = (float)ci.x, c2i = (float)ci.y;
     const float deltaf = (float)A.delta;
-    for (int t = sub; t < c; t += U * S) {
-        uint32_t wd[U];
-        float sc[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            wd[u] = (t + u * S < c) ? wbase[(int64_t)(t + u * S) * 64] : 0u;
-            sc[u] = (SC && t + u * S < c) ? A.scf32[b0 + (int64_t)(t + u * S) * 64] : 1.f;
-        }
+    __syncthreads();
+    pdx_walk4_mx(A, R, [&](const uint32_t (&wd)[4], int i) {
         // the group's bond forces are summed in FP32 (fused), then once into the FP64 sums
         float gx = 0.f, gy = 0.f, gz = 0.f;
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            if (t + u * S >= c) continue;
+        for (int u = 0; u < 4; u++) {
+            if (i + u >= R.ng) continue;  // uniform
             if (!(wd[u] & PDX_W16_ACT)) continue;  // one set: both copies of the bond agree
             const int slot = (int)(wd[u] & PDX_W16_SLOT);
             float4 a, b;
@@ -1183,7 +1123,7 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_osb_lds2_mx(pdx_step_args A)
             const float l = __builtin_amdgcn_sqrtf(L2 + num);
             const float e = num * __builtin_amdgcn_rcpf(l + Lb);
             float w = deltaf * __builtin_amdgcn_rcpf(Lb);
-            if (SC) w *= sc[u];
+            if (SC) w *= A.scf32[R.at(i + u)];
             // own term (c2_i L + c1_i e) V_j plus reverse term (c2 V)_j L + (c1 V)_j e
             const float fi = __builtin_fmaf(c1i, e, c2i * Lb) * a.w;
             const float fj = __builtin_fmaf(b.w, e, c2Vj * Lb);
@@ -1195,14 +1135,11 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_osb_lds2_mx(pdx_step_args A)
         bx += (double)gx;
         by += (double)gy;
         bz += (double)gz;
-    }
-#pragma unroll
-    for (int o = 1; o < S; o <<= 1) {
-        bx += __shfl_xor(bx, o);
-        by += __shfl_xor(by, o);
-        bz += __shfl_xor(bz, o);
-    }
-    static_assert(S == 4, "the tail takes four lanes per point");
+    });
+    pdx_fold(R, bx);
+    pdx_fold(R, by);
+    pdx_fold(R, bz);
+    if (p >= A.n || sub >= 4) return;  // the tail takes four lanes per point
     const double bb[3] = {bx, by, bz};
     point_tail4(A, p, ri, bb, sub, A.rho);
 }
@@ -1217,7 +1154,7 @@ __global__ __launch_bounds__(PDX_BLOCK) void k_osb_pass1(pdx_step_args A)
     const int64_t p = pdx_thread_point();
     if (p >= A.n) return;
     const int c = A.cnt[p];
-    const int64_t b0 = pdx_bond0(A.slice_ptr, p);
+    const int64_t b0 = A.rows.row(p);
     const double4 ri = A.rec_in[p];
     double wvol = 0.0, S = 0.0;
     int na = 0;
@@ -1260,7 +1197,7 @@ __global__ __launch_bounds__(PDX_BLOCK) void k_osb_pass2(pdx_step_args A)
     const int64_t p = pdx_thread_point();
     if (p >= A.n) return;
     const int c = A.cnt[p];
-    const int64_t b0 = pdx_bond0(A.slice_ptr, p);
+    const int64_t b0 = A.rows.row(p);
     const double4 ri = A.rec_in[p];
     const double2 ci = reinterpret_cast<const double2 *>(A.pstate)[p];
     double bx = 0.0, by = 0.0, bz = 0.0;
@@ -1290,390 +1227,273 @@ __global__ __launch_bounds__(PDX_BLOCK) void k_osb_pass2(pdx_step_args A)
     point_tail(A, p, ri, b, T, A.rho);
 }
 
-// OSB on the LDS-staged layout (four lanes per point, as the BB step).  Bond states live
-// in the 16-bit words.  With one parameter set the bond force of i-j,
+// OSB on the LDS-staged layout.  With one parameter set the bond force of i-j,
 //   (w / l) [(c2_i L + c1_i e) + (c2_j L + c1_j e)] V_j dx,
 // splits into an own part, c2_i A_i + c1_i B_i with A_i = sum (w/l) V_j L dx and
 // B_i = sum (w/l) V_j e dx, which pass 1 sums while it forms c1_i, c2_i, and a reverse
 // part, (w/l) [(c2 V)_j L + (c1 V)_j e] dx, which pass 2 gathers.  Pass 1 stages x|V
 // (32 B per neighbour-table entry) and stores (c1 V, c2 V) and the own part per point;
-// pass 2 stages x and (c1 V, c2 V) (40 B per entry), so a 2 M-point lattice's longest
-// table fits the LDS budget.  With several sets c1, c2 depend on the bond: pass 1 stores
-// (wvol, dilatation) and pass 2 stages x|V and those (48 B + the set index per entry).
-template <int S, int F>
-__global__ __launch_bounds__(PDX_BLOCK * S) void k_osb_lds1(pdx_step_args A)
+// pass 2 stages x and (c1 V, c2 V) (40 B per entry).  With the linear influence function
+// omega = delta / L the records carry delta V_j and delta (c1 V, c2 V)_j: the weighted volume is
+// sum (delta V_j) L and every other weight is one of the staged values times 1/(l L).
+//
+// With several sets c1, c2 depend on the bond (averaged G, K; force_density_point! with a
+// ParameterHandler, ordinary_state_based.jl:151-174).  Pass 1 leaves h = 1 / (2 wvol) and h times
+// the dilatation d per point; the bond's c2 L + c1 e of an end is then
+// (h d) (3 K - 5 G) L + h (15 G) e with G, K the sums of both ends' moduli, so pass 2 stages
+// x|V, (h, h d)_j and (15 G_j, 3 K_j - 5 G_j) (64 B) and divides nothing per bond.  Both ends'
+// copies of a bond fail against their own eps_c; the owner tracks the other copy in RACT.
+template <int S, int F, int PB, bool PK>
+__global__ __launch_bounds__(PB * S) void k_osb_lds1(pdx_step_args A)
 {
     constexpr bool MULTI = (F & PDX_FEAT_MULTI) != 0;
-    constexpr bool SPLIT = !MULTI;
+    constexpr bool KERN = (F & PDX_FEAT_KERN) != 0;
     constexpr bool SC = (F & PDX_FEAT_SC) != 0;
     constexpr bool CAP = (F & PDX_FEAT_CAP) != 0;
+    static_assert(!(PK && MULTI), "packed bonds hold one state bit");
     extern __shared__ double4 hrec[];
     const int64_t k = pdx_xcd_block();
-    const int64_t p0 = k * PDX_BLOCK;
+    const int64_t p0 = k * PB;
     if (p0 >= A.n) return;  // whole workgroup
     const int64_t h0 = A.halo_ptr[k];
     const int H = (int)(A.halo_ptr[k + 1] - h0);
-    // CAP: tables longer than the LDS budget are staged in tiles of HL entries (rows and
-    // tables sorted by neighbour: each lane meets the tiles in order)
+    // CAP: tables longer than the LDS budget are staged in tiles of HL entries
     const int HL = CAP ? pdx_lds_entries(A.halo_max, A.lds_budget, 32 + (MULTI ? 1 : 0)) : A.halo_max;
     const int32_t *const hidx = A.halo + h0;
     uint8_t *const hpid = reinterpret_cast<uint8_t *>(hrec + HL);
     auto stage = [&](int T0, int T1) {
-        for (int h = T0 + (int)threadIdx.x; h < T1; h += PDX_BLOCK * S) {
+        for (int h = T0 + (int)threadIdx.x; h < T1; h += PB * S) {
             const int32_t j = hidx[h];
-            // with the linear influence function the record carries delta V_j (omega V_j =
-            // (delta V_j) / L)
             const double4 r = A.rec_in[j];
-            hrec[h - T0] = (F & PDX_FEAT_KERN) ? r : make_double4(r.x, r.y, r.z, A.delta * r.w);
+            hrec[h - T0] = KERN ? r : make_double4(r.x, r.y, r.z, A.delta * r.w);
             if (MULTI) hpid[h - T0] = A.pid[j];
         }
     };
     const int sub = threadIdx.x % S;
     const int64_t p = p0 + threadIdx.x / S;
-    const bool valid = p < A.n;
-    if constexpr (!CAP) {
-        stage(0, H);
-        __syncthreads();
-        if (!valid) return;  // all S lanes of the point together
+    const int64_t q = p < A.n ? p : A.n - 1;
+    const pdx_lane<S, PK> R = pdx_lane_of<S, PK>(A, p0);
+    const double4 ri = A.rec_in[q];
+    double epsc = A.epsc, thr = A.epsc_lo;
+    pdx_pset Pi;
+    if (MULTI) {
+        Pi = A.psets[A.pid[q]];
+        thr = A.epsc_lo_min;  // of all sets: either copy of a bond may fail from there on
+    } else {
+        thr = fail_window<PK>(A, q, A.epsc_lo);
     }
-    const int c = valid ? A.cnt[p] : 0;
-    const int64_t b0 = valid ? pdx_bond0(A.slice_ptr, p) : 0;
-    uint16_t *const wbase = A.bw16 + b0;
-    const double *const Lbase = A.L + b0;
-    const double4 ri = valid ? A.rec_in[p] : make_double4(0.0, 0.0, 0.0, 0.0);
     double wvol = 0.0, Ssum = 0.0;
-    double ax = 0.0, ay = 0.0, az = 0.0, bx = 0.0, by = 0.0, bz = 0.0;  // A_i, B_i (SPLIT)
+    double ax = 0.0, ay = 0.0, az = 0.0, bx = 0.0, by = 0.0, bz = 0.0;  // A_i, B_i (one set)
     int na = 0;
-    double epsc = A.epsc, epsc_lo = A.epsc_lo, epsc_hi = A.epsc_hi, G = A.G, K = A.K;
-    if (MULTI && valid) {
-        const pdx_pset Pi = A.psets[A.pid[p]];
-        epsc = Pi.epsc;
-        epsc_lo = Pi.epsc_lo;
-        epsc_hi = Pi.epsc_hi;
-    }
-    // two bonds per lane in flight: their words and lengths are loaded before either is used
-    constexpr int U = 2;
-    int t0 = sub;
-    // the lane's bonds whose neighbours lie in the staged entries [T0, T1)
-    auto walk = [&](int T0, int T1) {
-        for (; t0 < c; t0 += U * S) {
-            uint32_t wdu[U];
-            double Lu[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const bool ok = t0 + u * S < c;
-                wdu[u] = ok ? wbase[(int64_t)(t0 + u * S) * 64] : 0u;
-                Lu[u] = ok ? Lbase[(int64_t)(t0 + u * S) * 64] : 1.0;
+    auto bond = [&](const bond_data<PK> &b, int i, int T0) {
+        const int ls = bond_slot(A, b) - T0;
+        const double4 rj = hrec[ls];
+        const double dx = rj.x - ri.x, dy = rj.y - ri.y, dz = rj.z - ri.z;
+        const double L = bond_len(A, b);
+        double rlL;
+        const double e = pdx_elong((dx * dx + dy * dy) + dz * dz, L, rlL);
+        bool act = bond_act(A, b);
+        if constexpr (MULTI) {
+            if ((b.w & PDX_W16_FP) && (b.w & (PDX_W16_ACT | PDX_W16_RACT)) && e >= thr * L) {
+                const double eps = e / L;
+                uint32_t nw = b.w;
+                if (eps > Pi.epsc) nw &= ~(uint32_t)PDX_W16_ACT;
+                if (eps > A.psets[hpid[ls]].epsc) nw &= ~(uint32_t)PDX_W16_RACT;
+                if (nw != b.w) A.bw16[R.at(i)] = (uint16_t)nw;
+                act = (nw & PDX_W16_ACT) != 0;
             }
-            int kk = U;
-            if (CAP) {
-                kk = 0;
-#pragma unroll
-                for (int u = 0; u < U; u++)
-                    if (kk == u && t0 + u * S < c && (int)(wdu[u] & PDX_W16_SLOT) < T1) kk = u + 1;
+        } else {
+            if (act && e >= thr * L && bond_breaks<PK>(A, hidx, b, e, L, epsc)) {
+                act = false;
+                R.kill(A, i, b);
             }
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const int t = t0 + u * S;
-                if (u >= kk || t >= c) continue;
-                const int64_t o = (int64_t)t * 64;
-                const uint32_t wd = wdu[u];
-                const double Lb = Lu[u];
-                const int ls = (int)(wd & PDX_W16_SLOT) - T0;
-                const double4 rj = hrec[ls];
-                const double dx = rj.x - ri.x, dy = rj.y - ri.y, dz = rj.z - ri.z;
-                double rl;
-                const double l = pdx_sqrt_rsq((dx * dx + dy * dy) + dz * dz, rl);
-                const double e = l - Lb;
-                const double rL = pdx_rcp1(Lb);
-                bool act;
-                if (MULTI) {
-                    // The neighbour fails its own copy of the bond against its eps_c; the stretch
-                    // is the same number at both ends, so the owner tracks that copy's state
-                    // (RACT) exactly, which the gather of pass 2 needs.
-                    const double eps = e * rL;
-                    const pdx_pset Pj = A.psets[hpid[ls]];
-                    uint32_t nw = wd;
-                    if ((wd & PDX_W16_ACT) && (wd & PDX_W16_FP) && eps >= epsc_lo)
-                        if ((eps > epsc_hi) ? true : ((e / Lb) > epsc)) nw &= ~PDX_W16_ACT;
-                    if ((wd & PDX_W16_RACT) && (wd & PDX_W16_FP) && eps >= Pj.epsc_lo)
-                        if ((eps > Pj.epsc_hi) ? true : ((e / Lb) > Pj.epsc)) nw &= ~PDX_W16_RACT;
-                    if (nw != wd) wbase[o] = (uint16_t)nw;
-                    act = (nw & PDX_W16_ACT) != 0;
-                } else {
-                    act = bond_fail16(wbase + o, wd, e, Lb, e * rL, epsc, epsc_lo, epsc_hi);
-                }
-                if (act) {
-                    // omega, or 1 / L with delta already in the record
-                    double w = (F & PDX_FEAT_KERN) ? pdx_omega(A.kernel, A.delta, Lb, rL) : rL;
-                    if (SC) w *= A.scf[b0 + o];  // omega * beta
-                    // w V_j formed once: wvol += (w V_j L) L, Ssum += (w V_j L) e
-                    const double wV = w * rj.w;
-                    const double wVL = wV * Lb;
-                    wvol = __builtin_fma(wVL, Lb, wvol);
-                    Ssum = __builtin_fma(wVL, e, Ssum);
-                    na++;
-                    if (SPLIT) {
-                        const double q = wV * rl;
-                        const double qL = q * Lb, qe = q * e;
-                        ax = __builtin_fma(qL, dx, ax);
-                        ay = __builtin_fma(qL, dy, ay);
-                        az = __builtin_fma(qL, dz, az);
-                        bx = __builtin_fma(qe, dx, bx);
-                        by = __builtin_fma(qe, dy, by);
-                        bz = __builtin_fma(qe, dz, bz);
-                    }
-                }
+        }
+        if (act) {
+            double V = rj.w;  // delta V_j, or V_j with another influence function
+            if (SC) V *= A.scf[R.at(i)];  // omega * beta
+            double wVL = V, wVl = V * rlL;  // omega V_j L and omega V_j / l
+            if (KERN) {
+                const double w = pdx_omega(A.kernel, A.delta, L, rlL * (e + L));
+                wVL = (w * V) * L;
+                wVl = (w * V) * (rlL * L);
             }
-            if (CAP && kk < U) {
-                t0 += kk * S;  // resume at the first bond past the tile (or the row's end)
-                return;
+            wvol = __builtin_fma(wVL, L, wvol);
+            Ssum = __builtin_fma(wVL, e, Ssum);
+            na++;
+            if (!MULTI) {
+                const double qL = wVl * L, qe = wVl * e;
+                ax = __builtin_fma(qL, dx, ax);
+                ay = __builtin_fma(qL, dy, ay);
+                az = __builtin_fma(qL, dz, az);
+                bx = __builtin_fma(qe, dx, bx);
+                by = __builtin_fma(qe, dy, by);
+                bz = __builtin_fma(qe, dz, bz);
             }
         }
     };
     if constexpr (!CAP) {
-        walk(0, H);
+        stage(0, H);
+        __syncthreads();
+        pdx_walk<2>(A, R, [&](const bond_data<PK> (&b)[2], int i) {
+            bond(b[0], i, 0);
+            if (i + 1 < R.ng) bond(b[1], i + 1, 0);
+        });
     } else {
+        int i = 0;
         for (int T0 = 0; T0 < H; T0 += HL) {
             const int T1 = H < T0 + HL ? H : T0 + HL;
             if (T0 > 0) __syncthreads();  // the previous tile is consumed
             stage(T0, T1);
             __syncthreads();
-            walk(T0, T1);
+            i = pdx_walk_tile<2>(A, R, i, T1, [&](const bond_data<PK> &b, int ib) { bond(b, ib, T0); });
         }
     }
-#pragma unroll
-    for (int o = 1; o < S; o <<= 1) {
-        wvol += __shfl_xor(wvol, o);
-        Ssum += __shfl_xor(Ssum, o);
-        na += __shfl_xor(na, o);
-        if (SPLIT) {
-            ax += __shfl_xor(ax, o);
-            ay += __shfl_xor(ay, o);
-            az += __shfl_xor(az, o);
-            bx += __shfl_xor(bx, o);
-            by += __shfl_xor(by, o);
-            bz += __shfl_xor(bz, o);
-        }
+    pdx_fold(R, wvol);
+    pdx_fold(R, Ssum);
+    pdx_fold(R, na);
+    if (!MULTI) {
+        pdx_fold(R, ax);
+        pdx_fold(R, ay);
+        pdx_fold(R, az);
+        pdx_fold(R, bx);
+        pdx_fold(R, by);
+        pdx_fold(R, bz);
     }
-    if (!valid) return;
-    if (SPLIT) {
-        // every lane holds the sums; lane d < 3 stores component d of the own part, lane 3
-        // the per-point pair and the counts
-        double c1 = 0.0, c2 = 0.0;
-        if (wvol != 0.0) {
-            const double dil = (3.0 / wvol) * Ssum;
-            c1 = (15.0 * G) / wvol;
-            c2 = dil * ((3.0 * K) / wvol - c1 / 3.0);
-        }
-        if (sub < 3) {
-            const double a = sub == 0 ? ax : (sub == 1 ? ay : az);
-            const double bb = sub == 0 ? bx : (sub == 1 ? by : bz);
-            A.pstate[2 * A.n + 3 * p + sub] = c2 * a + c1 * bb;
-            return;
-        }
-        reinterpret_cast<double2 *>(A.pstate)[p] = make_double2(c1 * ri.w, c2 * ri.w);
-        if (A.flags & (PDX_F_STORE | PDX_F_FORCE_ONLY)) {
-            A.nact_out[p] = na;
-            A.dmg_out[p] = 1.0 - (double)na / (double)c;
-        }
+    if (p >= A.n || sub > 3) return;
+    const bool counts = sub == 3 && (A.flags & (PDX_F_STORE | PDX_F_FORCE_ONLY)) != 0;
+    if (counts) {
+        A.nact_out[p] = na;
+        A.dmg_out[p] = 1.0 - (double)na / (double)A.cnt[p];
+    }
+    if (MULTI) {
+        const double h = wvol != 0.0 ? 1.0 / (2.0 * wvol) : 0.0;
+        const double dil = wvol != 0.0 ? (3.0 / wvol) * Ssum : 0.0;
+        if (sub == 3) reinterpret_cast<double2 *>(A.pstate)[p] = make_double2(h, h * dil);
         return;
     }
-    if (sub != 0) return;
+    // every lane holds the sums; lane d < 3 stores component d of the own part, lane 3 the
+    // per-point pair and the counts
     double c1 = 0.0, c2 = 0.0;
-    if (MULTI) {
-        // several sets: c1, c2 depend on the bond (averaged G, K); keep wvol and the dilatation
-        c1 = wvol;
-        c2 = wvol != 0.0 ? (3.0 / wvol) * Ssum : 0.0;
-    } else if (wvol != 0.0) {
+    if (wvol != 0.0) {
         const double dil = (3.0 / wvol) * Ssum;
-        c1 = (15.0 * G) / wvol;
-        c2 = dil * ((3.0 * K) / wvol - c1 / 3.0);
+        c1 = (15.0 * A.G) / wvol;
+        c2 = dil * ((3.0 * A.K) / wvol - c1 / 3.0);
     }
-    reinterpret_cast<double2 *>(A.pstate)[p] = make_double2(c1, c2);
-    if (A.flags & (PDX_F_STORE | PDX_F_FORCE_ONLY)) {
-        A.nact_out[p] = na;
-        A.dmg_out[p] = 1.0 - (double)na / (double)c;
+    if (sub < 3) {
+        const double a = sub == 0 ? ax : (sub == 1 ? ay : az);
+        const double bb = sub == 0 ? bx : (sub == 1 ? by : bz);
+        A.pstate[2 * A.n + 3 * p + sub] = c2 * a + c1 * bb;
+    } else {
+        reinterpret_cast<double2 *>(A.pstate)[p] = make_double2(c1 * ri.w, c2 * ri.w);
     }
 }
 
-// One set: the own part comes from pass 1, the loop gathers the reverse parts.
-// MULTI: several parameter sets (force_density_point! with a ParameterHandler,
-// ordinary_state_based.jl:151-174): pass 1 left (wvol, dilatation) per point and the bond
-// takes c1 = 15 (G_i + G_j) / (2 wvol), c2 = dil (3 (K_i + K_j) / (2 wvol) - c1 / 3) of each
-// end; a point with wvol = 0 contributes nothing (its loop returns early)
-template <int S, int F>
-__global__ __launch_bounds__(PDX_BLOCK * S) void k_osb_lds2(pdx_step_args A)
+template <int S, int F, int PB, bool PK>
+__global__ __launch_bounds__(PB * S) void k_osb_lds2(pdx_step_args A)
 {
     constexpr bool MULTI = (F & PDX_FEAT_MULTI) != 0;
-    constexpr bool SPLIT = !MULTI;
+    constexpr bool KERN = (F & PDX_FEAT_KERN) != 0;
     constexpr bool SC = (F & PDX_FEAT_SC) != 0;
     constexpr bool CAP = (F & PDX_FEAT_CAP) != 0;
     extern __shared__ double4 hrec[];
-    // CAP: tables longer than the LDS budget are staged in tiles of HL entries
-    const int HL = CAP ? pdx_lds_entries(A.halo_max, A.lds_budget, SPLIT ? 40 : 48 + 1) : A.halo_max;
-    // SPLIT: hrec holds (x, y, z, (c1 V)_j), hc2 (c2 V)_j; otherwise hrec x|V, hc (wvol, dil)
-    double2 *const hc = reinterpret_cast<double2 *>(hrec + HL);
+    const int HL = CAP ? pdx_lds_entries(A.halo_max, A.lds_budget, MULTI ? 64 : 40) : A.halo_max;
+    // one set: hrec (x, y, z, (c1 V)_j), hc2 (c2 V)_j; several: hrec x|V, then (h, h d)_j,
+    // (15 G_j, 3 K_j - 5 G_j)
     double *const hc2 = reinterpret_cast<double *>(hrec + HL);
+    double4 *const hm = hrec + HL;
     const int64_t k = pdx_xcd_block();
-    const int64_t p0 = k * PDX_BLOCK;
+    const int64_t p0 = k * PB;
     if (p0 >= A.n) return;  // whole workgroup
     const int64_t h0 = A.halo_ptr[k];
     const int H = (int)(A.halo_ptr[k + 1] - h0);
     const double2 *const cst = reinterpret_cast<const double2 *>(A.pstate);
     const int32_t *const hidx = A.halo + h0;
-    uint8_t *const hpid = reinterpret_cast<uint8_t *>(hc + HL);
     auto stage = [&](int T0, int T1) {
-        for (int h = T0 + (int)threadIdx.x; h < T1; h += PDX_BLOCK * S) {
+        for (int h = T0 + (int)threadIdx.x; h < T1; h += PB * S) {
             const int64_t j = hidx[h];
             const double4 r = A.rec_in[j];
             const double2 cj = cst[j];
-            if (SPLIT) {
+            if (MULTI) {
+                const pdx_pset &Pj = A.psets[A.pid[j]];
+                hrec[h - T0] = make_double4(r.x, r.y, r.z, KERN ? r.w : A.delta * r.w);
+                hm[h - T0] = make_double4(cj.x, cj.y, 15.0 * Pj.G, 3.0 * Pj.K - 5.0 * Pj.G);
+            } else {
                 // with the linear influence function: delta (c1 V)_j, delta (c2 V)_j
-                const double dl = (F & PDX_FEAT_KERN) ? 1.0 : A.delta;
+                const double dl = KERN ? 1.0 : A.delta;
                 hrec[h - T0] = make_double4(r.x, r.y, r.z, dl * cj.x);
                 hc2[h - T0] = dl * cj.y;
-            } else {
-                hrec[h - T0] = r;
-                hc[h - T0] = cj;
-                hpid[h - T0] = A.pid[j];
             }
         }
     };
     const int sub = threadIdx.x % S;
     const int64_t p = p0 + threadIdx.x / S;
-    const bool valid = p < A.n;
-    if constexpr (!CAP) {
-        stage(0, H);
-        __syncthreads();
-        if (!valid) return;  // all S lanes of the point together
-    }
-    const int c = valid ? A.cnt[p] : 0;
-    const int64_t b0 = valid ? pdx_bond0(A.slice_ptr, p) : 0;
-    const uint16_t *const wbase = A.bw16 + b0;
-    const double *const Lbase = A.L + b0;
-    const double4 ri = valid ? A.rec_in[p] : make_double4(0.0, 0.0, 0.0, 0.0);
-    const double2 ci = (MULTI && valid) ? cst[p] : make_double2(0.0, 0.0);
+    const int64_t q = p < A.n ? p : A.n - 1;
+    const pdx_lane<S, PK> R = pdx_lane_of<S, PK>(A, p0);
+    const double4 ri = A.rec_in[q];
+    const double2 ci = MULTI ? cst[q] : make_double2(0.0, 0.0);
     double bx = 0.0, by = 0.0, bz = 0.0;
-    if (SPLIT && sub == 0 && valid) {
+    if (!MULTI && sub == 0 && p < A.n) {  // the own part (pass 1)
         const double *own = A.pstate + 2 * A.n + 3 * p;
         bx = own[0];
         by = own[1];
         bz = own[2];
     }
-    double Gi = A.G, Ki = A.K, rho = A.rho;
-    if (MULTI && valid) {
-        const pdx_pset Pi = A.psets[A.pid[p]];
-        Gi = Pi.G;
-        Ki = Pi.K;
+    double gi = 0.0, ki = 0.0, rho = A.rho;
+    if (MULTI) {
+        const pdx_pset &Pi = A.psets[A.pid[q]];
+        gi = 15.0 * Pi.G;
+        ki = 3.0 * Pi.K - 5.0 * Pi.G;
         rho = Pi.rho;
     }
-    constexpr int U = 2;  // two bonds per lane in flight
-    int t0 = sub;
-    // the lane's bonds whose neighbours lie in the staged entries [T0, T1)
-    auto walk = [&](int T0, int T1) {
-        for (; t0 < c; t0 += U * S) {
-            uint32_t wdu[U];
-            double Lu[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const bool ok = t0 + u * S < c;
-                wdu[u] = ok ? wbase[(int64_t)(t0 + u * S) * 64] : 0u;
-                Lu[u] = ok ? Lbase[(int64_t)(t0 + u * S) * 64] : 1.0;
-            }
-            int kk = U;
-            if (CAP) {
-                kk = 0;
-#pragma unroll
-                for (int u = 0; u < U; u++)
-                    if (kk == u && t0 + u * S < c && (int)(wdu[u] & PDX_W16_SLOT) < T1) kk = u + 1;
-            }
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const int t = t0 + u * S;
-                if (u >= kk || t >= c) continue;
-                const int64_t o = (int64_t)t * 64;
-                const uint32_t wd = wdu[u];
-                const double Lb = Lu[u];
-                const bool act = (wd & PDX_W16_ACT) != 0;
-                const bool ract = MULTI ? (wd & PDX_W16_RACT) != 0 : act;  // one set: both copies agree
-                if (!act && !ract) continue;
-                const int ls = (int)(wd & PDX_W16_SLOT) - T0;
-                double4 rj;
-                double2 cj;
-                if (SPLIT) {
-                    rj = hrec[ls];
-                    cj = make_double2(rj.w, hc2[ls]);
-                } else {
-                    rj = hrec[ls];
-                    cj = hc[ls];
-                }
-                const double dx = rj.x - ri.x, dy = rj.y - ri.y, dz = rj.z - ri.z;
-                double rl;
-                const double l = pdx_sqrt_rsq((dx * dx + dy * dy) + dz * dz, rl);
-                const double rLb = pdx_rcp1(Lb);
-                // omega, or 1 / L where delta is already in the staged constants (one set)
-                double w = (F & PDX_FEAT_KERN) ? pdx_omega(A.kernel, A.delta, Lb, rLb) : (SPLIT ? rLb : A.delta * rLb);
-                if (SC) w *= A.scf[b0 + o];  // beta is symmetric: both ends' copies of the bond carry it
-                const double e = l - Lb;
-                if (SPLIT) {
-                    // the reverse part (c2 V)_j L + (c1 V)_j e
-                    const double s = (w * rl) * __builtin_fma(cj.x, e, cj.y * Lb);
-                    bx = __builtin_fma(s, dx, bx);
-                    by = __builtin_fma(s, dy, by);
-                    bz = __builtin_fma(s, dz, bz);
-                    continue;
-                }
-                double fi, fj;
-                if (MULTI) {
-                    const pdx_pset Pj = A.psets[hpid[ls]];
-                    const double Gs = Gi + Pj.G, Ks = Ki + Pj.K;
-                    fi = 0.0;
-                    fj = 0.0;
-                    if (act && ci.x != 0.0) {
-                        const double c1 = (15.0 * Gs) / (2.0 * ci.x);
-                        const double c2 = ci.y * ((3.0 * Ks) / (2.0 * ci.x) - c1 / 3.0);
-                        fi = c2 * Lb + c1 * e;
-                    }
-                    if (ract && cj.x != 0.0) {
-                        const double c1 = (15.0 * Gs) / (2.0 * cj.x);
-                        const double c2 = cj.y * ((3.0 * Ks) / (2.0 * cj.x) - c1 / 3.0);
-                        fj = c2 * Lb + c1 * e;
-                    }
-                } else {
-                    fi = ci.y * Lb + ci.x * e;
-                    fj = cj.y * Lb + cj.x * e;
-                }
-                const double s = (w * rl) * ((fi + fj) * rj.w);
-                bx = __builtin_fma(s, dx, bx);
-                by = __builtin_fma(s, dy, by);
-                bz = __builtin_fma(s, dz, bz);
-            }
-            if (CAP && kk < U) {
-                t0 += kk * S;  // resume at the first bond past the tile (or the row's end)
-                return;
-            }
+    auto bond = [&](const bond_data<PK> &b, int i, int T0) {
+        const bool act = bond_act(A, b);
+        bool ract = act;  // one set: both copies agree
+        if constexpr (MULTI) ract = (b.w & PDX_W16_RACT) != 0;
+        if (!act && !ract) return;
+        const int ls = bond_slot(A, b) - T0;
+        const double4 rj = hrec[ls];
+        const double dx = rj.x - ri.x, dy = rj.y - ri.y, dz = rj.z - ri.z;
+        const double L = bond_len(A, b);
+        double rlL;
+        const double e = pdx_elong((dx * dx + dy * dy) + dz * dz, L, rlL);
+        double w = rlL;  // omega / l with delta already in the record
+        if (KERN) w = pdx_omega(A.kernel, A.delta, L, rlL * (e + L)) * (rlL * L);
+        if (SC) w *= A.scf[R.at(i)];  // beta is symmetric
+        double f;
+        if (MULTI) {
+            const double4 m = hm[ls];
+            const double h1 = (act ? ci.x : 0.0) + (ract ? m.x : 0.0);
+            const double h2 = (act ? ci.y : 0.0) + (ract ? m.y : 0.0);
+            f = rj.w * __builtin_fma((gi + m.z) * e, h1, ((ki + m.w) * L) * h2);
+        } else {
+            f = __builtin_fma(rj.w, e, hc2[ls] * L);  // the reverse part (c2 V)_j L + (c1 V)_j e
         }
+        const double s = w * f;
+        bx = __builtin_fma(s, dx, bx);
+        by = __builtin_fma(s, dy, by);
+        bz = __builtin_fma(s, dz, bz);
     };
     if constexpr (!CAP) {
-        walk(0, H);
+        stage(0, H);
+        __syncthreads();
+        pdx_walk<2>(A, R, [&](const bond_data<PK> (&b)[2], int i) {
+            bond(b[0], i, 0);
+            if (i + 1 < R.ng) bond(b[1], i + 1, 0);
+        });
     } else {
+        int i = 0;
         for (int T0 = 0; T0 < H; T0 += HL) {
             const int T1 = H < T0 + HL ? H : T0 + HL;
             if (T0 > 0) __syncthreads();  // the previous tile is consumed
             stage(T0, T1);
             __syncthreads();
-            walk(T0, T1);
+            i = pdx_walk_tile<2>(A, R, i, T1, [&](const bond_data<PK> &b, int ib) { bond(b, ib, T0); });
         }
     }
-#pragma unroll
-    for (int o = 1; o < S; o <<= 1) {
-        bx += __shfl_xor(bx, o);
-        by += __shfl_xor(by, o);
-        bz += __shfl_xor(bz, o);
-    }
-    if (!valid) return;
-    static_assert(S == 4, "the tail takes four lanes per point");
+    pdx_fold(R, bx);
+    pdx_fold(R, by);
+    pdx_fold(R, bz);
+    if (p >= A.n || sub >= 4) return;  // the tail takes four lanes per point
     const double b[3] = {bx, by, bz};
     point_tail4(A, p, ri, b, sub, rho);
 }
@@ -1887,7 +1707,7 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_pass1(pdx_step_args A)
     const int64_t p = pdx_xcd_block() * PDX_BLOCK + threadIdx.x / S;
     if (p >= A.n) return;  // all S lanes of the point together
     const int c = A.cnt[p];
-    const int64_t b0 = pdx_bond0(A.slice_ptr, p);
+    const int64_t b0 = A.rows.row(p);
     const double4 ri = A.rec_in[p];
     const double4 Xi = A.Xr[p];
     const bool dead = A.killed[p] != 0;
@@ -1959,7 +1779,7 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_pass2(pdx_step_args A)
     const int64_t p = pdx_xcd_block() * PDX_BLOCK + threadIdx.x / S;
     if (p >= A.n) return;  // all S lanes of the point together
     const int c = A.cnt[p];
-    const int64_t b0 = pdx_bond0(A.slice_ptr, p);
+    const int64_t b0 = A.rows.row(p);
     const double4 ri = A.rec_in[p];
     const double4 Xi = A.Xr[p];
     const bool dead_i = A.killed[p] != 0;
@@ -2024,8 +1844,8 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_pass2(pdx_step_args A)
 // the next tile is staged.  Pass 1 entries: x|V, X (64 B); pass 2: x|V, X|beta [j alive],
 // [j alive] Q_j (136 B).  The arithmetic is that of k_cpd_pass1/2.
 // ----------------------------------------------------------------------------------------
-template <int S, int F>
-__global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_lds1(pdx_step_args A)
+template <int S, int F, int PB, bool PK>
+__global__ __launch_bounds__(PB * S) void k_cpd_lds1(pdx_step_args A)
 {
     // PDX_FEAT_MULTI: several parameter sets (force_density_point! with the params of the
     // point whose loop runs, correspondence.jl:183-191): eps_c of the owner per copy of a
@@ -2038,34 +1858,32 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_lds1(pdx_step_args A)
     double4 *const hX = hrec + TL;
     uint8_t *const hpid = reinterpret_cast<uint8_t *>(hrec + 2 * TL);
     const int64_t k = pdx_xcd_block();
-    const int64_t p0 = k * PDX_BLOCK;
+    const int64_t p0 = k * PB;
     if (p0 >= A.n) return;  // whole workgroup
     const int64_t h0 = A.halo_ptr[k];
     const int H = (int)(A.halo_ptr[k + 1] - h0);
     const int32_t *const hidx = A.halo + h0;
     const int sub = threadIdx.x % S;
     const int64_t p = p0 + threadIdx.x / S;
-    const bool valid = p < A.n;  // the block's threads all take part in the tile barriers
-    const int c = valid ? A.cnt[p] : 0;
-    const int64_t b0 = valid ? pdx_bond0(A.slice_ptr, p) : 0;
-    uint16_t *const wbase = A.bw16 + b0;
-    const double *const Lbase = A.L + b0;
-    const double4 ri = valid ? A.rec_in[p] : make_double4(0.0, 0.0, 0.0, 0.0);
-    const double4 Xi = valid ? A.Xr[p] : make_double4(0.0, 0.0, 0.0, 0.0);
-    const bool dead = valid && A.killed[p] != 0;
-    double epsc = A.epsc, epsc_lo = A.epsc_lo, epsc_hi = A.epsc_hi;
+    const int64_t pq = p < A.n ? p : A.n - 1;  // the block's threads all take part in the tile barriers
+    const pdx_lane<S, PK> R = pdx_lane_of<S, PK>(A, p0);
+    const double4 ri = A.rec_in[pq];
+    const double4 Xi = A.Xr[pq];
+    const bool dead = A.killed[pq] != 0;
+    double epsc = A.epsc, thr;
     double lam = A.lambda, mu = A.mu, Gp = A.G, Kp = A.K, nup = A.nu, beta = A.beta_zem;
-    if (MULTI && valid) {
-        const pdx_pset Pi = A.psets[A.pid[p]];
+    if (MULTI) {
+        const pdx_pset Pi = A.psets[A.pid[pq]];
         epsc = Pi.epsc;
-        epsc_lo = Pi.epsc_lo;
-        epsc_hi = Pi.epsc_hi;
+        thr = A.epsc_lo_min;  // of all sets: either copy of a bond may fail from there on
         lam = Pi.lam;
         mu = Pi.mu;
         Gp = Pi.G;
         Kp = Pi.K;
         nup = Pi.nu;
         beta = Pi.beta;
+    } else {
+        thr = fail_window<PK>(A, pq, A.epsc_lo);
     }
     double Km[6] = {0, 0, 0, 0, 0, 0};  // 00 10 20 11 21 22
     double Ft[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
@@ -2074,47 +1892,48 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_lds1(pdx_step_args A)
     constexpr bool ZWF = (F & PDX_FEAT_ZW) != 0;
     double S1[3] = {0, 0, 0}, S2[3] = {0, 0, 0};
     int na = 0;
-    int t = sub;
+    int ig = 0;
     for (int T0 = 0; T0 < H; T0 += TL) {
         const int T1 = H < T0 + TL ? H : T0 + TL;
         if (T0 > 0) __syncthreads();  // the previous tile is consumed
-        for (int h = T0 + (int)threadIdx.x; h < T1; h += PDX_BLOCK * S) {
+        for (int h = T0 + (int)threadIdx.x; h < T1; h += PB * S) {
             const int32_t j = hidx[h];
             hx[h - T0] = A.rec_in[j];
             hX[h - T0] = A.Xr[j];
             if (MULTI) hpid[h - T0] = A.pid[j];
         }
         __syncthreads();
-        t = pdx_walk_tile<1, S>(wbase, Lbase, t, c, T1, [&](uint32_t wd, double Lb, int tb) {
-            const int slot = (int)(wd & PDX_W16_SLOT);
+        ig = pdx_walk_tile<1>(A, R, ig, T1, [&](const bond_data<PK> &bd, int ib) {
+            const int slot = bond_slot(A, bd);
             const double4 rj = hx[slot - T0];
             const double4 Xj = hX[slot - T0];
             const double dx[3] = {rj.x - ri.x, rj.y - ri.y, rj.z - ri.z};
             const double DX[3] = {Xj.x - Xi.x, Xj.y - Xi.y, Xj.z - Xi.z};
+            const double Lb = bond_len(A, bd);
             double rl;
-            const double l = pdx_sqrt_rsq((dx[0] * dx[0] + dx[1] * dx[1]) + dx[2] * dx[2], rl);
-            const double e = l - Lb;
-            const double rL = pdx_rcp1(Lb);
-            bool act;
-            if (MULTI) {
+            const double e = pdx_sqrt_rsq((dx[0] * dx[0] + dx[1] * dx[1]) + dx[2] * dx[2], rl) - Lb;
+            bool act = bond_act(A, bd);
+            if constexpr (MULTI) {
                 // each end fails its copy of the bond against its own eps_c; the stretch is the
                 // same number at both ends
-                const double eps = e * rL;
-                const pdx_pset Pj = A.psets[hpid[slot - T0]];
-                uint32_t nw = wd;
-                if ((wd & PDX_W16_ACT) && (wd & PDX_W16_FP) && eps >= epsc_lo)
-                    if ((eps > epsc_hi) ? true : ((e / Lb) > epsc)) nw &= ~PDX_W16_ACT;
-                if ((wd & PDX_W16_RACT) && (wd & PDX_W16_FP) && eps >= Pj.epsc_lo)
-                    if ((eps > Pj.epsc_hi) ? true : ((e / Lb) > Pj.epsc)) nw &= ~PDX_W16_RACT;
-                if (nw != wd) wbase[(int64_t)tb * 64] = (uint16_t)nw;
-                act = (nw & PDX_W16_ACT) != 0;
+                if ((bd.w & PDX_W16_FP) && (bd.w & (PDX_W16_ACT | PDX_W16_RACT)) && e >= thr * Lb) {
+                    const double eps = e / Lb;
+                    uint32_t nw = bd.w;
+                    if (eps > epsc) nw &= ~(uint32_t)PDX_W16_ACT;
+                    if (eps > A.psets[hpid[slot - T0]].epsc) nw &= ~(uint32_t)PDX_W16_RACT;
+                    if (nw != bd.w) A.bw16[R.at(ib)] = (uint16_t)nw;
+                    act = (nw & PDX_W16_ACT) != 0;
+                }
             } else {
-                act = bond_fail16(wbase + (int64_t)tb * 64, wd, e, Lb, e * rL, epsc, epsc_lo, epsc_hi);
+                if (act && e >= thr * Lb && bond_breaks<PK>(A, hidx, bd, e, Lb, epsc)) {
+                    act = false;
+                    R.kill(A, ib, bd);
+                }
             }
             if (act && !dead) {
                 na++;
                 // K += w V_j DX DX', Ft += w V_j dx DX' as fused products of (w V_j DX)
-                const double temp = pdx_omega(A.kernel, A.delta, Lb, rL) * rj.w;
+                const double temp = pdx_omega(A.kernel, A.delta, Lb, pdx_rcp1(Lb)) * rj.w;
                 const double tD[3] = {temp * DX[0], temp * DX[1], temp * DX[2]};
                 Km[0] = fma(tD[0], DX[0], Km[0]);
                 Km[1] = fma(tD[1], DX[0], Km[1]);
@@ -2135,20 +1954,17 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_lds1(pdx_step_args A)
         });
     }
 #pragma unroll
-    for (int o = 1; o < S; o <<= 1) {
+    for (int q = 0; q < 6; q++) pdx_fold(R, Km[q]);
 #pragma unroll
-        for (int q = 0; q < 6; q++) Km[q] += __shfl_xor(Km[q], o);
+    for (int q = 0; q < 9; q++) pdx_fold(R, Ft[q]);
 #pragma unroll
-        for (int q = 0; q < 9; q++) Ft[q] += __shfl_xor(Ft[q], o);
-#pragma unroll
-        for (int r = 0; r < 3; r++) {
-            S1[r] += __shfl_xor(S1[r], o);
-            S2[r] += __shfl_xor(S2[r], o);
-        }
-        na += __shfl_xor(na, o);
+    for (int r = 0; r < 3; r++) {
+        pdx_fold(R, S1[r]);
+        pdx_fold(R, S2[r]);
     }
-    if (!valid || sub != 0) return;
-    const bool kill = cpd_point_state<ZWF>(A, p, Km, Ft, na, c, dead, lam, mu, Gp, Kp, nup, beta);
+    pdx_fold(R, na);
+    if (p >= A.n || sub != 0) return;
+    const bool kill = cpd_point_state<ZWF>(A, p, Km, Ft, na, A.cnt[p], dead, lam, mu, Gp, Kp, nup, beta);
     {
         // the own term of the point's bonds, Q_i S1 + beta S2, and a_i = Q_i X_i + beta x_i
         // (ZEMWan: C_1i in place of beta; zero for a dead point, whose state is zero), behind
@@ -2180,7 +1996,7 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_lds1(pdx_step_args A)
 // CPD pass 2 (correspondence.jl:234-249).  The own terms of the point's bonds, w V_j [Q_i DX +
 // beta dx] summed, came from pass 1 as Q_i S1 + beta S2; the neighbour's term of a bond,
 // Q_j DX + beta_j dx, is a_j - Q_j X_i - beta_j x_i with a_j = Q_j X_j + beta_j x_j from
-// pass 1, in coordinates relative to the block's first point (the staging moves a_j there),
+// pass 1, in coordinates relative to the first point of the run of 256 (the staging moves a_j there),
 // so that the products stay of the size of the block rather than of the coordinates.  ZW
 // (ZEMWan): the symmetric C_1 of each end in place of beta.  Table entries as 16-byte pairs:
 // [j alive] (Q_j, a_j), then [j alive] beta, V_j (112 B, 1463 entries in a 160 KB tile), or
@@ -2189,12 +2005,11 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_lds1(pdx_step_args A)
 // parameter sets): beta_j of the neighbour's set, the neighbour's term for the neighbour's
 // copy of the bond (RACT; the own terms followed the owner's copy, ACT, in pass 1), and the
 // point's own rho (velocity_verlet.jl:262-275).
-template <int S, int F>
-__global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_lds2_own(pdx_step_args A)
+template <int S, int F, int PB, bool PK>
+__global__ __launch_bounds__(PB * S) void k_cpd_lds2_own(pdx_step_args A)
 {
     constexpr bool MULTI = (F & PDX_FEAT_MULTI) != 0;
     constexpr bool ZW = (F & PDX_FEAT_ZW) != 0;
-    constexpr uint32_t NBIT = MULTI ? PDX_W16_RACT : PDX_W16_ACT;  // the neighbour's copy
     constexpr int NQ = ZW ? 15 : 9;  // state numbers per point
     constexpr int ND = ZW ? 10 : 7;  // 16-byte pairs per entry
     constexpr int IV = ZW ? 18 : 13;  // V_j in the entry
@@ -2203,7 +2018,7 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_lds2_own(pdx_step_args A)
     double2 *const hq = reinterpret_cast<double2 *>(hrec);
     const int TL = pdx_lds_entries(A.halo_max, A.lds_budget, 16 * ND);
     const int64_t k = pdx_xcd_block();
-    const int64_t p0 = k * PDX_BLOCK;
+    const int64_t p0 = k * PB;
     if (p0 >= A.n) return;  // whole workgroup
     const int64_t h0 = A.halo_ptr[k];
     const int H = (int)(A.halo_ptr[k + 1] - h0);
@@ -2211,11 +2026,9 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_lds2_own(pdx_step_args A)
     const int sub = threadIdx.x % S;
     const int64_t p = p0 + threadIdx.x / S;
     const bool valid = p < A.n;
-    const int c = valid ? A.cnt[p] : 0;
-    const int64_t b0 = valid ? pdx_bond0(A.slice_ptr, p) : 0;
-    const uint16_t *const wbase = A.bw16 + b0;
-    const double *const Lbase = A.L + b0;
-    const double4 OX = A.Xr[p0], Ox = A.rec_in[p0];
+    const pdx_lane<S, PK> R = pdx_lane_of<S, PK>(A, p0);
+    const int64_t po = p0 & ~(int64_t)(PDX_BLOCK - 1);
+    const double4 OX = A.Xr[po], Ox = A.rec_in[po];
     const double4 ri = valid ? A.rec_in[p] : Ox;
     const double4 Xi = valid ? A.Xr[p] : OX;
     const double xr[3] = {ri.x - Ox.x, ri.y - Ox.y, ri.z - Ox.z};
@@ -2224,11 +2037,11 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_lds2_own(pdx_step_args A)
     const double *const ext = A.pstate + NQ * A.n;
     const double rho = MULTI && valid ? A.psets[A.pid[p]].rho : A.rho;
     double b3[3] = {0.0, 0.0, 0.0};
-    int t = sub;
+    int ig = 0;
     for (int T0 = 0; T0 < H; T0 += TL) {
         const int T1 = H < T0 + TL ? H : T0 + TL;
         if (T0 > 0) __syncthreads();  // the previous tile is consumed
-        for (int h = T0 + (int)threadIdx.x; h < T1; h += PDX_BLOCK * S) {
+        for (int h = T0 + (int)threadIdx.x; h < T1; h += PB * S) {
             const int64_t j = hidx[h];
             const bool live = !A.killed[j];
             const double *const q = A.pstate + NQ * j;
@@ -2258,9 +2071,12 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_lds2_own(pdx_step_args A)
             for (int m = 0; m < ND; m++) d[m] = make_double2(e[2 * m], e[2 * m + 1]);
         }
         __syncthreads();
-        t = pdx_walk_tile<PDX_CPD_GROUP, S>(wbase, Lbase, t, c, T1, [&](uint32_t wd, double Lb, int) {
-            if (!(wd & NBIT)) return;
-            const double2 *const d = hq + ND * (int64_t)((int)(wd & PDX_W16_SLOT) - T0);
+        ig = pdx_walk_tile<PDX_CPD_GROUP>(A, R, ig, T1, [&](const bond_data<PK> &bd, int) {
+            bool on = bond_act(A, bd);
+            if constexpr (MULTI) on = (bd.w & PDX_W16_RACT) != 0;  // the neighbour's copy
+            if (!on) return;
+            const double Lb = bond_len(A, bd);
+            const double2 *const d = hq + ND * (int64_t)(bond_slot(A, bd) - T0);
             double e[2 * ND];
 #pragma unroll
             for (int m = 0; m < ND; m++) {
@@ -2281,13 +2097,10 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_lds2_own(pdx_step_args A)
         });
     }
 #pragma unroll
-    for (int o = 1; o < S; o <<= 1)
-#pragma unroll
-        for (int r = 0; r < 3; r++) b3[r] += __shfl_xor(b3[r], o);
-    if (!valid) return;
+    for (int r = 0; r < 3; r++) pdx_fold(R, b3[r]);
+    if (!valid || sub >= 4) return;  // the tail takes four lanes per point
 #pragma unroll
     for (int r = 0; r < 3; r++) b3[r] += ext[6 * p + r];  // the own terms (pass 1)
-    static_assert(S == 4, "the tail takes four lanes per point");
     point_tail4(A, p, ri, b3, sub, rho);
 }
 
@@ -2302,22 +2115,23 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_lds2_own(pdx_step_args A)
 // pass 2 stages (D, V), (U, beta [j alive]), [j alive] Q'_j (68 B per table entry) and
 // gathers both terms of every bond.
 // ----------------------------------------------------------------------------------------
-template <int U, int S, int F>
-__global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_pass1_mx(pdx_step_args A)
+template <int S, int F, int PB>
+__global__ __launch_bounds__(PB * S) void k_cpd_pass1_mx(pdx_step_args A)
 {
     constexpr bool CAP = (F & PDX_FEAT_CAP) != 0;
     extern __shared__ float4 hmx[];
     const int64_t k = pdx_xcd_block();
-    const int64_t p0 = k * PDX_BLOCK;
+    const int64_t p0 = k * PB;
     if (p0 >= A.n) return;  // whole workgroup
     const int64_t h0 = A.halo_ptr[k];
     const int H = (int)(A.halo_ptr[k + 1] - h0);
-    const double4 O = A.Xr[p0], xo = A.rec_in[p0];
+    const int64_t po = p0 & ~(int64_t)(PDX_BLOCK - 1);
+    const double4 O = A.Xr[po], xo = A.rec_in[po];
     const double uo0 = xo.x - O.x, uo1 = xo.y - O.y, uo2 = xo.z - O.z;
     const int HL = CAP ? pdx_lds_entries(A.halo_max, A.lds_budget, 32) : A.halo_max;
     const int Hs = H < HL ? H : HL;
     const int32_t *const hidx = A.halo + h0;
-    for (int h = threadIdx.x; h < Hs; h += PDX_BLOCK * S) {
+    for (int h = threadIdx.x; h < Hs; h += PB * S) {
         float4 a, b;
         mx_stage_xu(A, hidx[h], O, uo0, uo1, uo2, a, b);
         hmx[2 * h] = a;
@@ -2326,29 +2140,24 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_pass1_mx(pdx_step_args A)
     __syncthreads();
     const int sub = threadIdx.x % S;
     const int64_t p = p0 + threadIdx.x / S;
-    if (p >= A.n) return;  // all S lanes of the point together
-    const int c = A.cnt[p];
-    const int64_t b0 = pdx_bond0(A.slice_ptr, p);
-    uint16_t *const wbase = A.bw16 + b0;
-    const double4 ri = A.rec_in[p];
-    const double4 Xi = A.Xr[p];
+    const int64_t pq = p < A.n ? p : A.n - 1;
+    const pdx_lane<S, false> R = pdx_lane_of<S, false>(A, p0);
+    const double4 ri = A.rec_in[pq];
+    const double4 Xi = A.Xr[pq];
     const float xi = (float)(Xi.x - O.x), yi = (float)(Xi.y - O.y), zi = (float)(Xi.z - O.z);
     const float ui = (float)((ri.x - Xi.x) - uo0), vi = (float)((ri.y - Xi.y) - uo1),
                 wi = (float)((ri.z - Xi.z) - uo2);
-    const bool dead = A.killed[p] != 0;
+    const bool dead = A.killed[pq] != 0;
     double Km[6] = {0, 0, 0, 0, 0, 0};  // 00 10 20 11 21 22
     double Ht[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     int na = 0;
     const double epsc = A.epsc;
     const float epscf = (float)epsc, deltaf = (float)A.delta;
     const float win_lo = epscf * 0.9999f, win_hi = epscf * 1.0001f;
-    for (int t = sub; t < c; t += U * S) {
-        uint32_t wd[U];
+    pdx_walk4_mx(A, R, [&](const uint32_t (&wd)[4], int i) {
 #pragma unroll
-        for (int u = 0; u < U; u++) wd[u] = (t + u * S < c) ? wbase[(int64_t)(t + u * S) * 64] : 0u;
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            if (t + u * S >= c) continue;
+        for (int u = 0; u < 4; u++) {
+            if (i + u >= R.ng) continue;  // uniform
             const int slot = (int)(wd[u] & PDX_W16_SLOT);
             float4 a, b;
             if (!CAP || slot < HL) {
@@ -2368,20 +2177,10 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_pass1_mx(pdx_step_args A)
             const float rL = __builtin_amdgcn_rcpf(Lb);
             const float eps = (num * __builtin_amdgcn_rcpf(l + Lb)) * rL;
             bool act = (wd[u] & PDX_W16_ACT) != 0;
-            if (act && (wd[u] & PDX_W16_FP) && eps > win_lo) {
-                bool brk = eps > win_hi;
-                if (!brk) {
-                    const double L64 = A.L[b0 + (int64_t)(t + u * S) * 64];
-                    const double4 xj = A.rec_in[hidx[slot]];
-                    const double dx = xj.x - ri.x, dy = xj.y - ri.y, dz = xj.z - ri.z;
-                    double rl;
-                    const double l64 = pdx_sqrt_rsq((dx * dx + dy * dy) + dz * dz, rl);
-                    brk = ((l64 - L64) / L64) > epsc;
-                }
-                if (brk) {
-                    act = false;
-                    wbase[(int64_t)(t + u * S) * 64] = (uint16_t)(wd[u] & ~PDX_W16_ACT);
-                }
+            const int64_t o = R.at(i + u);
+            if (act && (wd[u] & PDX_W16_FP) && eps > win_lo && mx_breaks(A, hidx, wd[u], o, ri, eps, win_hi, epsc)) {
+                act = false;
+                A.bw16[o] = (uint16_t)(wd[u] & ~PDX_W16_ACT);
             }
             if (act && !dead) {
                 na++;
@@ -2399,16 +2198,14 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_pass1_mx(pdx_step_args A)
                     for (int r = 0; r < 3; r++) Ht[r + 3 * cc] += (double)(Uv[r] * wD[cc]);
             }
         }
-    }
+    });
 #pragma unroll
-    for (int o = 1; o < S; o <<= 1) {
+    for (int q = 0; q < 6; q++) pdx_fold(R, Km[q]);
 #pragma unroll
-        for (int q = 0; q < 6; q++) Km[q] += __shfl_xor(Km[q], o);
-#pragma unroll
-        for (int q = 0; q < 9; q++) Ht[q] += __shfl_xor(Ht[q], o);
-        na += __shfl_xor(na, o);
-    }
-    if (sub != 0) return;
+    for (int q = 0; q < 9; q++) pdx_fold(R, Ht[q]);
+    pdx_fold(R, na);
+    if (p >= A.n || sub != 0) return;
+    const int c = A.cnt[p];
     const double K9[9] = {Km[0], Km[1], Km[2], Km[1], Km[3], Km[4], Km[2], Km[4], Km[5]};
     double Kinv[9], Hm[9], Fm[9];
     m3_inv(K9, Kinv);
@@ -2460,23 +2257,24 @@ __device__ __forceinline__ void cpd_mx_entry(const pdx_step_args &A, int64_t j, 
     for (int r = 0; r < 9; r++) q[r] = live ? (float)A.pstate[9 * j + r] : 0.f;
 }
 
-template <int U, int S, int F>
-__global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_pass2_mx(pdx_step_args A)
+template <int S, int F, int PB>
+__global__ __launch_bounds__(PB * S) void k_cpd_pass2_mx(pdx_step_args A)
 {
     constexpr bool CAP = (F & PDX_FEAT_CAP) != 0;
     extern __shared__ float4 hmx[];  // [4 HL]: (D, V), (U, beta l), q0-3, q4-7; then q8 [HL]
     const int64_t k = pdx_xcd_block();
-    const int64_t p0 = k * PDX_BLOCK;
+    const int64_t p0 = k * PB;
     if (p0 >= A.n) return;  // whole workgroup
     const int64_t h0 = A.halo_ptr[k];
     const int H = (int)(A.halo_ptr[k + 1] - h0);
-    const double4 O = A.Xr[p0], xo = A.rec_in[p0];
+    const int64_t po = p0 & ~(int64_t)(PDX_BLOCK - 1);
+    const double4 O = A.Xr[po], xo = A.rec_in[po];
     const double uo0 = xo.x - O.x, uo1 = xo.y - O.y, uo2 = xo.z - O.z;
     const int HL = CAP ? pdx_lds_entries(A.halo_max, A.lds_budget, 68) : A.halo_max;
     const int Hs = H < HL ? H : HL;
     const int32_t *const hidx = A.halo + h0;
     float *const hq8 = reinterpret_cast<float *>(hmx + 4 * HL);
-    for (int h = threadIdx.x; h < Hs; h += PDX_BLOCK * S) {
+    for (int h = threadIdx.x; h < Hs; h += PB * S) {
         float4 a, b;
         float q[9];
         cpd_mx_entry(A, hidx[h], O, uo0, uo1, uo2, a, b, q);
@@ -2489,29 +2287,24 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_pass2_mx(pdx_step_args A)
     __syncthreads();
     const int sub = threadIdx.x % S;
     const int64_t p = p0 + threadIdx.x / S;
-    if (p >= A.n) return;  // all S lanes of the point together
-    const int c = A.cnt[p];
-    const int64_t b0 = pdx_bond0(A.slice_ptr, p);
-    const uint16_t *const wbase = A.bw16 + b0;
-    const double4 ri = A.rec_in[p];
-    const double4 Xi = A.Xr[p];
+    const int64_t pq = p < A.n ? p : A.n - 1;
+    const pdx_lane<S, false> R = pdx_lane_of<S, false>(A, p0);
+    const double4 ri = A.rec_in[pq];
+    const double4 Xi = A.Xr[pq];
     const float xi = (float)(Xi.x - O.x), yi = (float)(Xi.y - O.y), zi = (float)(Xi.z - O.z);
     const float ui = (float)((ri.x - Xi.x) - uo0), vi = (float)((ri.y - Xi.y) - uo1),
                 wi = (float)((ri.z - Xi.z) - uo2);
-    const bool live_i = !A.killed[p];
+    const bool live_i = !A.killed[pq];
     const float beta_i = live_i ? (float)A.beta_zem : 0.f;
     float Qi[9];
 #pragma unroll
-    for (int r = 0; r < 9; r++) Qi[r] = live_i ? (float)A.pstate[9 * p + r] : 0.f;
+    for (int r = 0; r < 9; r++) Qi[r] = live_i ? (float)A.pstate[9 * pq + r] : 0.f;
     const float deltaf = (float)A.delta;
     double b3[3] = {0.0, 0.0, 0.0};
-    for (int t = sub; t < c; t += U * S) {
-        uint32_t wd[U];
+    pdx_walk4_mx(A, R, [&](const uint32_t (&wd)[4], int i) {
 #pragma unroll
-        for (int u = 0; u < U; u++) wd[u] = (t + u * S < c) ? wbase[(int64_t)(t + u * S) * 64] : 0u;
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            if (t + u * S >= c) continue;
+        for (int u = 0; u < 4; u++) {
+            if (i + u >= R.ng) continue;  // uniform
             if (!(wd[u] & PDX_W16_ACT)) continue;
             const int slot = (int)(wd[u] & PDX_W16_SLOT);
             float4 a, b;
@@ -2539,12 +2332,10 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_pass2_mx(pdx_step_args A)
                 b3[r] += (double)(wv * tt);
             }
         }
-    }
+    });
 #pragma unroll
-    for (int o = 1; o < S; o <<= 1)
-#pragma unroll
-        for (int r = 0; r < 3; r++) b3[r] += __shfl_xor(b3[r], o);
-    static_assert(S == 4, "the tail takes four lanes per point");
+    for (int r = 0; r < 3; r++) pdx_fold(R, b3[r]);
+    if (p >= A.n || sub >= 4) return;  // the tail takes four lanes per point
     point_tail4(A, p, ri, b3, sub, A.rho);
 }
 
@@ -2588,7 +2379,7 @@ pdx_status pdx_fill_step_args(pdx_ctx *c, pdx_step_args *a, int64_t step, int fl
     a->rho = c->P.rho;
     a->dt = dt;
     a->dth = 0.5 * dt;
-    a->slice_ptr = c->slice_ptr;
+    a->rows = c->rows();
     a->cnt = c->cnt;
     a->bw = c->bw;
     a->bw16 = c->bw16;
@@ -2623,7 +2414,15 @@ pdx_status pdx_fill_step_args(pdx_ctx *c, pdx_step_args *a, int64_t step, int fl
     // (l - L) / L; outside [epsc_lo, epsc_hi] the two compare equal against eps_c, inside
     // the kernel takes the correctly rounded quotient
     a->epsc_lo = c->P.epsc - 1e-11 * fabs(c->P.epsc);
+    a->epsc_lo_min = a->epsc_lo;
+    for (const pdx_params &q : c->psets)
+        a->epsc_lo_min = std::min(a->epsc_lo_min, q.epsc - 1e-11 * fabs(q.epsc));
     a->epsc_hi = c->P.epsc + 1e-11 * fabs(c->P.epsc);
+    a->pk = c->pk;
+    a->pk_shift = c->pk_shift;
+    a->pk_mask = c->pk_mask;
+    a->pk_base = c->pk_base;
+    a->fp = c->d_fp;
     a->delta = c->P.delta;
     a->G = c->P.G;
     a->K = c->P.K;
@@ -2684,38 +2483,54 @@ static int kernel_vgprs(const void *fn)
     return v;
 }
 
-// Launch of an LDS-staged kernel whose table entries take `entry` bytes.  A capped variant
-// (tables longer than the budget) whose registers allow one block per CU anyway may take the
-// CU's whole LDS.  Measured at 576 k points: a tiled kernel gains from fewer tiles whenever
-// the table is longer than the budget; a kernel that reads the entries past the budget from
-// global memory gains once they are many (horizon 5.015 dx: ~80 % past the budget) and
-// loses a little when they are few (4.015 dx: ~15 %).
-static void launch_lds(pdx_ctx *c, const void *fn, bool capped, bool tiled, int entry, dim3 G,
-                       dim3 BL, const pdx_step_args &a)
+// Points per block and lanes per point of the LDS-staged kernels (c->cfg).
+template <int PB_, int S_>
+struct blk_cfg {
+    static constexpr int PB = PB_, S = S_;
+};
+template <class FN>
+static void with_cfg(const pdx_ctx *c, FN &&f)
+{
+    switch (c->cfg) {
+    case 1: f(blk_cfg<128, 4>{}); break;
+    case 2: f(blk_cfg<64, 8>{}); break;
+    case 3: f(blk_cfg<32, 16>{}); break;
+    default: f(blk_cfg<256, 4>{}); break;
+    }
+}
+
+// Launch of an LDS-staged kernel whose table entries take `entry` bytes, `bud` bytes of LDS
+// per block at the most.
+template <class CFG>
+static void launch_lds_bud(pdx_ctx *c, const void *fn, int entry, int bud, const pdx_step_args &a)
 {
     pdx_step_args af = a;
+    af.lds_budget = bud;
+    void *args[] = {&af};
+    const int64_t blocks = (c->n + CFG::PB - 1) / CFG::PB;
+    const dim3 G((unsigned)((blocks + PDX_NUM_XCD - 1) / PDX_NUM_XCD * PDX_NUM_XCD));
+    (void)hipLaunchKernel(fn, G, dim3(CFG::PB * CFG::S), args, lds_bytes(c, entry, bud), c->stream);
+}
+
+// A capped variant (tables longer than the budget) whose registers allow one block per CU
+// anyway may take the CU's whole LDS.  Measured at 576 k points: a tiled kernel gains from
+// fewer tiles whenever the table is longer than the budget; a kernel that reads the entries
+// past the budget from global memory gains once they are many (horizon 5.015 dx: ~80 % past
+// the budget) and loses a little when they are few (4.015 dx: ~15 %).
+template <class CFG>
+static void launch_lds(pdx_ctx *c, const void *fn, bool capped, bool tiled, int entry, const pdx_step_args &a)
+{
     int bud = pdx_lds_budget(c);
     const bool many_past = (int64_t)c->halo_max * entry > (int64_t)bud * 3 / 2;
     if (capped && (tiled || many_past) && kernel_vgprs(fn) > 64) bud = pdx_lds_budget_full(c);
-    af.lds_budget = bud;
-    void *args[] = {&af};
-    (void)hipLaunchKernel(fn, G, BL, args, lds_bytes(c, entry, bud), c->stream);
-}
-
-template <int F>
-static void launch_bb_feat(pdx_ctx *c, bool mixed, dim3 G, dim3 BL, size_t lds, const pdx_step_args &a)
-{
-    if (mixed && (F & PDX_FEAT_CAP))
-        launch_lds(c, (const void *)&k_bb_lds_mx<4, PDX_LDS_LANES, F>, true, false,
-                   32 + ((F & PDX_FEAT_MULTI) ? 1 : 0), G, BL, a);
-    else if (mixed) hipLaunchKernelGGL((k_bb_lds_mx<4, PDX_LDS_LANES, F>), G, BL, lds, c->stream, a);
-    else hipLaunchKernelGGL((k_bb_lds<2, PDX_LDS_LANES, F>), G, BL, lds, c->stream, a);
+    launch_lds_bud<CFG>(c, fn, entry, bud, a);
 }
 
 // feature masks 1..7 (PDX_FEAT_MULTI | PDX_FEAT_SC | PDX_FEAT_CAP); for OSB also those with
 // PDX_FEAT_KERN
 #define PDX_FEAT_SWITCH(feat, CALL)                                                         \
     switch (feat) {                                                                         \
+    case 0: CALL(0); break;                                                                 \
     case 1: CALL(1); break;                                                                 \
     case 2: CALL(2); break;                                                                 \
     case 3: CALL(3); break;                                                                 \
@@ -2738,12 +2553,56 @@ static void launch_bb_feat(pdx_ctx *c, bool mixed, dim3 G, dim3 BL, size_t lds, 
     default: PDX_FEAT_SWITCH(feat, CALL)                                                    \
     }
 
-template <int F>
-static void launch_osb_feat(pdx_ctx *c, int pass, dim3 G, dim3 BL, int entry, const pdx_step_args &a)
+template <int F, class CFG>
+static void launch_bb(pdx_ctx *c, CFG, bool mixed, int entry, const pdx_step_args &a)
 {
-    const void *fn = pass == 1 ? (const void *)&k_osb_lds1<PDX_LDS_LANES, F>
-                               : (const void *)&k_osb_lds2<PDX_LDS_LANES, F>;
-    launch_lds(c, fn, (F & PDX_FEAT_CAP) != 0, true, entry, G, BL, a);
+    // bonds per lane and unrolled iteration: the FP32 bond arithmetic of the mixed step is
+    // short enough that four loads in flight pay; FP64 is indifferent
+    const void *fn;
+    if (mixed) fn = (const void *)&k_bb_lds_mx<CFG::S, F, CFG::PB>;
+    else if constexpr (F & PDX_FEAT_MULTI) fn = (const void *)&k_bb_lds<2, CFG::S, F, CFG::PB, false>;
+    else fn = c->pk ? (const void *)&k_bb_lds<2, CFG::S, F, CFG::PB, true>
+                    : (const void *)&k_bb_lds<2, CFG::S, F, CFG::PB, false>;
+    if (mixed && (F & PDX_FEAT_CAP)) launch_lds<CFG>(c, fn, true, false, entry, a);
+    else launch_lds_bud<CFG>(c, fn, entry, pdx_lds_budget(c), a);
+}
+
+template <int F, class CFG>
+static void launch_osb(pdx_ctx *c, CFG, int pass, int entry, const pdx_step_args &a)
+{
+    const void *fn = pass == 1 ? (const void *)&k_osb_lds1<CFG::S, F, CFG::PB, false>
+                               : (const void *)&k_osb_lds2<CFG::S, F, CFG::PB, false>;
+    if constexpr (!(F & PDX_FEAT_MULTI))
+        if (c->pk) fn = pass == 1 ? (const void *)&k_osb_lds1<CFG::S, F, CFG::PB, true>
+                                  : (const void *)&k_osb_lds2<CFG::S, F, CFG::PB, true>;
+    launch_lds<CFG>(c, fn, (F & PDX_FEAT_CAP) != 0, true, entry, a);
+}
+
+template <int F, class CFG>
+static void launch_osb_mx(pdx_ctx *c, CFG, int pass, int entry, const pdx_step_args &a)
+{
+    const void *fn = pass == 1 ? (const void *)&k_osb_lds1_mx<CFG::S, F, CFG::PB>
+                               : (const void *)&k_osb_lds2_mx<CFG::S, F, CFG::PB>;
+    launch_lds<CFG>(c, fn, (F & PDX_FEAT_CAP) != 0, false, entry, a);
+}
+
+template <int F, class CFG>
+static void launch_cpd(pdx_ctx *c, CFG, int pass, int entry, int bud, const pdx_step_args &a)
+{
+    const void *fn = pass == 1 ? (const void *)&k_cpd_lds1<CFG::S, F, CFG::PB, false>
+                               : (const void *)&k_cpd_lds2_own<CFG::S, F, CFG::PB, false>;
+    if constexpr (!(F & PDX_FEAT_MULTI))
+        if (c->pk) fn = pass == 1 ? (const void *)&k_cpd_lds1<CFG::S, F, CFG::PB, true>
+                                  : (const void *)&k_cpd_lds2_own<CFG::S, F, CFG::PB, true>;
+    launch_lds_bud<CFG>(c, fn, entry, bud, a);
+}
+
+template <int F, class CFG>
+static void launch_cpd_mx(pdx_ctx *c, CFG, int pass, int entry, int bud, const pdx_step_args &a)
+{
+    const void *fn = pass == 1 ? (const void *)&k_cpd_pass1_mx<CFG::S, F, CFG::PB>
+                               : (const void *)&k_cpd_pass2_mx<CFG::S, F, CFG::PB>;
+    launch_lds_bud<CFG>(c, fn, entry, bud, a);
 }
 
 bool pdx_bb_jv_fusable(const pdx_ctx *c)
@@ -2758,19 +2617,26 @@ pdx_status pdx_launch_bb_jv(pdx_ctx *c, const double *u, const double *v, const 
     if (!pdx_bb_jv_fusable(c)) return pdx_fail(c, PDX_ERR_UNSUPPORTED, "fused J v: layout not supported");
     pdx_step_args a;
     PDX_TRY(pdx_fill_step_args(c, &a, 0, PDX_F_FORCE_ONLY | PDX_F_SCALE_VOL | PDX_F_FP64, 0.0, nullptr));
-    const int64_t blocks = (c->n + PDX_BLOCK - 1) / PDX_BLOCK;
-    const dim3 G((unsigned)((blocks + PDX_NUM_XCD - 1) / PDX_NUM_XCD * PDX_NUM_XCD));
-    const dim3 BL(PDX_BLOCK * PDX_LDS_LANES);
     const size_t two = (size_t)std::max(c->halo_max, 1) * 64 + 16;
     const char *env = std::getenv("PDX_JV_ONE_PASS");
     // (the static LDS of the sum adds 128 bytes)
     const bool one_pass = (int64_t)two + 256 <= c->lds_limit && !(env && env[0] == '0');
-    if (one_pass)
-        hipLaunchKernelGGL((k_bb_jv1<4, PDX_LDS_LANES>), G, BL, two, c->stream, a, u, v, un2, parts, np, sc,
-                           cmask, jv);
-    else
-        hipLaunchKernelGGL((k_bb_jv<2, PDX_LDS_LANES>), G, BL, lds_bytes(c, 32), c->stream, a, u, v, un2,
-                           parts, np, sc, cmask, jv);
+    with_cfg(c, [&](auto g) {
+        constexpr int PB = decltype(g)::PB, S = decltype(g)::S;
+        const int64_t blocks = (c->n + PB - 1) / PB;
+        const dim3 G((unsigned)((blocks + PDX_NUM_XCD - 1) / PDX_NUM_XCD * PDX_NUM_XCD));
+        const size_t lds = one_pass ? two : lds_bytes(c, 32);
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, G, dim3(PB * S), lds, c->stream, a, u, v, un2, parts, np, sc, cmask, jv);
+        };
+        if (c->pk) {
+            if (one_pass) go(k_bb_jv<S, PB, true, true>);
+            else go(k_bb_jv<S, PB, true, false>);
+        } else {
+            if (one_pass) go(k_bb_jv<S, PB, false, true>);
+            else go(k_bb_jv<S, PB, false, false>);
+        }
+    });
     PDX_HIP(c, hipGetLastError());
     return PDX_OK;
 }
@@ -2781,38 +2647,23 @@ pdx_status pdx_launch_step(pdx_ctx *c, const pdx_step_args &a)
     const bool mixed = c->precision == PDX_MIXED && !(a.flags & PDX_F_FP64);
     const int64_t blocks = (c->n + PDX_BLOCK - 1) / PDX_BLOCK;
     const dim3 G((unsigned)((blocks + PDX_NUM_XCD - 1) / PDX_NUM_XCD * PDX_NUM_XCD)), B(PDX_BLOCK);
+    const int cap32 = lds_capped(c, 32) ? PDX_FEAT_CAP : 0;
+    if (c->multi() && !c->d_psets)
+        return pdx_fail(c, PDX_ERR_STATE, "the parameter sets were set after pdx_build_bonds");
     switch (c->kind) {
     case PDX_BB:
         PDX_TRY(pdx_timed_begin(c));
         if (c->lds_mode) {
-            const size_t lds = lds_bytes(c, 32);
-            // four lanes per point (the halo table of a block limits the blocks per CU, so
-            // the lanes, not the blocks, supply the parallelism that hides the bond loads)
-            const dim3 BL(PDX_BLOCK * PDX_LDS_LANES);
-            // bonds per lane and unrolled iteration: the FP32 bond arithmetic of the mixed
-            // step is short enough that four loads in flight pay; FP64 is indifferent
-            const bool u4 = c->bb_unroll ? c->bb_unroll == 4 : mixed;
             // with several parameter sets each neighbour-table entry also carries the
             // neighbour's set
-            const int entry = 32 + (c->multi() ? 1 : 0);
+            const int entry = 32 + (c->multi() ? (mixed ? 1 : 8) : 0);
             const int feat = pdx_features(c) | (lds_capped(c, entry) ? PDX_FEAT_CAP : 0);
-            const size_t ldsf = lds_bytes(c, entry);
-#define PDX_BB_LAUNCH(F) launch_bb_feat<F>(c, mixed, G, BL, ldsf, a)
-            if (feat) {
-                PDX_FEAT_SWITCH(feat, PDX_BB_LAUNCH)
-            } else if (mixed) {
-                if (u4) hipLaunchKernelGGL((k_bb_lds_mx<4, PDX_LDS_LANES, 0>), G, BL, lds, c->stream, a);
-                else hipLaunchKernelGGL((k_bb_lds_mx<2, PDX_LDS_LANES, 0>), G, BL, lds, c->stream, a);
-            } else {
-                if (u4) hipLaunchKernelGGL((k_bb_lds<4, PDX_LDS_LANES, 0>), G, BL, lds, c->stream, a);
-                else hipLaunchKernelGGL((k_bb_lds<2, PDX_LDS_LANES, 0>), G, BL, lds, c->stream, a);
-            }
+#define PDX_BB_LAUNCH(F) with_cfg(c, [&](auto g) { launch_bb<F>(c, g, mixed, entry, a); })
+            PDX_FEAT_SWITCH(feat, PDX_BB_LAUNCH)
         } else if (mixed) {
-            if (c->bb_unroll == 4) hipLaunchKernelGGL((k_bb_step<true, 4>), G, B, 0, c->stream, a);
-            else hipLaunchKernelGGL((k_bb_step<true, 2>), G, B, 0, c->stream, a);
+            hipLaunchKernelGGL((k_bb_step<true, 2>), G, B, 0, c->stream, a);
         } else {
-            if (c->bb_unroll == 4) hipLaunchKernelGGL((k_bb_step<false, 4>), G, B, 0, c->stream, a);
-            else hipLaunchKernelGGL((k_bb_step<false, 2>), G, B, 0, c->stream, a);
+            hipLaunchKernelGGL((k_bb_step<false, 2>), G, B, 0, c->stream, a);
         }
         PDX_HIP(c, hipGetLastError());
         PDX_TRY(pdx_timed_end(c, "step"));
@@ -2820,58 +2671,36 @@ pdx_status pdx_launch_step(pdx_ctx *c, const pdx_step_args &a)
     case PDX_OSB:
         // (an influence function other than linear_kernel runs the FP64 passes)
         if (c->lds_mode && mixed && !c->multi() && c->P.kernel == PDX_KERNEL_LINEAR) {
-            const dim3 BL(PDX_BLOCK * PDX_LDS_LANES);
             // pass 1 entries (D, V), (U, 0): 32 B; pass 2 also (c2 V)_j: 36 B
             const int sc = c->corr ? PDX_FEAT_SC : 0;
-            const int feat = sc | (lds_capped(c, 32) ? PDX_FEAT_CAP : 0);
-            const int feat2 = sc | (lds_capped(c, 36) ? PDX_FEAT_CAP : 0);
-            const size_t lds = lds_bytes(c, 32), lds2 = lds_bytes(c, 36);
-            PDX_TRY(pdx_timed_begin(c));
-            switch (feat) {
-            case 0: hipLaunchKernelGGL((k_osb_lds1_mx<4, PDX_LDS_LANES, 0>), G, BL, lds, c->stream, a); break;
-            case PDX_FEAT_SC: hipLaunchKernelGGL((k_osb_lds1_mx<4, PDX_LDS_LANES, PDX_FEAT_SC>), G, BL, lds, c->stream, a); break;
-            case PDX_FEAT_CAP: launch_lds(c, (const void *)&k_osb_lds1_mx<4, PDX_LDS_LANES, PDX_FEAT_CAP>, true, false, 32, G, BL, a); break;
-            default: launch_lds(c, (const void *)&k_osb_lds1_mx<4, PDX_LDS_LANES, PDX_FEAT_SC | PDX_FEAT_CAP>, true, false, 32, G, BL, a); break;
+            const int feat[2] = {sc | cap32, sc | (lds_capped(c, 36) ? PDX_FEAT_CAP : 0)};
+            for (int pass = 1; pass <= 2; pass++) {
+                const int entry = pass == 1 ? 32 : 36;
+#define PDX_OSBMX_LAUNCH(F) with_cfg(c, [&](auto g) { launch_osb_mx<F>(c, g, pass, entry, a); })
+                PDX_TRY(pdx_timed_begin(c));
+                switch (feat[pass - 1]) {
+                case 0: PDX_OSBMX_LAUNCH(0); break;
+                case PDX_FEAT_SC: PDX_OSBMX_LAUNCH(PDX_FEAT_SC); break;
+                case PDX_FEAT_CAP: PDX_OSBMX_LAUNCH(PDX_FEAT_CAP); break;
+                default: PDX_OSBMX_LAUNCH(PDX_FEAT_SC | PDX_FEAT_CAP); break;
+                }
+                PDX_HIP(c, hipGetLastError());
+                PDX_TRY(pdx_timed_end(c, pass == 1 ? "pass1" : "step"));
             }
-            PDX_HIP(c, hipGetLastError());
-            PDX_TRY(pdx_timed_end(c, "pass1"));
-            PDX_TRY(pdx_timed_begin(c));
-            switch (feat2) {
-            case 0: hipLaunchKernelGGL((k_osb_lds2_mx<4, PDX_LDS_LANES, 0>), G, BL, lds2, c->stream, a); break;
-            case PDX_FEAT_SC: hipLaunchKernelGGL((k_osb_lds2_mx<4, PDX_LDS_LANES, PDX_FEAT_SC>), G, BL, lds2, c->stream, a); break;
-            case PDX_FEAT_CAP: launch_lds(c, (const void *)&k_osb_lds2_mx<4, PDX_LDS_LANES, PDX_FEAT_CAP>, true, false, 36, G, BL, a); break;
-            default: launch_lds(c, (const void *)&k_osb_lds2_mx<4, PDX_LDS_LANES, PDX_FEAT_SC | PDX_FEAT_CAP>, true, false, 36, G, BL, a); break;
-            }
-            PDX_HIP(c, hipGetLastError());
-            PDX_TRY(pdx_timed_end(c, "step"));
             break;
         }
         if (c->lds_mode) {
-            const dim3 BL(PDX_BLOCK * PDX_LDS_LANES);
             const int mb = c->multi() ? 1 : 0;  // the neighbours' parameter sets
-            // pass 2 entries: x and (c1 V, c2 V) with one set, x|V, (wvol, dil) and the set
-            const int e2 = mb ? 48 + mb : 40;
-            const int e1 = 32 + mb;
-            const int f1 = pdx_features(c) | (lds_capped(c, e1) ? PDX_FEAT_CAP : 0);
-            const int f2 = pdx_features(c) | (lds_capped(c, e2) ? PDX_FEAT_CAP : 0);
-#define PDX_OSB1_LAUNCH(F) launch_osb_feat<F>(c, 1, G, BL, e1, a)
-#define PDX_OSB2_LAUNCH(F) launch_osb_feat<F>(c, 2, G, BL, e2, a)
-            PDX_TRY(pdx_timed_begin(c));
-            if (f1) {
-                PDX_FEAT_SWITCH_OSB(f1, PDX_OSB1_LAUNCH)
-            } else {
-                launch_osb_feat<0>(c, 1, G, BL, e1, a);
+            for (int pass = 1; pass <= 2; pass++) {
+                // pass 2 entries: x and (c1 V, c2 V) with one set, x|V, (wvol, dil) and the set
+                const int entry = pass == 1 ? 32 + mb : (mb ? 64 : 40);
+                const int feat = pdx_features(c) | (lds_capped(c, entry) ? PDX_FEAT_CAP : 0);
+#define PDX_OSB_LAUNCH(F) with_cfg(c, [&](auto g) { launch_osb<F>(c, g, pass, entry, a); })
+                PDX_TRY(pdx_timed_begin(c));
+                PDX_FEAT_SWITCH_OSB(feat, PDX_OSB_LAUNCH)
+                PDX_HIP(c, hipGetLastError());
+                PDX_TRY(pdx_timed_end(c, pass == 1 ? "pass1" : "step"));
             }
-            PDX_HIP(c, hipGetLastError());
-            PDX_TRY(pdx_timed_end(c, "pass1"));
-            PDX_TRY(pdx_timed_begin(c));
-            if (f2) {
-                PDX_FEAT_SWITCH_OSB(f2, PDX_OSB2_LAUNCH)
-            } else {
-                launch_osb_feat<0>(c, 2, G, BL, e2, a);
-            }
-            PDX_HIP(c, hipGetLastError());
-            PDX_TRY(pdx_timed_end(c, "step"));
             break;
         }
         PDX_TRY(pdx_timed_begin(c));
@@ -2887,51 +2716,37 @@ pdx_status pdx_launch_step(pdx_ctx *c, const pdx_step_args &a)
         if (c->lds_mode) {
             // The CPD passes hold 97-122 VGPRs, so one 1024-thread block runs per CU: their
             // tables take the CU's whole LDS (fewer tiles, fewer entries read past the cap).
-            pdx_step_args af = a;
             const int bud = pdx_lds_budget_full(c);
-            af.lds_budget = bud;
-            const dim3 BL(PDX_BLOCK * PDX_LDS_LANES);
             if (mixed && !c->multi() && c->P.zem != PDX_ZEM_WAN &&
                 c->P.kernel == PDX_KERNEL_LINEAR) {  // otherwise the FP64 passes
-                // pass 1 entries (D, V), (U, 0): 32 B; pass 2 (D, V), (U, beta l), l Q': 68 B
-                const size_t l1 = lds_bytes(c, 32, bud), l2b = lds_bytes(c, 68, bud);
-                PDX_TRY(pdx_timed_begin(c));
-                if (lds_capped(c, 32, bud))
-                    hipLaunchKernelGGL((k_cpd_pass1_mx<1, PDX_LDS_LANES, PDX_FEAT_CAP>), G, BL, l1, c->stream, af);
-                else
-                    hipLaunchKernelGGL((k_cpd_pass1_mx<1, PDX_LDS_LANES, 0>), G, BL, l1, c->stream, af);
-                PDX_HIP(c, hipGetLastError());
-                PDX_TRY(pdx_timed_end(c, "pass1"));
-                PDX_TRY(pdx_timed_begin(c));
-                if (lds_capped(c, 68, bud))
-                    hipLaunchKernelGGL((k_cpd_pass2_mx<2, PDX_LDS_LANES, PDX_FEAT_CAP>), G, BL, l2b, c->stream, af);
-                else
-                    hipLaunchKernelGGL((k_cpd_pass2_mx<2, PDX_LDS_LANES, 0>), G, BL, l2b, c->stream, af);
-                PDX_HIP(c, hipGetLastError());
-                PDX_TRY(pdx_timed_end(c, "step"));
+                for (int pass = 1; pass <= 2; pass++) {
+                    // pass 1 entries (D, V), (U, 0): 32 B; pass 2 (D, V), (U, beta l), l Q': 68 B
+                    const int entry = pass == 1 ? 32 : 68;
+                    PDX_TRY(pdx_timed_begin(c));
+                    with_cfg(c, [&](auto g) {
+                        if (lds_capped(c, entry, bud)) launch_cpd_mx<PDX_FEAT_CAP>(c, g, pass, entry, bud, a);
+                        else launch_cpd_mx<0>(c, g, pass, entry, bud, a);
+                    });
+                    PDX_HIP(c, hipGetLastError());
+                    PDX_TRY(pdx_timed_end(c, pass == 1 ? "pass1" : "step"));
+                }
                 break;
             }
             const int fc = (c->multi() ? PDX_FEAT_MULTI : 0) | (c->P.zem == PDX_ZEM_WAN ? PDX_FEAT_ZW : 0);
-            // pass 2 entries 112 B, 160 B with ZEMWan
-            const int e1 = 64 + (c->multi() ? 1 : 0), e2 = c->P.zem == PDX_ZEM_WAN ? 160 : 112;
-            PDX_TRY(pdx_timed_begin(c));
-            switch (fc) {
-            case 0: hipLaunchKernelGGL((k_cpd_lds1<PDX_LDS_LANES, 0>), G, BL, lds_bytes(c, e1, bud), c->stream, af); break;
-            case PDX_FEAT_MULTI: hipLaunchKernelGGL((k_cpd_lds1<PDX_LDS_LANES, PDX_FEAT_MULTI>), G, BL, lds_bytes(c, e1, bud), c->stream, af); break;
-            case PDX_FEAT_ZW: hipLaunchKernelGGL((k_cpd_lds1<PDX_LDS_LANES, PDX_FEAT_ZW>), G, BL, lds_bytes(c, e1, bud), c->stream, af); break;
-            default: hipLaunchKernelGGL((k_cpd_lds1<PDX_LDS_LANES, PDX_FEAT_MULTI | PDX_FEAT_ZW>), G, BL, lds_bytes(c, e1, bud), c->stream, af); break;
+            for (int pass = 1; pass <= 2; pass++) {
+                // pass 2 entries 112 B, 160 B with ZEMWan
+                const int entry = pass == 1 ? 64 + (c->multi() ? 1 : 0) : (c->P.zem == PDX_ZEM_WAN ? 160 : 112);
+#define PDX_CPD_LAUNCH(F) with_cfg(c, [&](auto g) { launch_cpd<F>(c, g, pass, entry, bud, a); })
+                PDX_TRY(pdx_timed_begin(c));
+                switch (fc) {
+                case 0: PDX_CPD_LAUNCH(0); break;
+                case PDX_FEAT_MULTI: PDX_CPD_LAUNCH(PDX_FEAT_MULTI); break;
+                case PDX_FEAT_ZW: PDX_CPD_LAUNCH(PDX_FEAT_ZW); break;
+                default: PDX_CPD_LAUNCH(PDX_FEAT_MULTI | PDX_FEAT_ZW); break;
+                }
+                PDX_HIP(c, hipGetLastError());
+                PDX_TRY(pdx_timed_end(c, pass == 1 ? "pass1" : "step"));
             }
-            PDX_HIP(c, hipGetLastError());
-            PDX_TRY(pdx_timed_end(c, "pass1"));
-            PDX_TRY(pdx_timed_begin(c));
-            switch (fc) {
-            case 0: hipLaunchKernelGGL((k_cpd_lds2_own<PDX_LDS_LANES, 0>), G, BL, lds_bytes(c, e2, bud), c->stream, af); break;
-            case PDX_FEAT_MULTI: hipLaunchKernelGGL((k_cpd_lds2_own<PDX_LDS_LANES, PDX_FEAT_MULTI>), G, BL, lds_bytes(c, e2, bud), c->stream, af); break;
-            case PDX_FEAT_ZW: hipLaunchKernelGGL((k_cpd_lds2_own<PDX_LDS_LANES, PDX_FEAT_ZW>), G, BL, lds_bytes(c, e2, bud), c->stream, af); break;
-            default: hipLaunchKernelGGL((k_cpd_lds2_own<PDX_LDS_LANES, PDX_FEAT_MULTI | PDX_FEAT_ZW>), G, BL, lds_bytes(c, e2, bud), c->stream, af); break;
-            }
-            PDX_HIP(c, hipGetLastError());
-            PDX_TRY(pdx_timed_end(c, "step"));
             break;
         }
         PDX_TRY(pdx_timed_begin(c));

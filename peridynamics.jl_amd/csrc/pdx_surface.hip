@@ -10,7 +10,7 @@
 //   scfactor (calc_scfactor!, :161-204): per bond, the ellipsoid radius of the two ends'
 //     mean mfactors along the bond's direction angles theta, phi.
 //
-// One thread per point walks its SELL-64 row; the sums run in the device row order
+// One thread per point walks its row; the sums run in the device row order
 // (Morton order of the neighbours), so they agree with the reference's bond order to
 // rounding.  The step kernels then multiply every bond's weight by scfactor.
 #include <algorithm>
@@ -20,11 +20,6 @@
 #include "pdx_internal.h"
 
 #define ESC_STRETCH 1.001
-
-__device__ __forceinline__ int64_t esc_bond0(const int64_t *slice_ptr, int64_t p)
-{
-    return slice_ptr[p >> 6] + (p & 63);
-}
 
 // lambda, mu, bc, G, K of point i (several sets or one)
 struct esc_par {
@@ -52,7 +47,7 @@ __device__ __forceinline__ double esc_omega(int kid, double delta, double L)
     return kid == PDX_KERNEL_LINEAR ? delta / L : pdx_omega_other(kid, delta, L);
 }
 
-__global__ void k_esc_mfactor(int64_t n, int d, int32_t kind, int kid, const int64_t *slice_ptr,
+__global__ void k_esc_mfactor(int64_t n, int d, int32_t kind, int kid, pdx_rows rows,
                               const int32_t *cnt, const uint32_t *bw, const double *L,
                               const double4 *Xr, double delta, esc_par one, const pdx_pset *ps,
                               const uint8_t *pid, double *mfactor)
@@ -60,7 +55,7 @@ __global__ void k_esc_mfactor(int64_t n, int d, int32_t kind, int kid, const int
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int c = cnt[i];
-    const int64_t b0 = esc_bond0(slice_ptr, i);
+    const int64_t b0 = rows.row(i);
     const esc_par Pi = esc_params(i, one, ps, pid);
     const double4 Xi = Xr[i];
     const double3 xi = esc_stretched(Xi, d);
@@ -71,7 +66,7 @@ __global__ void k_esc_mfactor(int64_t n, int d, int32_t kind, int kid, const int
         double sl = 0.0, sm = 0.0;
         int na = 0;
         for (int t = 0; t < c; t++) {
-            const uint32_t wd = bw[b0 + (int64_t)t * 64];
+            const uint32_t wd = bw[rows.at(b0, t)];
             if (!(wd & PDX_BW_ACT)) continue;
             const esc_par Pj = esc_params(wd & PDX_BW_NBR, one, ps, pid);
             sl += (Pi.lam + Pj.lam) / 2.0;
@@ -86,14 +81,14 @@ __global__ void k_esc_mfactor(int64_t n, int d, int32_t kind, int kid, const int
     double psi = 0.0;
     if (kind == PDX_BB) {
         for (int t = 0; t < c; t++) {
-            const int64_t b = b0 + (int64_t)t * 64;
+            const int64_t b = rows.at(b0, t);
             const uint32_t wd = bw[b];
             const int64_t j = wd & PDX_BW_NBR;
             const double4 Xj = Xr[j];
             const double3 xj = esc_stretched(Xj, d);
             const double dx = xj.x - xi.x, dy = xj.y - xi.y, dz = xj.z - xi.z;
             const double l = sqrt((dx * dx + dy * dy) + dz * dz);
-            const double Lb = L[b];
+            const double Lb = pdx_ref_len(L, b, Xi, Xj);
             const double eps = (l - Lb) / Lb;
             const double w = (wd & PDX_BW_ACT) ? 1.0 : 0.0;
             const double bcb = (Pi.bc + esc_params(j, one, ps, pid).bc) / 2.0;
@@ -102,38 +97,38 @@ __global__ void k_esc_mfactor(int64_t n, int d, int32_t kind, int kid, const int
     } else {  // PDX_OSB
         double wvol = 0.0;
         for (int t = 0; t < c; t++) {
-            const int64_t b = b0 + (int64_t)t * 64;
+            const int64_t b = rows.at(b0, t);
             const uint32_t wd = bw[b];
             const double4 Xj = Xr[wd & PDX_BW_NBR];
             const double Dx = Xj.x - Xi.x, Dy = Xj.y - Xi.y, Dz = Xj.z - Xi.z;
-            const double w = (wd & PDX_BW_ACT) ? esc_omega(kid, delta, L[b]) : 0.0;
+            const double w = (wd & PDX_BW_ACT) ? esc_omega(kid, delta, pdx_ref_len(L, b, Xi, Xj)) : 0.0;
             wvol += ((w * 1.0) * ((Dx * Dx + Dy * Dy) + Dz * Dz)) * Xj.w;
         }
         if (wvol != 0.0) {  // a point without weighted volume keeps psi = 0
             const double c1 = 3.0 / wvol;
             double dil = 0.0;
             for (int t = 0; t < c; t++) {
-                const int64_t b = b0 + (int64_t)t * 64;
+                const int64_t b = rows.at(b0, t);
                 const uint32_t wd = bw[b];
                 const double4 Xj = Xr[wd & PDX_BW_NBR];
                 const double3 xj = esc_stretched(Xj, d);
                 const double dx = xj.x - xi.x, dy = xj.y - xi.y, dz = xj.z - xi.z;
                 const double l = sqrt((dx * dx + dy * dy) + dz * dz);
-                const double Lb = L[b];
+                const double Lb = pdx_ref_len(L, b, Xi, Xj);
                 const double w = (wd & PDX_BW_ACT) ? esc_omega(kid, delta, Lb) : 0.0;
                 dil += ((((w * 1.0) * c1) * Lb) * (l - Lb)) * Xj.w;
             }
             const double psi_vol = (0.5 * Pi.K) * (dil * dil);
             double psi_dev = 0.0;
             for (int t = 0; t < c; t++) {
-                const int64_t b = b0 + (int64_t)t * 64;
+                const int64_t b = rows.at(b0, t);
                 const uint32_t wd = bw[b];
                 const int64_t j = wd & PDX_BW_NBR;
                 const double4 Xj = Xr[j];
                 const double3 xj = esc_stretched(Xj, d);
                 const double dx = xj.x - xi.x, dy = xj.y - xi.y, dz = xj.z - xi.z;
                 const double l = sqrt((dx * dx + dy * dy) + dz * dz);
-                const double Lb = L[b];
+                const double Lb = pdx_ref_len(L, b, Xi, Xj);
                 const double e = l - Lb;
                 const double edev = e - ((1.0 / 3.0) * dil) * Lb;
                 const double w = (wd & PDX_BW_ACT) ? esc_omega(kid, delta, Lb) : 0.0;
@@ -147,18 +142,18 @@ __global__ void k_esc_mfactor(int64_t n, int d, int32_t kind, int kid, const int
     mfactor[(int64_t)d * n + i] = psi_t / psi;
 }
 
-__global__ void k_esc_scfactor(int64_t n, const int64_t *slice_ptr, const int32_t *cnt,
+__global__ void k_esc_scfactor(int64_t n, pdx_rows rows, const int32_t *cnt,
                                const uint32_t *bw, const double *L, const double4 *Xr,
                                const double *mfactor, double *scf, float *scf32)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int c = cnt[i];
-    const int64_t b0 = esc_bond0(slice_ptr, i);
+    const int64_t b0 = rows.row(i);
     const double4 Xi = Xr[i];
     const double right = (90.0 * M_PI) / 180.0;
     for (int t = 0; t < c; t++) {
-        const int64_t b = b0 + (int64_t)t * 64;
+        const int64_t b = rows.at(b0, t);
         const int64_t j = bw[b] & PDX_BW_NBR;
         const double4 Xj = Xr[j];
         const double ax = fabs(Xj.x - Xi.x), ay = fabs(Xj.y - Xi.y), az = fabs(Xj.z - Xi.z);
@@ -173,7 +168,7 @@ __global__ void k_esc_scfactor(int64_t n, const int64_t *slice_ptr, const int32_
                 ph = right;
             } else {
                 th = atan(ay / ax);
-                ph = acos(az / L[b]);
+                ph = acos(az / pdx_ref_len(L, b, Xi, Xj));
             }
             const double cx = cos(th) * sin(ph), cy = sin(th) * sin(ph), cz = cos(ph);
             scr = sqrt(1.0 / (((cx * cx) / (scx * scx) + (cy * cy) / (scy * scy)) + (cz * cz) / (scz * scz)));
@@ -209,12 +204,12 @@ pdx_status pdx_build_correction(pdx_ctx *c)
     const esc_par one = {c->P.lambda, c->P.mu, c->P.bc, c->P.G, c->P.K};
     const dim3 G((unsigned)((n + 255) / 256)), B(256);
     for (int d = 0; d < 3; d++)
-        hipLaunchKernelGGL(k_esc_mfactor, G, B, 0, c->stream, n, d, c->kind, (int)c->P.kernel, c->slice_ptr,
+        hipLaunchKernelGGL(k_esc_mfactor, G, B, 0, c->stream, n, d, c->kind, (int)c->P.kernel, c->rows(),
                            c->cnt, c->bw,
                            c->L, c->Xr, c->P.delta, one, c->multi() ? c->d_psets : nullptr,
                            c->multi() ? c->d_pid : nullptr, c->mfactor);
     PDX_HIP(c, hipGetLastError());
-    hipLaunchKernelGGL(k_esc_scfactor, G, B, 0, c->stream, n, c->slice_ptr, c->cnt, c->bw, c->L, c->Xr,
+    hipLaunchKernelGGL(k_esc_scfactor, G, B, 0, c->stream, n, c->rows(), c->cnt, c->bw, c->L, c->Xr,
                        c->mfactor, c->scf, c->scf32);
     PDX_HIP(c, hipGetLastError());
     PDX_HIP(c, hipStreamSynchronize(c->stream));
