@@ -104,6 +104,7 @@ struct pdx_ctx {
 
     // host copies in the caller's order
     std::vector<double> X, vol;
+    double mn[3] = {0, 0, 0}, mx[3] = {0, 0, 0};  // bounding box of X
     std::vector<uint8_t> fail_permit;
     std::vector<int32_t> perm;   // perm[m] = caller index of internal point m (Morton order)
     std::vector<int32_t> iperm;  // iperm[caller index] = internal index

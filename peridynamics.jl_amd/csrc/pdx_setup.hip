@@ -1,12 +1,13 @@
 // Context, body set-up and the bond system of libpdx.
 //
-// Bond system (reference: src/discretization/bond_system.jl:55-132, 142-176):
-//  - points are reordered along a Morton curve (host, once) so that the neighbours of a
+// Bond system (reference: src/discretization/bond_system.jl:55-132, 142-176), all on the device:
+//  - points are reordered along a Morton curve (radix sort, once) so that the neighbours of a
 //    point are close in memory; every get/set maps back to the caller's order;
-//  - the neighbour search runs on the device over a cell list with cell size = horizon
-//    (the GridNeighborhoodSearch of bond_system.jl:97-99); one wavefront per point counts
-//    the neighbours, a host prefix sum gives the CSR row pointers, and a second pass fills
-//    the bonds of every point ordered by ascending caller index;
+//  - the neighbour search runs over a cell list with cell size = horizon (the
+//    GridNeighborhoodSearch of bond_system.jl:97-99); one wavefront per point counts the
+//    neighbours, prefix sums give the rows, and a second pass fills the bonds of every point
+//    ordered by internal index;
+//  - the neighbour tables of the step kernels' blocks are built in LDS, one workgroup per block;
 //  - the pair distance is formed as PointNeighbors does: pos_diff = x_i - x_j,
 //    d2 = (p0*p0 + p1*p1) + p2*p2, accepted if d2 <= delta*delta, L = sqrt(d2), so that L
 //    is bit-identical to the reference's Bond.length;
@@ -17,8 +18,6 @@
 #include <cstdarg>
 #include <cstdlib>
 #include <cstring>
-#include <numeric>
-#include <thread>
 
 #include "pdx_internal.h"
 
@@ -175,8 +174,17 @@ extern "C" pdx_status pdx_set_points(pdx_ctx *c, int64_t n, const double *X, con
     c->fail_permit.assign(n, 1);
     if (fp)
         for (int64_t i = 0; i < n; i++) c->fail_permit[i] = fp[i] ? 1 : 0;
-    for (int64_t k = 0; k < 3 * n; k++)
-        if (!std::isfinite(X[k])) return pdx_fail(c, PDX_ERR_ARG, "non-finite position");
+    for (int d = 0; d < 3; d++) {
+        c->mn[d] = INFINITY;
+        c->mx[d] = -INFINITY;
+    }
+    for (int64_t i = 0; i < n; i++)
+        for (int d = 0; d < 3; d++) {
+            const double x = X[3 * i + d];
+            if (!std::isfinite(x)) return pdx_fail(c, PDX_ERR_ARG, "non-finite position");
+            c->mn[d] = std::min(c->mn[d], x);
+            c->mx[d] = std::max(c->mx[d], x);
+        }
     c->cracks.clear();
     c->n_src = 0;
     c->n_bcpts = 0;
@@ -282,9 +290,14 @@ extern "C" pdx_status pdx_add_precrack(pdx_ctx *c, int64_t na, const int32_t *a,
 }
 
 // ----------------------------------------------------------------------------------------
-// Morton order (host, once per body)
+// Morton order: 63-bit keys (three quantised coordinates, bits interleaved), a stable radix sort
+// of (key, caller index) eight bits a pass.  One wave sorts a run of RS_RUN keys per pass: it
+// ranks 64 keys at a time by matching their digits over the wave, so the order inside a run is
+// kept without a barrier.  Measured with the rest of the device set-up (see pdx_build_bonds).
 // ----------------------------------------------------------------------------------------
-static inline uint64_t spread3(uint64_t v)
+#define RS_RUN 2048
+
+__device__ __forceinline__ uint64_t spread3(uint64_t v)
 {
     v &= 0x1fffff;
     v = (v | v << 32) & 0x1f00000000ffffULL;
@@ -295,28 +308,233 @@ static inline uint64_t spread3(uint64_t v)
     return v;
 }
 
-static void morton_order(const std::vector<double> &X, int64_t n, std::vector<int32_t> &perm)
+__global__ void k_morton_keys(int64_t n, const double *X, double3 mn, double s, uint64_t *key, int32_t *val)
 {
-    double mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
-    for (int64_t i = 0; i < n; i++)
-        for (int d = 0; d < 3; d++) {
-            mn[d] = std::min(mn[d], X[3 * i + d]);
-            mx[d] = std::max(mx[d], X[3 * i + d]);
-        }
-    double ext = std::max({mx[0] - mn[0], mx[1] - mn[1], mx[2] - mn[2], 1e-300});
-    double s = 2097151.0 / ext;
-    std::vector<std::pair<uint64_t, int32_t>> key(n);
-    for (int64_t i = 0; i < n; i++) {
-        uint64_t q[3];
-        for (int d = 0; d < 3; d++) {
-            double t = (X[3 * i + d] - mn[d]) * s;
-            q[d] = (uint64_t)std::min(std::max(t, 0.0), 2097151.0);
-        }
-        key[i] = {spread3(q[0]) | spread3(q[1]) << 1 | spread3(q[2]) << 2, (int32_t)i};
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const double m[3] = {mn.x, mn.y, mn.z};
+    uint64_t q[3];
+    for (int d = 0; d < 3; d++) {
+        const double t = (X[3 * i + d] - m[d]) * s;
+        q[d] = (uint64_t)fmin(fmax(t, 0.0), 2097151.0);
     }
-    std::sort(key.begin(), key.end());
-    perm.resize(n);
-    for (int64_t m = 0; m < n; m++) perm[m] = key[m].second;
+    key[i] = spread3(q[0]) | spread3(q[1]) << 1 | spread3(q[2]) << 2;
+    val[i] = (int32_t)i;
+}
+
+// digits of every run: cnt[digit * runs + run]
+__global__ __launch_bounds__(64) void k_rs_hist(int64_t n, int shift, const uint64_t *key, int32_t *cnt)
+{
+    __shared__ int32_t h[256];
+    for (int d = threadIdx.x; d < 256; d += 64) h[d] = 0;
+    __syncthreads();
+    const int64_t b = (int64_t)blockIdx.x * RS_RUN;
+    for (int64_t k = b + threadIdx.x; k < b + RS_RUN && k < n; k += 64)
+        atomicAdd(&h[(key[k] >> shift) & 255], 1);
+    __syncthreads();
+    for (int d = threadIdx.x; d < 256; d += 64) cnt[(int64_t)d * gridDim.x + blockIdx.x] = h[d];
+}
+
+// exclusive sums over the runs of each digit (one workgroup per digit), and the digit's total
+__global__ __launch_bounds__(256) void k_rs_scan(int runs, int32_t *cnt, int32_t *total)
+{
+    __shared__ int32_t sh[256];
+    int32_t *c = cnt + (int64_t)blockIdx.x * runs;
+    int32_t carry = 0;
+    for (int k0 = 0; k0 < runs; k0 += 256) {
+        const int k = k0 + threadIdx.x;
+        const int32_t v = k < runs ? c[k] : 0;
+        sh[threadIdx.x] = v;
+        __syncthreads();
+        for (int o = 1; o < 256; o <<= 1) {
+            const int32_t a = (int)threadIdx.x >= o ? sh[threadIdx.x - o] : 0;
+            __syncthreads();
+            sh[threadIdx.x] += a;
+            __syncthreads();
+        }
+        if (k < runs) c[k] = carry + sh[threadIdx.x] - v;
+        carry += sh[255];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) total[blockIdx.x] = carry;
+}
+
+__global__ __launch_bounds__(64) void k_rs_scatter(int64_t n, int shift, const uint64_t *key, const int32_t *val,
+                                                   const int32_t *cnt, const int32_t *total, uint64_t *key_out,
+                                                   int32_t *val_out)
+{
+    __shared__ int32_t pos[256];
+    const int lane = threadIdx.x;
+    // first position of every digit: four digits per lane, then the sum over the lower lanes
+    int32_t t[4], s = 0;
+    for (int q = 0; q < 4; q++) {
+        t[q] = s;
+        s += total[4 * lane + q];
+    }
+    int32_t x = s;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int32_t y = __shfl_up(x, o);
+        if (lane >= o) x += y;
+    }
+    for (int q = 0; q < 4; q++)
+        pos[4 * lane + q] = x - s + t[q] + cnt[(int64_t)(4 * lane + q) * gridDim.x + blockIdx.x];
+    __syncthreads();
+    const int64_t b = (int64_t)blockIdx.x * RS_RUN;
+    for (int64_t k0 = b; k0 < b + RS_RUN && k0 < n; k0 += 64) {
+        const int64_t k = k0 + lane;
+        const bool in = k < n;
+        const uint64_t v = in ? key[k] : 0;
+        const int d = (int)((v >> shift) & 255);
+        // the lanes with the same digit
+        uint64_t same = __ballot(in);
+        for (int bit = 0; bit < 8; bit++) {
+            const uint64_t m = __ballot((d >> bit) & 1);
+            same &= ((d >> bit) & 1) ? m : ~m;
+        }
+        const int before = __popcll(same & ((1ULL << lane) - 1ULL));
+        int32_t p = 0;
+        if (in) p = pos[d] + before;
+        __syncthreads();  // (one wave: orders the reads of pos before its updates)
+        if (in) {
+            key_out[p] = v;
+            val_out[p] = val[k];
+            if (before == 0) pos[d] += __popcll(same);
+        }
+        __syncthreads();
+    }
+}
+
+// exclusive sums of n int32 values as int64: runs of SCAN_RUN, then the run totals, then both
+#define SCAN_RUN 4096
+__global__ __launch_bounds__(256) void k_scan_runs(int64_t n, const int32_t *in, int64_t *total)
+{
+    __shared__ int64_t sh[4];
+    const int64_t b = (int64_t)blockIdx.x * SCAN_RUN;
+    int64_t s = 0;
+    for (int64_t k = b + threadIdx.x; k < b + SCAN_RUN && k < n; k += 256) s += in[k];
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) total[blockIdx.x] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+}
+
+// one workgroup: exclusive sums of the run totals in place, the grand total behind them
+__global__ __launch_bounds__(1024) void k_scan_totals(int64_t runs, int64_t *total)
+{
+    __shared__ int64_t sh[1024];
+    int64_t carry = 0;
+    for (int64_t k0 = 0; k0 < runs; k0 += 1024) {
+        const int64_t k = k0 + threadIdx.x;
+        const int64_t v = k < runs ? total[k] : 0;
+        sh[threadIdx.x] = v;
+        __syncthreads();
+        for (int o = 1; o < 1024; o <<= 1) {
+            const int64_t a = (int)threadIdx.x >= o ? sh[threadIdx.x - o] : 0;
+            __syncthreads();
+            sh[threadIdx.x] += a;
+            __syncthreads();
+        }
+        if (k < runs) total[k] = carry + sh[threadIdx.x] - v;
+        carry += sh[1023];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) total[runs] = carry;
+}
+
+__global__ __launch_bounds__(256) void k_scan_out(int64_t n, const int32_t *in, const int64_t *total, int64_t *out)
+{
+    __shared__ int64_t sh[256];
+    const int64_t b = (int64_t)blockIdx.x * SCAN_RUN + (int64_t)threadIdx.x * (SCAN_RUN / 256);
+    int64_t s = 0;
+    for (int q = 0; q < SCAN_RUN / 256; q++) s += b + q < n ? in[b + q] : 0;
+    sh[threadIdx.x] = s;
+    __syncthreads();
+    for (int o = 1; o < 256; o <<= 1) {
+        const int64_t a = (int)threadIdx.x >= o ? sh[threadIdx.x - o] : 0;
+        __syncthreads();
+        sh[threadIdx.x] += a;
+        __syncthreads();
+    }
+    int64_t x = total[blockIdx.x] + sh[threadIdx.x] - s;
+    for (int q = 0; q < SCAN_RUN / 256; q++) {
+        if (b + q >= n) break;
+        out[b + q] = x;
+        x += in[b + q];
+    }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = total[gridDim.x];
+}
+
+// scratch of one set-up, freed with it
+struct setup_scratch {
+    std::vector<void *> p;
+    ~setup_scratch()
+    {
+        for (void *q : p) (void)hipFree(q);
+    }
+    template <class T>
+    pdx_status get(pdx_ctx *c, T **out, size_t count)
+    {
+        *out = nullptr;
+        const hipError_t e = hipMalloc((void **)out, std::max<size_t>(count * sizeof(T), 256));
+        if (e != hipSuccess)
+            return pdx_fail(c, PDX_ERR_OOM, "hipMalloc of %zu bytes failed: %s", count * sizeof(T), hipGetErrorString(e));
+        p.push_back(*out);
+        return PDX_OK;
+    }
+};
+
+static inline dim3 grid256(int64_t m) { return dim3((unsigned)((m + 255) / 256)); }
+
+// out[k] = in[0] + ... + in[k - 1], k = 0 .. n
+static pdx_status scan_i32(pdx_ctx *c, setup_scratch &S, int64_t n, const int32_t *in, int64_t *out)
+{
+    const int64_t runs = std::max<int64_t>(1, (n + SCAN_RUN - 1) / SCAN_RUN);
+    int64_t *total;
+    PDX_TRY(S.get(c, &total, runs + 1));
+    hipLaunchKernelGGL(k_scan_runs, dim3((unsigned)runs), dim3(256), 0, c->stream, n, in, total);
+    hipLaunchKernelGGL(k_scan_totals, dim3(1), dim3(1024), 0, c->stream, runs, total);
+    hipLaunchKernelGGL(k_scan_out, dim3((unsigned)runs), dim3(256), 0, c->stream, n, in, total, out);
+    PDX_HIP(c, hipGetLastError());
+    return PDX_OK;
+}
+
+__global__ void k_invert(int64_t n, const int32_t *perm, int32_t *iperm)
+{
+    const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (m < n) iperm[perm[m]] = (int32_t)m;
+}
+
+// perm and iperm on the device and the host, from the caller's positions on the device
+static pdx_status morton_order(pdx_ctx *c, setup_scratch &S, const double *dX, const double mn[3], const double mx[3])
+{
+    const int64_t n = c->n;
+    const double ext = std::max({mx[0] - mn[0], mx[1] - mn[1], mx[2] - mn[2], 1e-300});
+    const int64_t runs = (n + RS_RUN - 1) / RS_RUN;
+    uint64_t *key[2];
+    int32_t *val[2], *cnt, *total;
+    for (int q = 0; q < 2; q++) {
+        PDX_TRY(S.get(c, &key[q], n));
+        PDX_TRY(S.get(c, &val[q], n));
+    }
+    PDX_TRY(S.get(c, &cnt, 256 * runs));
+    PDX_TRY(S.get(c, &total, 256));
+    hipLaunchKernelGGL(k_morton_keys, grid256(n), dim3(256), 0, c->stream, n, dX, make_double3(mn[0], mn[1], mn[2]),
+                       2097151.0 / ext, key[0], val[0]);
+    for (int pass = 0; pass < 8; pass++) {
+        const int a = pass & 1, b = a ^ 1;
+        hipLaunchKernelGGL(k_rs_hist, dim3((unsigned)runs), dim3(64), 0, c->stream, n, 8 * pass, key[a], cnt);
+        hipLaunchKernelGGL(k_rs_scan, dim3(256), dim3(256), 0, c->stream, (int)runs, cnt, total);
+        hipLaunchKernelGGL(k_rs_scatter, dim3((unsigned)runs), dim3(64), 0, c->stream, n, 8 * pass, key[a], val[a],
+                           cnt, total, key[b], pass == 7 ? c->d_perm : val[b]);
+    }
+    hipLaunchKernelGGL(k_invert, grid256(n), dim3(256), 0, c->stream, n, c->d_perm, c->d_iperm);
+    PDX_HIP(c, hipGetLastError());
+    c->perm.resize(n);
+    c->iperm.resize(n);
+    PDX_HIP(c, hipMemcpyAsync(c->perm.data(), c->d_perm, sizeof(int32_t) * n, hipMemcpyDeviceToHost, c->stream));
+    PDX_HIP(c, hipMemcpyAsync(c->iperm.data(), c->d_iperm, sizeof(int32_t) * n, hipMemcpyDeviceToHost, c->stream));
+    PDX_HIP(c, hipStreamSynchronize(c->stream));
+    return PDX_OK;
 }
 
 // ----------------------------------------------------------------------------------------
@@ -342,6 +560,79 @@ struct search_args {
     unsigned long long *flags;
 };
 
+// the points in internal order: records x|V (reference, both current buffers), failure permission,
+// crack membership
+__global__ void k_gather_points(int64_t n, const int32_t *perm, const double *X, const double *vol,
+                                const uint8_t *fp_in, const uint16_t *cm_in, double4 *Xr, double4 *r0, double4 *r1,
+                                uint8_t *fp, uint16_t *cm)
+{
+    const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (m >= n) return;
+    const int64_t i = perm[m];
+    const double4 x = make_double4(X[3 * i], X[3 * i + 1], X[3 * i + 2], vol[i]);
+    Xr[m] = x;
+    r0[m] = x;
+    r1[m] = x;
+    fp[m] = fp_in[i];
+    if (cm) cm[m] = cm_in[i];
+}
+
+// cell of every point and the points per cell
+__global__ void k_cells(int64_t n, const double4 *Xr, double3 mn, double cs, int64_t gx, int64_t gy, int64_t gz,
+                        int32_t *pcell, int32_t *num)
+{
+    const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (m >= n) return;
+    const double4 x = Xr[m];
+    const int64_t qx = min(max((int64_t)floor((x.x - mn.x) / cs), (int64_t)0), gx - 1);
+    const int64_t qy = min(max((int64_t)floor((x.y - mn.y) / cs), (int64_t)0), gy - 1);
+    const int64_t qz = min(max((int64_t)floor((x.z - mn.z) / cs), (int64_t)0), gz - 1);
+    pcell[3 * m] = (int32_t)qx;
+    pcell[3 * m + 1] = (int32_t)qy;
+    pcell[3 * m + 2] = (int32_t)qz;
+    atomicAdd(&num[qx + gx * (qy + gy * qz)], 1);
+}
+
+// the points of every cell, in any order (the rows are sorted later); num counts down to zero
+__global__ void k_cell_points(int64_t n, const int32_t *pcell, int64_t gx, int64_t gy, const int64_t *start,
+                              int32_t *num, int32_t *pts)
+{
+    const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (m >= n) return;
+    const int64_t cell = pcell[3 * m] + gx * (pcell[3 * m + 1] + gy * (int64_t)pcell[3 * m + 2]);
+    pts[start[cell] + atomicSub(&num[cell], 1) - 1] = (int32_t)m;
+}
+
+// sum and maximum of the bond counts: out[0] += , out[1] = max
+__global__ __launch_bounds__(256) void k_count_totals(int64_t n, const int32_t *cnt, unsigned long long *out)
+{
+    unsigned long long s = 0;
+    int m = 0;
+    for (int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x; k < n; k += (int64_t)gridDim.x * 256) {
+        s += (unsigned long long)cnt[k];
+        m = max(m, cnt[k]);
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        s += __shfl_xor(s, o);
+        m = max(m, __shfl_xor(m, o));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        atomicAdd(&out[0], s);
+        atomicMax(&out[1], (unsigned long long)m);
+    }
+}
+
+// slots of every slice: 64 per row group of its widest row
+__global__ void k_slice_width(int64_t n, int64_t n_slices, pdx_rows rows, const int32_t *cnt, int32_t *width)
+{
+    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= n_slices) return;
+    const int P = 64 >> rows.ls;
+    int w = 0;
+    for (int64_t m = P * s; m < min(n, P * s + P); m++) w = max(w, cnt[m]);
+    width[s] = 64 * rows.groups(w);
+}
+
 // (A_i & B_j) | (B_i & A_j) per crack, at the even bit positions
 __device__ __forceinline__ uint32_t crack_hits(uint32_t mi, uint32_t mj)
 {
@@ -365,28 +656,27 @@ __global__ __launch_bounds__(PDX_BLOCK) void k_count_bonds(search_args s)
     int cx = s.pcell[3 * i], cy = s.pcell[3 * i + 1], cz = s.pcell[3 * i + 2];
     uint32_t mi = s.cmask ? s.cmask[i] : 0;
     int cnt = 0;
+    const int64_t x0 = max(cx - 1, 0), x1 = min((int64_t)cx + 1, s.gx - 1);
     for (int z = cz - 1; z <= cz + 1; z++) {
         if (z < 0 || z >= s.gz) continue;
         for (int y = cy - 1; y <= cy + 1; y++) {
             if (y < 0 || y >= s.gy) continue;
-            for (int x = cx - 1; x <= cx + 1; x++) {
-                if (x < 0 || x >= s.gx) continue;
-                int64_t cell = x + s.gx * (y + s.gy * (int64_t)z);
-                int64_t e = s.cell_start[cell + 1];
-                for (int64_t k = s.cell_start[cell] + lane; k < e; k += 64) {
-                    int32_t j = s.cell_pts[k];
-                    if (j == i) continue;
-                    double d2 = pair_d2(xi, s.Xr[j]);
-                    if (d2 <= s.r2) {
-                        if (sqrt(d2) < 2.220446049250313e-16) {
-                            if (atomicExch(&s.flags[1], 1ULL) == 0ULL) {
-                                s.flags[2] = (unsigned long long)s.perm[i];
-                                s.flags[3] = (unsigned long long)s.perm[j];
-                            }
+            // the cells x - 1 .. x + 1 are one run of the cell list
+            const int64_t row = s.gx * (y + s.gy * (int64_t)z);
+            const int64_t e = s.cell_start[row + x1 + 1];
+            for (int64_t k = s.cell_start[row + x0] + lane; k < e; k += 64) {
+                int32_t j = s.cell_pts[k];
+                if (j == i) continue;
+                double d2 = pair_d2(xi, s.Xr[j]);
+                if (d2 <= s.r2) {
+                    if (sqrt(d2) < 2.220446049250313e-16) {
+                        if (atomicExch(&s.flags[1], 1ULL) == 0ULL) {
+                            s.flags[2] = (unsigned long long)s.perm[i];
+                            s.flags[3] = (unsigned long long)s.perm[j];
                         }
-                        uint32_t h = s.cmask ? crack_hits(mi, s.cmask[j]) : 0u;
-                        if (!(h & s.filt_bits)) cnt++;
                     }
+                    uint32_t h = s.cmask ? crack_hits(mi, s.cmask[j]) : 0u;
+                    if (!(h & s.filt_bits)) cnt++;
                 }
             }
         }
@@ -397,8 +687,7 @@ __global__ __launch_bounds__(PDX_BLOCK) void k_count_bonds(search_args s)
 
 __global__ __launch_bounds__(PDX_BLOCK) void k_fill_bonds(search_args s)
 {
-    __shared__ int32_t cj[PDX_WAVES_PER_BLOCK][PDX_FILL_CAP];
-    __shared__ int32_t co[PDX_WAVES_PER_BLOCK][PDX_FILL_CAP];
+    __shared__ __align__(16) int32_t cj[PDX_WAVES_PER_BLOCK][PDX_FILL_CAP + 4];
     int64_t i = pdx_wave_point();
     if (i >= s.n) return;
     int lane = threadIdx.x & 63;
@@ -409,56 +698,60 @@ __global__ __launch_bounds__(PDX_BLOCK) void k_fill_bonds(search_args s)
     const int64_t b0 = s.rows.row(i);
     const int want = s.cnt[i];                          // <= PDX_FILL_CAP, checked on the host
     int base = 0;
+    const int64_t x0 = max(cx - 1, 0), x1 = min((int64_t)cx + 1, s.gx - 1);
     for (int z = cz - 1; z <= cz + 1; z++) {
         if (z < 0 || z >= s.gz) continue;
         for (int y = cy - 1; y <= cy + 1; y++) {
             if (y < 0 || y >= s.gy) continue;
-            for (int x = cx - 1; x <= cx + 1; x++) {
-                if (x < 0 || x >= s.gx) continue;
-                int64_t cell = x + s.gx * (y + s.gy * (int64_t)z);
-                int64_t st = s.cell_start[cell], e = s.cell_start[cell + 1];
-                for (int64_t k0 = st; k0 < e; k0 += 64) {
-                    int64_t k = k0 + lane;
-                    bool take = false;
-                    int32_t j = -1;
-                    if (k < e) {
-                        j = s.cell_pts[k];
-                        if (j != i) {
-                            double d2 = pair_d2(xi, s.Xr[j]);
-                            uint32_t h = s.cmask ? crack_hits(mi, s.cmask[j]) : 0u;
-                            take = (d2 <= s.r2) && !(h & s.filt_bits);
-                        }
+            const int64_t row = s.gx * (y + s.gy * (int64_t)z);
+            const int64_t st = s.cell_start[row + x0], e = s.cell_start[row + x1 + 1];
+            for (int64_t k0 = st; k0 < e; k0 += 64) {
+                int64_t k = k0 + lane;
+                bool take = false;
+                int32_t j = -1;
+                if (k < e) {
+                    j = s.cell_pts[k];
+                    if (j != i) {
+                        double d2 = pair_d2(xi, s.Xr[j]);
+                        uint32_t h = s.cmask ? crack_hits(mi, s.cmask[j]) : 0u;
+                        take = (d2 <= s.r2) && !(h & s.filt_bits);
                     }
-                    uint64_t m = __ballot(take);
-                    int pos = base + (int)__popcll(m & ((1ULL << lane) - 1ULL));
-                    if (take && pos < PDX_FILL_CAP) {
-                        cj[w][pos] = j;
-                        co[w][pos] = s.perm[j];
-                    }
-                    base += (int)__popcll(m);
                 }
+                uint64_t m = __ballot(take);
+                int pos = base + (int)__popcll(m & ((1ULL << lane) - 1ULL));
+                if (take && pos < PDX_FILL_CAP) cj[w][pos] = j;
+                base += (int)__popcll(m);
             }
         }
     }
+    const int cnt = min(base, want);
+    if (lane < 4) cj[w][cnt + lane] = 0x7fffffff;  // the ranking reads four at a time
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    int cnt = min(base, want);
-    for (int k = lane; k < cnt; k += 64) {
-        // rows are ordered by the neighbour's internal (Morton) index, so that the lanes of
-        // a gather read neighbouring records; pdx_get_bonds reorders rows by caller index
-        int32_t ok = cj[w][k];
-        int rank = 0;
-        for (int m2 = 0; m2 < cnt; m2++) rank += (cj[w][m2] < ok) ? 1 : 0;
-        int32_t j = cj[w][k];
-        double4 xj = s.Xr[j];
-        double d2 = pair_d2(xi, xj);
-        uint32_t h = s.cmask ? crack_hits(mi, s.cmask[j]) : 0u;
-        const uint32_t fpb = (s.fp[i] & s.fp[j]) ? PDX_BW_FP : 0u;
-        const uint32_t act = (h & ~s.filt_bits) ? 0u : PDX_BW_ACT;  // broken at t = 0 by a precrack
-        const int64_t b = s.rows.at(b0, rank);
-        s.bw[b] = (uint32_t)j | act | fpb;
-        s.L[b] = sqrt(d2);
+    // rows are ordered by the neighbour's internal (Morton) index, so that the lanes of a gather
+    // read neighbouring records and the tiles of a table are met in order; pdx_get_bonds reorders
+    // rows by caller index.  Two bonds per lane are ranked in one sweep over the row.
+    for (int k = lane; k < cnt; k += 128) {
+        const int32_t ja = cj[w][k], jb = k + 64 < cnt ? cj[w][k + 64] : 0x7fffffff;
+        int ra = 0, rb = 0;
+        for (int q = 0; q < cnt; q += 4) {
+            const int4 v = *reinterpret_cast<const int4 *>(&cj[w][q]);
+            ra += (v.x < ja ? 1 : 0) + (v.y < ja ? 1 : 0) + (v.z < ja ? 1 : 0) + (v.w < ja ? 1 : 0);
+            rb += (v.x < jb ? 1 : 0) + (v.y < jb ? 1 : 0) + (v.z < jb ? 1 : 0) + (v.w < jb ? 1 : 0);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            if (k + 64 * u >= cnt) break;
+            const int32_t j = u ? jb : ja;
+            const double d2 = pair_d2(xi, s.Xr[j]);
+            const uint32_t h = s.cmask ? crack_hits(mi, s.cmask[j]) : 0u;
+            const uint32_t fpb = (s.fp[i] & s.fp[j]) ? PDX_BW_FP : 0u;
+            const uint32_t act = (h & ~s.filt_bits) ? 0u : PDX_BW_ACT;  // broken at t = 0 by a precrack
+            const int64_t b = s.rows.at(b0, u ? rb : ra);
+            s.bw[b] = (uint32_t)j | act | fpb;
+            s.L[b] = sqrt(d2);
+        }
     }
 }
 
@@ -547,20 +840,17 @@ pdx_status pdx_download_vec(pdx_ctx *c, const double *dev, double *host, int com
 // ----------------------------------------------------------------------------------------
 // packed bonds
 // ----------------------------------------------------------------------------------------
-// bit patterns of the shortest and the longest bond (positive doubles order as their bits do):
-// range[0] starts at ~0, range[1] at 0
-__global__ __launch_bounds__(256) void k_len_range(int64_t n, pdx_rows rows, const int32_t *cnt,
-                                                   const double *L, unsigned long long *range)
+// bit patterns of the shortest and the longest active bond (positive doubles order as their bits
+// do): range[0] starts at ~0, range[1] at 0
+__global__ __launch_bounds__(256) void k_len_range(int64_t nb, const uint32_t *bw, const double *L,
+                                                   unsigned long long *range)
 {
     unsigned long long lo = ~0ULL, hi = 0ULL;
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < n) {
-        const int64_t b0 = rows.row(p);
-        for (int t = 0; t < cnt[p]; t++) {
-            const unsigned long long v = (unsigned long long)__double_as_longlong(L[rows.at(b0, t)]);
-            lo = v < lo ? v : lo;
-            hi = v > hi ? v : hi;
-        }
+    for (int64_t b = (int64_t)blockIdx.x * 256 + threadIdx.x; b < nb; b += (int64_t)gridDim.x * 256) {
+        if (!(bw[b] & PDX_BW_ACT)) continue;  // also the padding
+        const unsigned long long v = (unsigned long long)__double_as_longlong(L[b]);
+        lo = v < lo ? v : lo;
+        hi = v > hi ? v : hi;
     }
     for (int o = 32; o > 0; o >>= 1) {
         const unsigned long long a = __shfl_xor(lo, o), b = __shfl_xor(hi, o);
@@ -596,8 +886,8 @@ static pdx_status pack_bonds(pdx_ctx *c)
     if (c->precision != PDX_FP64 || c->multi() || c->nb <= 0) return PDX_OK;
     unsigned long long *range = c->d_flags + 4, h[2] = {~0ULL, 0ULL};
     PDX_HIP(c, hipMemcpyAsync(range, h, sizeof h, hipMemcpyHostToDevice, c->stream));
-    hipLaunchKernelGGL(k_len_range, dim3((unsigned)((c->n + 255) / 256)), dim3(256), 0, c->stream, c->n,
-                       c->rows(), c->cnt, c->L, range);
+    hipLaunchKernelGGL(k_len_range, dim3((unsigned)std::min<int64_t>((c->nb_alloc + 255) / 256, 2048)), dim3(256), 0,
+                       c->stream, c->nb_alloc, c->bw, c->L, range);
     PDX_HIP(c, hipGetLastError());
     PDX_HIP(c, hipMemcpyAsync(h, range, sizeof h, hipMemcpyDeviceToHost, c->stream));
     PDX_HIP(c, hipStreamSynchronize(c->stream));
@@ -605,6 +895,7 @@ static pdx_status pack_bonds(pdx_ctx *c)
     while ((1 << sb) < c->halo_max) sb++;
     const int shift = 64 - sb;
     const unsigned long long mask = (1ULL << shift) - 1;
+    if (h[0] > h[1]) h[0] = h[1] = 0;  // no active bond
     if (h[1] - h[0] >= mask) return PDX_OK;
     c->pk_shift = shift;
     c->pk_mask = mask;
@@ -621,102 +912,155 @@ static pdx_status pack_bonds(pdx_ctx *c)
 }
 
 // ----------------------------------------------------------------------------------------
-// LDS halos of the BB step.  For every block of PDX_BLOCK consecutive (Morton) points the
-// sorted, de-duplicated list of the points its bonds reach; every bond is rewritten as a
-// 16-bit slot into its block's list.  Built on the host, in parallel over blocks, once.
-// Returns false (and leaves the global-gather layout in use) if a halo does not fit.
+// Neighbour tables of the LDS-staged kernels: for every block of PB consecutive (Morton) points
+// the sorted list of the points its bonds reach; every bond gets a 16-bit slot into its block's
+// list.  One workgroup per block: the neighbours go into a hash table in LDS, its entries are
+// compacted and sorted there, and the bonds look their slots up by bisection.  Run twice: the
+// first run (WRITE = false) only counts.
 // ----------------------------------------------------------------------------------------
+#define HALO_T 512
+#define HALO_HASH 16384
+#define HALO_LIST (PDX_W16_SLOT + 1)  // longest table that the slots address
+
+template <bool WRITE>
+__global__ __launch_bounds__(HALO_T) void k_halo(int64_t n, int PB, pdx_rows rows, const int32_t *cnt,
+                                                 const uint32_t *bw, int32_t *count, const int64_t *hptr,
+                                                 int32_t *halo, uint16_t *w16)
+{
+    extern __shared__ int32_t lds[];
+    int32_t *const hash = lds, *const list = lds + HALO_HASH;
+    __shared__ int num, pos;
+    const int64_t p0 = (int64_t)blockIdx.x * PB;
+    const int P = 64 >> rows.ls, S = 1 << rows.ls, lane = threadIdx.x & 63;
+    const int64_t s1 = (min(p0 + PB, n) + P - 1) / P;
+    for (int q = threadIdx.x; q < HALO_HASH; q += HALO_T) hash[q] = -1;
+    if (threadIdx.x == 0) num = pos = 0;
+    __syncthreads();
+    // lane -> point of the slice and its bonds: group g holds bond t(g) (pdx_rows::at)
+    const int sub = lane & (S - 1), kk = sub >> 2, m = S >> 2;
+    auto bond_no = [&](int g) { return 16 * ((g >> 2) * m + kk) + 4 * (g & 3) + (sub & 3); };
+    for (int64_t s = p0 / P + (threadIdx.x >> 6); s < s1; s += HALO_T / 64) {
+        const int64_t p = s * P + (lane >> rows.ls), b0 = rows.ptr[s];
+        const int c = p < n ? cnt[p] : 0;
+        const int ng = (int)((rows.ptr[s + 1] - b0) >> 6);
+        for (int g = 0; g < ng; g++) {
+            if (bond_no(g) >= c) continue;
+            const int32_t j = (int32_t)(bw[b0 + (int64_t)g * 64 + lane] & PDX_BW_NBR);
+            uint32_t h = ((uint32_t)j * 2654435761u) >> 18;
+            // at most HALO_LIST entries and one more per thread go in, so a probe ends at j or a free cell
+            while (true) {
+                const int32_t e = hash[h];
+                if (e == j) break;
+                if (e == -1) {
+                    if (*(volatile int *)&num > HALO_LIST) break;
+                    const int32_t old = atomicCAS(&hash[h], -1, j);
+                    if (old == -1) atomicAdd(&num, 1);
+                    if (old == -1 || old == j) break;
+                }
+                h = (h + 1) & (HALO_HASH - 1);
+            }
+        }
+    }
+    __syncthreads();
+    const int H = num;
+    if (!WRITE) {
+        if (threadIdx.x == 0) count[blockIdx.x] = H;
+        return;
+    }
+    for (int q = threadIdx.x; q < HALO_HASH; q += HALO_T)
+        if (hash[q] >= 0) list[atomicAdd(&pos, 1)] = hash[q];
+    int np = 1;
+    while (np < H) np <<= 1;
+    __syncthreads();
+    for (int q = H + (int)threadIdx.x; q < np; q += HALO_T) list[q] = 0x7fffffff;
+    __syncthreads();
+    for (int k = 2; k <= np; k <<= 1)
+        for (int d = k >> 1; d > 0; d >>= 1) {
+            for (int q = threadIdx.x; q < np / 2; q += HALO_T) {
+                const int a = 2 * q - (q & (d - 1)), b = a + d;
+                const int32_t x = list[a], y = list[b];
+                if ((x > y) == ((a & k) == 0)) {
+                    list[a] = y;
+                    list[b] = x;
+                }
+            }
+            __syncthreads();
+        }
+    int32_t *const out = halo + hptr[blockIdx.x];
+    for (int q = threadIdx.x; q < H; q += HALO_T) out[q] = list[q];
+    for (int64_t s = p0 / P + (threadIdx.x >> 6); s < s1; s += HALO_T / 64) {
+        const int64_t p = s * P + (lane >> rows.ls), b0 = rows.ptr[s];
+        const int c = p < n ? cnt[p] : 0;
+        const int ng = (int)((rows.ptr[s + 1] - b0) >> 6);
+        // the slots past the row's end repeat its last neighbour, not active
+        const uint32_t last = c > 0 ? bw[rows.at(rows.row(p), c - 1)] & PDX_BW_NBR : 0u;
+        for (int g = 0; g < ng; g++) {
+            const int64_t b = b0 + (int64_t)g * 64 + lane;
+            const uint32_t w = bond_no(g) < c ? bw[b] : last;
+            const int32_t j = (int32_t)(w & PDX_BW_NBR);
+            int lo = 0, hi = H;
+            while (lo < hi) {
+                const int mid = (lo + hi) >> 1;
+                if (list[mid] < j) lo = mid + 1;
+                else hi = mid;
+            }
+            w16[b] = c > 0 ? (uint16_t)(lo | ((w & PDX_BW_ACT) ? PDX_W16_ACT | PDX_W16_RACT : 0u) |
+                                        ((w & PDX_BW_FP) ? PDX_W16_FP : 0u))
+                           : (uint16_t)0;
+        }
+    }
+}
+
+// the largest of n counts
+__global__ __launch_bounds__(256) void k_max_i32(int64_t n, const int32_t *in, unsigned long long *out)
+{
+    int m = 0;
+    for (int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x; k < n; k += (int64_t)gridDim.x * 256) m = max(m, in[k]);
+    for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o));
+    if ((threadIdx.x & 63) == 0) atomicMax(out, (unsigned long long)m);
+}
+
+// Builds the tables and the 16-bit words; *ok = false (and no LDS layout) if a table does not fit.
 static pdx_status build_halos(pdx_ctx *c, bool *ok)
 {
     *ok = false;
-    const int64_t n = c->n, nba = c->nb_alloc;
-    const int64_t n_slices = c->n_slices();
-    const int64_t PB = c->pb;
-    const int64_t nblk = (n + PB - 1) / PB;
-    hipDeviceProp_t prop;
-    PDX_HIP(c, hipGetDeviceProperties(&prop, c->device));
-    const int64_t lds_limit = std::min<int64_t>((int64_t)prop.sharedMemPerBlock, 160 * 1024);
-    c->lds_limit = lds_limit - 64;
+    const int64_t n = c->n, PB = c->pb, nblk = (n + PB - 1) / PB;
+    int lds = 0;
+    PDX_HIP(c, hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, c->device));
     // 64 bytes of slack for the alignment pad of a trailing byte table.  A table longer than
-    // what LDS holds is still served: the kernels stage what fits and read the rest from
-    // global memory (or stage it in tiles), so only the 13-bit slot field limits a table.
-    const int64_t slot_limit = PDX_W16_SLOT + 1;
-    std::vector<int64_t> sp(n_slices + 1);
-    std::vector<int32_t> cn(n);
-    std::vector<uint32_t> w(nba);
-    PDX_HIP(c, hipMemcpy(sp.data(), c->slice_ptr, sizeof(int64_t) * (n_slices + 1), hipMemcpyDeviceToHost));
-    PDX_HIP(c, hipMemcpy(cn.data(), c->cnt, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
-    const pdx_rows hr{sp.data(), c->ls};
-    PDX_HIP(c, hipMemcpy(w.data(), c->bw, sizeof(uint32_t) * nba, hipMemcpyDeviceToHost));
-    std::vector<std::vector<int32_t>> tab(nblk);
-    std::vector<uint16_t> w16(nba, 0);
-    std::vector<uint8_t> used(nba, 0);
-    std::vector<int> too_big(nblk, 0), unsorted(nblk, 0);
-    unsigned nth = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
-    auto work = [&](int64_t k0, int64_t k1) {
-        std::vector<int32_t> tmp;
-        for (int64_t k = k0; k < k1; k++) {
-            tmp.clear();
-            const int64_t pe = std::min(n, (k + 1) * PB);
-            for (int64_t p = k * PB; p < pe; p++) {
-                const int64_t b0 = hr.row(p);
-                for (int t = 0; t < cn[p]; t++) tmp.push_back((int32_t)(w[hr.at(b0, t)] & PDX_BW_NBR));
-            }
-            std::sort(tmp.begin(), tmp.end());
-            tmp.erase(std::unique(tmp.begin(), tmp.end()), tmp.end());
-            if ((int64_t)tmp.size() > slot_limit) {
-                too_big[k] = 1;
-                continue;
-            }
-            for (int64_t p = k * PB; p < pe; p++) {
-                const int64_t b0 = hr.row(p);
-                int64_t prev = -1;
-                for (int t = 0; t < cn[p]; t++) {
-                    const int64_t b = hr.at(b0, t);
-                    const int32_t j = (int32_t)(w[b] & PDX_BW_NBR);
-                    const uint32_t slot = (uint32_t)(std::lower_bound(tmp.begin(), tmp.end(), j) - tmp.begin());
-                    if ((int64_t)slot <= prev) unsorted[k] = 1;
-                    prev = slot;
-                    used[b] = 1;
-                    w16[b] = (uint16_t)(slot | ((w[b] & PDX_BW_ACT) ? PDX_W16_ACT | PDX_W16_RACT : 0u) |
-                                        ((w[b] & PDX_BW_FP) ? PDX_W16_FP : 0u));
-                }
-                // the slots past the row's end repeat its last neighbour, inactive
-                const int64_t ng = (sp[(p >> (6 - c->ls)) + 1] - sp[p >> (6 - c->ls)]) >> 6;
-                for (int64_t g = 0; g < ng; g++)
-                    for (int l = 0; l < (1 << c->ls); l++)
-                        if (!used[b0 + 64 * g + l]) w16[b0 + 64 * g + l] = (uint16_t)(prev < 0 ? 0 : prev);
-            }
-            tab[k] = tmp;
-        }
-    };
-    std::vector<std::thread> th;
-    const int64_t per = (nblk + nth - 1) / nth;
-    for (unsigned t = 0; t < nth; t++) {
-        const int64_t k0 = t * per, k1 = std::min(nblk, k0 + per);
-        if (k0 < k1) th.emplace_back(work, k0, k1);
-    }
-    for (auto &t : th) t.join();
-    // keep the global-gather kernels if a table outgrows the slot field, or if a row's slots
-    // do not increase (the tiled staging walks every row in slot order)
-    for (int64_t k = 0; k < nblk; k++)
-        if (too_big[k] || unsorted[k]) return PDX_OK;
-    std::vector<int64_t> hp(nblk + 1, 0);
-    int64_t hmax = 0;
-    for (int64_t k = 0; k < nblk; k++) {
-        hp[k + 1] = hp[k] + (int64_t)tab[k].size();
-        hmax = std::max<int64_t>(hmax, (int64_t)tab[k].size());
-    }
-    std::vector<int32_t> halo(std::max<int64_t>(hp[nblk], 1));
-    for (int64_t k = 0; k < nblk; k++) std::copy(tab[k].begin(), tab[k].end(), halo.begin() + hp[k]);
-    PDX_TRY(pdx_alloc(c, &c->bw16, nba));
+    // what LDS holds is still served: the kernels stage it in tiles or stage what fits and read
+    // the rest from global memory, so only the 13-bit slot field limits a table.
+    c->lds_limit = std::min<int64_t>(lds, 160 * 1024) - 64;
+    setup_scratch S;
+    int32_t *count;
+    PDX_TRY(S.get(c, &count, nblk));
+    const size_t hl = sizeof(int32_t) * (HALO_HASH + HALO_LIST);
+    hipLaunchKernelGGL(k_halo<false>, dim3((unsigned)nblk), dim3(HALO_T), hl, c->stream, n, (int)PB, c->rows(),
+                       c->cnt, c->bw, count, nullptr, nullptr, nullptr);
+    PDX_HIP(c, hipGetLastError());
     PDX_TRY(pdx_alloc(c, &c->halo_ptr, nblk + 1));
-    PDX_TRY(pdx_alloc(c, &c->halo, halo.size()));
-    PDX_HIP(c, hipMemcpy(c->bw16, w16.data(), sizeof(uint16_t) * nba, hipMemcpyHostToDevice));
-    PDX_HIP(c, hipMemcpy(c->halo_ptr, hp.data(), sizeof(int64_t) * (nblk + 1), hipMemcpyHostToDevice));
-    PDX_HIP(c, hipMemcpy(c->halo, halo.data(), sizeof(int32_t) * halo.size(), hipMemcpyHostToDevice));
-    c->halo_max = (int32_t)hmax;
-    c->halo_total = hp[nblk];
+    PDX_TRY(scan_i32(c, S, nblk, count, c->halo_ptr));
+    unsigned long long *mx = c->d_flags + 6, h[1] = {0};
+    int64_t total = 0;
+    PDX_HIP(c, hipMemcpyAsync(mx, h, sizeof h, hipMemcpyHostToDevice, c->stream));
+    hipLaunchKernelGGL(k_max_i32, dim3((unsigned)std::min<int64_t>((nblk + 255) / 256, 256)), dim3(256), 0, c->stream,
+                       nblk, count, mx);
+    PDX_HIP(c, hipMemcpyAsync(h, mx, sizeof h, hipMemcpyDeviceToHost, c->stream));
+    PDX_HIP(c, hipMemcpyAsync(&total, c->halo_ptr + nblk, sizeof total, hipMemcpyDeviceToHost, c->stream));
+    PDX_HIP(c, hipStreamSynchronize(c->stream));
+    // a longer table: the global-gather kernels
+    if (h[0] > HALO_LIST) {
+        FREE(c->halo_ptr);
+        c->dev_bytes -= (int64_t)sizeof(int64_t) * (nblk + 1);
+        return PDX_OK;
+    }
+    PDX_TRY(pdx_alloc(c, &c->bw16, c->nb_alloc));
+    PDX_TRY(pdx_alloc(c, &c->halo, std::max<int64_t>(total, 1)));
+    hipLaunchKernelGGL(k_halo<true>, dim3((unsigned)nblk), dim3(HALO_T), hl, c->stream, n, (int)PB, c->rows(),
+                       c->cnt, c->bw, count, c->halo_ptr, c->halo, c->bw16);
+    PDX_HIP(c, hipGetLastError());
+    c->halo_max = (int32_t)h[0];
+    c->halo_total = total;
     c->lds_mode = true;
     *ok = true;
     return pack_bonds(c);
@@ -758,28 +1102,30 @@ static void choose_blocks(pdx_ctx *c, bool lds)
 }
 
 // the rows of the chosen layout: slice pointers, bond words and lengths
-static pdx_status fill_rows(pdx_ctx *c, search_args &s, const std::vector<int32_t> &counts)
+static pdx_status fill_rows(pdx_ctx *c, search_args &s)
 {
     if (c->bw) c->dev_bytes -= (int64_t)(sizeof(uint32_t) + sizeof(double)) * c->nb_alloc;
     FREE(c->slice_ptr);
     FREE(c->bw);
     FREE(c->L);
-    const int64_t n = c->n, n_slices = c->n_slices(), P = 64 >> c->ls;
-    std::vector<int64_t> slice_ptr(n_slices + 1, 0);
-    for (int64_t sl = 0; sl < n_slices; sl++) {
-        int32_t w = 0;
-        for (int64_t m = P * sl; m < std::min(n, P * sl + P); m++) w = std::max(w, counts[m]);
-        slice_ptr[sl + 1] = slice_ptr[sl] + 64 * (int64_t)c->rows().groups(w);
-    }
-    const int64_t nba = c->nb_alloc = slice_ptr[n_slices];
-    if (nba >= ((int64_t)1 << 40)) return pdx_fail(c, PDX_ERR_UNSUPPORTED, "too many bonds");
+    const int64_t n = c->n, n_slices = c->n_slices();
+    setup_scratch S;
+    int32_t *width;
+    PDX_TRY(S.get(c, &width, n_slices));
     PDX_TRY(pdx_alloc(c, &c->slice_ptr, n_slices + 1));
+    hipLaunchKernelGGL(k_slice_width, grid256(n_slices), dim3(256), 0, c->stream, n, n_slices, c->rows(), c->cnt, width);
+    PDX_TRY(scan_i32(c, S, n_slices, width, c->slice_ptr));
+    int64_t nba = 0;
+    PDX_HIP(c, hipMemcpyAsync(&nba, c->slice_ptr + n_slices, sizeof nba, hipMemcpyDeviceToHost, c->stream));
+    PDX_HIP(c, hipStreamSynchronize(c->stream));
+    c->nb_alloc = nba;
+    if (nba >= ((int64_t)1 << 40)) return pdx_fail(c, PDX_ERR_UNSUPPORTED, "too many bonds");
     PDX_TRY(pdx_alloc(c, &c->bw, nba));
     PDX_TRY(pdx_alloc(c, &c->L, nba));
-    PDX_HIP(c, hipMemcpy(c->slice_ptr, slice_ptr.data(), sizeof(int64_t) * (n_slices + 1), hipMemcpyHostToDevice));
     // padding slots: bond word 0, length 1
     PDX_HIP(c, hipMemsetAsync(c->bw, 0, sizeof(uint32_t) * nba, c->stream));
-    hipLaunchKernelGGL(k_fill_value, dim3((unsigned)((nba + 255) / 256)), dim3(256), 0, c->stream, nba, 1.0, c->L);
+    if (nba > 0)
+        hipLaunchKernelGGL(k_fill_value, grid256(nba), dim3(256), 0, c->stream, nba, 1.0, c->L);
     s.rows = c->rows();
     s.cnt = c->cnt;
     s.bw = c->bw;
@@ -791,7 +1137,10 @@ static pdx_status fill_rows(pdx_ctx *c, search_args &s, const std::vector<int32_
 }
 
 // ----------------------------------------------------------------------------------------
-// pdx_build_bonds
+// pdx_build_bonds.  The host takes part only to size allocations (four synchronisations).  A
+// 576 k-point BB body of 61 M bonds: 8.6 ms (fill 1.5, tables 1.7, count 1.3, packing 0.5, sort 0.5
+// ms of kernels, the rest allocations and the upload) against 0.27 s with the sort, the cell list
+// and the tables on the host (the tables alone moved the 32-bit words to the host and back).
 // ----------------------------------------------------------------------------------------
 extern "C" pdx_status pdx_build_bonds(pdx_ctx *c, int64_t *n_bonds_out)
 {
@@ -806,27 +1155,9 @@ extern "C" pdx_status pdx_build_bonds(pdx_ctx *c, int64_t *n_bonds_out)
         pdx_free_all(c);
         c->cracks = keep;
     }
-    // Morton order
-    morton_order(c->X, n, c->perm);
-    c->iperm.assign(n, 0);
-    for (int64_t m = 0; m < n; m++) c->iperm[c->perm[m]] = (int32_t)m;
-    std::vector<double4> Xm(n);
-    std::vector<uint8_t> fpm(n);
-    for (int64_t m = 0; m < n; m++) {
-        int64_t i = c->perm[m];
-        Xm[m] = make_double4(c->X[3 * i], c->X[3 * i + 1], c->X[3 * i + 2], c->vol[i]);
-        fpm[m] = c->fail_permit[i];
-    }
     // cell list over the internal order, cell size = horizon
     double cs = c->P.delta;
-    double mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
-    for (int64_t m = 0; m < n; m++) {
-        const double v3[3] = {Xm[m].x, Xm[m].y, Xm[m].z};
-        for (int d = 0; d < 3; d++) {
-            mn[d] = std::min(mn[d], v3[d]);
-            mx[d] = std::max(mx[d], v3[d]);
-        }
-    }
+    double *const mn = c->mn, *const mx = c->mx;
     for (;;) {
         double ncell = 1;
         for (int d = 0; d < 3; d++) ncell *= std::floor((mx[d] - mn[d]) / cs) + 1.0;
@@ -835,34 +1166,15 @@ extern "C" pdx_status pdx_build_bonds(pdx_ctx *c, int64_t *n_bonds_out)
     }
     int64_t g[3];
     for (int d = 0; d < 3; d++) g[d] = (int64_t)std::floor((mx[d] - mn[d]) / cs) + 1;
-    int64_t ncell = g[0] * g[1] * g[2];
-    std::vector<int32_t> pcell(3 * n);
-    std::vector<int64_t> cell_start(ncell + 1, 0);
-    std::vector<int64_t> cid(n);
-    for (int64_t m = 0; m < n; m++) {
-        const double v3[3] = {Xm[m].x, Xm[m].y, Xm[m].z};
-        for (int d = 0; d < 3; d++) {
-            int64_t q = (int64_t)std::floor((v3[d] - mn[d]) / cs);
-            q = std::min(std::max(q, (int64_t)0), g[d] - 1);
-            pcell[3 * m + d] = (int32_t)q;
-        }
-        cid[m] = pcell[3 * m] + g[0] * (pcell[3 * m + 1] + g[1] * (int64_t)pcell[3 * m + 2]);
-        cell_start[cid[m] + 1]++;
-    }
-    for (int64_t k = 0; k < ncell; k++) cell_start[k + 1] += cell_start[k];
-    std::vector<int32_t> cell_pts(n);
-    {
-        std::vector<int64_t> fill(cell_start.begin(), cell_start.end() - 1);
-        for (int64_t m = 0; m < n; m++) cell_pts[fill[cid[m]]++] = (int32_t)m;
-    }
+    const int64_t ncell = g[0] * g[1] * g[2];
     // crack membership masks
     std::vector<uint16_t> cmask;
     uint32_t filt_bits = 0;
     if (!c->cracks.empty()) {
         cmask.assign(n, 0);
         for (size_t k = 0; k < c->cracks.size(); k++) {
-            for (int32_t i : c->cracks[k].a) cmask[c->iperm[i]] |= (uint16_t)(1u << (2 * k));
-            for (int32_t i : c->cracks[k].b) cmask[c->iperm[i]] |= (uint16_t)(1u << (2 * k + 1));
+            for (int32_t i : c->cracks[k].a) cmask[i] |= (uint16_t)(1u << (2 * k));
+            for (int32_t i : c->cracks[k].b) cmask[i] |= (uint16_t)(1u << (2 * k + 1));
             if (c->cracks[k].filter) filt_bits |= 1u << (2 * k);
         }
     }
@@ -879,51 +1191,39 @@ extern "C" pdx_status pdx_build_bonds(pdx_ctx *c, int64_t *n_bonds_out)
     PDX_TRY(pdx_alloc(c, &c->nact, n));
     PDX_TRY(pdx_alloc(c, &c->killed, n));
     PDX_TRY(pdx_alloc(c, &c->bcslot, n));
-    int32_t *d_pcell = nullptr, *d_cell_pts = nullptr, *d_counts = nullptr;
-    int64_t *d_cell_start = nullptr;
-    uint16_t *d_cmask = nullptr;
-    auto cleanup = [&]() {
-        FREE(d_pcell);
-        FREE(d_cell_pts);
-        FREE(d_counts);
-        FREE(d_cell_start);
-        FREE(d_cmask);
-    };
-#define TRY_C(expr)                                                                         \
-    do {                                                                                    \
-        pdx_status s_ = (expr);                                                             \
-        if (s_ != PDX_OK) {                                                                 \
-            cleanup();                                                                      \
-            return s_;                                                                      \
-        }                                                                                   \
-    } while (0)
-#define HIP_C(call)                                                                         \
-    do {                                                                                    \
-        hipError_t e_ = (call);                                                             \
-        if (e_ != hipSuccess) {                                                             \
-            cleanup();                                                                      \
-            return pdx_fail(c, PDX_ERR_HIP, "%s failed: %s", #call, hipGetErrorString(e_)); \
-        }                                                                                   \
-    } while (0)
-    HIP_C(hipMalloc((void **)&d_pcell, sizeof(int32_t) * 3 * n));
-    HIP_C(hipMalloc((void **)&d_cell_pts, sizeof(int32_t) * n));
-    HIP_C(hipMalloc((void **)&d_counts, sizeof(int32_t) * n));
-    HIP_C(hipMalloc((void **)&d_cell_start, sizeof(int64_t) * (ncell + 1)));
-    TRY_C(pdx_alloc(c, &c->d_fp, n));
-    if (!cmask.empty()) HIP_C(hipMalloc((void **)&d_cmask, sizeof(uint16_t) * n));
-    HIP_C(hipMemcpy(c->Xr, Xm.data(), sizeof(double4) * n, hipMemcpyHostToDevice));
-    HIP_C(hipMemcpy(c->rec[0], Xm.data(), sizeof(double4) * n, hipMemcpyHostToDevice));
-    HIP_C(hipMemcpy(c->rec[1], Xm.data(), sizeof(double4) * n, hipMemcpyHostToDevice));
-    HIP_C(hipMemcpy(c->d_perm, c->perm.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice));
-    HIP_C(hipMemcpy(c->d_iperm, c->iperm.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice));
-    HIP_C(hipMemcpy(d_pcell, pcell.data(), sizeof(int32_t) * 3 * n, hipMemcpyHostToDevice));
-    HIP_C(hipMemcpy(d_cell_pts, cell_pts.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice));
-    HIP_C(hipMemcpy(d_cell_start, cell_start.data(), sizeof(int64_t) * (ncell + 1),
-                    hipMemcpyHostToDevice));
-    HIP_C(hipMemcpy(c->d_fp, fpm.data(), n, hipMemcpyHostToDevice));
-    if (d_cmask)
-        HIP_C(hipMemcpy(d_cmask, cmask.data(), sizeof(uint16_t) * n, hipMemcpyHostToDevice));
-    HIP_C(hipMemset(c->d_flags, 0, 8 * sizeof(unsigned long long)));
+    PDX_TRY(pdx_alloc(c, &c->d_fp, n));
+    setup_scratch S;
+    double *dX, *dV;
+    uint8_t *dfp;
+    uint16_t *dcm_in = nullptr, *d_cmask = nullptr;
+    int32_t *d_pcell, *d_cell_pts, *d_num;
+    int64_t *d_cell_start;
+    PDX_TRY(S.get(c, &dX, 3 * n));
+    PDX_TRY(S.get(c, &dV, n));
+    PDX_TRY(S.get(c, &dfp, n));
+    PDX_TRY(S.get(c, &d_pcell, 3 * n));
+    PDX_TRY(S.get(c, &d_cell_pts, n));
+    PDX_TRY(S.get(c, &d_num, ncell));
+    PDX_TRY(S.get(c, &d_cell_start, ncell + 1));
+    if (!cmask.empty()) {
+        PDX_TRY(S.get(c, &dcm_in, n));
+        PDX_TRY(S.get(c, &d_cmask, n));
+        PDX_HIP(c, hipMemcpyAsync(dcm_in, cmask.data(), sizeof(uint16_t) * n, hipMemcpyHostToDevice, c->stream));
+    }
+    PDX_HIP(c, hipMemcpyAsync(dX, c->X.data(), sizeof(double) * 3 * n, hipMemcpyHostToDevice, c->stream));
+    PDX_HIP(c, hipMemcpyAsync(dV, c->vol.data(), sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
+    PDX_HIP(c, hipMemcpyAsync(dfp, c->fail_permit.data(), n, hipMemcpyHostToDevice, c->stream));
+    PDX_HIP(c, hipMemsetAsync(c->d_flags, 0, 8 * sizeof(unsigned long long), c->stream));
+    PDX_HIP(c, hipMemsetAsync(d_num, 0, sizeof(int32_t) * ncell, c->stream));
+    PDX_TRY(morton_order(c, S, dX, mn, mx));
+    hipLaunchKernelGGL(k_gather_points, grid256(n), dim3(256), 0, c->stream, n, c->d_perm, dX, dV, dfp, dcm_in, c->Xr,
+                       c->rec[0], c->rec[1], c->d_fp, d_cmask);
+    const double3 mn3 = make_double3(mn[0], mn[1], mn[2]);
+    hipLaunchKernelGGL(k_cells, grid256(n), dim3(256), 0, c->stream, n, c->Xr, mn3, cs, g[0], g[1], g[2], d_pcell, d_num);
+    PDX_TRY(scan_i32(c, S, ncell, d_num, d_cell_start));
+    hipLaunchKernelGGL(k_cell_points, grid256(n), dim3(256), 0, c->stream, n, d_pcell, g[0], g[1], d_cell_start, d_num,
+                       d_cell_pts);
+    PDX_HIP(c, hipGetLastError());
     // Each (Xr) record keeps the volume in .w for the bond passes; the reference record's
     // .w holds the volume too (only .xyz are read as the reference position).
 
@@ -941,74 +1241,62 @@ extern "C" pdx_status pdx_build_bonds(pdx_ctx *c, int64_t *n_bonds_out)
     s.cmask = d_cmask;
     s.filt_bits = filt_bits;
     s.fp = c->d_fp;
-    s.counts = d_counts;
+    PDX_TRY(pdx_alloc(c, &c->cnt, n));
+    s.counts = c->cnt;
     s.flags = c->d_flags;
     hipLaunchKernelGGL(k_count_bonds, dim3((unsigned)pdx_wave_grid(n)), dim3(PDX_BLOCK), 0, c->stream, s);
-    HIP_C(hipGetLastError());
-    std::vector<int32_t> counts(n);
-    HIP_C(hipMemcpyAsync(counts.data(), d_counts, sizeof(int32_t) * n, hipMemcpyDeviceToHost,
-                         c->stream));
+    hipLaunchKernelGGL(k_count_totals, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 512)), dim3(256), 0, c->stream, n,
+                       c->cnt, c->d_flags + 4);
+    PDX_HIP(c, hipGetLastError());
     unsigned long long hflags[8];
-    HIP_C(hipMemcpyAsync(hflags, c->d_flags, sizeof hflags, hipMemcpyDeviceToHost, c->stream));
-    HIP_C(hipStreamSynchronize(c->stream));
-    if (hflags[1]) {
-        cleanup();
+    PDX_HIP(c, hipMemcpyAsync(hflags, c->d_flags, sizeof hflags, hipMemcpyDeviceToHost, c->stream));
+    PDX_HIP(c, hipStreamSynchronize(c->stream));
+    if (hflags[1])
         return pdx_fail(c, PDX_ERR_DUPLICATE_POINT,
                         "point duplicate found! Point #%llu has a duplicate #%llu which will lead to NaNs",
                         hflags[2] + 1, hflags[3] + 1);
-    }
-    int32_t maxc = 0;
-    int64_t nb = 0;
-    for (int64_t m = 0; m < n; m++) {
-        maxc = std::max(maxc, counts[m]);
-        nb += counts[m];
-    }
-    if (maxc > PDX_FILL_CAP) {
-        cleanup();
-        return pdx_fail(c, PDX_ERR_UNSUPPORTED, "a point has %d bonds (> %d)", maxc, PDX_FILL_CAP);
-    }
+    const int64_t nb = (int64_t)hflags[4];
+    if (hflags[5] > PDX_FILL_CAP)
+        return pdx_fail(c, PDX_ERR_UNSUPPORTED, "a point has %d bonds (> %d)", (int)hflags[5], PDX_FILL_CAP);
     c->nb = nb;
     choose_blocks(c, !getenv("PDX_NO_LDS"));
-    TRY_C(pdx_alloc(c, &c->cnt, n));
-    HIP_C(hipMemcpy(c->cnt, counts.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice));
-    TRY_C(fill_rows(c, s, counts));
+    PDX_TRY(fill_rows(c, s));
     // the LDS-staged layout; tables it cannot address go to the global-gather layout
     if (c->ls > 0) {
         bool ok = false;
-        TRY_C(build_halos(c, &ok));
+        PDX_TRY(build_halos(c, &ok));
         if (!ok) {
             choose_blocks(c, false);
-            TRY_C(fill_rows(c, s, counts));
+            PDX_TRY(fill_rows(c, s));
         }
     }
     hipLaunchKernelGGL(k_init_point_state, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
                        c->stream, n, c->rows(), c->cnt, c->bw, c->nact, c->damage);
-    HIP_C(hipGetLastError());
+    PDX_HIP(c, hipGetLastError());
     // zero dynamic state
     for (double *p : {c->u, c->vh, c->v, c->a, c->bint, c->bext})
-        HIP_C(hipMemsetAsync(p, 0, sizeof(double) * 3 * n, c->stream));
-    HIP_C(hipMemsetAsync(c->killed, 0, n, c->stream));
-    HIP_C(hipMemsetAsync(c->bcslot, 0xff, sizeof(int32_t) * n, c->stream));
-    HIP_C(hipStreamSynchronize(c->stream));
+        PDX_HIP(c, hipMemsetAsync(p, 0, sizeof(double) * 3 * n, c->stream));
+    PDX_HIP(c, hipMemsetAsync(c->killed, 0, n, c->stream));
+    PDX_HIP(c, hipMemsetAsync(c->bcslot, 0xff, sizeof(int32_t) * n, c->stream));
+    PDX_HIP(c, hipStreamSynchronize(c->stream));
     c->bext_nonzero = false;
     c->cur = 0;
     c->n_src = 0;
     c->n_bcpts = 0;
     // material state between the passes
     // OSB: the per-point pair of pass 1, then (LDS layout, one set) the own force part
-    if (c->kind == PDX_OSB) TRY_C(pdx_alloc(c, &c->pstate, 5 * n));
+    if (c->kind == PDX_OSB) PDX_TRY(pdx_alloc(c, &c->pstate, 5 * n));
     if (c->kind == PDX_CPD) {
         // Q per point; with ZEMWan also the stabilisation stiffness C_1 (15 numbers per point).
         // The LDS passes keep six more per point behind those: the own bond terms and
         // a = Q X + beta x (ZEMWan: Q X + C_1 x)
-        TRY_C(pdx_alloc(c, &c->pstate, (c->P.zem == PDX_ZEM_WAN ? 21 : 15) * n));
-        TRY_C(pdx_alloc(c, &c->defgrad, 9 * n));
-        TRY_C(pdx_alloc(c, &c->cauchy, 9 * n));
-        HIP_C(hipMemsetAsync(c->defgrad, 0, sizeof(double) * 9 * n, c->stream));
-        HIP_C(hipMemsetAsync(c->cauchy, 0, sizeof(double) * 9 * n, c->stream));
-        HIP_C(hipStreamSynchronize(c->stream));
+        PDX_TRY(pdx_alloc(c, &c->pstate, (c->P.zem == PDX_ZEM_WAN ? 21 : 15) * n));
+        PDX_TRY(pdx_alloc(c, &c->defgrad, 9 * n));
+        PDX_TRY(pdx_alloc(c, &c->cauchy, 9 * n));
+        PDX_HIP(c, hipMemsetAsync(c->defgrad, 0, sizeof(double) * 9 * n, c->stream));
+        PDX_HIP(c, hipMemsetAsync(c->cauchy, 0, sizeof(double) * 9 * n, c->stream));
+        PDX_HIP(c, hipStreamSynchronize(c->stream));
     }
-    cleanup();
     // FP32 lengths for the global-gather mixed BB step (the LDS-staged steps take L = |D|)
     if (c->precision == PDX_MIXED && !c->lds_mode) {
         const int64_t nba = c->nb_alloc;
@@ -1031,8 +1319,6 @@ extern "C" pdx_status pdx_build_bonds(pdx_ctx *c, int64_t *n_bonds_out)
     c->bonds_built = true;
     if (n_bonds_out) *n_bonds_out = nb;
     return PDX_OK;
-#undef TRY_C
-#undef HIP_C
 }
 
 pdx_status pdx_caller_bond_slots(pdx_ctx *c, std::vector<int64_t> &slots)
@@ -1304,6 +1590,19 @@ __global__ __launch_bounds__(PDX_BLOCK) void k_timestep(int64_t n, pdx_rows rows
     }
 }
 
+// minimum over each workgroup's share of v (NaN entries are passed over, as std::min does)
+__global__ __launch_bounds__(256) void k_min(int64_t n, const double *v, double *out)
+{
+    __shared__ double sh[4];
+    double m = INFINITY;
+    for (int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x; k < n; k += (int64_t)gridDim.x * 256)
+        m = v[k] < m ? v[k] : m;
+    for (int o = 32; o > 0; o >>= 1) m = fmin(m, __shfl_xor(m, o));
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) out[blockIdx.x] = fmin(fmin(sh[0], sh[1]), fmin(sh[2], sh[3]));
+}
+
 extern "C" pdx_status pdx_stable_timestep(pdx_ctx *c, double safety, double *dt_out)
 {
     if (!c || !dt_out) return PDX_ERR_ARG;
@@ -1316,12 +1615,14 @@ extern "C" pdx_status pdx_stable_timestep(pdx_ctx *c, double safety, double *dt_
                        c->stream, c->n, c->rows(), c->cnt, c->bw, c->L, c->Xr, c->d_perm, c->P.bc,
                        c->P.rho, c->multi() ? c->d_psets : nullptr, c->multi() ? c->d_pid : nullptr, tmp);
     PDX_HIP(c, hipGetLastError());
-    std::vector<double> dt(c->n);
-    PDX_HIP(c, hipMemcpyAsync(dt.data(), tmp, sizeof(double) * c->n, hipMemcpyDeviceToHost,
-                              c->stream));
+    const int nb = (int)std::min<int64_t>((c->n + 255) / 256, 256);
+    hipLaunchKernelGGL(k_min, dim3(nb), dim3(256), 0, c->stream, c->n, tmp, tmp + c->n);
+    PDX_HIP(c, hipGetLastError());
+    double dt[256];
+    PDX_HIP(c, hipMemcpyAsync(dt, tmp + c->n, sizeof(double) * nb, hipMemcpyDeviceToHost, c->stream));
     PDX_HIP(c, hipStreamSynchronize(c->stream));
     double mn = INFINITY;
-    for (double d : dt) mn = std::min(mn, d);
+    for (int k = 0; k < nb; k++) mn = std::min(mn, dt[k]);
     *dt_out = mn * safety;
     return PDX_OK;
 }

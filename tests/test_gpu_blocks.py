@@ -101,3 +101,24 @@ def test_relaxation_force_density(need_gpu, oracle, kind, shape):
     assert scaled_error(dh.get("b_int"), orc) <= FP64_TOL
     assert np.array_equal(dh.get("n_active_bonds"), orc.n_active)
     dh.close()
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (2, 1, 1), (65, 1, 1), (70, 50, 40)])
+def test_bond_lists_of_the_device_set_up(need_gpu, oracle, shape):
+    """Bond lists, lengths and the stable time step of bodies from one point to many sort and
+    scan runs, with a precrack through the larger one."""
+    say("device set-up", shape)
+    b = body_of("BB", shape, 3.015)
+    y = b.position[1]
+    if shape[1] > 1:
+        pd.point_set(b, "a", (y > 0) & (y < 6e-3) & (b.position[0] < 0))
+        pd.point_set(b, "b", (y <= 0) & (y > -6e-3) & (b.position[0] < 0))
+        pd.precrack(b, "a", "b")
+    dh = pd.MI355XBodyDataHandler(b)
+    orc = oracle_for(oracle, b, "BB")
+    act = bonds_equal(dh, orc)
+    assert np.array_equal(act, orc.active)
+    assert np.array_equal(dh.get("n_active_bonds"), orc.n_active)
+    if shape[0] > 1:
+        assert dh.calc_stable_timestep() == orc.stable_dt()
+    dh.close()
