@@ -8,9 +8,139 @@
 // caller launches next overlap with the copy, and the host writes the files of one export
 // while the device computes the next ones.  Two slots alternate, so one export can be
 // written out while the next is copied.
+#include <algorithm>
+#include <atomic>
 #include <cstring>
+#include <thread>
 
 #include "pdx_internal.h"
+
+// ----------------------------------------------------------------------------------------
+// A field into the caller's memory.  The runtime's copy into pageable memory runs at the speed of
+// one thread that takes the page faults of a fresh array and copies out of a staging buffer.  Here
+// the gather into the caller's order writes straight into a pinned ring, over the bus, a slot per
+// launch, and the calling thread with up to seven helpers carries the values over in pieces; the
+// helpers touch the pages of their next piece while it is still under way.  24 MB into a new array:
+// 6.6 ms in one piece by the runtime; the bus alone 0.47 ms (by the gather as by the copy engine;
+// in slots of 2 MB with an event each 0.51 against the engine's 0.60, in slots of 512 KB 0.68 against
+// 1.1); out of pinned memory with 1 / 2 / 4 / 8 threads 6.0 / 3.8 / 2.2 / 1.4 ms.  A single piece is
+// copied by the calling thread alone (8 KB: 12 us, 26 us by the runtime).
+// ----------------------------------------------------------------------------------------
+#define PIN_PIECE ((size_t)512 << 10)
+
+void pdx_pin_free(pdx_ctx *c)
+{
+    if (c->pin) (void)hipHostFree(c->pin);
+    c->pin = nullptr;
+    c->pin_slots = 0;
+    for (hipEvent_t &e : c->pin_ev) {
+        if (e) (void)hipEventDestroy(e);
+        e = nullptr;
+    }
+}
+
+// room for `slots` slots; false: not to be had
+static bool pin_reserve(pdx_ctx *c, int slots)
+{
+    for (int k = 0; k < slots; k++)
+        if (!c->pin_ev[k] && hipEventCreateWithFlags(&c->pin_ev[k], hipEventDisableTiming) != hipSuccess) {
+            c->pin_ev[k] = nullptr;
+            (void)hipGetLastError();
+            return false;
+        }
+    if (c->pin_slots >= slots) return true;
+    if (c->pin) (void)hipHostFree(c->pin);
+    c->pin_slots = 0;
+    if (hipHostMalloc((void **)&c->pin, slots * PDX_PIN_CHUNK, hipHostMallocDefault) != hipSuccess) {
+        c->pin = nullptr;
+        (void)hipGetLastError();
+        return false;
+    }
+    c->pin_slots = slots;
+    return true;
+}
+
+pdx_status pdx_download_vec(pdx_ctx *c, const double *dev, double *host, int comps, int stride)
+{
+    constexpr int64_t SLOT = PDX_PIN_CHUNK / sizeof(double), PIECE = PIN_PIECE / sizeof(double), PER = SLOT / PIECE;
+    const int64_t cnt = c->n * comps;
+    const int64_t nch = (cnt + SLOT - 1) / SLOT, npc = (cnt + PIECE - 1) / PIECE;
+    const int slots = (int)std::min<int64_t>(nch, PDX_PIN_SLOTS);
+    if (!pin_reserve(c, slots)) {
+        PDX_TRY(pdx_gather_range(c, dev, comps, stride, 0, cnt, c->stage));
+        PDX_HIP(c, hipMemcpyAsync(host, c->stage, sizeof(double) * cnt, hipMemcpyDeviceToHost, c->stream));
+        PDX_HIP(c, hipStreamSynchronize(c->stream));
+        return PDX_OK;
+    }
+    double *const pin = c->pin;
+    if (npc == 1) {
+        PDX_TRY(pdx_gather_range(c, dev, comps, stride, 0, cnt, pin));
+        PDX_HIP(c, hipStreamSynchronize(c->stream));
+        memcpy(host, pin, sizeof(double) * cnt);
+        return PDX_OK;
+    }
+    // Chunk k passes through slot k % slots in PER pieces.  `ready` pieces have arrived, `next` is the
+    // first one that nobody has taken, left[s] counts the pieces carried out of slot s.
+    std::atomic<int64_t> ready{0}, next{0};
+    std::atomic<int64_t> left[PDX_PIN_SLOTS] = {};
+    std::atomic<bool> stop{false};
+    auto carry = [&](int64_t k) {
+        const int64_t s = (k / PER) % slots;
+        memcpy(host + k * PIECE, pin + s * SLOT + (k % PER) * PIECE, sizeof(double) * std::min(PIECE, cnt - k * PIECE));
+        left[s].fetch_add(1, std::memory_order_release);
+    };
+    auto helper = [&]() {
+        for (int64_t k; (k = next.fetch_add(1)) < npc;) {
+            volatile double *const h = host + k * PIECE;
+            for (int64_t o = 0; o < std::min(PIECE, cnt - k * PIECE); o += 512) h[o] = 0.0;
+            while (ready.load(std::memory_order_acquire) <= k) {
+                if (stop.load()) return;
+                std::this_thread::yield();
+            }
+            carry(k);
+        }
+    };
+    pdx_status st = PDX_OK;
+    int64_t issued = 0, arrived = 0;
+    // every chunk whose slot is free goes on the stream
+    auto issue = [&]() -> pdx_status {
+        for (; issued < nch; issued++) {
+            const int64_t s = issued % slots;
+            if (left[s].load(std::memory_order_acquire) < issued / slots * PER) break;
+            PDX_TRY(pdx_gather_range(c, dev, comps, stride, issued * SLOT, std::min(cnt, (issued + 1) * SLOT), pin + s * SLOT));
+            PDX_HIP(c, hipEventRecord(c->pin_ev[s], c->stream));
+        }
+        return PDX_OK;
+    };
+    auto arrive = [&]() -> pdx_status {
+        PDX_HIP(c, hipEventSynchronize(c->pin_ev[arrived % slots]));
+        arrived++;
+        ready.store(std::min(npc, arrived * PER), std::memory_order_release);
+        return PDX_OK;
+    };
+    st = issue();
+    const int64_t want = std::min<int64_t>(std::min<int64_t>(7, npc - 1), (int64_t)std::thread::hardware_concurrency() - 1);
+    std::thread th[7];
+    int nth = 0;
+    try {
+        for (; nth < want; nth++) th[nth] = std::thread(helper);
+    } catch (...) {
+        // no more threads to be had: those there are, and this one, do the work
+    }
+    while (st == PDX_OK && (arrived < nch || next.load() < npc)) {
+        st = issue();
+        if (st == PDX_OK && arrived < issued) {
+            st = arrive();
+            if (arrived < issued && nth > 0) continue;  // the next one first: the helpers wait for it
+        }
+        int64_t k = next.load();  // a piece that has arrived and that nobody has taken
+        if (k < ready.load() && next.compare_exchange_strong(k, k + 1)) carry(k);
+        else std::this_thread::yield();
+    }
+    if (st != PDX_OK) stop.store(true);
+    for (int k = 0; k < nth; k++) th[k].join();
+    return st;
+}
 
 #define PDX_EXPORT_MAX_FIELDS 16
 

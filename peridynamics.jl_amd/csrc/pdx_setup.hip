@@ -138,6 +138,7 @@ extern "C" void pdx_destroy(pdx_ctx *c)
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     pdx_export_free(c);
+    pdx_pin_free(c);
     pdx_free_all(c);
     FREE(c->d_flags);
     (void)pdx_timed_flush(c);
@@ -794,15 +795,22 @@ __global__ void k_scatter_in(int64_t n, int comps, int stride, const int32_t *pe
     dev[m * stride + d] = stage[(int64_t)perm[m] * comps + d];
 }
 
-// stage[i*comps + d] = dev[iperm[i]*stride + d]
-__global__ void k_gather_out(int64_t n, int comps, int stride, const int32_t *iperm,
-                             const double *dev, double *stage)
+// dst[t - t0] = dev[iperm[t / comps] * stride + t % comps]
+__global__ void k_gather_out(int64_t t0, int64_t t1, int comps, int stride, const int32_t *iperm, const double *dev,
+                             double *dst)
 {
-    int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n * comps) return;
-    int64_t i = t / comps;
-    int d = (int)(t - i * comps);
-    stage[t] = dev[(int64_t)iperm[i] * stride + d];
+    const int64_t t = t0 + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= t1) return;
+    const int64_t i = t / comps;
+    const int d = (int)(t - i * comps);
+    dst[t - t0] = dev[(int64_t)iperm[i] * stride + d];
+}
+
+pdx_status pdx_gather_range(pdx_ctx *c, const double *dev, int comps, int stride, int64_t t0, int64_t t1, double *dst)
+{
+    hipLaunchKernelGGL(k_gather_out, grid256(t1 - t0), dim3(256), 0, c->stream, t0, t1, comps, stride, c->d_iperm, dev, dst);
+    PDX_HIP(c, hipGetLastError());
+    return PDX_OK;
 }
 
 pdx_status pdx_upload_vec(pdx_ctx *c, const double *host, double *dev, int comps)
@@ -820,19 +828,6 @@ pdx_status pdx_upload_strided(pdx_ctx *c, const double *host, double *dev, int c
     hipLaunchKernelGGL(k_scatter_in, dim3(blocks), dim3(256), 0, c->stream, c->n, comps, stride,
                        c->d_perm, c->stage, dev);
     PDX_HIP(c, hipGetLastError());
-    PDX_HIP(c, hipStreamSynchronize(c->stream));
-    return PDX_OK;
-}
-
-pdx_status pdx_download_vec(pdx_ctx *c, const double *dev, double *host, int comps, int stride)
-{
-    int64_t cnt = c->n * comps;
-    int64_t blocks = (cnt + 255) / 256;
-    hipLaunchKernelGGL(k_gather_out, dim3(blocks), dim3(256), 0, c->stream, c->n, comps, stride,
-                       c->d_iperm, dev, c->stage);
-    PDX_HIP(c, hipGetLastError());
-    PDX_HIP(c, hipMemcpyAsync(host, c->stage, sizeof(double) * cnt, hipMemcpyDeviceToHost,
-                              c->stream));
     PDX_HIP(c, hipStreamSynchronize(c->stream));
     return PDX_OK;
 }
@@ -1484,17 +1479,11 @@ pdx_status pdx_gather_field(pdx_ctx *c, int field, double *dst)
         double *tmp = c->stage + 4 * c->n;  // second half of the staging buffer
         hipLaunchKernelGGL(k_int_to_double, dim3((c->n + 255) / 256), dim3(256), 0, c->stream,
                            c->n, c->nact, tmp);
-        hipLaunchKernelGGL(k_gather_out, dim3((c->n + 255) / 256), dim3(256), 0, c->stream,
-                           c->n, 1, 1, c->d_iperm, tmp, dst);
         PDX_HIP(c, hipGetLastError());
-        return PDX_OK;
+        return pdx_gather_range(c, tmp, 1, 1, 0, c->n, dst);
     }
     PDX_TRY(pdx_field_ptr(c, field, &p, &comps, &stride));
-    const int64_t cnt = c->n * comps;
-    hipLaunchKernelGGL(k_gather_out, dim3((cnt + 255) / 256), dim3(256), 0, c->stream, c->n, comps,
-                       stride, c->d_iperm, p, dst);
-    PDX_HIP(c, hipGetLastError());
-    return PDX_OK;
+    return pdx_gather_range(c, p, comps, stride, 0, c->n * comps, dst);
 }
 
 extern "C" pdx_status pdx_get_field(pdx_ctx *c, int32_t field, double *host)

@@ -278,7 +278,7 @@ class Context:
 
     def get_field(self, name):
         fid, comps = FIELDS[name]
-        out = np.zeros((self.n, comps), np.float64)
+        out = np.empty((self.n, comps), np.float64)
         self.call("pdx_get_field", fid, ptr(out))
         return out if comps > 1 else out[:, 0]
 

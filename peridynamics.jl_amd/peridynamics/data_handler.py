@@ -27,7 +27,7 @@ class MI355XBodyDataHandler:
         if np.any(body.params_map == 0):
             raise _arg_error("not all points have material parameters (material!)")
         # distinct parameter sets in use (ParameterHandler, parameter_handler.jl:36-55)
-        used = sorted(set(int(k) for k in body.params_map))
+        used = [int(k) for k in np.unique(body.params_map)]
         keys = []
         set_of_key = {}
         for k in used:
@@ -97,17 +97,14 @@ class MI355XBodyDataHandler:
         for fld, (sd, pd) in conds.items():
             sets = [body.point_sets[s] for s, _, _ in sd + pd]
             pts = np.unique(np.concatenate(sets)) if sets else np.zeros(0, np.int64)
-            slot = {int(p): k for k, p in enumerate(pts)}
             src = -np.ones((len(pts), 3), np.int32)
             for s, d, f in sd:
-                idx = [slot[int(p)] for p in body.point_sets[s]]
-                src[idx, d] = n_src
+                src[np.searchsorted(pts, body.point_sets[s]), d] = n_src
                 self._sd.append((n_src, f))
                 n_src += 1
             for s, d, f in pd:
                 ps = body.point_sets[s]
-                idx = [slot[int(p)] for p in ps]
-                src[idx, d] = n_src + np.arange(len(ps))
+                src[np.searchsorted(pts, ps), d] = n_src + np.arange(len(ps))
                 self._pd.append((n_src, ps, f))
                 n_src += len(ps)
             tables[fld] = (pts, src)
@@ -128,7 +125,7 @@ class MI355XBodyDataHandler:
             for s, f in self._sd:
                 vals[k, s] = float(f(t))
             for base, ps, f in self._pd:
-                vals[k, base:base + len(ps)] = eval_posdep(f, X[:, ps], t)
+                vals[k, base:base + len(ps)] = eval_posdep(f, X.take(ps, axis=1), t)
         return vals
 
     # ------------------------------------------------------------------ reference interface
@@ -230,7 +227,7 @@ class MI355XBodyDataHandler:
         if body.single_dim_bcs or body.posdep_single_dim_bcs:
             raise _arg_error("NewtonKrylov solver does not support all boundary condition types!\n"
                              "Specify only position-dependent boundary conditions!")
-        for k in sorted(set(int(k) for k in body.params_map)):
+        for k in (int(k) for k in np.unique(body.params_map)):
             if body.point_params[k - 1].has_fracture():
                 i = int(np.argmax(body.params_map == k))
                 raise _arg_error("NewtonKrylov solver currently does not support damage or "
