@@ -521,8 +521,7 @@ inline int pdx_lds_budget(const pdx_ctx *c)
     const int64_t b = c->lds_budget_env > 0 ? c->lds_budget_env : half;
     return (int)std::min<int64_t>(b, c->lds_limit);
 }
-// for kernels whose registers allow one 1024-thread block per CU anyway (the CPD passes):
-// the whole LDS of the CU
+// the whole LDS of the CU, for kernels whose registers allow one 1024-thread block per CU anyway
 inline int pdx_lds_budget_full(const pdx_ctx *c)
 {
     const int64_t b = c->lds_budget_env > 0 ? c->lds_budget_env : c->lds_limit;

@@ -1069,14 +1069,15 @@ static pdx_status build_halos(pdx_ctx *c, bool *ok)
 //   BB FP64   6 k 14.3 /  9.8 /  7.1 /  6.4    14 k 16.7 / 11.8 /  8.7 /  8.8
 //            25 k 17.2 / 12.4 / 12.5 / 13.4   100 k 31.5 / 30.6 / 30.5 / 35.0
 //             2 M  560 /  515 /  598 /  729
-//   CPD FP64  6 k 44.8 / 30.9 / 24.1 / 21.7    14 k 52.9 / 36.5 / 28.8 / 32.0
-//            25 k 55.4 / 37.8 / 46.5 / 53.5    54 k 63.6 / 65.4 / 84.8 / 91.4
-// so the blocks are the largest that still give 160 of them.  The correspondence kernels go up to
-// 256 points (one block of 1024 threads per CU by their registers; 128 points: 2658 against 2034
-// at 2 M), as do the mixed steps of bodies beyond a million points (334 against 356 at 2 M); the
-// others stop at 128, whose blocks share a CU three at a time.  Horizons beyond about 4 spacings stop
-// at 64 points, whose neighbour tables still fit a block's share of the LDS (5.015 spacings, 121 k
-// points, BB: 216 / 169 / 157 / 159; OSB at 400 k: 1042 / 1074 / 897 / 942).
+//   CPD FP64  6 k  n/a / 28.0 / 21.8 / 18.7    14 k  n/a / 38.4 / 29.7 / 27.6
+//            25 k  n/a / 40.2 / 39.4 / 46.3    54 k 61.8 / 59.0 / 67.8
+//           512 k  490 /  458 /  588            2 M 2218 / 1750
+// so the blocks are the largest that still give 160 of them.  FP64 stops at 128 points, whose
+// blocks share a CU two or three at a time; the mixed BB and OSB steps of bodies beyond a million
+// points go to 256 (334 against 356 at 2 M).  Horizons beyond about 4 spacings stop at 64 points,
+// whose neighbour tables still fit a block's share of the LDS (5.015 spacings, 121 k points, BB:
+// 216 / 169 / 157 / 159; OSB at 400 k: 1042 / 1074 / 897 / 942; CPD at 100 k: 629 / 517 / 403; 4.015
+// spacings, CPD at 100 k: 280 / 210 / 191).
 static void choose_blocks(pdx_ctx *c, bool lds)
 {
     if (!lds) {
@@ -1087,8 +1088,8 @@ static void choose_blocks(pdx_ctx *c, bool lds)
     }
     static const int pbs[4] = {256, 128, 64, 32}, lss[4] = {2, 2, 3, 4};
     int first = 1;
-    if (c->kind == PDX_CPD || (c->precision == PDX_MIXED && c->n > 1000000)) first = 0;
-    else if (c->nb > 180 * c->n) first = 2;
+    if (c->nb > 180 * c->n) first = 2;
+    else if (c->kind != PDX_CPD && c->precision == PDX_MIXED && c->n > 1000000) first = 0;
     int k = first;
     while (k < 3 && c->n < (int64_t)160 * pbs[k]) k++;
     c->cfg = k;

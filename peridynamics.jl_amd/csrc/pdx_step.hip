@@ -795,21 +795,21 @@ __global__ __launch_bounds__(PB * S) void k_bb_jv(pdx_step_args A, const double 
 // bond word is read: L comes from D.  The Velocity Verlet tail stays FP64.
 // ----------------------------------------------------------------------------------------
 
-// the lane's bond words, four row groups at a time, the next four in flight
-template <int S, class GROUP>
-__device__ __forceinline__ void pdx_walk4_mx(const pdx_step_args &A, const pdx_lane<S, false> &R, GROUP &&group)
+// the lane's bond words, U row groups at a time, the next U in flight
+template <int U, int S, class GROUP>
+__device__ __forceinline__ void pdx_walk_mx(const pdx_step_args &A, const pdx_lane<S, false> &R, GROUP &&group)
 {
     if (R.ng == 0) return;
-    uint32_t c[4];
+    uint32_t c[U];
 #pragma unroll
-    for (int u = 0; u < 4; u++) c[u] = A.bw16[R.at(u)];
-    for (int i = 0; i < R.ng; i += 4) {
-        uint32_t nx[4];
+    for (int u = 0; u < U; u++) c[u] = A.bw16[R.at(u)];
+    for (int i = 0; i < R.ng; i += U) {
+        uint32_t nx[U];
 #pragma unroll
-        for (int u = 0; u < 4; u++) nx[u] = A.bw16[R.at(i + 4 + u)];
+        for (int u = 0; u < U; u++) nx[u] = A.bw16[R.at(i + U + u)];
         group(c, i);
 #pragma unroll
-        for (int u = 0; u < 4; u++) c[u] = nx[u];
+        for (int u = 0; u < U; u++) c[u] = nx[u];
     }
 }
 
@@ -841,7 +841,7 @@ __global__ __launch_bounds__(PB * S) void k_bb_lds_mx(pdx_step_args A)
     constexpr bool MULTI = (F & PDX_FEAT_MULTI) != 0;
     constexpr bool SC = (F & PDX_FEAT_SC) != 0;
     constexpr bool CAP = (F & PDX_FEAT_CAP) != 0;
-    extern __shared__ float4 hmx[];  // [2 H]: (X - O, V), (u - u_O, 0)
+    extern __shared__ float4 hmx[];  // [HL] (X - O, V), [HL] (u - u_O, 0)
     const int64_t k = pdx_xcd_block();
     const int64_t p0 = k * PB;
     if (p0 >= A.n) return;  // whole workgroup
@@ -859,7 +859,7 @@ __global__ __launch_bounds__(PB * S) void k_bb_lds_mx(pdx_step_args A)
     for (int h = threadIdx.x; h < Hs; h += PB * S) {
         const int64_t j = hidx[h];
         if (MULTI) hpid[h] = A.pid[j];
-        mx_stage_xu(A, j, O, uo0, uo1, uo2, hmx[2 * h], hmx[2 * h + 1]);
+        mx_stage_xu(A, j, O, uo0, uo1, uo2, hmx[h], hmx[HL + h]);
     }
     const int sub = threadIdx.x % S;
     const int64_t p = p0 + threadIdx.x / S;
@@ -883,7 +883,7 @@ __global__ __launch_bounds__(PB * S) void k_bb_lds_mx(pdx_step_args A)
     }
     const float win_lo = epscf * 0.9999f, win_hi = epscf * 1.0001f;
     __syncthreads();
-    pdx_walk4_mx(A, R, [&](const uint32_t (&wd)[4], int i) {
+    pdx_walk_mx<4>(A, R, [&](const uint32_t (&wd)[4], int i) {
         // the group's bond forces are summed in FP32 (fused), then once into the FP64 sums
         float gx = 0.f, gy = 0.f, gz = 0.f;
 #pragma unroll
@@ -894,8 +894,8 @@ __global__ __launch_bounds__(PB * S) void k_bb_lds_mx(pdx_step_args A)
             float4 a, b;
             int32_t jg = 0;
             if (!CAP || slot < HL) {
-                a = hmx[2 * slot];
-                b = hmx[2 * slot + 1];
+                a = hmx[slot];
+                b = hmx[HL + slot];
             } else {  // past the staged entries: the same values from global memory
                 jg = hidx[slot];
                 mx_stage_xu(A, jg, O, uo0, uo1, uo2, a, b);
@@ -971,7 +971,7 @@ __global__ __launch_bounds__(PB * S) void k_osb_lds1_mx(pdx_step_args A)
     const int Hs = H < HL ? H : HL;
     const int32_t *const hidx = A.halo + h0;
     for (int h = threadIdx.x; h < Hs; h += PB * S)
-        mx_stage_xu(A, hidx[h], O, uo0, uo1, uo2, hmx[2 * h], hmx[2 * h + 1]);
+        mx_stage_xu(A, hidx[h], O, uo0, uo1, uo2, hmx[h], hmx[HL + h]);
     const int sub = threadIdx.x % S;
     const int64_t p = p0 + threadIdx.x / S;
     const int64_t q = p < A.n ? p : A.n - 1;
@@ -987,7 +987,7 @@ __global__ __launch_bounds__(PB * S) void k_osb_lds1_mx(pdx_step_args A)
     const float epscf = (float)epsc, deltaf = (float)A.delta;
     const float win_lo = epscf * 0.9999f, win_hi = epscf * 1.0001f;
     __syncthreads();
-    pdx_walk4_mx(A, R, [&](const uint32_t (&wd)[4], int i) {
+    pdx_walk_mx<4>(A, R, [&](const uint32_t (&wd)[4], int i) {
         // the group's sums in FP32 (fused), then once into the FP64 sums
         float gv = 0.f, gs = 0.f;
 #pragma unroll
@@ -997,8 +997,8 @@ __global__ __launch_bounds__(PB * S) void k_osb_lds1_mx(pdx_step_args A)
             const int slot = (int)(wd[u] & PDX_W16_SLOT);
             float4 a, b;
             if (!CAP || slot < HL) {
-                a = hmx[2 * slot];
-                b = hmx[2 * slot + 1];
+                a = hmx[slot];
+                b = hmx[HL + slot];
             } else {  // past the staged entries: the same values from global memory
                 mx_stage_xu(A, hidx[slot], O, uo0, uo1, uo2, a, b);
             }
@@ -1074,8 +1074,8 @@ __global__ __launch_bounds__(PB * S) void k_osb_lds2_mx(pdx_step_args A)
         const double2 cj = cst[j];
         const double Vj = A.Xr[j].w;
         b.w = (float)(cj.x * Vj);
-        hmx[2 * h] = a;
-        hmx[2 * h + 1] = b;
+        hmx[h] = a;
+        hmx[HL + h] = b;
         hc2[h] = (float)(cj.y * Vj);
     }
     const int sub = threadIdx.x % S;
@@ -1092,7 +1092,7 @@ __global__ __launch_bounds__(PB * S) void k_osb_lds2_mx(pdx_step_args A)
     const float c1i = (float)ci.x, c2i = (float)ci.y;
     const float deltaf = (float)A.delta;
     __syncthreads();
-    pdx_walk4_mx(A, R, [&](const uint32_t (&wd)[4], int i) {
+    pdx_walk_mx<4>(A, R, [&](const uint32_t (&wd)[4], int i) {
         // the group's bond forces are summed in FP32 (fused), then once into the FP64 sums
         float gx = 0.f, gy = 0.f, gz = 0.f;
 #pragma unroll
@@ -1103,8 +1103,8 @@ __global__ __launch_bounds__(PB * S) void k_osb_lds2_mx(pdx_step_args A)
             float4 a, b;
             float c2Vj;
             if (!CAP || slot < HL) {
-                a = hmx[2 * slot];
-                b = hmx[2 * slot + 1];
+                a = hmx[slot];
+                b = hmx[HL + slot];
                 c2Vj = hc2[slot];
             } else {
                 const int64_t j = hidx[slot];
@@ -1828,21 +1828,83 @@ __global__ __launch_bounds__(PDX_BLOCK * S) void k_cpd_pass2(pdx_step_args A)
     point_tail4(A, p, ri, b3, sub, A.rho);
 }
 
-// bonds per group of CPD pass 2's bond walk (pdx_walk_tile): the loads of the next group are
-// in flight while a group is evaluated.  Measured at 512 k points, pass 2 with ZEMSilling:
-// 0.330 / 0.306 / 0.319 / 0.328 / 0.365 ms for groups of 1 / 2 / 3 / 4 / 8 (ZEMWan within
-// 1 % for 2 to 4).  Pass 1, whose bond arithmetic is longer, runs fastest with groups of 1.
-#ifndef PDX_CPD_GROUP
-#define PDX_CPD_GROUP 2
-#endif
+// The bond walk of the FP64 CPD passes.  STAGE(T0, T1) brings entries [T0, T1) of the block's table
+// into LDS, with the barrier behind it, BOND(T0, b, i) evaluates a bond of the staged tile.  A table
+// that fits is walked U bonds at a time by wave-uniform counts (pass 1 at 512 k points: 240 us by
+// tiles, 229 / 196 / 194 / 204 for U = 1 / 2 / 3 / 4); a longer one in tiles of the table: a point's
+// bonds are sorted by neighbour, as the table is, so each lane walks as far as its neighbours lie
+// in the tile and resumes there in the next (pass 2: 265 / 253 / 260 / 263 for U = 2 / 3 / 4 / 6, 359
+// for 8).
+template <int U, int S, bool PK, class STAGE, class BOND>
+__device__ __forceinline__ void cpd_walk(const pdx_step_args &A, const pdx_lane<S, PK> &R, int H, int TL, STAGE &&stage,
+                                         BOND &&bond)
+{
+    if (H <= TL) {  // uniform over the block
+        stage(0, H);
+        pdx_walk<U>(A, R, [&](const bond_data<PK> (&b)[U], int i) {
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (U == 1 || i + u < R.ng) bond(0, b[u], i + u);
+        });
+        return;
+    }
+    int ig = 0;
+    for (int T0 = 0; T0 < H; T0 += TL) {
+        const int T1 = H < T0 + TL ? H : T0 + TL;
+        if (T0 > 0) __syncthreads();  // the previous tile is consumed
+        stage(T0, T1);
+        ig = pdx_walk_tile<U>(A, R, ig, T1, [&](const bond_data<PK> &b, int i) { bond(T0, b, i); });
+    }
+}
+
+// The sums of a point's S lanes, a share in each of them: lane s gets the sums of v[s], v[S + s], ... in
+// v[0], v[1], ...  Every sum has the pairwise order of pdx_fold, at a quarter of its shuffles.
+template <int O, int S, int N>
+__device__ __forceinline__ void pdx_fold_part(double *v)
+{
+    if constexpr (O < S) {
+        constexpr int M = (N + 1) / 2;
+        const bool up = (threadIdx.x & O) != 0;
+#pragma unroll
+        for (int m = 0; m < M; m++) {
+            const double a = v[2 * m], b = 2 * m + 1 < N ? v[2 * m + 1] : 0.0;
+            v[m] = (up ? b : a) + __shfl_xor(up ? a : b, O);
+        }
+        pdx_fold_part<2 * O, S, M>(v);
+    }
+}
+
+// The N sums of every point of the block, in hs[q PB + point], for one thread per point.  The
+// staged table is consumed by then, and its LDS is reused.  The point part of a correspondence
+// step (two 3 x 3 inverses, the stress, some 700 FP64 instructions) then runs in full waves
+// instead of one lane in S of all of them (512 k points, with the squared pre-check of the failure
+// window in place of a root per bond: pass 1 275 -> 245 us; without the point part it takes 208).
+template <int S, int PB, int N, bool PK>
+__device__ __forceinline__ void cpd_hand_over(const pdx_lane<S, PK> &R, double *v, double *hs)
+{
+    const int sub = threadIdx.x % S, pt = threadIdx.x / S;
+    if (S > 4 && R.order && sub >= 4) {
+#pragma unroll
+        for (int q = 0; q < N; q++) v[q] = 0.0;
+    }
+    pdx_fold_part<1, S, N>(v);
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < (N + S - 1) / S; m++)
+        if (S * m + sub < N) hs[(S * m + sub) * PB + pt] = v[m];
+    __syncthreads();
+}
 
 // ----------------------------------------------------------------------------------------
-// CPD passes on the LDS-staged layout (FP64), for neighbour tables longer than one LDS
-// budget: the block's table is staged in tiles of TL entries.  A point's bonds are sorted
-// by neighbour index, as is the table, so each lane's bonds fall into the tiles in order:
-// the lane walks its bonds while their slots lie in the staged tile and resumes there after
-// the next tile is staged.  Pass 1 entries: x|V, X (64 B); pass 2: x|V, X|beta [j alive],
-// [j alive] Q_j (136 B).  The arithmetic is that of k_cpd_pass1/2.
+// CPD passes on the LDS-staged layout (FP64).  Pass 1 entries: x, V, X (56 B); pass 2: see below.
+// The arithmetic of pass 1 is that of k_cpd_pass1.
+//
+// Bound by the bond walk's instructions and LDS reads: at 512 k points (60 M bonds) the vector units
+// are busy 56 % of pass 1's time and 36 % of pass 2's, the LDS 40 and 47 %, and a pass without its
+// walk takes 62 (46) of 245 (258) us.  What helped, us of both passes at 512 k points: blocks of 128
+// points, two to a CU, 500 -> 458 (256 points leave one block per CU, whose staging and point part
+// nothing hides); walking a table that fits by wave-uniform counts instead of by tiles 545 -> 501 in
+// the same blocks.  A point's own lanes S at 8 (64-point blocks) cost 588: longer tables per point.
 // ----------------------------------------------------------------------------------------
 template <int S, int F, int PB, bool PK>
 __global__ __launch_bounds__(PB * S) void k_cpd_lds1(pdx_step_args A)
@@ -1853,118 +1915,124 @@ __global__ __launch_bounds__(PB * S) void k_cpd_lds1(pdx_step_args A)
     // of the point
     constexpr bool MULTI = (F & PDX_FEAT_MULTI) != 0;
     extern __shared__ double4 hrec[];
-    const int TL = pdx_lds_entries(A.halo_max, A.lds_budget, 64 + (MULTI ? 1 : 0));
-    double4 *const hx = hrec;
-    double4 *const hX = hrec + TL;
-    uint8_t *const hpid = reinterpret_cast<uint8_t *>(hrec + 2 * TL);
+    const int TL = pdx_lds_entries(A.halo_max, A.lds_budget, 56 + (MULTI ? 1 : 0));
+    // pairs x, y | z, V | X, Y and then Z, each an array of its own
+    double2 *const hx = reinterpret_cast<double2 *>(hrec);
+    double *const hZ = reinterpret_cast<double *>(hx + 3 * TL);
+    uint8_t *const hpid = reinterpret_cast<uint8_t *>(hZ + TL);
     const int64_t k = pdx_xcd_block();
     const int64_t p0 = k * PB;
     if (p0 >= A.n) return;  // whole workgroup
     const int64_t h0 = A.halo_ptr[k];
     const int H = (int)(A.halo_ptr[k + 1] - h0);
     const int32_t *const hidx = A.halo + h0;
-    const int sub = threadIdx.x % S;
-    const int64_t p = p0 + threadIdx.x / S;
-    const int64_t pq = p < A.n ? p : A.n - 1;  // the block's threads all take part in the tile barriers
+    const int64_t pq = p0 + threadIdx.x / S < A.n ? p0 + threadIdx.x / S : A.n - 1;  // all threads meet the barriers
     const pdx_lane<S, PK> R = pdx_lane_of<S, PK>(A, p0);
     const double4 ri = A.rec_in[pq];
     const double4 Xi = A.Xr[pq];
     const bool dead = A.killed[pq] != 0;
     double epsc = A.epsc, thr;
+    if (MULTI) {
+        epsc = A.psets[A.pid[pq]].epsc;
+        thr = A.epsc_lo_min;  // of all sets: either copy of a bond may fail from there on
+    } else {
+        thr = fail_window<PK>(A, pq, A.epsc_lo);
+    }
+    // from this squared elongation on a bond may lie in the failure window
+    const double thr2 = thr >= 0.0 ? (1.0 + thr) * (1.0 + thr) * (1.0 - 1e-12) : 0.0;
+    constexpr bool ZWF = (F & PDX_FEAT_ZW) != 0;
+    // K (00 10 20 11 21 22), Ft, and the sums of w V_j DX and w V_j dx over the owner's copies of
+    // the bonds for the own bond terms of pass 2; then the active bonds
+    double sum[22] = {};
+    double *const Km = sum, *const Ft = sum + 6, *const S1 = sum + 15, *const S2 = sum + 18;
+    int na = 0;
+    const auto stage = [&](int T0, int T1) {
+        for (int h = T0 + (int)threadIdx.x; h < T1; h += PB * S) {
+            const int32_t j = hidx[h];
+            const double4 x = A.rec_in[j], X = A.Xr[j];
+            hx[h - T0] = make_double2(x.x, x.y);
+            hx[TL + h - T0] = make_double2(x.z, x.w);
+            hx[2 * TL + h - T0] = make_double2(X.x, X.y);
+            hZ[h - T0] = X.z;
+            if (MULTI) hpid[h - T0] = A.pid[j];
+        }
+        __syncthreads();
+    };
+    const auto bond = [&](int T0, const bond_data<PK> &bd, int ib) {
+                    const int slot = bond_slot(A, bd);
+                    const double2 *const hj = hx + (slot - T0);
+                    const double2 xy = hj[0], zV = hj[TL], XY = hj[2 * TL];
+                    const double dx[3] = {xy.x - ri.x, xy.y - ri.y, zV.x - ri.z};
+                    const double DX[3] = {XY.x - Xi.x, XY.y - Xi.y, hZ[slot - T0] - Xi.z};
+                    const double Lb = bond_len(A, bd);
+                    const double d2 = (dx[0] * dx[0] + dx[1] * dx[1]) + dx[2] * dx[2];
+                    bool act = bond_act(A, bd);
+                    // (the length is needed only here)
+                    const bool look = d2 >= thr2 * (Lb * Lb);
+                    double e = 0.0;
+                    if (look) {
+                        double rl;
+                        e = pdx_sqrt_rsq(d2, rl) - Lb;
+                    }
+                    if constexpr (MULTI) {
+                        // each end fails its copy of the bond against its own eps_c; the stretch is the
+                        // same number at both ends
+                        if (look && (bd.w & PDX_W16_FP) && (bd.w & (PDX_W16_ACT | PDX_W16_RACT)) && e >= thr * Lb) {
+                            const double eps = e / Lb;
+                            uint32_t nw = bd.w;
+                            if (eps > epsc) nw &= ~(uint32_t)PDX_W16_ACT;
+                            if (eps > A.psets[hpid[slot - T0]].epsc) nw &= ~(uint32_t)PDX_W16_RACT;
+                            if (nw != bd.w) A.bw16[R.at(ib)] = (uint16_t)nw;
+                            act = (nw & PDX_W16_ACT) != 0;
+                        }
+                    } else {
+                        if (look && act && e >= thr * Lb && bond_breaks<PK>(A, hidx, bd, e, Lb, epsc)) {
+                            act = false;
+                            R.kill(A, ib, bd);
+                        }
+                    }
+                    if (act && !dead) {
+                        na++;
+                        // K += w V_j DX DX', Ft += w V_j dx DX' as fused products of (w V_j DX)
+                        const double temp = pdx_omega(A.kernel, A.delta, Lb, pdx_rcp1(Lb)) * zV.y;
+                        const double tD[3] = {temp * DX[0], temp * DX[1], temp * DX[2]};
+                        Km[0] = fma(tD[0], DX[0], Km[0]);
+                        Km[1] = fma(tD[1], DX[0], Km[1]);
+                        Km[2] = fma(tD[2], DX[0], Km[2]);
+                        Km[3] = fma(tD[1], DX[1], Km[3]);
+                        Km[4] = fma(tD[2], DX[1], Km[4]);
+                        Km[5] = fma(tD[2], DX[2], Km[5]);
+        #pragma unroll
+                        for (int cc = 0; cc < 3; cc++)
+        #pragma unroll
+                            for (int r = 0; r < 3; r++) Ft[r + 3 * cc] = fma(tD[cc], dx[r], Ft[r + 3 * cc]);
+        #pragma unroll
+                        for (int r = 0; r < 3; r++) {
+                            S1[r] += tD[r];
+                            S2[r] = fma(temp, dx[r], S2[r]);
+                        }
+                    }
+    };
+    cpd_walk<2>(A, R, H, TL, stage, bond);
+    sum[21] = na;
+    double *const hs = reinterpret_cast<double *>(hrec);
+    cpd_hand_over<S, PB, 22>(R, sum, hs);
+    const int64_t p = p0 + threadIdx.x;
+    if (threadIdx.x >= PB || p >= A.n) return;
+#pragma unroll
+    for (int q = 0; q < 22; q++) sum[q] = hs[q * PB + threadIdx.x];
     double lam = A.lambda, mu = A.mu, Gp = A.G, Kp = A.K, nup = A.nu, beta = A.beta_zem;
     if (MULTI) {
-        const pdx_pset Pi = A.psets[A.pid[pq]];
-        epsc = Pi.epsc;
-        thr = A.epsc_lo_min;  // of all sets: either copy of a bond may fail from there on
+        const pdx_pset Pi = A.psets[A.pid[p]];
         lam = Pi.lam;
         mu = Pi.mu;
         Gp = Pi.G;
         Kp = Pi.K;
         nup = Pi.nu;
         beta = Pi.beta;
-    } else {
-        thr = fail_window<PK>(A, pq, A.epsc_lo);
     }
-    double Km[6] = {0, 0, 0, 0, 0, 0};  // 00 10 20 11 21 22
-    double Ft[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    // the sums of w V_j DX and w V_j dx over the owner's copies of the bonds, for the own
-    // bond terms of pass 2
-    constexpr bool ZWF = (F & PDX_FEAT_ZW) != 0;
-    double S1[3] = {0, 0, 0}, S2[3] = {0, 0, 0};
-    int na = 0;
-    int ig = 0;
-    for (int T0 = 0; T0 < H; T0 += TL) {
-        const int T1 = H < T0 + TL ? H : T0 + TL;
-        if (T0 > 0) __syncthreads();  // the previous tile is consumed
-        for (int h = T0 + (int)threadIdx.x; h < T1; h += PB * S) {
-            const int32_t j = hidx[h];
-            hx[h - T0] = A.rec_in[j];
-            hX[h - T0] = A.Xr[j];
-            if (MULTI) hpid[h - T0] = A.pid[j];
-        }
-        __syncthreads();
-        ig = pdx_walk_tile<1>(A, R, ig, T1, [&](const bond_data<PK> &bd, int ib) {
-            const int slot = bond_slot(A, bd);
-            const double4 rj = hx[slot - T0];
-            const double4 Xj = hX[slot - T0];
-            const double dx[3] = {rj.x - ri.x, rj.y - ri.y, rj.z - ri.z};
-            const double DX[3] = {Xj.x - Xi.x, Xj.y - Xi.y, Xj.z - Xi.z};
-            const double Lb = bond_len(A, bd);
-            double rl;
-            const double e = pdx_sqrt_rsq((dx[0] * dx[0] + dx[1] * dx[1]) + dx[2] * dx[2], rl) - Lb;
-            bool act = bond_act(A, bd);
-            if constexpr (MULTI) {
-                // each end fails its copy of the bond against its own eps_c; the stretch is the
-                // same number at both ends
-                if ((bd.w & PDX_W16_FP) && (bd.w & (PDX_W16_ACT | PDX_W16_RACT)) && e >= thr * Lb) {
-                    const double eps = e / Lb;
-                    uint32_t nw = bd.w;
-                    if (eps > epsc) nw &= ~(uint32_t)PDX_W16_ACT;
-                    if (eps > A.psets[hpid[slot - T0]].epsc) nw &= ~(uint32_t)PDX_W16_RACT;
-                    if (nw != bd.w) A.bw16[R.at(ib)] = (uint16_t)nw;
-                    act = (nw & PDX_W16_ACT) != 0;
-                }
-            } else {
-                if (act && e >= thr * Lb && bond_breaks<PK>(A, hidx, bd, e, Lb, epsc)) {
-                    act = false;
-                    R.kill(A, ib, bd);
-                }
-            }
-            if (act && !dead) {
-                na++;
-                // K += w V_j DX DX', Ft += w V_j dx DX' as fused products of (w V_j DX)
-                const double temp = pdx_omega(A.kernel, A.delta, Lb, pdx_rcp1(Lb)) * rj.w;
-                const double tD[3] = {temp * DX[0], temp * DX[1], temp * DX[2]};
-                Km[0] = fma(tD[0], DX[0], Km[0]);
-                Km[1] = fma(tD[1], DX[0], Km[1]);
-                Km[2] = fma(tD[2], DX[0], Km[2]);
-                Km[3] = fma(tD[1], DX[1], Km[3]);
-                Km[4] = fma(tD[2], DX[1], Km[4]);
-                Km[5] = fma(tD[2], DX[2], Km[5]);
-#pragma unroll
-                for (int cc = 0; cc < 3; cc++)
-#pragma unroll
-                    for (int r = 0; r < 3; r++) Ft[r + 3 * cc] = fma(tD[cc], dx[r], Ft[r + 3 * cc]);
-#pragma unroll
-                for (int r = 0; r < 3; r++) {
-                    S1[r] += tD[r];
-                    S2[r] = fma(temp, dx[r], S2[r]);
-                }
-            }
-        });
-    }
-#pragma unroll
-    for (int q = 0; q < 6; q++) pdx_fold(R, Km[q]);
-#pragma unroll
-    for (int q = 0; q < 9; q++) pdx_fold(R, Ft[q]);
-#pragma unroll
-    for (int r = 0; r < 3; r++) {
-        pdx_fold(R, S1[r]);
-        pdx_fold(R, S2[r]);
-    }
-    pdx_fold(R, na);
-    if (p >= A.n || sub != 0) return;
-    const bool kill = cpd_point_state<ZWF>(A, p, Km, Ft, na, A.cnt[p], dead, lam, mu, Gp, Kp, nup, beta);
+    const bool kill =
+        cpd_point_state<ZWF>(A, p, Km, Ft, (int)sum[21], A.cnt[p], A.killed[p] != 0, lam, mu, Gp, Kp, nup, beta);
     {
         // the own term of the point's bonds, Q_i S1 + beta S2, and a_i = Q_i X_i + beta x_i
         // (ZEMWan: C_1i in place of beta; zero for a dead point, whose state is zero), behind
@@ -2017,6 +2085,10 @@ __global__ __launch_bounds__(PB * S) void k_cpd_lds2_own(pdx_step_args A)
     extern __shared__ double4 hrec[];
     double2 *const hq = reinterpret_cast<double2 *>(hrec);
     const int TL = pdx_lds_entries(A.halo_max, A.lds_budget, 16 * ND);
+    // Strides of entries and of pairs.  112-byte entries lie one after the other (their first words
+    // fall on all 16 groups of four banks); 160-byte ones would meet on 8, so their pairs are
+    // arrays of their own (54 k points 55.1 -> 51.1 us, 512 k 418.6 -> 396).
+    const int EH = ZW ? 1 : ND, EM = ZW ? TL : 1;
     const int64_t k = pdx_xcd_block();
     const int64_t p0 = k * PB;
     if (p0 >= A.n) return;  // whole workgroup
@@ -2037,10 +2109,7 @@ __global__ __launch_bounds__(PB * S) void k_cpd_lds2_own(pdx_step_args A)
     const double *const ext = A.pstate + NQ * A.n;
     const double rho = MULTI && valid ? A.psets[A.pid[p]].rho : A.rho;
     double b3[3] = {0.0, 0.0, 0.0};
-    int ig = 0;
-    for (int T0 = 0; T0 < H; T0 += TL) {
-        const int T1 = H < T0 + TL ? H : T0 + TL;
-        if (T0 > 0) __syncthreads();  // the previous tile is consumed
+    const auto stage = [&](int T0, int T1) {
         for (int h = T0 + (int)threadIdx.x; h < T1; h += PB * S) {
             const int64_t j = hidx[h];
             const bool live = !A.killed[j];
@@ -2066,36 +2135,37 @@ __global__ __launch_bounds__(PB * S) void k_cpd_lds2_own(pdx_step_args A)
                     o = fma(e[12], O3x[r], o);
                 e[9 + r] = live ? aj[r] - o : 0.0;
             }
-            double2 *const d = hq + ND * (int64_t)(h - T0);
+            double2 *const d = hq + (h - T0) * EH;
 #pragma unroll
-            for (int m = 0; m < ND; m++) d[m] = make_double2(e[2 * m], e[2 * m + 1]);
+            for (int m = 0; m < ND; m++) d[m * EM] = make_double2(e[2 * m], e[2 * m + 1]);
         }
         __syncthreads();
-        ig = pdx_walk_tile<PDX_CPD_GROUP>(A, R, ig, T1, [&](const bond_data<PK> &bd, int) {
-            bool on = bond_act(A, bd);
-            if constexpr (MULTI) on = (bd.w & PDX_W16_RACT) != 0;  // the neighbour's copy
-            if (!on) return;
-            const double Lb = bond_len(A, bd);
-            const double2 *const d = hq + ND * (int64_t)(bond_slot(A, bd) - T0);
-            double e[2 * ND];
-#pragma unroll
-            for (int m = 0; m < ND; m++) {
-                const double2 v = d[m];
-                e[2 * m] = v.x;
-                e[2 * m + 1] = v.y;
-            }
-            const double wv = pdx_omega(A.kernel, A.delta, Lb, pdx_rcp1(Lb)) * e[IV];  // w V_j
-#pragma unroll
-            for (int r = 0; r < 3; r++) {
-                double o = fma(e[r + 6], Xr[2], fma(e[r + 3], Xr[1], e[r] * Xr[0]));
-                if (ZW)
-                    o = fma(e[12 + SY[r + 6]], xr[2], fma(e[12 + SY[r + 3]], xr[1], fma(e[12 + SY[r]], xr[0], o)));
-                else
-                    o = fma(e[12], xr[r], o);
-                b3[r] = fma(wv, e[9 + r] - o, b3[r]);
-            }
-        });
-    }
+    };
+    const auto bond = [&](int T0, const bond_data<PK> &bd, int) {
+                    bool on = bond_act(A, bd);
+                    if constexpr (MULTI) on = (bd.w & PDX_W16_RACT) != 0;  // the neighbour's copy
+                    if (!on) return;
+                    const double Lb = bond_len(A, bd);
+                    const double2 *const d = hq + (bond_slot(A, bd) - T0) * EH;
+                    double e[2 * ND];
+        #pragma unroll
+                    for (int m = 0; m < ND; m++) {
+                        const double2 v = d[m * EM];
+                        e[2 * m] = v.x;
+                        e[2 * m + 1] = v.y;
+                    }
+                    const double wv = pdx_omega(A.kernel, A.delta, Lb, pdx_rcp1(Lb)) * e[IV];  // w V_j
+        #pragma unroll
+                    for (int r = 0; r < 3; r++) {
+                        double o = fma(e[r + 6], Xr[2], fma(e[r + 3], Xr[1], e[r] * Xr[0]));
+                        if (ZW)
+                            o = fma(e[12 + SY[r + 6]], xr[2], fma(e[12 + SY[r + 3]], xr[1], fma(e[12 + SY[r]], xr[0], o)));
+                        else
+                            o = fma(e[12], xr[r], o);
+                        b3[r] = fma(wv, e[9 + r] - o, b3[r]);
+                    }
+    };
+    cpd_walk<3>(A, R, H, TL, stage, bond);
 #pragma unroll
     for (int r = 0; r < 3; r++) pdx_fold(R, b3[r]);
     if (!valid || sub >= 4) return;  // the tail takes four lanes per point
@@ -2114,6 +2184,12 @@ __global__ __launch_bounds__(PB * S) void k_cpd_lds2_own(pdx_step_args A)
 // without the cancellation of d - F D in FP32.  Pass 1 stores Q' (9 numbers per point);
 // pass 2 stages (D, V), (U, beta [j alive]), [j alive] Q'_j (68 B per table entry) and
 // gathers both terms of every bond.
+// Pass 1 is bound by its vector instructions (busy 82 % of the time: 15 FP32 products per bond are
+// converted and summed in FP64), so one bond at a time without a stretch that only a bond near its
+// critical one needs; pass 2 by LDS reads, whose 64-byte entries met on two groups of banks
+// (75 % of the LDS cycles were conflicts) until every quarter became an array of its own.
+// Both passes at 512 k points: 468 us with four bonds per step and entries in one piece, 355 now,
+// 308 in blocks of 128 points.
 // ----------------------------------------------------------------------------------------
 template <int S, int F, int PB>
 __global__ __launch_bounds__(PB * S) void k_cpd_pass1_mx(pdx_step_args A)
@@ -2134,35 +2210,35 @@ __global__ __launch_bounds__(PB * S) void k_cpd_pass1_mx(pdx_step_args A)
     for (int h = threadIdx.x; h < Hs; h += PB * S) {
         float4 a, b;
         mx_stage_xu(A, hidx[h], O, uo0, uo1, uo2, a, b);
-        hmx[2 * h] = a;
-        hmx[2 * h + 1] = b;
+        hmx[h] = a;
+        hmx[HL + h] = b;
     }
     __syncthreads();
-    const int sub = threadIdx.x % S;
-    const int64_t p = p0 + threadIdx.x / S;
-    const int64_t pq = p < A.n ? p : A.n - 1;
+    const int64_t pq = p0 + threadIdx.x / S < A.n ? p0 + threadIdx.x / S : A.n - 1;
     const pdx_lane<S, false> R = pdx_lane_of<S, false>(A, p0);
     const double4 ri = A.rec_in[pq];
     const double4 Xi = A.Xr[pq];
     const float xi = (float)(Xi.x - O.x), yi = (float)(Xi.y - O.y), zi = (float)(Xi.z - O.z);
     const float ui = (float)((ri.x - Xi.x) - uo0), vi = (float)((ri.y - Xi.y) - uo1),
                 wi = (float)((ri.z - Xi.z) - uo2);
-    const bool dead = A.killed[pq] != 0;
-    double Km[6] = {0, 0, 0, 0, 0, 0};  // 00 10 20 11 21 22
-    double Ht[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    const bool dead_i = A.killed[pq] != 0;
+    double sum[16] = {};  // K (00 10 20 11 21 22), Ht; then the active bonds
+    double *const Km = sum, *const Ht = sum + 6;
     int na = 0;
     const double epsc = A.epsc;
     const float epscf = (float)epsc, deltaf = (float)A.delta;
     const float win_lo = epscf * 0.9999f, win_hi = epscf * 1.0001f;
-    pdx_walk4_mx(A, R, [&](const uint32_t (&wd)[4], int i) {
+    // l^2 / L^2 - 1 from which on the stretch may exceed win_lo
+    const float num_lo = win_lo >= 0.f ? 0.999f * win_lo * (2.f + win_lo) : -INFINITY;
+    pdx_walk_mx<1>(A, R, [&](const uint32_t (&wd)[1], int i) {
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
+        for (int u = 0; u < 1; u++) {
             if (i + u >= R.ng) continue;  // uniform
             const int slot = (int)(wd[u] & PDX_W16_SLOT);
             float4 a, b;
             if (!CAP || slot < HL) {
-                a = hmx[2 * slot];
-                b = hmx[2 * slot + 1];
+                a = hmx[slot];
+                b = hmx[HL + slot];
             } else {
                 mx_stage_xu(A, hidx[slot], O, uo0, uo1, uo2, a, b);
             }
@@ -2173,16 +2249,18 @@ __global__ __launch_bounds__(PB * S) void k_cpd_pass1_mx(pdx_step_args A)
             const float UU = __builtin_fmaf(Uv[2], Uv[2], __builtin_fmaf(Uv[1], Uv[1], Uv[0] * Uv[0]));
             const float num = __builtin_fmaf(2.f, DU, UU);  // l^2 - L^2
             const float Lb = __builtin_amdgcn_sqrtf(L2);
-            const float l = __builtin_amdgcn_sqrtf(L2 + num);
             const float rL = __builtin_amdgcn_rcpf(Lb);
-            const float eps = (num * __builtin_amdgcn_rcpf(l + Lb)) * rL;
             bool act = (wd[u] & PDX_W16_ACT) != 0;
-            const int64_t o = R.at(i + u);
-            if (act && (wd[u] & PDX_W16_FP) && eps > win_lo && mx_breaks(A, hidx, wd[u], o, ri, eps, win_hi, epsc)) {
-                act = false;
-                A.bw16[o] = (uint16_t)(wd[u] & ~PDX_W16_ACT);
+            if (act && (wd[u] & PDX_W16_FP) && num >= num_lo * L2) {
+                const int64_t o = R.at(i + u);
+                const float l = __builtin_amdgcn_sqrtf(L2 + num);
+                const float eps = (num * __builtin_amdgcn_rcpf(l + Lb)) * rL;
+                if (eps > win_lo && mx_breaks(A, hidx, wd[u], o, ri, eps, win_hi, epsc)) {
+                    act = false;
+                    A.bw16[o] = (uint16_t)(wd[u] & ~PDX_W16_ACT);
+                }
             }
-            if (act && !dead) {
+            if (act && !dead_i) {
                 na++;
                 const float wv = (deltaf * rL) * a.w;  // w V_j
                 const float wD[3] = {wv * D[0], wv * D[1], wv * D[2]};  // the products of w V_j D
@@ -2199,12 +2277,15 @@ __global__ __launch_bounds__(PB * S) void k_cpd_pass1_mx(pdx_step_args A)
             }
         }
     });
+    sum[15] = na;
+    double *const hs = reinterpret_cast<double *>(hmx);
+    cpd_hand_over<S, PB, 16>(R, sum, hs);
+    const int64_t p = p0 + threadIdx.x;
+    if (threadIdx.x >= PB || p >= A.n) return;
 #pragma unroll
-    for (int q = 0; q < 6; q++) pdx_fold(R, Km[q]);
-#pragma unroll
-    for (int q = 0; q < 9; q++) pdx_fold(R, Ht[q]);
-    pdx_fold(R, na);
-    if (p >= A.n || sub != 0) return;
+    for (int q = 0; q < 16; q++) sum[q] = hs[q * PB + threadIdx.x];
+    na = (int)sum[15];
+    const bool dead = A.killed[p] != 0;
     const int c = A.cnt[p];
     const double K9[9] = {Km[0], Km[1], Km[2], Km[1], Km[3], Km[4], Km[2], Km[4], Km[5]};
     double Kinv[9], Hm[9], Fm[9];
@@ -2261,7 +2342,7 @@ template <int S, int F, int PB>
 __global__ __launch_bounds__(PB * S) void k_cpd_pass2_mx(pdx_step_args A)
 {
     constexpr bool CAP = (F & PDX_FEAT_CAP) != 0;
-    extern __shared__ float4 hmx[];  // [4 HL]: (D, V), (U, beta l), q0-3, q4-7; then q8 [HL]
+    extern __shared__ float4 hmx[];  // [HL] each: (D, V), (U, beta l), q0-3, q4-7; then q8 [HL]
     const int64_t k = pdx_xcd_block();
     const int64_t p0 = k * PB;
     if (p0 >= A.n) return;  // whole workgroup
@@ -2278,10 +2359,10 @@ __global__ __launch_bounds__(PB * S) void k_cpd_pass2_mx(pdx_step_args A)
         float4 a, b;
         float q[9];
         cpd_mx_entry(A, hidx[h], O, uo0, uo1, uo2, a, b, q);
-        hmx[4 * h] = a;
-        hmx[4 * h + 1] = b;
-        hmx[4 * h + 2] = make_float4(q[0], q[1], q[2], q[3]);
-        hmx[4 * h + 3] = make_float4(q[4], q[5], q[6], q[7]);
+        hmx[h] = a;
+        hmx[HL + h] = b;
+        hmx[2 * HL + h] = make_float4(q[0], q[1], q[2], q[3]);
+        hmx[3 * HL + h] = make_float4(q[4], q[5], q[6], q[7]);
         hq8[h] = q[8];
     }
     __syncthreads();
@@ -2301,18 +2382,18 @@ __global__ __launch_bounds__(PB * S) void k_cpd_pass2_mx(pdx_step_args A)
     for (int r = 0; r < 9; r++) Qi[r] = live_i ? (float)A.pstate[9 * pq + r] : 0.f;
     const float deltaf = (float)A.delta;
     double b3[3] = {0.0, 0.0, 0.0};
-    pdx_walk4_mx(A, R, [&](const uint32_t (&wd)[4], int i) {
+    pdx_walk_mx<2>(A, R, [&](const uint32_t (&wd)[2], int i) {
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
+        for (int u = 0; u < 2; u++) {
             if (i + u >= R.ng) continue;  // uniform
             if (!(wd[u] & PDX_W16_ACT)) continue;
             const int slot = (int)(wd[u] & PDX_W16_SLOT);
             float4 a, b;
             float q[9];
             if (!CAP || slot < HL) {
-                a = hmx[4 * slot];
-                b = hmx[4 * slot + 1];
-                const float4 q0 = hmx[4 * slot + 2], q1 = hmx[4 * slot + 3];
+                a = hmx[slot];
+                b = hmx[HL + slot];
+                const float4 q0 = hmx[2 * HL + slot], q1 = hmx[3 * HL + slot];
                 q[0] = q0.x; q[1] = q0.y; q[2] = q0.z; q[3] = q0.w;
                 q[4] = q1.x; q[5] = q1.y; q[6] = q1.z; q[7] = q1.w;
                 q[8] = hq8[slot];
@@ -2488,28 +2569,31 @@ template <int PB_, int S_>
 struct blk_cfg {
     static constexpr int PB = PB_, S = S_;
 };
-template <class FN>
+// (BIG: the kernel also runs in blocks of 256 points; no correspondence kernel does)
+template <bool BIG = true, class FN>
 static void with_cfg(const pdx_ctx *c, FN &&f)
 {
     switch (c->cfg) {
-    case 1: f(blk_cfg<128, 4>{}); break;
+    case 0:
+        if constexpr (BIG) f(blk_cfg<256, 4>{});
+        break;
     case 2: f(blk_cfg<64, 8>{}); break;
     case 3: f(blk_cfg<32, 16>{}); break;
-    default: f(blk_cfg<256, 4>{}); break;
+    default: f(blk_cfg<128, 4>{}); break;
     }
 }
 
 // Launch of an LDS-staged kernel whose table entries take `entry` bytes, `bud` bytes of LDS
-// per block at the most.
+// per block at the most for the table and `least` bytes in any case.
 template <class CFG>
-static void launch_lds_bud(pdx_ctx *c, const void *fn, int entry, int bud, const pdx_step_args &a)
+static void launch_lds_bud(pdx_ctx *c, const void *fn, int entry, int bud, const pdx_step_args &a, size_t least = 0)
 {
     pdx_step_args af = a;
     af.lds_budget = bud;
     void *args[] = {&af};
     const int64_t blocks = (c->n + CFG::PB - 1) / CFG::PB;
     const dim3 G((unsigned)((blocks + PDX_NUM_XCD - 1) / PDX_NUM_XCD * PDX_NUM_XCD));
-    (void)hipLaunchKernel(fn, G, dim3(CFG::PB * CFG::S), args, lds_bytes(c, entry, bud), c->stream);
+    (void)hipLaunchKernel(fn, G, dim3(CFG::PB * CFG::S), args, std::max(lds_bytes(c, entry, bud), least), c->stream);
 }
 
 // A capped variant (tables longer than the budget) whose registers allow one block per CU
@@ -2518,12 +2602,13 @@ static void launch_lds_bud(pdx_ctx *c, const void *fn, int entry, int bud, const
 // past the budget from global memory gains once they are many (horizon 5.015 dx: ~80 % past
 // the budget) and loses a little when they are few (4.015 dx: ~15 %).
 template <class CFG>
-static void launch_lds(pdx_ctx *c, const void *fn, bool capped, bool tiled, int entry, const pdx_step_args &a)
+static void launch_lds(pdx_ctx *c, const void *fn, bool capped, bool tiled, int entry, const pdx_step_args &a,
+                       size_t least = 0)
 {
     int bud = pdx_lds_budget(c);
     const bool many_past = (int64_t)c->halo_max * entry > (int64_t)bud * 3 / 2;
     if (capped && (tiled || many_past) && kernel_vgprs(fn) > 64) bud = pdx_lds_budget_full(c);
-    launch_lds_bud<CFG>(c, fn, entry, bud, a);
+    launch_lds_bud<CFG>(c, fn, entry, bud, a, least);
 }
 
 // feature masks 1..7 (PDX_FEAT_MULTI | PDX_FEAT_SC | PDX_FEAT_CAP); for OSB also those with
@@ -2587,22 +2672,25 @@ static void launch_osb_mx(pdx_ctx *c, CFG, int pass, int entry, const pdx_step_a
 }
 
 template <int F, class CFG>
-static void launch_cpd(pdx_ctx *c, CFG, int pass, int entry, int bud, const pdx_step_args &a)
+static void launch_cpd(pdx_ctx *c, CFG, int pass, int entry, const pdx_step_args &a)
 {
     const void *fn = pass == 1 ? (const void *)&k_cpd_lds1<CFG::S, F, CFG::PB, false>
                                : (const void *)&k_cpd_lds2_own<CFG::S, F, CFG::PB, false>;
     if constexpr (!(F & PDX_FEAT_MULTI))
         if (c->pk) fn = pass == 1 ? (const void *)&k_cpd_lds1<CFG::S, F, CFG::PB, true>
                                   : (const void *)&k_cpd_lds2_own<CFG::S, F, CFG::PB, true>;
-    launch_lds_bud<CFG>(c, fn, entry, bud, a);
+    // Tables up to half of the CU's LDS, so that two blocks share it and one walks its bonds while the
+    // other stages or finishes its points: with the whole LDS for one block 512 k points took 489
+    // against 458 us, ZEMWan 720 against 618, 5.015 spacings at 100 k points 428 against 403.
+    launch_lds_bud<CFG>(c, fn, entry, pdx_lds_budget(c), a, pass == 1 ? 22 * sizeof(double) * CFG::PB : 0);  // cpd_hand_over
 }
 
 template <int F, class CFG>
-static void launch_cpd_mx(pdx_ctx *c, CFG, int pass, int entry, int bud, const pdx_step_args &a)
+static void launch_cpd_mx(pdx_ctx *c, CFG, int pass, int entry, const pdx_step_args &a)
 {
     const void *fn = pass == 1 ? (const void *)&k_cpd_pass1_mx<CFG::S, F, CFG::PB>
                                : (const void *)&k_cpd_pass2_mx<CFG::S, F, CFG::PB>;
-    launch_lds_bud<CFG>(c, fn, entry, bud, a);
+    launch_lds<CFG>(c, fn, (F & PDX_FEAT_CAP) != 0, false, entry, a, pass == 1 ? 16 * sizeof(double) * CFG::PB : 0);
 }
 
 bool pdx_bb_jv_fusable(const pdx_ctx *c)
@@ -2714,18 +2802,15 @@ pdx_status pdx_launch_step(pdx_ctx *c, const pdx_step_args &a)
         break;
     case PDX_CPD:
         if (c->lds_mode) {
-            // The CPD passes hold 97-122 VGPRs, so one 1024-thread block runs per CU: their
-            // tables take the CU's whole LDS (fewer tiles, fewer entries read past the cap).
-            const int bud = pdx_lds_budget_full(c);
             if (mixed && !c->multi() && c->P.zem != PDX_ZEM_WAN &&
                 c->P.kernel == PDX_KERNEL_LINEAR) {  // otherwise the FP64 passes
                 for (int pass = 1; pass <= 2; pass++) {
                     // pass 1 entries (D, V), (U, 0): 32 B; pass 2 (D, V), (U, beta l), l Q': 68 B
                     const int entry = pass == 1 ? 32 : 68;
                     PDX_TRY(pdx_timed_begin(c));
-                    with_cfg(c, [&](auto g) {
-                        if (lds_capped(c, entry, bud)) launch_cpd_mx<PDX_FEAT_CAP>(c, g, pass, entry, bud, a);
-                        else launch_cpd_mx<0>(c, g, pass, entry, bud, a);
+                    with_cfg<false>(c, [&](auto g) {
+                        if (lds_capped(c, entry)) launch_cpd_mx<PDX_FEAT_CAP>(c, g, pass, entry, a);
+                        else launch_cpd_mx<0>(c, g, pass, entry, a);
                     });
                     PDX_HIP(c, hipGetLastError());
                     PDX_TRY(pdx_timed_end(c, pass == 1 ? "pass1" : "step"));
@@ -2735,8 +2820,8 @@ pdx_status pdx_launch_step(pdx_ctx *c, const pdx_step_args &a)
             const int fc = (c->multi() ? PDX_FEAT_MULTI : 0) | (c->P.zem == PDX_ZEM_WAN ? PDX_FEAT_ZW : 0);
             for (int pass = 1; pass <= 2; pass++) {
                 // pass 2 entries 112 B, 160 B with ZEMWan
-                const int entry = pass == 1 ? 64 + (c->multi() ? 1 : 0) : (c->P.zem == PDX_ZEM_WAN ? 160 : 112);
-#define PDX_CPD_LAUNCH(F) with_cfg(c, [&](auto g) { launch_cpd<F>(c, g, pass, entry, bud, a); })
+                const int entry = pass == 1 ? 56 + (c->multi() ? 1 : 0) : (c->P.zem == PDX_ZEM_WAN ? 160 : 112);
+#define PDX_CPD_LAUNCH(F) with_cfg<false>(c, [&](auto g) { launch_cpd<F>(c, g, pass, entry, a); })
                 PDX_TRY(pdx_timed_begin(c));
                 switch (fc) {
                 case 0: PDX_CPD_LAUNCH(0); break;

@@ -122,3 +122,29 @@ def test_bond_lists_of_the_device_set_up(need_gpu, oracle, shape):
     if shape[0] > 1:
         assert dh.calc_stable_timestep() == orc.stable_dt()
     dh.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("zem", ["silling", "wan"])
+@pytest.mark.parametrize("horizon", [3.015, 4.015, 5.015])
+def test_correspondence_failure_and_tiles(need_gpu, oracle, horizon, zem, precision):
+    """Correspondence bodies whose neighbour tables fit one LDS tile (3.015 spacings) and take
+    several (wider horizons), with bonds on both sides of the critical stretch: the squared
+    pre-check of the failure window may not lose one."""
+    say("correspondence tiles", horizon, zem, precision)
+    b = body_of("CPD", (23, 21, 12), horizon, Gc=100.0)
+    if zem == "wan":
+        b.mat.zem = pd.ZEMWan()
+    dh = pd.MI355XBodyDataHandler(b, precision=precision)
+    orc = oracle_for(oracle, b, "CPD")
+    X = b.xyz
+    x = X + displacement_field(X, 1e-5)
+    for _ in range(2):
+        dh.set("position", x)
+        dh.calc_force_density()
+        orc.force(x)
+        assert np.array_equal(dh.get("n_active_bonds"), orc.n_active)
+        assert 0 < orc.n_active.sum() < dh.n_bonds
+        assert scaled_error(dh.get("b_int"), orc) <= (FP64_TOL if precision == "fp64" else MIXED_TOL)
+        x = x + displacement_field(X[:, [1, 2, 0]], 5e-6)
+    dh.close()
