@@ -12,6 +12,9 @@
 //          (relaxation_step!, :335-343)
 //   v = (v_half_old + v_half) / 2, v_half_old = v_half, b_int_old = b_int
 //   (relaxation_updates!, :345-350)
+// Three launches per step: the force; the partial sums of cn1 and cn2, with the force-density
+// conditions of the step (k_dr_damping); cn from the partial sums, the update and the beginning of
+// the next step (k_dr_advance).
 // Lambda per point (calc_density_matrix!, :166-176):
 //   damping_factor * 1 / 4 * dt^2 * n_bonds * (5 pi delta^2 bc), the same for x, y, z.
 #include <cmath>
@@ -30,15 +33,13 @@ __global__ void k_dr_density(int64_t n, const int32_t *cnt, double lam, double d
     density[i] = ((((lam * 1.0) / 4.0) * (dt * dt)) * (double)cnt[i]) * k;
 }
 
-// velocity BCs on v_half (apply_boundary_conditions!), then u and x
-__global__ void k_dr_begin(int64_t n, const int32_t *bcslot, const int32_t *slot_src,
-                           const double *bcv, double dt, double *vh, double *u, double4 *rec)
+// dof t at the beginning of a step: its velocity condition on v_half
+// (apply_boundary_conditions!), then u and x
+__device__ __forceinline__ void dr_begin_dof(int64_t t, double v, const int32_t *bcslot, const int32_t *slot_src,
+                                             const double *bcv, double dt, double *vh, double *u, double4 *rec)
 {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= 3 * n) return;
     const int64_t i = t / 3;
     const int d = (int)(t - 3 * i);
-    double v = vh[t];
     const int32_t s = bcslot[i];
     if (s >= 0 && bcv) {
         const int32_t src = slot_src[3 * s + d];
@@ -54,6 +55,14 @@ __global__ void k_dr_begin(int64_t n, const int32_t *bcslot, const int32_t *slot
     *x = *x + du;
 }
 
+__global__ void k_dr_begin(int64_t n, const int32_t *bcslot, const int32_t *slot_src,
+                           const double *bcv, double dt, double *vh, double *u, double4 *rec)
+{
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= 3 * n) return;
+    dr_begin_dof(t, vh[t], bcslot, slot_src, bcv, dt, vh, u, rec);
+}
+
 __device__ __forceinline__ void two_sum(double a, double b, double &s, double &e)
 {
     s = a + b;
@@ -61,13 +70,16 @@ __device__ __forceinline__ void two_sum(double a, double b, double &s, double &e
     e = (a - (s - v)) + (b - v);
 }
 
-// compensated partial sums of cn1 and cn2: part[4 blk + (cn1, cn1_c, cn2, cn2_c)]
+// compensated partial sums of cn1 and cn2: part[4 blk + (cn1, cn1_c, cn2, cn2_c)]; also the
+// force-density conditions of the step (fd.n > 0), which only the update behind it reads
 __global__ __launch_bounds__(256) void k_dr_damping(int64_t m, const double *u, const double *vh,
                                                     const double *vh_old, const double *bint,
                                                     const double *bint_old, const double *density,
-                                                    double dt, double *part)
+                                                    double dt, double *part, pdx_fd_bcs fd)
 {
     __shared__ double sh[4][256];
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < 3 * fd.n; t += (int64_t)gridDim.x * 256)
+        pdx_fd_dof(fd, t);
     double c1 = 0.0, c1c = 0.0, c2 = 0.0, c2c = 0.0, e;
     for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < m; t += (int64_t)gridDim.x * 256) {
         const double ut = u[t];
@@ -100,8 +112,8 @@ __global__ __launch_bounds__(256) void k_dr_damping(int64_t m, const double *u, 
     if (threadIdx.x < 4) part[4 * blockIdx.x + threadIdx.x] = sh[threadIdx.x][0];
 }
 
-// combine the partial sums (two_sum) and finish_damping: cn into out[0]
-__global__ __launch_bounds__(256) void k_dr_finish(int nblk, const double *part, double *out)
+// cn from the partial sums (two_sum) and finish_damping; every thread of a block of 256 calls it
+__device__ __forceinline__ double dr_finish(int nblk, const double *part)
 {
     __shared__ double sh[4][256];
     double c1 = 0.0, c1c = 0.0, c2 = 0.0, c2c = 0.0, s, e;
@@ -129,36 +141,48 @@ __global__ __launch_bounds__(256) void k_dr_finish(int nblk, const double *part,
         }
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        const double cn1 = sh[0][0] + sh[1][0], cn2 = sh[2][0] + sh[3][0];
-        double cn = 0.0;
-        if (cn2 != 0.0 && cn1 / cn2 > 0.0) cn = 2.0 * sqrt(cn1 / cn2);
-        if (cn > 2.0) cn = 1.9;
-        out[0] = cn;
-    }
+    const double cn1 = sh[0][0] + sh[1][0], cn2 = sh[2][0] + sh[3][0];
+    double cn = 0.0;
+    if (cn2 != 0.0 && cn1 / cn2 > 0.0) cn = 2.0 * sqrt(cn1 / cn2);
+    if (cn > 2.0) cn = 1.9;
+    return cn;
 }
 
-// relaxation_first_step! / relaxation_step! and relaxation_updates!
-__global__ void k_dr_update(int64_t m, int first, double dt, const double *cnp, const double *bint,
-                            const double *bext, const double *density, double *vh, double *vh_old,
-                            double *v, double *bint_old)
+__global__ __launch_bounds__(256) void k_dr_finish(int nblk, const double *part, double *out)
 {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= m) return;
-    const double rho = density[t / 3];
-    const double bt = bint[t] + (bext ? bext[t] : 0.0);
-    double vn;
-    if (first) {
-        vn = ((0.5 * dt) * bt) / rho;
-    } else {
-        const double cn = *cnp;
-        const double a = bt / rho;
-        vn = ((2.0 - cn * dt) * vh[t] + (2.0 * dt) * a) / (2.0 + cn * dt);
+    const double cn = dr_finish(nblk, part);
+    if (threadIdx.x == 0) out[0] = cn;
+}
+
+// cn, relaxation_first_step! / relaxation_step! and relaxation_updates!, then (more) the
+// beginning of the next step with its condition values bcv.  Every block forms cn for itself, in
+// the same order, from at most 1024 partial sums (32 KB from the L2): a launch for it between the
+// two passes took 4.7 us, the beginning of a step as a pass of its own 5.6, the force-density
+// conditions 4.6, of 66 us per step at 100 k points.
+__global__ __launch_bounds__(256) void k_dr_advance(int64_t m, int first, int more, double dt, int nblk, const double *part,
+                                                    const double *bint, const double *bext, const double *density,
+                                                    double *vh, double *vh_old, double *v, double *bint_old,
+                                                    const int32_t *bcslot, const int32_t *slot_src, const double *bcv,
+                                                    double *u, double4 *rec)
+{
+    const double cn = first ? 0.0 : dr_finish(nblk, part);
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < m; t += (int64_t)gridDim.x * 256) {
+        const double rho = density[t / 3];
+        const double bi = bint[t];
+        const double bt = bi + (bext ? bext[t] : 0.0);
+        double vn;
+        if (first) {
+            vn = ((0.5 * dt) * bt) / rho;
+        } else {
+            const double a = bt / rho;
+            vn = ((2.0 - cn * dt) * vh[t] + (2.0 * dt) * a) / (2.0 + cn * dt);
+        }
+        v[t] = 0.5 * (vh_old[t] + vn);
+        vh_old[t] = vn;
+        bint_old[t] = bi;
+        if (more) dr_begin_dof(t, vn, bcslot, slot_src, bcv, dt, vh, u, rec);
+        else vh[t] = vn;
     }
-    vh[t] = vn;
-    v[t] = 0.5 * (vh_old[t] + vn);
-    vh_old[t] = vn;
-    bint_old[t] = bint[t];
 }
 
 static pdx_status dr_ensure(pdx_ctx *c)
@@ -201,7 +225,7 @@ extern "C" pdx_status pdx_dr_damping(pdx_ctx *c, double dt, double *cn_out)
     const int64_t m = 3 * c->n;
     const int nb = (int)std::min<int64_t>(DR_BLOCKS, (m + 255) / 256);
     hipLaunchKernelGGL(k_dr_damping, dim3(nb), dim3(256), 0, c->stream, m, c->u, c->vh, c->dr_vh_old,
-                       c->bint, c->dr_bint_old, c->dr_density, dt, c->dr_part);
+                       c->bint, c->dr_bint_old, c->dr_density, dt, c->dr_part, pdx_fd_bcs{});
     hipLaunchKernelGGL(k_dr_finish, dim3(1), dim3(256), 0, c->stream, nb, c->dr_part,
                        c->dr_part + 4 * DR_BLOCKS);
     PDX_HIP(c, hipGetLastError());
@@ -235,28 +259,30 @@ extern "C" pdx_status pdx_dr_run(pdx_ctx *c, int64_t first, int64_t n_steps, dou
     PDX_TRY(pdx_reset_flags(c));
     const int64_t m = 3 * c->n;
     const int nb = (int)std::min<int64_t>(DR_BLOCKS, (m + 255) / 256);
-    double *cnp = c->dr_part + 4 * DR_BLOCKS;
+    auto bcv_of = [&](int64_t k) { return c->n_src > 0 ? c->bcvals + c->n_src * k : nullptr; };
+    hipLaunchKernelGGL(k_dr_begin, grid_of(m), dim3(256), 0, c->stream, c->n, c->bcslot, c->slot_src,
+                       bcv_of(0), dt, c->vh, c->u, c->rec[c->cur]);
+    PDX_HIP(c, hipGetLastError());
     for (int64_t k = 0; k < n_steps; k++) {
         const int64_t step = first + k;
-        const double *bcv = c->n_src > 0 ? c->bcvals + c->n_src * k : nullptr;
-        hipLaunchKernelGGL(k_dr_begin, grid_of(m), dim3(256), 0, c->stream, c->n, c->bcslot, c->slot_src,
-                           bcv, dt, c->vh, c->u, c->rec[c->cur]);
-        PDX_HIP(c, hipGetLastError());
-        PDX_TRY(pdx_apply_fd_bcs(c, bcv));
+        const int firstflag = step == 1 ? 1 : 0;
         pdx_step_args a;
         // (the adaptive damping amplifies the rounding of the sums from step to step: they keep one
         // order for every block size)
         PDX_TRY(pdx_fill_step_args(c, &a, step, PDX_F_FORCE_ONLY | PDX_F_ORDER, dt, nullptr));
         PDX_TRY(pdx_launch_step(c, a));
-        const int firstflag = step == 1 ? 1 : 0;
-        if (!firstflag) {
+        if (firstflag)
+            PDX_TRY(pdx_apply_fd_bcs(c, bcv_of(k)));
+        else
             hipLaunchKernelGGL(k_dr_damping, dim3(nb), dim3(256), 0, c->stream, m, c->u, c->vh,
-                               c->dr_vh_old, c->bint, c->dr_bint_old, c->dr_density, dt, c->dr_part);
-            hipLaunchKernelGGL(k_dr_finish, dim3(1), dim3(256), 0, c->stream, nb, c->dr_part, cnp);
-        }
-        hipLaunchKernelGGL(k_dr_update, grid_of(m), dim3(256), 0, c->stream, m, firstflag, dt, cnp,
-                           c->bint, c->bext_nonzero ? c->bext : nullptr, c->dr_density, c->vh,
-                           c->dr_vh_old, c->v, c->dr_bint_old);
+                               c->dr_vh_old, c->bint, c->dr_bint_old, c->dr_density, dt, c->dr_part,
+                               pdx_fd_table(c, bcv_of(k)));
+        const int more = k + 1 < n_steps ? 1 : 0;
+        hipLaunchKernelGGL(k_dr_advance, dim3((unsigned)std::min<int64_t>(2 * DR_BLOCKS, (m + 255) / 256)), dim3(256), 0,
+                           c->stream, m, firstflag, more, dt, nb, c->dr_part, c->bint,
+                           c->bext_nonzero ? c->bext : nullptr, c->dr_density, c->vh, c->dr_vh_old, c->v,
+                           c->dr_bint_old, c->bcslot, c->slot_src, more ? bcv_of(k + 1) : nullptr, c->u,
+                           c->rec[c->cur]);
         PDX_HIP(c, hipGetLastError());
     }
     int64_t nan_step = -1;

@@ -511,7 +511,24 @@ pdx_status pdx_launch_bb_jv(pdx_ctx *c, const double *u, const double *v, const 
                             const double *parts, int np, double sc, const uint8_t *cmask,
                             double *jv);
 pdx_status pdx_launch_prologue(pdx_ctx *c, int64_t step, double dt, const double *bcv_dev);
-pdx_status pdx_apply_fd_bcs(pdx_ctx *c, const double *bcv_row);  // b_ext conditions of one step
+// force-density conditions of one step: dof 3 pts[k] + d of b_ext takes value src[3k + d] of the
+// step's row (non-finite: unchanged)
+struct pdx_fd_bcs {
+    int64_t n;
+    const int32_t *pts, *src;
+    const double *bcv;
+    double *bext;
+};
+__device__ __forceinline__ void pdx_fd_dof(const pdx_fd_bcs &fd, int64_t t)
+{
+    const int64_t k = t / 3;
+    const int32_t s = fd.src[t];
+    if (s < 0) return;
+    const double val = fd.bcv[s];
+    if (isfinite(val)) fd.bext[3 * (int64_t)fd.pts[k] + (t - 3 * k)] = val;
+}
+pdx_fd_bcs pdx_fd_table(const pdx_ctx *c, const double *bcv_row);  // n = 0: none
+pdx_status pdx_apply_fd_bcs(pdx_ctx *c, const double *bcv_row);
 pdx_status pdx_build_correction(pdx_ctx *c);  // EnergySurfaceCorrection factors
 // LDS bytes for a block's neighbour table: half the CU's LDS (two 1024-thread blocks per
 // CU), minus room for the parameter-set bytes' alignment

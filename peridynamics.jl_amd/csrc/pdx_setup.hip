@@ -1692,25 +1692,25 @@ extern "C" pdx_status pdx_set_force_density_bcs(pdx_ctx *c, int64_t npts, const 
     return PDX_OK;
 }
 
-// b_ext of the constrained dofs from one row of condition values (non-finite: unchanged)
-__global__ void k_fd_bcs(int64_t npts, const int32_t *pts, const int32_t *src, const double *bcv,
-                         double *bext)
+// b_ext of the constrained dofs from one row of condition values
+__global__ void k_fd_bcs(pdx_fd_bcs fd)
 {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= 3 * npts) return;
-    const int64_t k = t / 3;
-    const int d = (int)(t - 3 * k);
-    const int32_t s = src[t];
-    if (s < 0) return;
-    const double val = bcv[s];
-    if (isfinite(val)) bext[3 * (int64_t)pts[k] + d] = val;
+    if (t < 3 * fd.n) pdx_fd_dof(fd, t);
+}
+
+pdx_fd_bcs pdx_fd_table(const pdx_ctx *c, const double *bcv_row)
+{
+    pdx_fd_bcs fd{};
+    if (c->n_fdpts > 0 && bcv_row) fd = {c->n_fdpts, c->fd_pts, c->fd_src, bcv_row, c->bext};
+    return fd;
 }
 
 pdx_status pdx_apply_fd_bcs(pdx_ctx *c, const double *bcv_row)
 {
-    if (c->n_fdpts <= 0 || !bcv_row) return PDX_OK;
-    hipLaunchKernelGGL(k_fd_bcs, dim3((unsigned)((3 * c->n_fdpts + 255) / 256)), dim3(256), 0, c->stream,
-                       c->n_fdpts, c->fd_pts, c->fd_src, bcv_row, c->bext);
+    const pdx_fd_bcs fd = pdx_fd_table(c, bcv_row);
+    if (fd.n <= 0) return PDX_OK;
+    hipLaunchKernelGGL(k_fd_bcs, dim3((unsigned)((3 * fd.n + 255) / 256)), dim3(256), 0, c->stream, fd);
     PDX_HIP(c, hipGetLastError());
     return PDX_OK;
 }

@@ -148,3 +148,29 @@ def test_correspondence_failure_and_tiles(need_gpu, oracle, horizon, zem, precis
         assert scaled_error(dh.get("b_int"), orc) <= (FP64_TOL if precision == "fp64" else MIXED_TOL)
         x = x + displacement_field(X[:, [1, 2, 0]], 5e-6)
     dh.close()
+
+
+@pytest.mark.parametrize("shape", ["tiny", "64x8", "256x4 cpd"])
+def test_relaxation_steps_in_one_call(need_gpu, shape):
+    """Relaxation steps of one call, where a step's update also begins the next one, equal the same
+    steps in calls of their own, with time-dependent velocity and force-density conditions that
+    leave out some steps (NaN)."""
+    say("relaxation calls", shape)
+    out = []
+    for cap in (7, 1):
+        b = body_of("BB", SHAPES[shape], 3.015, Gc=None)
+        x = b.position[0]
+        pd.point_set(b, "left", x < x.min() + 1.1e-3)
+        pd.point_set(b, "right", x > x.max() - 1.1e-3)
+        pd.velocity_bc(lambda t: np.nan if t == 3.0 else 1e-9 * t, b, "left", "x")
+        pd.forcedensity_bc(lambda t: np.nan if t in (2.0, 5.0) else 1e5 * t, b, "right", "x")
+        dh = pd.MI355XBodyDataHandler(b)
+        dh.ctx.dr_init(1.0, 1.0)
+        for n in range(1, 8, cap):
+            dh.ctx.dr_run(n, cap, 1.0, dh.bc_values(range(n, n + cap), 1.0))
+        out.append([dh.get(f) for f in ("displacement", "velocity", "velocity_half", "velocity_half_old", "b_int",
+                                        "b_int_old", "b_ext", "position")])
+        dh.close()
+    assert np.abs(out[0][0]).max() > 0
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
