@@ -362,23 +362,53 @@ __device__ __forceinline__ void cgs_block_store1(double x, double *partial, int 
     }
 }
 
-// partial (column q, one per block) = V_q . w for q < nv
+// V_q of one dof, q < 32 NC, eight loads per branch (past nv the last vector again: it is not used)
+template <int NC>
+__device__ __forceinline__ void cgs_load(double (&v)[NC][CGS_REG], int nv, const double *V, int64_t ldv, int64_t i)
+{
+#pragma unroll
+    for (int g = 0; g < NC * CGS_REG; g += 8) {
+#pragma unroll
+        for (int q = g; q < g + 8; q++) v[q / CGS_REG][q % CGS_REG] = 0.0;
+        if (g < nv) {
+#pragma unroll
+            for (int q = g; q < g + 8; q++) v[q / CGS_REG][q % CGS_REG] = V[(int64_t)min(q, nv - 1) * ldv + i];
+        }
+    }
+}
+
+// The one-dof-per-thread forms load all vectors at once, so that a basis of up to 64 vectors is one
+// round of loads.  They are bound by that round's latency and the reductions: at 43 k dofs (169 blocks)
+// the dots took 12.5 us on average over a cycle of 60 columns with two rounds of predicated loads
+// beyond 32 vectors, and the update with its dots 21.4 us there (V read twice, the first time one
+// vector after the other).  A solve of 532 columns at 43 k dofs 38.9 -> 33.5 ms, of 720 columns at
+// 302 k dofs 101 -> 90.6 ms, of 240 columns at 525 k dofs (one dof per thread no longer) 56.4 either way.
+
+// partial (column q, one per block) = V_q . w for q < nv; nv <= 32 NC and one dof per thread
+template <int NC>
 __global__ __launch_bounds__(CGS_T) void k_cgs_dots(int64_t m, int nv, const double *V, int64_t ldv,
                                                   const double *w, double *partial)
 {
     __shared__ double sh[CGS_NW][CGS_REG];
-    const int64_t i0 = (int64_t)blockIdx.x * CGS_T, stride = (int64_t)gridDim.x * CGS_T;
-    if (m <= stride && nv <= CGS_REG) {
-        // one dof per thread: the products go straight into the register array
-        const int64_t i = i0 + threadIdx.x;
-        double s[CGS_REG];
-        const double wi = i < m ? w[i] : 0.0;
+    const int64_t i = (int64_t)blockIdx.x * CGS_T + threadIdx.x, ic = i < m ? i : m - 1;
+    const double wi = i < m ? w[i] : 0.0;
+    double s[NC][CGS_REG];
+    cgs_load<NC>(s, nv, V, ldv, ic);
 #pragma unroll
-        for (int q = 0; q < CGS_REG; q++) s[q] = (q < nv && i < m) ? V[(int64_t)q * ldv + i] * wi : 0.0;
-        pdx_wave_reduce32(s);
-        cgs_block_store(s, nv, sh, partial, 0);
-        return;
+    for (int c = 0; c < NC; c++) {
+#pragma unroll
+        for (int q = 0; q < CGS_REG; q++) s[c][q] = i < m ? s[c][q] * wi : 0.0;
+        pdx_wave_reduce32(s[c]);
+        cgs_block_store(s[c], min(CGS_REG, nv - c * CGS_REG), sh, partial, c * CGS_REG);
     }
+}
+
+// the same for several dofs per thread or a longer basis
+__global__ __launch_bounds__(CGS_T) void k_cgs_dots_loop(int64_t m, int nv, const double *V, int64_t ldv,
+                                                       const double *w, double *partial)
+{
+    __shared__ double sh[CGS_NW][CGS_REG];
+    const int64_t i0 = (int64_t)blockIdx.x * CGS_T, stride = (int64_t)gridDim.x * CGS_T;
     for (int k0 = 0; k0 < nv; k0 += CGS_REG) {
         const int kn = min(CGS_REG, nv - k0);
         const double *Vk = V + (int64_t)k0 * ldv;
@@ -397,34 +427,33 @@ __global__ __launch_bounds__(CGS_T) void k_cgs_dots(int64_t m, int nv, const dou
 }
 
 // w -= V h; partial columns q < nv: V_q . w (the updated w), column nv: w . w.  One dof
-// per thread (m <= CGS_T x blocks) and nv <= 32: the products overwrite the loaded V values,
-// so only one 32-wide register array is live; h is read from LDS.
+// per thread (m <= CGS_T x blocks) and nv <= 32 NC: the products overwrite the loaded V values; h is
+// read from LDS (zero past nv).
+template <int NC>
 __global__ __launch_bounds__(CGS_T) void k_cgs_axdn(int64_t m, int nv, const double *h, const double *V,
                                                   int64_t ldv, double *w, double *partial)
 {
     __shared__ double sh[CGS_NW][CGS_REG];
-    __shared__ double hs[CGS_REG];
-    if (threadIdx.x < CGS_REG) hs[threadIdx.x] = (int)threadIdx.x < nv ? h[threadIdx.x] : 0.0;
+    __shared__ double hs[NC * CGS_REG];
+    const int64_t i = (int64_t)blockIdx.x * CGS_T + threadIdx.x, ic = i < m ? i : m - 1;
+    const double ht = (int)threadIdx.x < nv ? h[threadIdx.x] : 0.0;
+    double x = w[ic];
+    double v[NC][CGS_REG];
+    cgs_load<NC>(v, nv, V, ldv, ic);
+    if (threadIdx.x < NC * CGS_REG) hs[threadIdx.x] = ht;
     __syncthreads();
-    const int64_t i = (int64_t)blockIdx.x * CGS_T + threadIdx.x;
-    double v[CGS_REG];
-    double x = 0.0;
 #pragma unroll
-    for (int q = 0; q < CGS_REG; q++) v[q] = 0.0;
-    if (i < m) {
+    for (int q = 0; q < NC * CGS_REG; q++)
+        if (q < nv) x -= hs[q] * v[q / CGS_REG][q % CGS_REG];
+    if (i < m) w[i] = x;
+    else x = 0.0;
 #pragma unroll
-        for (int q = 0; q < CGS_REG; q++)
-            if (q < nv) v[q] = V[(int64_t)q * ldv + i];
-        x = w[i];
+    for (int c = 0; c < NC; c++) {
 #pragma unroll
-        for (int q = 0; q < CGS_REG; q++)
-            if (q < nv) x -= hs[q] * v[q];
-        w[i] = x;
+        for (int q = 0; q < CGS_REG; q++) v[c][q] = i < m ? v[c][q] * x : 0.0;
+        pdx_wave_reduce32(v[c]);
+        cgs_block_store(v[c], min(CGS_REG, nv - c * CGS_REG), sh, partial, c * CGS_REG);
     }
-#pragma unroll
-    for (int q = 0; q < CGS_REG; q++) v[q] *= x;
-    pdx_wave_reduce32(v);
-    cgs_block_store(v, nv, sh, partial, 0);
     cgs_block_store1(x * x, partial, nv);
 }
 
@@ -591,7 +620,7 @@ pdx_status pdx_nk_jv_dev(pdx_ctx *c, const double *v, double *jv, double scale, 
     const double sc = scale * std::cbrt(2.220446049250313e-16);
     if (!parts) {
         const int nb = cgs_blocks(k->m);
-        hipLaunchKernelGGL(k_cgs_dots, dim3(nb), dim3(CGS_T), 0, c->stream, k->m, 1, v, k->m, v, k->vparts);
+        hipLaunchKernelGGL(k_cgs_dots_loop, dim3(nb), dim3(CGS_T), 0, c->stream, k->m, 1, v, k->m, v, k->vparts);
         parts = k->vparts;
         np = nb;
     }
@@ -1443,7 +1472,7 @@ static pdx_status nk_norm2_dev(pdx_ctx *c, const double *x, double *out_dev)
 {
     pdx_nk *k = c->nk;
     const int nb = cgs_blocks(k->m);
-    hipLaunchKernelGGL(k_cgs_dots, dim3(nb), dim3(CGS_T), 0, c->stream, k->m, 1, x, k->m, x, k->red);
+    hipLaunchKernelGGL(k_cgs_dots_loop, dim3(nb), dim3(CGS_T), 0, c->stream, k->m, 1, x, k->m, x, k->red);
     hipLaunchKernelGGL(k_reduce_cols, dim3(1), dim3(256), 0, c->stream, nb, (const double *)k->red, out_dev);
     PDX_HIP(c, hipGetLastError());
     return PDX_OK;
@@ -1520,15 +1549,12 @@ static pdx_status fgmres(pdx_ctx *c, const double *b, int restart, int maxiter, 
             // partial sums that the Arnoldi step reduces into h2; then the next basis vector
             // (w - V h2) / |w - V h2| and its preconditioned image
             const int nv = j + 1;
-            hipLaunchKernelGGL(k_cgs_dots, dim3(CB), dim3(CGS_T), 0, s, m, nv, (const double *)k->Vb, m,
-                               (const double *)w, k->red);
+            const bool one = m <= (int64_t)CB * CGS_T && nv <= 2 * CGS_REG;
+            hipLaunchKernelGGL(!one ? k_cgs_dots_loop : nv > CGS_REG ? k_cgs_dots<2> : k_cgs_dots<1>, dim3(CB),
+                               dim3(CGS_T), 0, s, m, nv, (const double *)k->Vb, m, (const double *)w, k->red);
             hipLaunchKernelGGL(k_reduce_cols, dim3((unsigned)nv), dim3(256), 0, s, CB, (const double *)k->red, G.h1);
-            if (nv <= CGS_REG && m <= (int64_t)CB * CGS_T)
-                hipLaunchKernelGGL(k_cgs_axdn, dim3(CB), dim3(CGS_T), 0, s, m, nv, (const double *)G.h1,
-                                   (const double *)k->Vb, m, w, k->red);
-            else
-                hipLaunchKernelGGL(k_cgs_axdn_loop, dim3(CB), dim3(CGS_T), 0, s, m, nv, (const double *)G.h1,
-                                   (const double *)k->Vb, m, w, k->red);
+            hipLaunchKernelGGL(!one ? k_cgs_axdn_loop : nv > CGS_REG ? k_cgs_axdn<2> : k_cgs_axdn<1>, dim3(CB),
+                               dim3(CGS_T), 0, s, m, nv, (const double *)G.h1, (const double *)k->Vb, m, w, k->red);
             const int last_allowed = (it + enq + 1 >= maxiter) ? 1 : 0;
             const int tok = k->col_tok = k->col_tok % 0x3fffffff + 1;  // 1 .. 2^30 - 1: 2 tok + 1 fits an int
             k->tok[j % PDX_NK_SLOTS] = tok;
