@@ -1072,7 +1072,10 @@ static pdx_status build_halos(pdx_ctx *c, bool *ok)
 //   CPD FP64  6 k  n/a / 28.0 / 21.8 / 18.7    14 k  n/a / 38.4 / 29.7 / 27.6
 //            25 k  n/a / 40.2 / 39.4 / 46.3    54 k 61.8 / 59.0 / 67.8
 //           512 k  490 /  458 /  588            2 M 2218 / 1750
-// so the blocks are the largest that still give 160 of them.  FP64 stops at 128 points, whose
+// so the blocks are the largest that still give 160 of them, and those of 32 points, where twice as
+// many cost little, hold until 64-point blocks number 256 (12 k to 16 k points, 64 against 32: BB
+// 9.2 / 9.1, mixed BB 9.8 / 9.1, OSB 17.3 / 17.0, CPD 29.5 / 27.2; the load step of 14 k points
+// 33.5 against 31.9 ms).  FP64 stops at 128 points, whose
 // blocks share a CU two or three at a time; the mixed BB and OSB steps of bodies beyond a million
 // points go to 256 (334 against 356 at 2 M).  Horizons beyond about 4 spacings stop at 64 points,
 // whose neighbour tables still fit a block's share of the LDS (5.015 spacings, 121 k points, BB:
@@ -1091,7 +1094,7 @@ static void choose_blocks(pdx_ctx *c, bool lds)
     if (c->nb > 180 * c->n) first = 2;
     else if (c->kind != PDX_CPD && c->precision == PDX_MIXED && c->n > 1000000) first = 0;
     int k = first;
-    while (k < 3 && c->n < (int64_t)160 * pbs[k]) k++;
+    while (k < 3 && c->n < (int64_t)(k == 2 ? 256 : 160) * pbs[k]) k++;
     c->cfg = k;
     c->pb = pbs[k];
     c->ls = lss[k];

@@ -11,10 +11,10 @@ from test_gpu_parity import (FP64_TOL, MIXED_TOL, bonds_equal, displacement_fiel
 
 pytestmark = pytest.mark.gpu
 
-# below 160 blocks of 64 points: 32 points x 16 lanes; below 160 of 128: 64 x 8; then 128 x 4
-# (correspondence bodies from 160 blocks of 256: 256 x 4)
-SHAPES = {"tiny": (3, 3, 3), "32x16": (37, 25, 11), "64x8": (31, 30, 11), "64x8 last": (40, 39, 13),
-          "128x4": (41, 40, 13), "256x4 cpd": (61, 43, 16)}
+# below 256 blocks of 64 points: 32 points x 16 lanes; below 160 of 128: 64 x 8; then 128 x 4
+SHAPES = {"tiny": (3, 3, 3), "32x16": (37, 25, 11), "32x16 more": (31, 30, 11),
+          "64x8": (32, 32, 16), "64x8 last": (40, 39, 13),
+          "128x4": (41, 40, 13), "128x4 more": (61, 43, 16)}
 
 
 def body_of(kind, shape, horizon, isolated=False, Gc=100.0):
@@ -150,7 +150,7 @@ def test_correspondence_failure_and_tiles(need_gpu, oracle, horizon, zem, precis
     dh.close()
 
 
-@pytest.mark.parametrize("shape", ["tiny", "64x8", "256x4 cpd"])
+@pytest.mark.parametrize("shape", ["tiny", "64x8", "128x4 more"])
 def test_relaxation_steps_in_one_call(need_gpu, shape):
     """Relaxation steps of one call, where a step's update also begins the next one, equal the same
     steps in calls of their own, with time-dependent velocity and force-density conditions that
