@@ -94,6 +94,7 @@ struct pdx_gnn;  // learned preconditioner (pdx_gnn.hip)
 // the pinned ring of pdx_download_vec: slots, and bytes per slot
 #define PDX_PIN_SLOTS 8
 #define PDX_PIN_CHUNK ((size_t)2 << 20)
+#define PDX_PIN_RENT ((size_t)8 << 20)
 
 struct pdx_ctx {
     int device = 0;
@@ -153,10 +154,9 @@ struct pdx_ctx {
     double *defgrad = nullptr, *cauchy = nullptr;  // 9n (CPD)
     int32_t *d_perm = nullptr, *d_iperm = nullptr;
     double *stage = nullptr;               // 9n staging for permuted transfers
-    // pinned ring of pdx_download_vec: PDX_PIN_SLOTS slots at most, one event per slot
-    double *pin = nullptr;
-    int pin_slots = 0;
+    // pdx_download_vec: one event per slot of its ring, and bytes transferred without one
     hipEvent_t pin_ev[PDX_PIN_SLOTS] = {};
+    size_t pin_rent = 0;
     // bonds in sliced ELL (pdx_rows)
     int64_t *slice_ptr = nullptr;          // n_slices() + 1
     int ls = 0;                            // log2 of the lanes per point
@@ -545,7 +545,8 @@ inline int pdx_lds_budget_full(const pdx_ctx *c)
     return (int)std::min<int64_t>(b, c->lds_limit);
 }
 void pdx_export_free(pdx_ctx *c);              // the export pipeline's buffers and stream
-void pdx_pin_free(pdx_ctx *c);                 // the pinned ring of pdx_download_vec
+void pdx_pin_open();                           // a context more / less that may use the pinned rings
+void pdx_pin_close(pdx_ctx *c);
 // values [t0, t1) of a field in the caller's point order, to dst (device or pinned memory)
 pdx_status pdx_gather_range(pdx_ctx *c, const double *dev, int comps, int stride, int64_t t0, int64_t t1, double *dst);
 // device pointer, components and stride of a field (PDX_FIELD_*)

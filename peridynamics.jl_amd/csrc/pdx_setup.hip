@@ -128,6 +128,7 @@ extern "C" pdx_status pdx_create(pdx_ctx **out, int32_t device, int32_t precisio
         delete c;
         return PDX_ERR_OOM;
     }
+    pdx_pin_open();
     *out = c;
     return PDX_OK;
 }
@@ -138,7 +139,7 @@ extern "C" void pdx_destroy(pdx_ctx *c)
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     pdx_export_free(c);
-    pdx_pin_free(c);
+    pdx_pin_close(c);
     pdx_free_all(c);
     FREE(c->d_flags);
     (void)pdx_timed_flush(c);

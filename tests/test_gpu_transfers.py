@@ -47,3 +47,29 @@ def test_condition_sources_of_listed_points(need_gpu):
     assert np.array_equal(vh[one, 0], np.full(90, 0.25))
     assert np.array_equal(vh[two, 1], 100.0 * X[two, 0] + X[two, 1] * vv.dt)
     dh.close()
+
+
+def test_transfers_of_several_threads(need_gpu):
+    """Four threads, each with a body of its own, more than the process keeps rings for."""
+    import threading
+    shapes = [(64, 64, 32), (61, 53, 37), (30, 30, 30), (100, 100, 30)]
+    wrong = []
+
+    def work(k):
+        pos, vol = pd.lattice_block(*shapes[k], 1e-3)
+        b = pd.Body(pd.BBMaterial(), pos, vol)
+        pd.material(b, horizon=1.2e-3, rho=2700.0, E=70e9)
+        dh = pd.MI355XBodyDataHandler(b)
+        v = np.random.default_rng(k).standard_normal((b.n_points, 3))
+        dh.set("velocity", v)
+        for _ in range(5):
+            if not (np.array_equal(dh.get("velocity"), v) and np.array_equal(dh.get("volume"), b.volume)):
+                wrong.append(k)
+        dh.close()
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
