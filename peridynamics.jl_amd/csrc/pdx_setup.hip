@@ -293,11 +293,18 @@ extern "C" pdx_status pdx_add_precrack(pdx_ctx *c, int64_t na, const int32_t *a,
 
 // ----------------------------------------------------------------------------------------
 // Morton order: 63-bit keys (three quantised coordinates, bits interleaved), a stable radix sort
-// of (key, caller index) eight bits a pass.  One wave sorts a run of RS_RUN keys per pass: it
+// of (key, caller index) eight bits a pass.  One wave sorts a run of keys per pass: it
 // ranks 64 keys at a time by matching their digits over the wave, so the order inside a run is
 // kept without a barrier.  Measured with the rest of the device set-up (see pdx_build_bonds).
 // ----------------------------------------------------------------------------------------
-#define RS_RUN 2048
+// (256 to 2048 keys: as long as 512 runs remain, so that a small body's waves go through few rounds
+// of 64 keys in series; at 6 k points a pass of 21.6 us came from 32 such rounds)
+static int64_t rs_run(int64_t n)
+{
+    int64_t run = 256;
+    while (run < 2048 && n > 512 * run) run *= 2;
+    return run;
+}
 
 __device__ __forceinline__ uint64_t spread3(uint64_t v)
 {
@@ -325,13 +332,13 @@ __global__ void k_morton_keys(int64_t n, const double *X, double3 mn, double s, 
 }
 
 // digits of every run: cnt[digit * runs + run]
-__global__ __launch_bounds__(64) void k_rs_hist(int64_t n, int shift, const uint64_t *key, int32_t *cnt)
+__global__ __launch_bounds__(64) void k_rs_hist(int64_t n, int run, int shift, const uint64_t *key, int32_t *cnt)
 {
     __shared__ int32_t h[256];
     for (int d = threadIdx.x; d < 256; d += 64) h[d] = 0;
     __syncthreads();
-    const int64_t b = (int64_t)blockIdx.x * RS_RUN;
-    for (int64_t k = b + threadIdx.x; k < b + RS_RUN && k < n; k += 64)
+    const int64_t b = (int64_t)blockIdx.x * run;
+    for (int64_t k = b + threadIdx.x; k < b + run && k < n; k += 64)
         atomicAdd(&h[(key[k] >> shift) & 255], 1);
     __syncthreads();
     for (int d = threadIdx.x; d < 256; d += 64) cnt[(int64_t)d * gridDim.x + blockIdx.x] = h[d];
@@ -361,7 +368,7 @@ __global__ __launch_bounds__(256) void k_rs_scan(int runs, int32_t *cnt, int32_t
     if (threadIdx.x == 0) total[blockIdx.x] = carry;
 }
 
-__global__ __launch_bounds__(64) void k_rs_scatter(int64_t n, int shift, const uint64_t *key, const int32_t *val,
+__global__ __launch_bounds__(64) void k_rs_scatter(int64_t n, int run, int shift, const uint64_t *key, const int32_t *val,
                                                    const int32_t *cnt, const int32_t *total, uint64_t *key_out,
                                                    int32_t *val_out)
 {
@@ -381,8 +388,8 @@ __global__ __launch_bounds__(64) void k_rs_scatter(int64_t n, int shift, const u
     for (int q = 0; q < 4; q++)
         pos[4 * lane + q] = x - s + t[q] + cnt[(int64_t)(4 * lane + q) * gridDim.x + blockIdx.x];
     __syncthreads();
-    const int64_t b = (int64_t)blockIdx.x * RS_RUN;
-    for (int64_t k0 = b; k0 < b + RS_RUN && k0 < n; k0 += 64) {
+    const int64_t b = (int64_t)blockIdx.x * run;
+    for (int64_t k0 = b; k0 < b + run && k0 < n; k0 += 64) {
         const int64_t k = k0 + lane;
         const bool in = k < n;
         const uint64_t v = in ? key[k] : 0;
@@ -511,7 +518,8 @@ static pdx_status morton_order(pdx_ctx *c, setup_scratch &S, const double *dX, c
 {
     const int64_t n = c->n;
     const double ext = std::max({mx[0] - mn[0], mx[1] - mn[1], mx[2] - mn[2], 1e-300});
-    const int64_t runs = (n + RS_RUN - 1) / RS_RUN;
+    const int run = (int)rs_run(n);
+    const int64_t runs = (n + run - 1) / run;
     uint64_t *key[2];
     int32_t *val[2], *cnt, *total;
     for (int q = 0; q < 2; q++) {
@@ -524,9 +532,9 @@ static pdx_status morton_order(pdx_ctx *c, setup_scratch &S, const double *dX, c
                        2097151.0 / ext, key[0], val[0]);
     for (int pass = 0; pass < 8; pass++) {
         const int a = pass & 1, b = a ^ 1;
-        hipLaunchKernelGGL(k_rs_hist, dim3((unsigned)runs), dim3(64), 0, c->stream, n, 8 * pass, key[a], cnt);
+        hipLaunchKernelGGL(k_rs_hist, dim3((unsigned)runs), dim3(64), 0, c->stream, n, run, 8 * pass, key[a], cnt);
         hipLaunchKernelGGL(k_rs_scan, dim3(256), dim3(256), 0, c->stream, (int)runs, cnt, total);
-        hipLaunchKernelGGL(k_rs_scatter, dim3((unsigned)runs), dim3(64), 0, c->stream, n, 8 * pass, key[a], val[a],
+        hipLaunchKernelGGL(k_rs_scatter, dim3((unsigned)runs), dim3(64), 0, c->stream, n, run, 8 * pass, key[a], val[a],
                            cnt, total, key[b], pass == 7 ? c->d_perm : val[b]);
     }
     hipLaunchKernelGGL(k_invert, grid256(n), dim3(256), 0, c->stream, n, c->d_perm, c->d_iperm);
@@ -618,9 +626,15 @@ __global__ __launch_bounds__(256) void k_count_totals(int64_t n, const int32_t *
         s += __shfl_xor(s, o);
         m = max(m, __shfl_xor(m, o));
     }
+    __shared__ unsigned long long sh[2][4];  // one pair of atomics per block
     if ((threadIdx.x & 63) == 0) {
-        atomicAdd(&out[0], s);
-        atomicMax(&out[1], (unsigned long long)m);
+        sh[0][threadIdx.x >> 6] = s;
+        sh[1][threadIdx.x >> 6] = (unsigned long long)m;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        atomicAdd(&out[0], (sh[0][0] + sh[0][1]) + (sh[0][2] + sh[0][3]));
+        atomicMax(&out[1], max(max(sh[1][0], sh[1][1]), max(sh[1][2], sh[1][3])));
     }
 }
 
@@ -853,7 +867,19 @@ __global__ __launch_bounds__(256) void k_len_range(int64_t nb, const uint32_t *b
         lo = a < lo ? a : lo;
         hi = b > hi ? b : hi;
     }
+    // one pair of atomics per block: they all meet on one address (four pairs from each of 2048 blocks
+    // took 0.2 to 0.33 ms)
+    __shared__ unsigned long long sh[2][4];
     if ((threadIdx.x & 63) == 0) {
+        sh[0][threadIdx.x >> 6] = lo;
+        sh[1][threadIdx.x >> 6] = hi;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 4; w++) {
+            lo = sh[0][w] < lo ? sh[0][w] : lo;
+            hi = sh[1][w] > hi ? sh[1][w] : hi;
+        }
         atomicMin(&range[0], lo);
         atomicMax(&range[1], hi);
     }
@@ -882,7 +908,7 @@ static pdx_status pack_bonds(pdx_ctx *c)
     if (c->precision != PDX_FP64 || c->multi() || c->nb <= 0) return PDX_OK;
     unsigned long long *range = c->d_flags + 4, h[2] = {~0ULL, 0ULL};
     PDX_HIP(c, hipMemcpyAsync(range, h, sizeof h, hipMemcpyHostToDevice, c->stream));
-    hipLaunchKernelGGL(k_len_range, dim3((unsigned)std::min<int64_t>((c->nb_alloc + 255) / 256, 2048)), dim3(256), 0,
+    hipLaunchKernelGGL(k_len_range, dim3((unsigned)std::min<int64_t>((c->nb_alloc + 1023) / 1024, 2048)), dim3(256), 0,
                        c->stream, c->nb_alloc, c->bw, c->L, range);
     PDX_HIP(c, hipGetLastError());
     PDX_HIP(c, hipMemcpyAsync(h, range, sizeof h, hipMemcpyDeviceToHost, c->stream));
@@ -1245,7 +1271,7 @@ extern "C" pdx_status pdx_build_bonds(pdx_ctx *c, int64_t *n_bonds_out)
     s.counts = c->cnt;
     s.flags = c->d_flags;
     hipLaunchKernelGGL(k_count_bonds, dim3((unsigned)pdx_wave_grid(n)), dim3(PDX_BLOCK), 0, c->stream, s);
-    hipLaunchKernelGGL(k_count_totals, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 512)), dim3(256), 0, c->stream, n,
+    hipLaunchKernelGGL(k_count_totals, dim3((unsigned)std::min<int64_t>((n + 1023) / 1024, 256)), dim3(256), 0, c->stream, n,
                        c->cnt, c->d_flags + 4);
     PDX_HIP(c, hipGetLastError());
     unsigned long long hflags[8];
@@ -1816,6 +1842,12 @@ extern "C" pdx_status pdx_layout(pdx_ctx *c, int32_t *lds_mode, int64_t *bond_sl
     if (halo_entries) *halo_entries = c->lds_mode ? c->halo_total : 0;
     if (halo_max) *halo_max = c->lds_mode ? c->halo_max : 0;
     return PDX_OK;
+}
+
+extern "C" int32_t pdx_bond_bytes(const pdx_ctx *c)
+{
+    if (!c || !c->bonds_built) return 0;
+    return c->pk ? 8 : c->lds_mode ? 10 : 12;
 }
 
 pdx_status pdx_reset_flags(pdx_ctx *c)
