@@ -45,7 +45,8 @@ def step_bytes(n_points, n_bonds, precision, layout):
     per point: read x|V (32), u (24), v_half (24), bond count (4), BC slot (4); write x|V
                (32), u (24), v_half (24)  -> 168 B, plus 8 B per 64-point slice pointer;
                the mixed LDS step also reads the reference record X|V (32) -> 200 B;
-    per bond:  LDS-staged FP64: 16-bit bond word (2) + FP64 reference length (8);
+    per bond:  LDS-staged FP64: 16-bit bond word (2) + FP64 reference length (8), or both in one
+               64-bit word (8; layout["bond_bytes"]);
                LDS-staged mixed: the 16-bit bond word only (2; L = |X_j - X_i|);
                global-gather layout: 32-bit bond word (4) + length (8 FP64 / 4 FP32);
     per neighbour-table entry (LDS layouts): its 4-byte point index.
@@ -53,8 +54,9 @@ def step_bytes(n_points, n_bonds, precision, layout):
     n_slices = (n_points + 63) // 64
     if layout["lds_mode"]:
         if precision == "fp64":
-            return (10 * n_bonds + 168 * n_points + 8 * n_slices + 4 * layout["halo_entries"],
-                    "10*N_b + 168*N_p + 8*N_slices + 4*N_halo")
+            per_bond = layout.get("bond_bytes", 10)
+            return (per_bond * n_bonds + 168 * n_points + 8 * n_slices + 4 * layout["halo_entries"],
+                    f"{per_bond}*N_b + 168*N_p + 8*N_slices + 4*N_halo")
         return (2 * n_bonds + 200 * n_points + 8 * n_slices + 4 * layout["halo_entries"],
                 "2*N_b + 200*N_p + 8*N_slices + 4*N_halo")
     per_bond = 12 if precision == "fp64" else 8
@@ -290,8 +292,9 @@ def state_based_bytes(kind, n_points, n_bonds, layout, precision="fp64", zem="Si
     else:
         per_pt = (607 if zem == "Wan" else 511) if layout["lds_mode"] else 415
     if layout["lds_mode"]:
-        return (20 * n_bonds + per_pt * n_points + 8 * layout["halo_entries"],
-                f"20*N_b + {per_pt}*N_p + 8*N_halo")
+        per_bond = 2 * layout.get("bond_bytes", 10)
+        return (per_bond * n_bonds + per_pt * n_points + 8 * layout["halo_entries"],
+                f"{per_bond}*N_b + {per_pt}*N_p + 8*N_halo")
     return 24 * n_bonds + per_pt * n_points, f"24*N_b + {per_pt}*N_p"
 
 

@@ -339,6 +339,9 @@ pdx_status pdx_info(pdx_ctx *ctx, int64_t *n_points, int64_t *n_bonds, int64_t *
  * neighbour table.  Used to state the step kernel's algorithmic bytes. */
 pdx_status pdx_layout(pdx_ctx *ctx, int32_t *lds_mode, int64_t *bond_slots,
                       int64_t *halo_entries, int32_t *halo_max);
+/* Bytes of a bond slot that an FP64 step reads: 8 (one packed word), 10 (16-bit word and length)
+ * or 12 (global-gather layout); 0 before pdx_build_bonds. */
+int32_t pdx_bond_bytes(const pdx_ctx *ctx);
 
 #ifdef __cplusplus
 }
