@@ -167,7 +167,7 @@ struct pdx_ctx {
     uint32_t *bw = nullptr;                // bond words: neighbour | active | fail_permit
     double *L = nullptr;                   // reference lengths, null with packed bonds (pdx_ref_len)
     float *Lf = nullptr;                   // reference lengths (mixed layout)
-    // LDS-staged BB step: per block of PDX_BLOCK points, the sorted list of every point
+    // LDS-staged steps: per block of `pb` points, the sorted list of every point
     // its bonds reach (the halo); bonds then address the halo with 16-bit words
     // (bits 0-13 slot, bit 14 active, bit 15 fail_permit)
     bool lds_mode = false;
@@ -530,7 +530,7 @@ __device__ __forceinline__ void pdx_fd_dof(const pdx_fd_bcs &fd, int64_t t)
 pdx_fd_bcs pdx_fd_table(const pdx_ctx *c, const double *bcv_row);  // n = 0: none
 pdx_status pdx_apply_fd_bcs(pdx_ctx *c, const double *bcv_row);
 pdx_status pdx_build_correction(pdx_ctx *c);  // EnergySurfaceCorrection factors
-// LDS bytes for a block's neighbour table: half the CU's LDS (two 1024-thread blocks per
+// LDS bytes for a block's neighbour table: half the CU's LDS (two blocks per
 // CU), minus room for the parameter-set bytes' alignment
 inline int pdx_lds_budget(const pdx_ctx *c)
 {

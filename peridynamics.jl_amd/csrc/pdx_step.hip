@@ -39,8 +39,8 @@ __device__ __forceinline__ int64_t pdx_thread_point()
 }
 
 // Neighbour-table entries a block stages in LDS: all of them up to a budget that leaves
-// room for two 1024-thread blocks per CU; a block whose table is longer reads the entries
-// past the budget from global memory (through the caches).  ENTRY = LDS bytes per entry.
+// room for two blocks per CU; a block whose table is longer reads the entries past the budget
+// from global memory (through the caches) or stages the table in tiles.  ENTRY = LDS bytes per entry.
 __host__ __device__ __forceinline__ int pdx_lds_entries(int halo_max, int budget, int entry)
 {
     const int cap = budget / entry;
@@ -2596,18 +2596,20 @@ static void launch_lds_bud(pdx_ctx *c, const void *fn, int entry, int bud, const
     (void)hipLaunchKernel(fn, G, dim3(CFG::PB * CFG::S), args, std::max(lds_bytes(c, entry, bud), least), c->stream);
 }
 
-// A capped variant (tables longer than the budget) whose registers allow one block per CU
-// anyway may take the CU's whole LDS.  Measured at 576 k points: a tiled kernel gains from
-// fewer tiles whenever the table is longer than the budget; a kernel that reads the entries
-// past the budget from global memory gains once they are many (horizon 5.015 dx: ~80 % past
-// the budget) and loses a little when they are few (4.015 dx: ~15 %).
+// A capped variant (tables longer than the budget) may take the CU's whole LDS.  A tiled kernel
+// does if its block holds a CU alone anyway (1024 threads of more than 64 VGPRs): fewer tiles.  In
+// smaller blocks it keeps to half, so that two share the CU (us per OSB step, half against whole:
+// 318 / 382 at 121 k points and 5.015 spacings, 2780 / 3130 at 576 k and 6.015; several sets 688 / 835
+// at 512 k and 4.015).  A kernel that reads the entries past the budget from global memory does once
+// they are many (more than half a budget; mixed CPD at 5.015 spacings 283 / 356) and loses a little
+// when they are few.
 template <class CFG>
 static void launch_lds(pdx_ctx *c, const void *fn, bool capped, bool tiled, int entry, const pdx_step_args &a,
                        size_t least = 0)
 {
     int bud = pdx_lds_budget(c);
-    const bool many_past = (int64_t)c->halo_max * entry > (int64_t)bud * 3 / 2;
-    if (capped && (tiled || many_past) && kernel_vgprs(fn) > 64) bud = pdx_lds_budget_full(c);
+    const bool many_past = !tiled && (int64_t)c->halo_max * entry > (int64_t)bud * 3 / 2;
+    if (capped && ((tiled && CFG::PB * CFG::S == 1024) || many_past) && kernel_vgprs(fn) > 64) bud = pdx_lds_budget_full(c);
     launch_lds_bud<CFG>(c, fn, entry, bud, a, least);
 }
 
