@@ -1108,6 +1108,11 @@ static pdx_status build_halos(pdx_ctx *c, bool *ok)
 // whose neighbour tables still fit a block's share of the LDS (5.015 spacings, 121 k points, BB:
 // 216 / 169 / 157 / 159; OSB at 400 k: 1042 / 1074 / 897 / 942; CPD at 100 k: 629 / 517 / 403; 4.015
 // spacings, CPD at 100 k: 280 / 210 / 191).
+// The mixed BB and OSB steps go back to 256 points beyond about 4.5 spacings (350 bonds per point),
+// where a block of 64 has 40 table entries per point that the short FP32 arithmetic does not hide, if
+// the last round of these blocks, one to a CU, fills 80 % of it on average (5.015 spacings, 256 against
+// 64: BB 54 k 54.0 / 57.7, 121 k 104.5 / 117.7, 576 k 482 / 501, OSB 206 / 221 and 942 / 966 at the last two;
+// 200 k points, 3.05 rounds, 200 / 185 and 393 / 344).
 static void choose_blocks(pdx_ctx *c, bool lds)
 {
     if (!lds) {
@@ -1118,7 +1123,9 @@ static void choose_blocks(pdx_ctx *c, bool lds)
     }
     static const int pbs[4] = {256, 128, 64, 32}, lss[4] = {2, 2, 3, 4};
     int first = 1;
-    if (c->nb > 180 * c->n) first = 2;
+    const int64_t b256 = (c->n + 255) / 256, r256 = (b256 + 255) / 256;  // blocks, and their rounds over 256 CUs
+    if (c->kind != PDX_CPD && c->precision == PDX_MIXED && c->nb > 350 * c->n && 5 * b256 >= 4 * 256 * r256) first = 0;
+    else if (c->nb > 180 * c->n) first = 2;
     else if (c->kind != PDX_CPD && c->precision == PDX_MIXED && c->n > 1000000) first = 0;
     int k = first;
     while (k < 3 && c->n < (int64_t)(k == 2 ? 256 : 160) * pbs[k]) k++;

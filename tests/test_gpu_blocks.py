@@ -174,3 +174,22 @@ def test_relaxation_steps_in_one_call(need_gpu, shape):
     assert np.abs(out[0][0]).max() > 0
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("kind", ["BB", "OSB"])
+@pytest.mark.parametrize("shape", [(48, 37, 30), (44, 36, 30)])
+def test_mixed_wide_horizon(need_gpu, oracle, kind, shape):
+    """Mixed steps at 5.015 spacings in 256-point blocks (209 of them) and, where these would
+    leave a quarter of the device idle (186), in 64-point ones."""
+    say("mixed wide", kind, shape)
+    b = body_of(kind, shape, 5.015, Gc=None)
+    dh = pd.MI355XBodyDataHandler(b, precision="mixed")
+    orc = oracle_for(oracle, b, kind)
+    X = b.xyz
+    x = X + displacement_field(X, 3e-5)
+    dh.set("position", x)
+    dh.calc_force_density()
+    orc.force(x)
+    assert scaled_error(dh.get("b_int"), orc) <= MIXED_TOL
+    assert np.array_equal(dh.get("n_active_bonds"), orc.n_active)
+    dh.close()
