@@ -342,15 +342,20 @@ __device__ __forceinline__ void pdx_wave_reduce32(double (&s)[32])
     s[0] += __shfl_xor(s[0], 1);
 }
 
-// sum of parts[0, np) by a whole workgroup: every thread returns it, and the order of the
-// additions depends only on np and the workgroup size (sh: one double per wave)
+// Sum of parts[0, np) by a whole workgroup of full waves; every thread returns it.  The order of the
+// additions depends on np alone, not on the workgroup: it is that of 1024 threads, whose waves the
+// present ones take in turn (sh: PDX_SUM_WAVES doubles).  J v is bound by its bonds, not by this: in
+// workgroups of 512 threads a second turn is only needed beyond 512 partial sums.
+#define PDX_SUM_WAVES 16
 __device__ __forceinline__ double pdx_block_sum_parts(const double *parts, int np, double *sh)
 {
-    double s = 0.0;
-    for (int t = threadIdx.x; t < np; t += blockDim.x) s += parts[t];
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-    const int nw = (int)((blockDim.x + 63) >> 6);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+    const int nw = min(PDX_SUM_WAVES, (np + 63) >> 6);  // the others hold zeros
+    for (int w = (int)threadIdx.x >> 6; w < nw; w += (int)blockDim.x >> 6) {
+        double s = 0.0;
+        for (int t = 64 * w + (int)(threadIdx.x & 63); t < np; t += 64 * PDX_SUM_WAVES) s += parts[t];
+        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+        if ((threadIdx.x & 63) == 0) sh[w] = s;
+    }
     __syncthreads();
     double tot = 0.0;
     for (int q = 0; q < nw; q++) tot += sh[q];
@@ -505,7 +510,7 @@ pdx_status pdx_launch_step(pdx_ctx *c, const pdx_step_args &a);  // one step of 
 // J v = (F(u + e v) V - F(u - e v) V) / (2 e) of the bond-based material in one kernel, the
 // constrained rows (cmask) = v; true when the context's layout allows it (FP64 LDS step
 // with one parameter set, no surface correction, a neighbour table that fits the LDS)
-// ||v||^2 = the sum of the np partial sums `parts` (pdx_block_sum_parts at 1024 threads)
+// ||v||^2 = the sum of the np partial sums `parts` (pdx_block_sum_parts)
 bool pdx_bb_jv_fusable(const pdx_ctx *c);
 pdx_status pdx_launch_bb_jv(pdx_ctx *c, const double *u, const double *v, const double *un2,
                             const double *parts, int np, double sc, const uint8_t *cmask,

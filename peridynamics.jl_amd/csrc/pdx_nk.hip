@@ -602,11 +602,10 @@ static pdx_status force_scaled(pdx_ctx *c, const double4 *rec_in, double *out)
 static pdx_status nk_norm2_dev(pdx_ctx *c, const double *x, double *out_dev);
 static pdx_status nk_refresh_unorm(pdx_ctx *c) { return nk_norm2_dev(c, c->u, c->nk->dsc + NK_UN2); }
 
-// sum of np partial sums into out[0] (the order of pdx_block_sum_parts at 1024 threads, as
-// the one-kernel J v forms ||v||^2)
+// sum of np partial sums into out[0] (pdx_block_sum_parts, as the one-kernel J v forms ||v||^2)
 __global__ __launch_bounds__(1024) void k_sum_parts(const double *parts, int np, double *out)
 {
-    __shared__ double sh[16];
+    __shared__ double sh[PDX_SUM_WAVES];
     const double t = pdx_block_sum_parts(parts, np, sh);
     if (threadIdx.x == 0) out[0] = t;
 }

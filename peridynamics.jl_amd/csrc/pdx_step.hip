@@ -700,7 +700,7 @@ __global__ __launch_bounds__(PB * S) void k_bb_jv(pdx_step_args A, const double 
                                                   double sc, const uint8_t *cmask, double *jv)
 {
     extern __shared__ double4 hrec[];  // ONE: [0, H) + positions, [H, 2H) - positions
-    __shared__ double shs[PB * S / 64];
+    __shared__ double shs[PDX_SUM_WAVES];
     const int64_t k = pdx_xcd_block();
     const int64_t p0 = k * PB;
     if (p0 >= A.n) return;  // whole workgroup
