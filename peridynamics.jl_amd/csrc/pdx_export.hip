@@ -36,6 +36,9 @@
 // counts for 128 KB more), which is about when it has cost as much as a ring: a first pass over
 // displacement, velocity and damage of 9 k points takes 110 us by the runtime, 550 with a new ring and
 // 75 with one in use; of 512 k points 2.34, 2.38 and 0.91 ms.
+// The gather writes a ring with a kernel's stores and host threads read it behind an event, so the
+// memory is coherent by its own flag (and the events release to the system), not by the runtime's
+// default, which the environment can change (HIP_HOST_COHERENT).
 static std::mutex pin_mutex;
 static int pin_contexts = 0;
 static double *pin_idle[2] = {};
@@ -54,7 +57,7 @@ static double *pin_borrow(pdx_ctx *c, size_t bytes)
     c->pin_rent += bytes + ((size_t)128 << 10);
     if (c->pin_rent < PDX_PIN_RENT) return nullptr;
     void *p = nullptr;
-    if (hipHostMalloc(&p, PDX_PIN_SLOTS * PDX_PIN_CHUNK, hipHostMallocPortable) != hipSuccess) {
+    if (hipHostMalloc(&p, PDX_PIN_SLOTS * PDX_PIN_CHUNK, hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
         (void)hipGetLastError();
         return nullptr;
     }
@@ -104,7 +107,8 @@ void pdx_pin_close(pdx_ctx *c)
 static bool pin_events(pdx_ctx *c, int slots)
 {
     for (int k = 0; k < slots; k++)
-        if (!c->pin_ev[k] && hipEventCreateWithFlags(&c->pin_ev[k], hipEventDisableTiming) != hipSuccess) {
+        if (!c->pin_ev[k] &&
+            hipEventCreateWithFlags(&c->pin_ev[k], hipEventDisableTiming | hipEventReleaseToSystem) != hipSuccess) {
             c->pin_ev[k] = nullptr;
             (void)hipGetLastError();
             return false;
