@@ -166,6 +166,15 @@ extern "C" pdx_status pdx_set_points(pdx_ctx *c, int64_t n, const double *X, con
     if (!c) return PDX_ERR_ARG;
     if (n <= 0 || !X || !vol) return pdx_fail(c, PDX_ERR_ARG, "invalid points (n=%lld)", (long long)n);
     if (n >= PDX_MAX_POINTS) return pdx_fail(c, PDX_ERR_UNSUPPORTED, "too many points");
+    // all positions are looked at before the context changes: refused points leave the old ones in place
+    double mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
+    for (int64_t i = 0; i < n; i++)
+        for (int d = 0; d < 3; d++) {
+            const double x = X[3 * i + d];
+            if (!std::isfinite(x)) return pdx_fail(c, PDX_ERR_ARG, "non-finite position");
+            mn[d] = std::min(mn[d], x);
+            mx[d] = std::max(mx[d], x);
+        }
     PDX_HIP(c, hipSetDevice(c->device));
     PDX_HIP(c, hipStreamSynchronize(c->stream));
     pdx_free_all(c);
@@ -176,17 +185,8 @@ extern "C" pdx_status pdx_set_points(pdx_ctx *c, int64_t n, const double *X, con
     c->fail_permit.assign(n, 1);
     if (fp)
         for (int64_t i = 0; i < n; i++) c->fail_permit[i] = fp[i] ? 1 : 0;
-    for (int d = 0; d < 3; d++) {
-        c->mn[d] = INFINITY;
-        c->mx[d] = -INFINITY;
-    }
-    for (int64_t i = 0; i < n; i++)
-        for (int d = 0; d < 3; d++) {
-            const double x = X[3 * i + d];
-            if (!std::isfinite(x)) return pdx_fail(c, PDX_ERR_ARG, "non-finite position");
-            c->mn[d] = std::min(c->mn[d], x);
-            c->mx[d] = std::max(c->mx[d], x);
-        }
+    std::copy(mn, mn + 3, c->mn);
+    std::copy(mx, mx + 3, c->mx);
     c->cracks.clear();
     c->n_src = 0;
     c->n_bcpts = 0;
@@ -1182,6 +1182,9 @@ extern "C" pdx_status pdx_build_bonds(pdx_ctx *c, int64_t *n_bonds_out)
     if (c->kind < 0) return pdx_fail(c, PDX_ERR_STATE, "pdx_set_material first");
     PDX_HIP(c, hipSetDevice(c->device));
     const int64_t n = c->n;
+    for (int d = 0; d < 3; d++)  // (the cells are counted from the extent)
+        if (!std::isfinite(c->mx[d] - c->mn[d]))
+            return pdx_fail(c, PDX_ERR_UNSUPPORTED, "the extent of the body is not a finite number");
     if (c->bonds_built) {
         // rebuilding: drop everything but the points
         std::vector<pdx_crack> keep = c->cracks;
