@@ -139,7 +139,7 @@ struct pdx_ctx {
     int64_t xtag[2] = {0, 0};
     int64_t xbegun = 0, xwaited = 0;
     std::vector<pdx_crack> cracks;
-    bool bonds_built = false;
+    bool bonds_built = false, bonds_begun = false;  // begun: pdx_build_bonds has allocated
 
     // device state, internal (Morton) order
     double4 *rec[2] = {nullptr, nullptr};  // (x, y, z, volume) current positions, ping-pong

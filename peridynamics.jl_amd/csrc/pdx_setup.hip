@@ -103,7 +103,7 @@ void pdx_free_all(pdx_ctx *c)
     FREE(c->bcvals);
     free_bonds(c);
     c->dev_bytes = 0;
-    c->bonds_built = false;
+    c->bonds_built = c->bonds_begun = false;
     c->bcvals_cap = 0;
 }
 
@@ -1185,12 +1185,14 @@ extern "C" pdx_status pdx_build_bonds(pdx_ctx *c, int64_t *n_bonds_out)
     for (int d = 0; d < 3; d++)  // (the cells are counted from the extent)
         if (!std::isfinite(c->mx[d] - c->mn[d]))
             return pdx_fail(c, PDX_ERR_UNSUPPORTED, "the extent of the body is not a finite number");
-    if (c->bonds_built) {
-        // rebuilding: drop everything but the points
+    if (c->bonds_begun) {
+        // again, or after a build that ended in an error and left arrays of its sizes behind (pdx_alloc
+        // keeps what is there): drop everything but the points
         std::vector<pdx_crack> keep = c->cracks;
         pdx_free_all(c);
         c->cracks = keep;
     }
+    c->bonds_begun = true;
     // cell list over the internal order, cell size = horizon
     double cs = c->P.delta;
     double *const mn = c->mn, *const mx = c->mx;
