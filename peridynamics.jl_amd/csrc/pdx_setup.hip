@@ -784,16 +784,25 @@ __global__ void k_init_point_state(int64_t n, pdx_rows rows, const int32_t *cnt,
     damage[i] = 1.0 - (double)na / (double)cnt[i];
 }
 
+// Kernels over the bond slots.  A launch takes fewer than 2^32 threads, and a body of 37 M points at
+// 3.015 spacings (8 M at 5.015) has more slots than that, so their threads go over the slots in
+// strides; the grid covers bodies of up to 2^30 slots in one.
+static inline dim3 slot_grid(int64_t slots)
+{
+    return dim3((unsigned)std::min<int64_t>((slots + 255) / 256, (int64_t)1 << 22));
+}
+
+#define PDX_SLOT_LOOP(k, n)                                                                               \
+    for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < (n); k += (int64_t)gridDim.x * blockDim.x)
+
 __global__ void k_fill_value(int64_t n, double v, double *out)
 {
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n) out[k] = v;
+    PDX_SLOT_LOOP(k, n) out[k] = v;
 }
 
 __global__ void k_L_to_float(int64_t nb, const double *L, float *Lf)
 {
-    int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < nb) Lf[k] = (float)L[k];
+    PDX_SLOT_LOOP(k, nb) Lf[k] = (float)L[k];
 }
 
 // ----------------------------------------------------------------------------------------
@@ -889,12 +898,13 @@ __global__ __launch_bounds__(256) void k_len_range(int64_t nb, const uint32_t *b
 __global__ void k_pack_bonds(int64_t nb, const uint16_t *w16, double *L, int shift, unsigned long long mask,
                              unsigned long long base)
 {
-    const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nb) return;
-    const uint32_t w = w16[b];
-    const unsigned long long v = (unsigned long long)__double_as_longlong(L[b]) - base;
-    L[b] = __longlong_as_double(
-        (long long)((unsigned long long)(w & PDX_W16_SLOT) << shift | ((w & PDX_W16_ACT) ? v : mask)));
+    PDX_SLOT_LOOP(b, nb)
+    {
+        const uint32_t w = w16[b];
+        const unsigned long long v = (unsigned long long)__double_as_longlong(L[b]) - base;
+        L[b] = __longlong_as_double(
+            (long long)((unsigned long long)(w & PDX_W16_SLOT) << shift | ((w & PDX_W16_ACT) ? v : mask)));
+    }
 }
 
 // One 64-bit word per bond in place of the 16-bit word and the FP64 length (FP64 contexts with
@@ -922,7 +932,7 @@ static pdx_status pack_bonds(pdx_ctx *c)
     c->pk_shift = shift;
     c->pk_mask = mask;
     c->pk_base = h[0];
-    hipLaunchKernelGGL(k_pack_bonds, dim3((unsigned)((c->nb_alloc + 255) / 256)), dim3(256), 0, c->stream,
+    hipLaunchKernelGGL(k_pack_bonds, slot_grid(c->nb_alloc), dim3(256), 0, c->stream,
                        c->nb_alloc, c->bw16, c->L, shift, mask, h[0]);
     PDX_HIP(c, hipGetLastError());
     PDX_HIP(c, hipStreamSynchronize(c->stream));
@@ -1158,7 +1168,8 @@ static pdx_status fill_rows(pdx_ctx *c, search_args &s)
     // padding slots: bond word 0, length 1
     PDX_HIP(c, hipMemsetAsync(c->bw, 0, sizeof(uint32_t) * nba, c->stream));
     if (nba > 0)
-        hipLaunchKernelGGL(k_fill_value, grid256(nba), dim3(256), 0, c->stream, nba, 1.0, c->L);
+        hipLaunchKernelGGL(k_fill_value, slot_grid(nba), dim3(256), 0, c->stream, nba, 1.0, c->L);
+    PDX_HIP(c, hipGetLastError());
     s.rows = c->rows();
     s.cnt = c->cnt;
     s.bw = c->bw;
@@ -1339,8 +1350,7 @@ extern "C" pdx_status pdx_build_bonds(pdx_ctx *c, int64_t *n_bonds_out)
     if (c->precision == PDX_MIXED && !c->lds_mode) {
         const int64_t nba = c->nb_alloc;
         PDX_TRY(pdx_alloc(c, &c->Lf, nba));
-        hipLaunchKernelGGL(k_L_to_float, dim3((unsigned)((nba + 255) / 256)), dim3(256), 0, c->stream,
-                           nba, c->L, c->Lf);
+        hipLaunchKernelGGL(k_L_to_float, slot_grid(nba), dim3(256), 0, c->stream, nba, c->L, c->Lf);
         PDX_HIP(c, hipGetLastError());
     }
     PDX_TRY(upload_psets(c));
