@@ -99,6 +99,7 @@ struct pdx_gnn;  // learned preconditioner (pdx_gnn.hip)
 struct pdx_ctx {
     int device = 0;
     int precision = PDX_FP64;
+    int bb_unroll = 0;               // PDX_BB_UNROLL: bonds per lane and unrolled iteration of the BB step, 0 = default
     int64_t lds_limit = 160 * 1024;  // dynamic LDS bytes a workgroup may use
     int32_t lds_budget_env = 0;      // PDX_LDS_BUDGET (bytes), 0 = default
     hipStream_t stream = nullptr;

@@ -118,6 +118,10 @@ extern "C" pdx_status pdx_create(pdx_ctx **out, int32_t device, int32_t precisio
     pdx_ctx *c = new pdx_ctx();
     c->device = device;
     c->precision = precision;
+    if (const char *e = getenv("PDX_BB_UNROLL")) {
+        const int v = atoi(e);
+        if (v == 2 || v == 4) c->bb_unroll = v;
+    }
     if (const char *e = getenv("PDX_LDS_BUDGET")) c->lds_budget_env = atoi(e);
     if (hipSetDevice(device) != hipSuccess || hipStreamCreate(&c->stream) != hipSuccess ||
         hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess) {

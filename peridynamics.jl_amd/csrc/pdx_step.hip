@@ -651,7 +651,7 @@ __global__ __launch_bounds__(PB * S) void k_bb_lds(pdx_step_args A)
             if (T0 > 0) __syncthreads();  // the previous tile is consumed
             stage(T0, T1);
             __syncthreads();
-            i = pdx_walk_tile<2>(A, R, i, T1, [&](const bond_data<PK> &b, int ib) {
+            i = pdx_walk_tile<U>(A, R, i, T1, [&](const bond_data<PK> &b, int ib) {
                 const bond_data<PK> one[1] = {b};
                 bb_group<1, F>(A, R, hidx, hrec, hb, T0, ri, bc, thr, epsc, one, ib, f);
             });
@@ -835,7 +835,7 @@ __device__ __forceinline__ bool mx_breaks(const pdx_step_args &A, const int32_t 
     return ((l - L) / L) > epsc;
 }
 
-template <int S, int F, int PB>
+template <int U, int S, int F, int PB>
 __global__ __launch_bounds__(PB * S) void k_bb_lds_mx(pdx_step_args A)
 {
     constexpr bool MULTI = (F & PDX_FEAT_MULTI) != 0;
@@ -883,11 +883,11 @@ __global__ __launch_bounds__(PB * S) void k_bb_lds_mx(pdx_step_args A)
     }
     const float win_lo = epscf * 0.9999f, win_hi = epscf * 1.0001f;
     __syncthreads();
-    pdx_walk_mx<4>(A, R, [&](const uint32_t (&wd)[4], int i) {
+    pdx_walk_mx<U>(A, R, [&](const uint32_t (&wd)[U], int i) {
         // the group's bond forces are summed in FP32 (fused), then once into the FP64 sums
         float gx = 0.f, gy = 0.f, gz = 0.f;
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
+        for (int u = 0; u < U; u++) {
             if (i + u >= R.ng) continue;  // uniform
             const int64_t o = R.at(i + u);
             const int slot = (int)(wd[u] & PDX_W16_SLOT);
@@ -2643,13 +2643,17 @@ static void launch_lds(pdx_ctx *c, const void *fn, bool capped, bool tiled, int 
 template <int F, class CFG>
 static void launch_bb(pdx_ctx *c, CFG, bool mixed, int entry, const pdx_step_args &a)
 {
-    // bonds per lane and unrolled iteration: the FP32 bond arithmetic of the mixed step is
-    // short enough that four loads in flight pay; FP64 is indifferent
+    // Bonds per lane and unrolled iteration (PDX_BB_UNROLL = 2 | 4): four in the mixed step, whose FP32
+    // bond arithmetic is short enough that four loads in flight pay, two in FP64
+    const bool u4 = c->bb_unroll ? c->bb_unroll == 4 : mixed;
     const void *fn;
-    if (mixed) fn = (const void *)&k_bb_lds_mx<CFG::S, F, CFG::PB>;
-    else if constexpr (F & PDX_FEAT_MULTI) fn = (const void *)&k_bb_lds<2, CFG::S, F, CFG::PB, false>;
-    else fn = c->pk ? (const void *)&k_bb_lds<2, CFG::S, F, CFG::PB, true>
-                    : (const void *)&k_bb_lds<2, CFG::S, F, CFG::PB, false>;
+    if (mixed)
+        fn = u4 ? (const void *)&k_bb_lds_mx<4, CFG::S, F, CFG::PB> : (const void *)&k_bb_lds_mx<2, CFG::S, F, CFG::PB>;
+    else
+        fn = u4 ? (const void *)&k_bb_lds<4, CFG::S, F, CFG::PB, false> : (const void *)&k_bb_lds<2, CFG::S, F, CFG::PB, false>;
+    if constexpr (!(F & PDX_FEAT_MULTI))
+        if (!mixed && c->pk)
+            fn = u4 ? (const void *)&k_bb_lds<4, CFG::S, F, CFG::PB, true> : (const void *)&k_bb_lds<2, CFG::S, F, CFG::PB, true>;
     if (mixed && (F & PDX_FEAT_CAP)) launch_lds<CFG>(c, fn, true, false, entry, a);
     else launch_lds_bud<CFG>(c, fn, entry, pdx_lds_budget(c), a);
 }
@@ -2751,9 +2755,11 @@ pdx_status pdx_launch_step(pdx_ctx *c, const pdx_step_args &a)
 #define PDX_BB_LAUNCH(F) with_cfg(c, [&](auto g) { launch_bb<F>(c, g, mixed, entry, a); })
             PDX_FEAT_SWITCH(feat, PDX_BB_LAUNCH)
         } else if (mixed) {
-            hipLaunchKernelGGL((k_bb_step<true, 2>), G, B, 0, c->stream, a);
+            if (c->bb_unroll == 4) hipLaunchKernelGGL((k_bb_step<true, 4>), G, B, 0, c->stream, a);
+            else hipLaunchKernelGGL((k_bb_step<true, 2>), G, B, 0, c->stream, a);
         } else {
-            hipLaunchKernelGGL((k_bb_step<false, 2>), G, B, 0, c->stream, a);
+            if (c->bb_unroll == 4) hipLaunchKernelGGL((k_bb_step<false, 4>), G, B, 0, c->stream, a);
+            else hipLaunchKernelGGL((k_bb_step<false, 2>), G, B, 0, c->stream, a);
         }
         PDX_HIP(c, hipGetLastError());
         PDX_TRY(pdx_timed_end(c, "step"));
