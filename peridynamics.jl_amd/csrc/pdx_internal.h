@@ -101,6 +101,7 @@ struct pdx_ctx {
     int precision = PDX_FP64;
     int bb_unroll = 0;               // PDX_BB_UNROLL: bonds per lane and unrolled iteration of the BB step, 0 = default
     int64_t lds_limit = 160 * 1024;  // dynamic LDS bytes a workgroup may use
+    int32_t block_points_env = 0;    // PDX_BLOCK_POINTS (32, 64, 128 or 256), 0 = by the body (choose_blocks)
     int32_t lds_budget_env = 0;      // PDX_LDS_BUDGET (bytes), 0 = default
     hipStream_t stream = nullptr;
     std::string err;

@@ -122,6 +122,7 @@ extern "C" pdx_status pdx_create(pdx_ctx **out, int32_t device, int32_t precisio
         const int v = atoi(e);
         if (v == 2 || v == 4) c->bb_unroll = v;
     }
+    if (const char *e = getenv("PDX_BLOCK_POINTS")) c->block_points_env = atoi(e);
     if (const char *e = getenv("PDX_LDS_BUDGET")) c->lds_budget_env = atoi(e);
     if (hipSetDevice(device) != hipSuccess || hipStreamCreate(&c->stream) != hipSuccess ||
         hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess) {
@@ -1143,6 +1144,9 @@ static void choose_blocks(pdx_ctx *c, bool lds)
     else if (c->kind != PDX_CPD && c->precision == PDX_MIXED && c->n > 1000000) first = 0;
     int k = first;
     while (k < 3 && c->n < (int64_t)(k == 2 ? 256 : 160) * pbs[k]) k++;
+    // PDX_BLOCK_POINTS: one of the four sizes whatever the body (no correspondence kernel has 256)
+    for (int q = c->kind == PDX_CPD ? 1 : 0; q < 4; q++)
+        if (c->block_points_env == pbs[q]) k = q;
     c->cfg = k;
     c->pb = pbs[k];
     c->ls = lss[k];
