@@ -43,7 +43,8 @@ def step_bytes(n_points, n_bonds, precision, layout):
     record counts once, as its own point's).
 
     per point: read x|V (32), u (24), v_half (24), bond count (4), BC slot (4); write x|V
-               (32), u (24), v_half (24)  -> 168 B, plus 8 B per 64-point slice pointer;
+               (32), u (24), v_half (24)  -> 168 B, plus 8 B per slice pointer (layout["slice_points"]
+               points: 64 in the global-gather layout, 16, 8 or 4 in the LDS-staged one);
                the mixed LDS step also reads the reference record X|V (32) -> 200 B;
     per bond:  LDS-staged FP64: 16-bit bond word (2) + FP64 reference length (8), or both in one
                64-bit word (8; layout["bond_bytes"]);
@@ -51,7 +52,8 @@ def step_bytes(n_points, n_bonds, precision, layout):
                global-gather layout: 32-bit bond word (4) + length (8 FP64 / 4 FP32);
     per neighbour-table entry (LDS layouts): its 4-byte point index.
     A bond word is written back only when the bond breaks (not counted)."""
-    n_slices = (n_points + 63) // 64
+    per_slice = layout.get("slice_points", 64)
+    n_slices = (n_points + per_slice - 1) // per_slice
     if layout["lds_mode"]:
         if precision == "fp64":
             per_bond = layout.get("bond_bytes", 10)

@@ -342,6 +342,9 @@ pdx_status pdx_layout(pdx_ctx *ctx, int32_t *lds_mode, int64_t *bond_slots,
 /* Bytes of a bond slot that an FP64 step reads: 8 (one packed word), 10 (16-bit word and length)
  * or 12 (global-gather layout); 0 before pdx_build_bonds. */
 int32_t pdx_bond_bytes(const pdx_ctx *ctx);
+/* Points of a slice of the bond rows, each with an 8-byte pointer: 64 in the global-gather layout,
+ * 16, 8 or 4 in the LDS-staged one (by the block size); 0 before pdx_build_bonds. */
+int32_t pdx_slice_points(const pdx_ctx *ctx);
 
 #ifdef __cplusplus
 }

@@ -1880,6 +1880,8 @@ extern "C" int32_t pdx_bond_bytes(const pdx_ctx *c)
     return c->pk ? 8 : c->lds_mode ? 10 : 12;
 }
 
+extern "C" int32_t pdx_slice_points(const pdx_ctx *c) { return c && c->bonds_built ? 64 >> c->ls : 0; }
+
 pdx_status pdx_reset_flags(pdx_ctx *c)
 {
     unsigned long long init[2] = {~0ULL, 0ULL};

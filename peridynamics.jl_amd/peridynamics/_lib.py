@@ -154,6 +154,7 @@ SIGNATURES = {
     "pdx_kernel_time": (_ST, [_P, ctypes.c_char_p, ctypes.POINTER(_D), ctypes.POINTER(_I64)]),
     "pdx_info": (_ST, [_P, ctypes.POINTER(_I64), ctypes.POINTER(_I64), ctypes.POINTER(_I64)]),
     "pdx_bond_bytes": (_I32, [_P]),
+    "pdx_slice_points": (_I32, [_P]),
     "pdx_layout": (_ST, [_P, ctypes.POINTER(_I32), ctypes.POINTER(_I64), ctypes.POINTER(_I64),
                          ctypes.POINTER(_I32)]),
 }
@@ -490,9 +491,11 @@ class Context:
         return a.value, b.value, c.value
 
     def layout(self):
-        """{"lds_mode", "bond_slots", "halo_entries", "halo_max", "bond_bytes"} of the device bond lists."""
+        """{"lds_mode", "bond_slots", "halo_entries", "halo_max", "bond_bytes", "slice_points"} of the
+        device bond lists."""
         m, s, h = _I32(), _I64(), _I64()
         hm = _I32()
         self.call("pdx_layout", ctypes.byref(m), ctypes.byref(s), ctypes.byref(h), ctypes.byref(hm))
         return {"lds_mode": bool(m.value), "bond_slots": s.value, "halo_entries": h.value,
-                "halo_max": hm.value, "bond_bytes": self.lib.pdx_bond_bytes(self.h)}
+                "halo_max": hm.value, "bond_bytes": self.lib.pdx_bond_bytes(self.h),
+                "slice_points": self.lib.pdx_slice_points(self.h)}
