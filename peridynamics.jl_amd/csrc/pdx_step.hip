@@ -412,9 +412,10 @@ struct pdx_lane {
     }
 };
 
-// p0 = the block's first point; waves past the last point have no bonds
+// p0 = the block's first point; waves past the last point have no bonds.  quads: the caller keeps the
+// order of PDX_F_ORDER by pdx_add_quad instead
 template <int S, bool PK>
-__device__ __forceinline__ pdx_lane<S, PK> pdx_lane_of(const pdx_step_args &A, int64_t p0)
+__device__ __forceinline__ pdx_lane<S, PK> pdx_lane_of(const pdx_step_args &A, int64_t p0, bool quads = false)
 {
     constexpr int LS = pdx_log2<S>();
     const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -422,7 +423,7 @@ __device__ __forceinline__ pdx_lane<S, PK> pdx_lane_of(const pdx_step_args &A, i
     R.lane = threadIdx.x & 63;
     R.ng = 0;
     R.b0 = 0;
-    R.order = S > 4 && (A.flags & PDX_F_ORDER) != 0;
+    R.order = S > 4 && !quads && (A.flags & PDX_F_ORDER) != 0;
     if (p0 + wv * (64 / S) < A.n) {
         const int64_t *const q = A.rows.ptr + (p0 >> (6 - LS)) + wv;
         R.b0 = q[0];
@@ -442,6 +443,23 @@ __device__ __forceinline__ void pdx_fold(const pdx_lane<S, PK> &R, T &x)
     if (S > 4 && R.order && (threadIdx.x & (S - 1)) >= 4) x = 0;
 #pragma unroll
     for (int o = 1; o < S; o <<= 1) x += __shfl_xor(x, o);
+}
+
+// PDX_F_ORDER where a lane adds its bonds by quadruples of row groups (the mixed kernels): g, the sum
+// of the lane's quadruple, goes into x in the order of four lanes per point, the quadruples of the
+// point's groups of four lanes one after the other, in every group.  A row is so walked once.  50
+// relaxation steps of 10 k to 20 k points, blocks of 256 points and four lanes / smaller blocks whose
+// groups each walk the whole row, as the FP64 kernels do / this: BB 1.40 / 1.43 to 1.48 / 0.91 to 1.04 ms,
+// OSB 2.13 / 2.25 to 2.33 / 1.31 to 1.57.  In any other launch: x += g.
+template <int S>
+__device__ __forceinline__ void pdx_add_quad(bool order, double &x, float g)
+{
+    if (S > 4 && order) {
+#pragma unroll
+        for (int k = 0; k < S / 4; k++) x += (double)__shfl(g, (int)(threadIdx.x & 63 & ~(S - 1)) | (k << 2) | (int)(threadIdx.x & 3));
+    } else {
+        x += (double)g;
+    }
 }
 
 // Walks the lane's bonds U at a time, the next U loaded before the current ones are evaluated.
@@ -864,7 +882,9 @@ __global__ __launch_bounds__(PB * S) void k_bb_lds_mx(pdx_step_args A)
     const int sub = threadIdx.x % S;
     const int64_t p = p0 + threadIdx.x / S;
     const int64_t q = p < A.n ? p : A.n - 1;
-    const pdx_lane<S, false> R = pdx_lane_of<S, false>(A, p0);
+    constexpr bool QUADS = U == 4;
+    pdx_lane<S, false> R = pdx_lane_of<S, false>(A, p0, QUADS);
+    const bool order = QUADS && (A.flags & PDX_F_ORDER) != 0;
     const double4 ri = A.rec_in[q];
     const double4 Xi = A.Xr[q];
     const float xi = (float)(Xi.x - O.x), yi = (float)(Xi.y - O.y), zi = (float)(Xi.z - O.z);
@@ -921,14 +941,15 @@ __global__ __launch_bounds__(PB * S) void k_bb_lds_mx(pdx_step_args A)
             gz = __builtin_fmaf(sf, Dz + Uz, gz);
             na += act ? 1 : 0;
         }
-        bx += (double)gx;
-        by += (double)gy;
-        bz += (double)gz;
+        pdx_add_quad<S>(order, bx, gx);
+        pdx_add_quad<S>(order, by, gy);
+        pdx_add_quad<S>(order, bz, gz);
     });
+    pdx_fold(R, na);
+    R.order |= order;
     pdx_fold(R, bx);
     pdx_fold(R, by);
     pdx_fold(R, bz);
-    pdx_fold(R, na);
     if (p >= A.n) return;
     const int c = A.cnt[p];
     if (c == 0) bx = by = bz = 0.0;
@@ -975,7 +996,8 @@ __global__ __launch_bounds__(PB * S) void k_osb_lds1_mx(pdx_step_args A)
     const int sub = threadIdx.x % S;
     const int64_t p = p0 + threadIdx.x / S;
     const int64_t q = p < A.n ? p : A.n - 1;
-    const pdx_lane<S, false> R = pdx_lane_of<S, false>(A, p0);
+    pdx_lane<S, false> R = pdx_lane_of<S, false>(A, p0, true);
+    const bool order = (A.flags & PDX_F_ORDER) != 0;
     const double4 ri = A.rec_in[q];
     const double4 Xi = A.Xr[q];
     const float xi = (float)(Xi.x - O.x), yi = (float)(Xi.y - O.y), zi = (float)(Xi.z - O.z);
@@ -1027,12 +1049,13 @@ __global__ __launch_bounds__(PB * S) void k_osb_lds1_mx(pdx_step_args A)
                 na++;
             }
         }
-        wvol += (double)gv;
-        Ssum += (double)gs;
+        pdx_add_quad<S>(order, wvol, gv);
+        pdx_add_quad<S>(order, Ssum, gs);
     });
+    pdx_fold(R, na);
+    R.order = order;
     pdx_fold(R, wvol);
     pdx_fold(R, Ssum);
-    pdx_fold(R, na);
     if (p >= A.n || sub != 0) return;
     double c1 = 0.0, c2 = 0.0;
     if (wvol != 0.0) {
@@ -1081,7 +1104,8 @@ __global__ __launch_bounds__(PB * S) void k_osb_lds2_mx(pdx_step_args A)
     const int sub = threadIdx.x % S;
     const int64_t p = p0 + threadIdx.x / S;
     const int64_t q = p < A.n ? p : A.n - 1;
-    const pdx_lane<S, false> R = pdx_lane_of<S, false>(A, p0);
+    pdx_lane<S, false> R = pdx_lane_of<S, false>(A, p0, true);
+    const bool order = (A.flags & PDX_F_ORDER) != 0;
     const double4 ri = A.rec_in[q];
     const double4 Xi = A.Xr[q];
     const float xi = (float)(Xi.x - O.x), yi = (float)(Xi.y - O.y), zi = (float)(Xi.z - O.z);
@@ -1132,10 +1156,11 @@ __global__ __launch_bounds__(PB * S) void k_osb_lds2_mx(pdx_step_args A)
             gy = __builtin_fmaf(sf, Dy + Uy, gy);
             gz = __builtin_fmaf(sf, Dz + Uz, gz);
         }
-        bx += (double)gx;
-        by += (double)gy;
-        bz += (double)gz;
+        pdx_add_quad<S>(order, bx, gx);
+        pdx_add_quad<S>(order, by, gy);
+        pdx_add_quad<S>(order, bz, gz);
     });
+    R.order = order;
     pdx_fold(R, bx);
     pdx_fold(R, by);
     pdx_fold(R, bz);
