@@ -1107,27 +1107,29 @@ static pdx_status build_halos(pdx_ctx *c, bool *ok)
 // 128 x 4, 64 x 8 or 32 x 16.  A small body needs many small blocks (a 6400-point one is 25 blocks of
 // 256 points on 256 CUs) and many lanes per point (its step is one chain of load latencies per
 // lane); a large one wants the larger blocks' smaller neighbour tables per point.  Measured, us
-// per step, blocks of 256 / 128 / 64 / 32 points (3.015 spacings):
-//   BB FP64   6 k 14.3 /  9.8 /  7.1 /  6.4    14 k 16.7 / 11.8 /  8.7 /  8.8
-//            25 k 17.2 / 12.4 / 12.5 / 13.4   100 k 31.5 / 30.6 / 30.5 / 35.0
-//             2 M  560 /  515 /  598 /  729
-//   CPD FP64  6 k  n/a / 28.0 / 21.8 / 18.7    14 k  n/a / 38.4 / 29.7 / 27.6
-//            25 k  n/a / 40.2 / 39.4 / 46.3    54 k 61.8 / 59.0 / 67.8
-//           512 k  490 /  458 /  588            2 M 2218 / 1750
+// per step, the best of five runs of 100 or 200 steps (at 2 M points their mean is 1 % longer, single
+// launches vary by 10 %), blocks of 256 / 128 / 64 / 32 points, 3.015 spacings:
+//   BB FP64   6 k 14.9 / 10.3 /  7.7 /  6.6    14 k 17.5 / 12.0 /  9.1 /  9.0
+//            25 k 17.8 / 12.2 / 12.5 / 13.0   100 k 31.4 / 30.7 / 30.8 / 35.3
+//             2 M  569 /  530 /  628 /  762
+//   CPD FP64  6 k  n/a / 27.9 / 21.7 / 18.5    14 k  n/a / 38.2 / 29.4 / 27.9
+//            25 k  n/a / 40.4 / 39.1 / 46.5    54 k  n/a / 60.4 / 68.0 / 78.8
+//           512 k  n/a /  450 /  580 /  762     2 M  n/a / 1731 / 2219 / 2965
 // so the blocks are the largest that still give 160 of them, and those of 32 points, where twice as
 // many cost little, hold until 64-point blocks number 256 (12 k to 16 k points, 64 against 32: BB
-// 9.2 / 9.1, mixed BB 9.8 / 9.1, OSB 17.3 / 17.0, CPD 29.5 / 27.2; the load step of 14 k points
-// 33.5 against 31.9 ms).  FP64 stops at 128 points, whose
-// blocks share a CU two or three at a time; the mixed BB and OSB steps of bodies beyond a million
-// points go to 256 (334 against 356 at 2 M).  Horizons beyond about 4 spacings stop at 64 points,
-// whose neighbour tables still fit a block's share of the LDS (5.015 spacings, 121 k points, BB:
-// 216 / 169 / 157 / 159; OSB at 400 k: 1042 / 1074 / 897 / 942; CPD at 100 k: 629 / 517 / 403; 4.015
-// spacings, CPD at 100 k: 280 / 210 / 191).
-// The mixed BB and OSB steps go back to 256 points beyond about 4.5 spacings (350 bonds per point),
-// where a block of 64 has 40 table entries per point that the short FP32 arithmetic does not hide, if
-// the last round of these blocks, one to a CU, fills 80 % of it on average (5.015 spacings, 256 against
-// 64: BB 54 k 54.0 / 57.7, 121 k 104.5 / 117.7, 576 k 482 / 501, OSB 206 / 221 and 942 / 966 at the last two;
-// 200 k points, 3.05 rounds, 200 / 185 and 393 / 344).
+// 9.0 / 8.8, mixed BB 8.8 / 8.7, OSB 17.2 / 17.1, CPD 29.4 / 27.2; the load step of 14 k points
+// 33.5 against 31.9 ms).  FP64 stops at 128 points, whose blocks share a CU two or three at a time (OSB
+// at 2 M 1022 / 1029 / 1186 / 1446).  Horizons beyond about 4 spacings stop at 64 points, whose
+// neighbour tables still fit a block's share of the LDS (5.015 spacings: BB at 121 k 215 / 174 / 160 /
+// 163, OSB at 400 k 1050 / 935 / 918 / 968, CPD at 100 k n/a / 504 / 395 / 375, mixed BB 256 against 64
+// points 54 / 52 at 54 k, 105 / 106 at 121 k, 327 / 295 at 400 k, 478 / 442 at 576 k, mixed OSB 932 / 893
+// there; 4.015 spacings: CPD at 100 k n/a / 214 / 192 / 211).
+// The mixed BB and OSB steps of bodies beyond a million points go to 256 points (340 against 361 and 647
+// against 677 at 2 M, 200x200x50).  That line is coarse: four 128-point blocks share a CU where every table
+// fits a quarter of its LDS (1279 entries), else three, and which it is depends on how the Morton
+// curve folds into the body (BB, 256 against 128: 1 M points 164 / 157, 1.1 M 179 / 194, 1.3 M 214 / 208,
+// 1.6 M 251 / 273, 1.7 M 224 / 219, 2.6 M 404 / 395; OSB 316 / 317, 339 / 360, 409 / 410, 479 / 507, 419 / 407,
+// 779 / 788).
 static void choose_blocks(pdx_ctx *c, bool lds)
 {
     if (!lds) {
@@ -1138,9 +1140,7 @@ static void choose_blocks(pdx_ctx *c, bool lds)
     }
     static const int pbs[4] = {256, 128, 64, 32}, lss[4] = {2, 2, 3, 4};
     int first = 1;
-    const int64_t b256 = (c->n + 255) / 256, r256 = (b256 + 255) / 256;  // blocks, and their rounds over 256 CUs
-    if (c->kind != PDX_CPD && c->precision == PDX_MIXED && c->nb > 350 * c->n && 5 * b256 >= 4 * 256 * r256) first = 0;
-    else if (c->nb > 180 * c->n) first = 2;
+    if (c->nb > 180 * c->n) first = 2;
     else if (c->kind != PDX_CPD && c->precision == PDX_MIXED && c->n > 1000000) first = 0;
     int k = first;
     while (k < 3 && c->n < (int64_t)(k == 2 ? 256 : 160) * pbs[k]) k++;
