@@ -324,11 +324,12 @@ __device__ __forceinline__ double4 pdx_rec_vbc(double4 r, double bc) { return ma
 // wave-uniform, and lanes whose row is shorter evaluate padding slots (inactive, the row's last
 // neighbour), which add zero.
 //
-// Measured, FP64 steps at 2 M points (3.015 spacings), us: per-lane loops over rows interleaved by
-// 64 points, 256 x 4 blocks BB 642, OSB 1295; the same loops over row groups BB 578; this walk
-// with words and lengths apart BB 578 (128 x 4 blocks; 626 with 256 x 4), OSB 1133; with packed
-// bonds BB 515, OSB 1010 (a slot costs 8 bytes instead of 10, 232 M of them: 4.3 TB/s of the
-// 5.0 TB/s that a device copy reaches).  The look-ahead is worth 5 to 10 % (BB 100 k points 33.0
+// Measured, FP64 steps at 2 M points (3.015 spacings), us, the best of a few runs each: per-lane loops
+// over rows interleaved by 64 points, 256 x 4 blocks BB 621 to 642, OSB 1295; the same loops over row groups
+// BB 578; this walk with words and lengths apart BB 578 (128 x 4 blocks; 626 with 256 x 4), OSB 1133;
+// with packed bonds BB 515 to 530, OSB 1010 to 1030 (a slot costs 8 bytes instead of 10, 232 M of
+// them: 4.3 TB/s of the 5.0 TB/s that a device copy reaches).  Averages over 100 launches: BB 545 to
+// 560, one launch 518 to 760.  The look-ahead is worth 5 to 10 % (BB 100 k points 33.0
 // without, 30.6 with), and two bonds per step of the walk 5 % over one (BB 1 M 266 against 261 at
 // 76 against 54 VGPRs); forcing 64 VGPRs spills and triples the time.
 //
@@ -1902,8 +1903,9 @@ __device__ __forceinline__ void pdx_fold_part(double *v)
 // The N sums of every point of the block, in hs[q PB + point], for one thread per point.  The
 // staged table is consumed by then, and its LDS is reused.  The point part of a correspondence
 // step (two 3 x 3 inverses, the stress, some 700 FP64 instructions) then runs in full waves
-// instead of one lane in S of all of them (512 k points, with the squared pre-check of the failure
-// window in place of a root per bond: pass 1 275 -> 245 us; without the point part it takes 208).
+// instead of one lane in S of all of them (512 k points in 256-point blocks, with the squared pre-check
+// of the failure window in place of a root per bond: pass 1 275 -> 245 us, 208 without the point part;
+// 197 to 208 in 128-point blocks).
 template <int S, int PB, int N, bool PK>
 __device__ __forceinline__ void cpd_hand_over(const pdx_lane<S, PK> &R, double *v, double *hs)
 {
@@ -1924,12 +1926,13 @@ __device__ __forceinline__ void cpd_hand_over(const pdx_lane<S, PK> &R, double *
 // CPD passes on the LDS-staged layout (FP64).  Pass 1 entries: x, V, X (56 B); pass 2: see below.
 // The arithmetic of pass 1 is that of k_cpd_pass1.
 //
-// Bound by the bond walk's instructions and LDS reads: at 512 k points (60 M bonds) the vector units
-// are busy 56 % of pass 1's time and 36 % of pass 2's, the LDS 40 and 47 %, and a pass without its
-// walk takes 62 (46) of 245 (258) us.  What helped, us of both passes at 512 k points: blocks of 128
-// points, two to a CU, 500 -> 458 (256 points leave one block per CU, whose staging and point part
-// nothing hides); walking a table that fits by wave-uniform counts instead of by tiles 545 -> 501 in
-// the same blocks.  A point's own lanes S at 8 (64-point blocks) cost 588: longer tables per point.
+// Bound by the bond walk's instructions and LDS reads: at 512 k points (60 M bonds, 128-point blocks)
+// the vector units are busy 63 % of pass 1's time and 43 % of pass 2's, the LDS 37 and 49 %, nearly half
+// of that in bank conflicts (with 256-point blocks 56, 37, 40 and 47 %; there a pass without its walk
+// took 62 (46) of 245 (258) us).  What helped, us of both passes at 512 k points: blocks of 128 points,
+// two to a CU, 500 -> 458 (256 points leave one block per CU, whose staging and point part nothing
+// hides); walking a table that fits by wave-uniform counts instead of by tiles 545 -> 501 in the same
+// blocks.  A point's own lanes S at 8 (64-point blocks) cost 580 to 588: longer tables per point.
 // ----------------------------------------------------------------------------------------
 template <int S, int F, int PB, bool PK>
 __global__ __launch_bounds__(PB * S) void k_cpd_lds1(pdx_step_args A)
@@ -2092,8 +2095,8 @@ __global__ __launch_bounds__(PB * S) void k_cpd_lds1(pdx_step_args A)
 // pass 1, in coordinates relative to the first point of the run of 256 (the staging moves a_j there),
 // so that the products stay of the size of the block rather than of the coordinates.  ZW
 // (ZEMWan): the symmetric C_1 of each end in place of beta.  Table entries as 16-byte pairs:
-// [j alive] (Q_j, a_j), then [j alive] beta, V_j (112 B, 1463 entries in a 160 KB tile), or
-// with ZEMWan [j alive] C_1j (six entries), V_j and a pad (160 B, 1024 entries), against
+// [j alive] (Q_j, a_j), then [j alive] beta, V_j (112 B, 730 entries in a tile of half the LDS), or
+// with ZEMWan [j alive] C_1j (six entries), V_j and a pad (160 B, 511 entries), against
 // the 136 B (184 B) of x, X and the state in a per-bond form.  PDX_FEAT_MULTI (several
 // parameter sets): beta_j of the neighbour's set, the neighbour's term for the neighbour's
 // copy of the bond (RACT; the own terms followed the owner's copy, ACT, in pass 1), and the
@@ -2209,12 +2212,12 @@ __global__ __launch_bounds__(PB * S) void k_cpd_lds2_own(pdx_step_args A)
 // without the cancellation of d - F D in FP32.  Pass 1 stores Q' (9 numbers per point);
 // pass 2 stages (D, V), (U, beta [j alive]), [j alive] Q'_j (68 B per table entry) and
 // gathers both terms of every bond.
-// Pass 1 is bound by its vector instructions (busy 82 % of the time: 15 FP32 products per bond are
-// converted and summed in FP64), so one bond at a time without a stretch that only a bond near its
-// critical one needs; pass 2 by LDS reads, whose 64-byte entries met on two groups of banks
-// (75 % of the LDS cycles were conflicts) until every quarter became an array of its own.
-// Both passes at 512 k points: 468 us with four bonds per step and entries in one piece, 355 now,
-// 308 in blocks of 128 points.
+// Pass 1 is bound by its vector instructions (issued at 84 % of the CU's rate: 15 FP32 products per bond
+// are converted and summed in FP64), so one bond at a time without a stretch that only a bond near its
+// critical one needs; pass 2 by LDS reads (busy 48 % of the time) and instructions (65 %).  Its 64-byte
+// entries met on two groups of banks (75 % of the LDS cycles were conflicts, now 51 %) until every
+// quarter became an array of its own.  Both passes at 512 k points: 468 us with four bonds per step and
+// entries in one piece, 355 now in blocks of 256 points, 308 to 320 in those of 128.
 // ----------------------------------------------------------------------------------------
 template <int S, int F, int PB>
 __global__ __launch_bounds__(PB * S) void k_cpd_pass1_mx(pdx_step_args A)
